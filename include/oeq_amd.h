@@ -71,19 +71,18 @@ typedef enum {
     OEQ_ROLE_CONV_FORWARD = 2,      /* main forward kernel (either mode) */
     OEQ_ROLE_CONV_BACKWARD = 3,     /* main backward kernel (either mode) */
     OEQ_ROLE_CONV_FIXUP_BACKWARD = 4,/* deterministic mode: sender-ordered segmented reduction */
-    OEQ_ROLE_SEGMENT_PTR = 5,       /* builds CSR pointers from a sorted index list */
+    OEQ_ROLE_SEGMENT_PTR = 5,       /* builds CSR pointers from one or two sorted index lists */
     OEQ_ROLE_FILL_ZERO = 6,         /* clears a buffer (used instead of memset: capture-safe) */
     OEQ_ROLE_TP_BACKWARD_WREDUCE = 7,/* shared weights: second pass of the weight-gradient reduction */
     OEQ_ROLE_SEGMENT_SUM = 8,       /* ordered sum of rows over the segments of a sorted key list */
-    OEQ_ROLE_GROUP_COUNT = 9,       /* grouping an unsorted key list: histogram, */
-    OEQ_ROLE_GROUP_SCAN = 10,       /*   exclusive scan (one block), */
+    OEQ_ROLE_GROUP_COUNT = 9,       /* grouping one or two unsorted key lists: histogram, */
+    OEQ_ROLE_GROUP_SCAN = 10,       /*   exclusive scan, and the table of extra walk positions of long segments, */
     OEQ_ROLE_GROUP_SCATTER = 11,    /*   scatter of the item indices into their key's segment, */
     OEQ_ROLE_GROUP_ORDER = 12,      /*   and ascending order of the indices within each segment */
     OEQ_ROLE_DOUBLE_BACKWARD_A = 13,/* second order: gradient w.r.t. the output gradient (forward-shaped) */
     OEQ_ROLE_DOUBLE_BACKWARD_B = 14,/* second order: gradients w.r.t. X, Y, W (backward-shaped) */
     OEQ_ROLE_ORDER_HOP = 15,        /* convolution walk order: one hop of the node clustering */
-    OEQ_ROLE_HUB_COUNT = 16,        /* long edge segments cut into chunks: extra walk positions per node, */
-    OEQ_ROLE_HUB_FILL = 17,         /*   and the list of those positions */
+    OEQ_ROLE_INDEX_SMALL = 16,      /* the whole index of a small edge list in one launch */
     OEQ_ROLE_CONV_FIXUP_FORWARD = 18,/* adds the rows written by the extra chunks to their nodes' rows, in chunk order */
     OEQ_ROLE_CONV_BACKWARD_DX = 19, /* OEQ_DX_SENDER_WALK: the sender gradients by a walk over the senders' edge segments
                                        (forward-shaped: argument list of OEQ_ROLE_CONV_FORWARD with dZ for X, the
@@ -145,6 +144,7 @@ typedef struct {
                                    highest-priority node within this many edges and walked cluster by cluster,
                                    so that nodes sharing senders run side by side and the gathered sender rows
                                    are served by the L2; 0 = nodes are walked by index */
+    int32_t order_min_nodes;    /* ... for graphs of at least this many nodes; smaller ones are walked by index */
     int32_t hub_limit;          /* conv, walk modes: > 0 = a node with more edges than this is walked in chunks of
                                    this many edges by different wave groups (the first chunk at the node's own walk
                                    position, the others at extra positions listed in the index), so that the time

@@ -493,8 +493,8 @@ def _conv_index(ks, nodes: int, nnz: int, r: torch.Tensor, c: torch.Tensor, p: O
     # the sender side is cheap to add when the caller brings the sender-major permutation, costly when the
     # library has to group the edges by sender itself: then only the calls that need it build it
     sender_side = need_sender_side or (not grouped and p is not None and p.numel() == nnz)
-    key = (dims["deterministic"], dims.get("order_hops", 0), dims.get("hub_limit", 0), nodes, nnz, r.data_ptr(),
-           c.data_ptr(),
+    key = (dims["deterministic"], dims.get("order_hops", 0), dims.get("order_min_nodes", 0), dims.get("hub_limit", 0),
+           nodes, nnz, r.data_ptr(), c.data_ptr(),
            p.data_ptr() if (p is not None and not grouped) else 0, stream, r.device.index)
     versions = (_version_of(r), _version_of(c), _version_of(p) if (p is not None and not grouped) else 0)
     # an edge tensor without a version counter could be rewritten unnoticed: such a call builds its index

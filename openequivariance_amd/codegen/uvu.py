@@ -2310,7 +2310,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
                     conv_segw=4, conv_split=1, conv_dd=1, dd_acc=0, dd_g=2, dd_wa=2, dd_wb=2, dd_fp=0, dd_fw=32,
                     dd_gres=-1, dd_split=1, dd_segw=4, dd_merge=0, dd_need=200, dd_ngrp=0, conv_gbud=0, conv_ngrp=0, conv_fit=300, conv_fw=0, conv_pf=0,
                     conv_dxm=-1, conv_q=0, conv_hops=2, conv_qpin=1, conv_qaf=48, conv_qab=24, tp_mask=0, tp_forms=1,
-                    conv_hub=256, conv_dxs=-1))
+                    conv_hub=256, conv_dxs=-1, conv_omin=32768))
     assert deterministic or not kahan, "kahan=True requires deterministic=True"
     # knobs somebody set: the rules below leave those alone
     user_tune = os.environ.get("OEQ_AMD_TUNE", "")
@@ -2520,14 +2520,13 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
             descs += uvu_double.add_conv_kernels(s, low, em, t, xcd, G_b, compute_units, kahan)
         # counting sort: of the edge indices by node (GROUPED mode) and of the nodes by cluster (walk order)
         descs += [
-            (rt.ROLE_GROUP_COUNT, "oeq_group_count", 256, 256 * 4, compute_units * 16),
-            (rt.ROLE_GROUP_SCAN, "oeq_group_scan", 1024, 1, 1),
-            (rt.ROLE_GROUP_SCATTER, "oeq_group_scatter", 256, 256 * 4, compute_units * 16),
+            (rt.ROLE_GROUP_COUNT, "oeq_group_count", 256, 256, compute_units * 16),
+            (rt.ROLE_GROUP_SCAN, "oeq_group_scan", 1024, 1, 0),
+            (rt.ROLE_GROUP_SCATTER, "oeq_group_scatter", 256, 256, compute_units * 16),
             (rt.ROLE_GROUP_ORDER, "oeq_group_order", 256, 4, compute_units * 32),
             (rt.ROLE_ORDER_HOP, "oeq_order_hop", 256, 256, compute_units * 16),
-            # long edge segments in chunks: table of the extra walk positions, and the sum of their rows
-            (rt.ROLE_HUB_COUNT, "oeq_hub_count", 256, 256, compute_units * 16),
-            (rt.ROLE_HUB_FILL, "oeq_hub_fill", 256, 256, compute_units * 16),
+            (rt.ROLE_INDEX_SMALL, "oeq_index_small", 1024, 1, 2),
+            # long edge segments in chunks: the sum of the chunks' rows
             (rt.ROLE_CONV_FIXUP_FORWARD, "fixup_forward", 256, 1, compute_units * 32),
         ]
     else:
@@ -2544,7 +2543,8 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     dims = dict(L1_dim=low.L1, L2_dim=low.L2, L3_dim=low.L3, weight_numel=low.WN, elem_size=low.elem_size,
                 shared_weights=int(low.shared_weights), deterministic=mode,
                 wpartial_per_block=G_b if (walk and low.shared_weights) else 0, dx_mode=dx_mode,
-                n_chunks=em.NCH, order_hops=max(0, t["conv_hops"]) if walk else 0, hub_limit=hub_limit)
+                n_chunks=em.NCH, order_hops=max(0, t["conv_hops"]) if walk else 0,
+                order_min_nodes=t["conv_omin"], hub_limit=hub_limit)
     src = s.text()
     if dx_mode == UvuEmitter.DX_SENDER_WALK and t["conv_dxs"] < 0:
         # the sender walk was chosen by its rule, not asked for: not with a kernel that does not fit its registers

@@ -43,7 +43,8 @@ class UvwEmitter:
         assert low.mode == "uvw"
         from .uvu import tuning
         self.tune = tuning(dict(uvw_unroll=16, uvw_tile=24576, uvw_regdw=1, conv_hops=2, conv_fuse_uvw=1, uvw_dd=1,
-                                uvw_dda_split=0, uvw_dda_unroll=4, conv_hub=256))
+                                uvw_dda_split=0, uvw_dda_unroll=4, conv_hub=256,
+                                conv_omin=32768))
         self.TILE_BYTES = self.tune["uvw_tile"]
         self.low = low
         self.T = low.ctype
@@ -1041,13 +1042,12 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         (rt.ROLE_CONV_BACKWARD, "backward", blk_b, 1, max_b),
         (rt.ROLE_TP_BACKWARD_WREDUCE, "oeq_wreduce", 256, 64, 0),
         (rt.ROLE_CONV_FIXUP_BACKWARD, "fixup_backward", 256, 1, 0),
-        (rt.ROLE_GROUP_COUNT, "oeq_group_count", 256, 256 * 4, cu * 16),
-        (rt.ROLE_GROUP_SCAN, "oeq_group_scan", 1024, 1, 1),
-        (rt.ROLE_GROUP_SCATTER, "oeq_group_scatter", 256, 256 * 4, cu * 16),
+        (rt.ROLE_GROUP_COUNT, "oeq_group_count", 256, 256, cu * 16),
+        (rt.ROLE_GROUP_SCAN, "oeq_group_scan", 1024, 1, 0),
+        (rt.ROLE_GROUP_SCATTER, "oeq_group_scatter", 256, 256, cu * 16),
         (rt.ROLE_GROUP_ORDER, "oeq_group_order", 256, 4, cu * 32),
         (rt.ROLE_ORDER_HOP, "oeq_order_hop", 256, 256, cu * 16),
-        (rt.ROLE_HUB_COUNT, "oeq_hub_count", 256, 256, cu * 16),
-        (rt.ROLE_HUB_FILL, "oeq_hub_fill", 256, 256, cu * 16),
+        (rt.ROLE_INDEX_SMALL, "oeq_index_small", 1024, 1, 2),
         (rt.ROLE_CONV_FIXUP_FORWARD, "fixup_forward", 256, 1, cu * 32),
     ]
     t = em.tune
@@ -1056,7 +1056,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     dims = dict(L1_dim=low.L1, L2_dim=low.L2, L3_dim=low.L3, weight_numel=low.WN, elem_size=low.elem_size,
                 shared_weights=int(shared), deterministic=rt.CONV_SORTED if deterministic else rt.CONV_GROUPED,
                 wpartial_per_block=em.backward_waves if shared else 0, dx_mode=rt.DX_TERMS, n_chunks=1,
-                order_hops=max(0, t["conv_hops"]), hub_limit=hub_limit)
+                order_hops=max(0, t["conv_hops"]), order_min_nodes=t["conv_omin"], hub_limit=hub_limit)
     return s.text(), dims, descs
 
 

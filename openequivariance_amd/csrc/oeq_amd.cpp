@@ -79,6 +79,19 @@ size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 // codegen/common.py use the same number).
 constexpr int64_t OEQ_LONG_LIST = 126;
 
+// One side of an index under construction, passed by value to its kernels (oeq_side in codegen/common.py).
+struct IndexSide {
+    const int64_t *keys = nullptr, *list = nullptr;
+    uint32_t *counts = nullptr, *slots = nullptr, *unordered = nullptr;
+    int64_t *perm = nullptr, *ptr = nullptr, *hubptr = nullptr, *hubnode = nullptr;
+};
+
+// Segments per tile of oeq_group_scan, and the blocks it gets per side (each sums what lies before its range).
+constexpr int64_t kScanTile = 1024, kScanBlocks = 32;
+// Largest edge list that oeq_index_small takes (its LDS; beyond it one block is also slower than the whole device:
+// 80 000 edges would be 80 per thread).
+constexpr int64_t kSmallItems = 16384, kSmallSegments = 4096;
+
 }  // namespace
 
 struct oeq_kernels {
@@ -161,11 +174,11 @@ struct oeq_kernels {
         return !slots[dev].modules.empty();
     }
 
-    int launch(int role, int64_t units, void** args, void* stream) {
+    int launch(int role, int64_t units, void** args, void* stream, unsigned blocks = 0) {
         const std::vector<hipFunction_t>* fns = nullptr;
         int rc = functions(role, &fns);
         if (rc) return rc;
-        unsigned grid = grid_for(role, units);
+        unsigned grid = blocks ? blocks : grid_for(role, units);
         if (no_events || !timing.load(std::memory_order_relaxed)) {
             for (hipFunction_t fn : *fns)
                 HIP_TRY(hipModuleLaunchKernel(fn, grid, 1, 1, roles[role].block, 1, 1, 0, (hipStream_t)stream, args,
@@ -193,36 +206,40 @@ struct oeq_kernels {
         return launch(OEQ_ROLE_FILL_ZERO, (n + 15) / 16, args, stream);
     }
 
-    int segment_ptr(int64_t n_items, int64_t n_segments, const int64_t* keys, const int64_t* perm, int64_t* ptr,
-                    void* stream) {
-        void* args[] = {&n_items, &n_segments, &keys, &perm, &ptr};
-        return launch(OEQ_ROLE_SEGMENT_PTR, n_items + 1, args, stream);
+    // Segment starts of one or two sorted lists (codegen/common.py: oeq_segment_ptr).
+    int segment_ptr(int64_t n_items, int64_t n_segments, IndexSide a, IndexSide b, void* stream) {
+        void* args[] = {&n_items, &n_segments, &a, &b};
+        return launch(OEQ_ROLE_SEGMENT_PTR, (n_items + 1) * (b.ptr ? 2 : 1), args, stream);
     }
 
-    // Counting sort of the item indices 0..n_items-1 by key: ptr[0..n_segments] = segment starts,
-    // perm = item indices grouped by key, ascending within a group (so the result depends on the key
-    // list only); cursor (n_segments + 1 entries and the long-segment list, see ptr_bytes_of) and unordered
-    // (n_items) are scratch.
-    int group_by_key(int64_t n_items, int64_t n_segments, const int64_t* keys, int64_t* ptr, int64_t* cursor,
-                     int64_t* unordered, int64_t* perm, void* stream) {
-        int rc = fill_zero(ptr, (size_t)(n_segments + 1) * sizeof(int64_t), stream);
+    // Segment starts from the histograms (grouping) and the table of extra walk positions, `limit` edges a chunk.
+    int scan(int64_t n_items, int64_t n_segments, int64_t limit, int64_t capacity, IndexSide a, IndexSide b,
+             void* stream) {
+        void* args[] = {&n_items, &n_segments, &limit, &capacity, &a, &b};
+        const int64_t per_side = std::min<int64_t>(kScanBlocks, (n_segments + kScanTile) / kScanTile);
+        return launch(OEQ_ROLE_GROUP_SCAN, 0, args, stream, (unsigned)(per_side * (b.ptr ? 2 : 1)));
+    }
+
+    // Counting sort of the item indices 0..n_items-1 by key, for one or two key lists: ptr[0..n_segments] =
+    // segment starts, perm = item indices grouped by key, ascending within a group (so the result depends on
+    // the key list only). The histograms of the sides lie next to each other: one fill clears them.
+    int group_by_key(int64_t n_items, int64_t n_segments, int64_t limit, int64_t capacity, IndexSide a, IndexSide b,
+                     void* stream) {
+        if (n_items > 0xffffffffLL)
+            return fail(OEQ_ERR_INVALID, "grouping %lld items: at most 2^32 - 1 are supported", (long long)n_items);
+        char* last = (char*)(b.ptr ? b.counts : a.counts);
+        int rc = fill_zero(a.counts, (size_t)(last - (char*)a.counts) + (size_t)(n_segments + 1) * sizeof(uint32_t),
+                           stream);
         if (rc) return rc;
-        void* cargs[] = {&n_items, &keys, &ptr, &n_segments};
-        rc = launch(OEQ_ROLE_GROUP_COUNT, n_items, cargs, stream);
-        if (rc) return rc;
-        int64_t n = n_segments + 1;
-        void* sargs[] = {&n, &ptr, &cursor};
-        rc = launch(OEQ_ROLE_GROUP_SCAN, 1, sargs, stream);
-        if (rc) return rc;
-        void* pargs[] = {&n_items, &keys, &cursor, &unordered, &n_segments};
-        rc = launch(OEQ_ROLE_GROUP_SCATTER, n_items, pargs, stream);
-        if (rc) return rc;
-        // the scan left the segments longer than a wave should rank by itself behind the cursor entries
-        const int64_t* long_list = cursor + n_segments + 1;
-        void* oargs[] = {&n_segments, &ptr, &unordered, &perm, &long_list, &n_items};
+        const int64_t sides = b.ptr ? 2 : 1;
+        void* args[] = {&n_items, &n_segments, &a, &b};
+        rc = launch(OEQ_ROLE_GROUP_COUNT, n_items * sides, args, stream);
+        if (!rc) rc = scan(n_items, n_segments, limit, capacity, a, b, stream);
+        if (!rc) rc = launch(OEQ_ROLE_GROUP_SCATTER, n_items * sides, args, stream);
         // one wave per segment, and at least one thread per 16 items so that few nodes with many items
         // still bring a grid wide enough for the long segments
-        return launch(OEQ_ROLE_GROUP_ORDER, std::max(n_segments, n_items / 64), oargs, stream);
+        if (!rc) rc = launch(OEQ_ROLE_GROUP_ORDER, std::max(n_segments * sides, n_items / 64), args, stream);
+        return rc;
     }
 };
 
@@ -262,7 +279,7 @@ int static_scratch(void** out) {
 extern "C" {
 
 const char* oeq_last_error(void) { return g_error.c_str(); }
-int oeq_abi_version(void) { return 6; }
+int oeq_abi_version(void) { return 7; }
 
 int oeq_get_device_props(int device, oeq_device_props* out) {
     if (!out) return fail(OEQ_ERR_INVALID, "oeq_get_device_props: out is NULL");
@@ -410,7 +427,9 @@ int oeq_segment_sum(oeq_kernels* k, int64_t n_segments, int64_t n_items, int64_t
     if (!workspace || workspace_bytes < need)
         return fail(OEQ_ERR_INVALID, "oeq_segment_sum: workspace too small (%zu < %zu bytes)", workspace_bytes, need);
     int64_t* ptr = (int64_t*)workspace;
-    int rc = k->segment_ptr(n_items, n_segments, keys, perm, ptr, stream);
+    IndexSide side;
+    side.keys = keys, side.list = perm, side.ptr = ptr;
+    int rc = k->segment_ptr(n_items, n_segments, side, IndexSide(), stream);
     if (rc) return rc;
     void* args[] = {&n_segments, &n_items, &row_len, &src, &dst, &perm, &ptr};
     return k->launch(OEQ_ROLE_SEGMENT_SUM, n_segments, args, stream);
@@ -418,7 +437,7 @@ int oeq_segment_sum(oeq_kernels* k, int64_t n_segments, int64_t n_items, int64_t
 
 size_t oeq_grouped_sum_workspace_bytes(const oeq_kernels* k, int64_t n_segments, int64_t n_items) {
     (void)k;
-    // [ptr | cursor | perm | scratch perm]
+    // [ptr | histogram | perm | place of every item, items in that order]
     return 2 * align_up((size_t)(n_segments + 1 + 1 + OEQ_LONG_LIST) * sizeof(int64_t), 256) +
            2 * align_up((size_t)n_items * sizeof(int64_t), 256);
 }
@@ -437,10 +456,13 @@ int oeq_grouped_sum(oeq_kernels* k, int64_t n_segments, int64_t n_items, int64_t
     const size_t pb = align_up((size_t)(n_segments + 1 + 1 + OEQ_LONG_LIST) * sizeof(int64_t), 256);
     const size_t qb = align_up((size_t)n_items * sizeof(int64_t), 256);
     int64_t* ptr = (int64_t*)workspace;
-    int64_t* cursor = (int64_t*)((char*)workspace + pb);
     int64_t* perm = (int64_t*)((char*)workspace + 2 * pb);
-    int64_t* scratch = (int64_t*)((char*)workspace + 2 * pb + qb);
-    int rc = k->group_by_key(n_items, n_segments, keys, ptr, cursor, scratch, perm, stream);
+    IndexSide side;
+    side.keys = keys, side.ptr = ptr, side.perm = perm;
+    side.counts = (uint32_t*)((char*)workspace + pb);
+    side.slots = (uint32_t*)((char*)workspace + 2 * pb + qb);
+    side.unordered = side.slots + n_items;
+    int rc = k->group_by_key(n_items, n_segments, 0, 0, side, IndexSide(), stream);
     if (rc) return rc;
     const int64_t* cperm = perm;
     void* args[] = {&n_segments, &n_items, &row_len, &src, &dst, &cperm, &ptr};
@@ -557,9 +579,7 @@ static size_t conv_wpartial_bytes(const oeq_kernels* k, int64_t walk_positions, 
 // segments (kernel sets without the table kernels, and the allocation-free entry point).
 static int64_t hub_limit_of(const oeq_kernels* k) {
     if (oeq_kernels::no_hubs || k->dims.hub_limit <= 0) return 0;
-    if (!k->roles[OEQ_ROLE_HUB_COUNT].present || !k->roles[OEQ_ROLE_HUB_FILL].present ||
-        !k->roles[OEQ_ROLE_CONV_FIXUP_FORWARD].present)
-        return 0;
+    if (!k->roles[OEQ_ROLE_GROUP_SCAN].present || !k->roles[OEQ_ROLE_CONV_FIXUP_FORWARD].present) return 0;
     return k->dims.hub_limit;
 }
 // every extra position follows a full chunk of its node, so there are at most nnz / limit of them
@@ -588,16 +608,25 @@ static size_t hub_rows_bytes(const oeq_kernels* k, int role, int64_t nnz) {
 // `keep` are temporaries of the build.
 struct IndexLayout {
     size_t rowptr = SIZE_MAX, colptr = SIZE_MAX, rperm = SIZE_MAX, sperm = SIZE_MAX, order = SIZE_MAX,
-           hubptr = SIZE_MAX, hubnode = SIZE_MAX, shubptr = SIZE_MAX, shubnode = SIZE_MAX, hubcur = SIZE_MAX,
-           keep = 0, cursor = SIZE_MAX, scratch = SIZE_MAX, key_a = SIZE_MAX, key_b = SIZE_MAX, optr = SIZE_MAX,
-           ocursor = SIZE_MAX, oscratch = SIZE_MAX, total = 0;
+           hubptr = SIZE_MAX, hubnode = SIZE_MAX, shubptr = SIZE_MAX, shubnode = SIZE_MAX, keep = 0, counts = SIZE_MAX,
+           scratch = SIZE_MAX, scratch2 = SIZE_MAX, key_a = SIZE_MAX, key_b = SIZE_MAX, optr = SIZE_MAX,
+           ocounts = SIZE_MAX, oscratch = SIZE_MAX, total = 0;
 };
+
+// The nodes are walked in an order derived from the graph where that pays: hops in the kernel set, and at least
+// order_min_nodes nodes. Below, the rows of X come from the Infinity Cache whatever the order (fp32, 32 edges a node:
+// forward 1 867 us against 1 803 at 20 000 nodes of 8 KB rows, backward 4 533 / 4 553; 395 / 387 and 974 / 957 at 6 001
+// nodes of 4.6 KB; no difference at 2 000), and the order costs 100 us and more of every index build; at 50 000
+// nodes of 8 KB rows it saves 1.1 ms of 19.6.
+static bool walks_in_order(const oeq_kernels* k, int64_t node_count) {
+    return k->dims.order_hops > 0 && k->roles[OEQ_ROLE_ORDER_HOP].present && node_count >= k->dims.order_min_nodes;
+}
 
 static IndexLayout index_layout(const oeq_kernels* k, int64_t node_count, int64_t nnz, bool sender_side) {
     IndexLayout w;
     const size_t pb = ptr_bytes_of(node_count), qb = perm_bytes_of(nnz);
     const bool grouped = k->dims.deterministic == OEQ_CONV_GROUPED;
-    const bool ordered = k->dims.order_hops > 0 && k->roles[OEQ_ROLE_ORDER_HOP].present;
+    const bool ordered = walks_in_order(k, node_count);
     auto take = [&w](size_t bytes) { size_t at = w.total; w.total += bytes; return at; };
     w.rowptr = take(pb);
     if (sender_side) w.colptr = take(pb);
@@ -614,16 +643,16 @@ static IndexLayout index_layout(const oeq_kernels* k, int64_t node_count, int64_
         }
     }
     w.keep = w.total;
-    if (hub_cap) w.hubcur = take(pb);
     if (grouped) {
-        w.cursor = take(pb);
+        w.counts = take(pb);  // (32 bits per node and side)
         w.scratch = take(qb);
+        if (sender_side) w.scratch2 = take(qb);
     }
     if (ordered) {
         w.key_a = take(pb);
         w.key_b = take(pb);
         w.optr = take(pb);
-        w.ocursor = take(pb);
+        w.ocounts = take(pb);
         w.oscratch = take(pb);
     }
     return w;
@@ -708,31 +737,35 @@ static int build_index(oeq_kernels* k, const char* who, const IndexLayout& w, in
     WalkIndex ix;
     int rc = bind_index(k, who, w, index, index_bytes, transpose_perm, &ix);
     if (rc) return rc;
-    const bool sender_side = w.colptr != SIZE_MAX;
-    if (k->dims.deterministic == OEQ_CONV_SORTED) {
-        rc = k->segment_ptr(nnz, node_count, rows, nullptr, ix.rowptr, stream);
-        if (!rc && sender_side) rc = k->segment_ptr(nnz, node_count, cols, transpose_perm, ix.colptr, stream);
+    const bool sender_side = w.colptr != SIZE_MAX, grouped = k->dims.deterministic == OEQ_CONV_GROUPED;
+    const int64_t limit = ix.hubptr ? ix.hub_limit : 0, cap = hub_capacity(k, nnz);
+    IndexSide a, b;
+    a.keys = rows, a.ptr = ix.rowptr, a.hubptr = ix.hubptr, a.hubnode = ix.hubnode;
+    if (sender_side) b.keys = cols, b.ptr = ix.colptr, b.hubptr = ix.shubptr, b.hubnode = ix.shubnode;
+    if (grouped) {
+        a.perm = ix.rperm;
+        a.counts = (uint32_t*)at_offset(index, w.counts);
+        a.slots = (uint32_t*)at_offset(index, w.scratch);
+        a.unordered = a.slots + nnz;
+        if (sender_side) {
+            b.perm = (int64_t*)ix.sperm;
+            b.counts = (uint32_t*)((char*)a.counts + align_up((size_t)(node_count + 1) * sizeof(uint32_t), 256));
+            b.slots = (uint32_t*)at_offset(index, w.scratch2);
+            b.unordered = b.slots + nnz;
+        }
     } else {
-        int64_t* cursor = (int64_t*)at_offset(index, w.cursor);
-        int64_t* scratch = (int64_t*)at_offset(index, w.scratch);
-        rc = k->group_by_key(nnz, node_count, rows, ix.rowptr, cursor, scratch, ix.rperm, stream);
-        if (!rc && sender_side)
-            rc = k->group_by_key(nnz, node_count, cols, ix.colptr, cursor, scratch, (int64_t*)ix.sperm, stream);
+        b.list = transpose_perm;
     }
-    // extra positions of long segments: count per node, exclusive scan, list the nodes
-    auto hub_table = [&](int64_t* segptr, int64_t* hubptr, int64_t* hubnode) {
-        int64_t limit = ix.hub_limit, cap = hub_capacity(k, nnz), n1 = node_count + 1;
-        int64_t* hubcur = (int64_t*)at_offset(index, w.hubcur);
-        void* cargs[] = {&node_count, &nnz, &segptr, &limit, &hubptr};
-        int r = k->launch(OEQ_ROLE_HUB_COUNT, n1, cargs, stream);
-        void* sargs[] = {&n1, &hubptr, &hubcur};
-        if (!r) r = k->launch(OEQ_ROLE_GROUP_SCAN, 1, sargs, stream);
-        void* fargs[] = {&node_count, &cap, &hubptr, &hubnode};
-        if (!r) r = k->launch(OEQ_ROLE_HUB_FILL, node_count, fargs, stream);
-        return r;
-    };
-    if (!rc && ix.hubptr) rc = hub_table(ix.rowptr, ix.hubptr, ix.hubnode);
-    if (!rc && ix.shubptr) rc = hub_table(ix.colptr, ix.shubptr, ix.shubnode);
+    if (nnz <= kSmallItems && node_count <= kSmallSegments && k->roles[OEQ_ROLE_INDEX_SMALL].present) {
+        int64_t n = nnz, ns = node_count, lim = limit, c = cap;
+        void* args[] = {&n, &ns, &lim, &c, &a, &b};
+        rc = k->launch(OEQ_ROLE_INDEX_SMALL, 0, args, stream, b.ptr ? 2u : 1u);
+    } else if (grouped) {
+        rc = k->group_by_key(nnz, node_count, limit, cap, a, b, stream);
+    } else {
+        rc = k->segment_ptr(nnz, node_count, a, b, stream);
+        if (!rc && limit) rc = k->scan(nnz, node_count, limit, cap, a, b, stream);
+    }
     if (rc || !ix.order) return rc;
     // Walk order: cluster the nodes by the highest-priority node within `order_hops` edges, then list them
     // cluster by cluster (a counting sort by cluster key, ascending node index inside a cluster, so that the
@@ -749,9 +782,12 @@ static int build_index(oeq_kernels* k, const char* who, const IndexLayout& w, in
         if (rc) return rc;
         key_in = key_out;
     }
-    return k->group_by_key(node_count, node_count, key_in, (int64_t*)at_offset(index, w.optr),
-                           (int64_t*)at_offset(index, w.ocursor), (int64_t*)at_offset(index, w.oscratch), ix.order,
-                           stream);
+    IndexSide o;
+    o.keys = key_in, o.ptr = (int64_t*)at_offset(index, w.optr), o.perm = ix.order;
+    o.counts = (uint32_t*)at_offset(index, w.ocounts);
+    o.slots = (uint32_t*)at_offset(index, w.oscratch);
+    o.unordered = o.slots + node_count;
+    return k->group_by_key(node_count, node_count, 0, 0, o, IndexSide(), stream);
 }
 
 static bool walk_mode(const oeq_kernels* k) { return k->dims.deterministic != OEQ_CONV_ATOMIC; }

@@ -50,14 +50,13 @@ ROLE_GROUP_ORDER = 12
 ROLE_DOUBLE_BACKWARD_A = 13
 ROLE_DOUBLE_BACKWARD_B = 14
 ROLE_ORDER_HOP = 15
-ROLE_HUB_COUNT = 16
-ROLE_HUB_FILL = 17
+ROLE_INDEX_SMALL = 16
 ROLE_CONV_FIXUP_FORWARD = 18
 ROLE_CONV_BACKWARD_DX = 19
 
 CONV_ATOMIC, CONV_SORTED, CONV_GROUPED = 0, 1, 2
 DX_TERMS, DX_ATOMIC, DX_ARRIVAL, DX_SENDER_WALK = 0, 1, 2, 3
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 
 class OeqError(RuntimeError):
@@ -102,6 +101,7 @@ class _ProblemDims(ctypes.Structure):
         ("dx_mode", ctypes.c_int32),
         ("n_chunks", ctypes.c_int32),
         ("order_hops", ctypes.c_int32),
+        ("order_min_nodes", ctypes.c_int32),
         ("hub_limit", ctypes.c_int32),
     ]
 
