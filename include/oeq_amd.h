@@ -83,11 +83,14 @@ typedef enum {
     OEQ_ROLE_DOUBLE_BACKWARD_B = 14,/* second order: gradients w.r.t. X, Y, W (backward-shaped) */
     OEQ_ROLE_ORDER_HOP = 15,        /* convolution walk order: one hop of the node clustering */
     OEQ_ROLE_INDEX_SMALL = 16,      /* the whole index of a small edge list in one launch */
+    OEQ_ROLE_CONV_FORWARD_SPLIT = 17,/* small graphs: OEQ_ROLE_CONV_FORWARD with a node's edges dealt out to several waves */
     OEQ_ROLE_CONV_FIXUP_FORWARD = 18,/* adds the rows written by the extra chunks to their nodes' rows, in chunk order */
     OEQ_ROLE_CONV_BACKWARD_DX = 19, /* OEQ_DX_SENDER_WALK: the sender gradients by a walk over the senders' edge segments
                                        (forward-shaped: argument list of OEQ_ROLE_CONV_FORWARD with dZ for X, the
                                        receivers for the senders and the sender-side index) */
-    OEQ_ROLE_COUNT = 20
+    OEQ_ROLE_CONV_BACKWARD_DX_SPLIT = 20,  /* the same for OEQ_ROLE_CONV_BACKWARD_DX */
+    OEQ_ROLE_DOUBLE_BACKWARD_A_SPLIT = 21, /* and for OEQ_ROLE_DOUBLE_BACKWARD_A */
+    OEQ_ROLE_COUNT = 22
 } oeq_role;
 
 /* How the convolution kernels of a set find the edges of a node (oeq_problem_dims.deterministic):
@@ -127,6 +130,10 @@ typedef struct {
     uint32_t max_blocks;        /* 0 = one block per ceil(units/units_per_block) */
     uint32_t grid_multiple;     /* 0/1 = none; else the grid is rounded up to a multiple of this (kernels that
                                    remap blockIdx so that each XCD walks a contiguous range of units) */
+    int32_t fill_units;         /* backward-shaped walk kernels: walk positions the device holds at once; on graphs
+                                   with few nodes for it a node's edges are dealt out to several positions
+                                   (0: never; -n: to n positions whatever the graph) */
+    uint32_t max_nodes;         /* *_SPLIT roles: the largest graph that runs them */
 } oeq_kernel_desc;
 
 typedef struct {

@@ -998,11 +998,13 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
 
     # ---------------------------------------------------------- conv forward
     def _edge_loop(self, s: Src, first: str, last: str, load: Callable[[str, str], None],
-                   compute: Callable[[str, str], None], pipelined: int, before_edge: Callable[[str], None] = None):
-        """Walk edges ``first, first+R, ... < last``. Pipelined: two operand
-        sets (A, B); the next edge's loads are issued before the current edge is
+                   compute: Callable[[str, str], None], pipelined: int, before_edge: Callable[[str], None] = None,
+                   split: int = 1):
+        """Walk edges ``first, first+R, ... < last`` (with ``split`` > 1 every ``split``-th step of that). Pipelined:
+        two operand sets (A, B); the next edge's loads are issued before the current edge is
         computed. ``load(buf, e)`` / ``compute(buf, e)`` emit code."""
-        R = self.R
+        R = self.R * split
+        assert split == 1 or pipelined <= 2
         # The compiler takes a direct global->LDS load to write only the bytes at the pointer it is given,
         # not the 64 lanes' worth behind it, so it would move reads of the staging buffer across the load
         # or across the wait for it. The empty asm statements pin them: no memory access crosses one.
@@ -1093,13 +1095,13 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
             s(vmcnt(0))
             self._emit_stage_read(s, "A")
             s(lgkm0)
-            s.open(f"if (e + 1 < {last})")
-            self._emit_stage_issue(s, "e + 1")
+            s.open(f"if (e + {split} < {last})")
+            self._emit_stage_issue(s, f"e + {split}")
             s.close()
             if before_edge:
                 before_edge("e")
             compute("A", "e")
-            s("++e;")
+            s(f"e += {split};" if split > 1 else "++e;")
             s.close()
             return
         if not pipelined:
@@ -1149,11 +1151,14 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
 
     # Trailing parameters of every kernel that walks receivers: the table of long edge segments cut into
     # chunks (see _node_loop_open). Forward-shaped kernels also take the rows that the extra chunks write.
+    # Backward-shaped kernels take ``parts`` instead: on small graphs a node's segment is dealt out to that many
+    # walk positions.
     HUB_PARAMS = (", const i64* __restrict__ hubptr, const i64* __restrict__ hubnode, i64 hub_limit, "
                   "i64 hub_units")
     HUB_ROWS_PARAM = ", T* __restrict__ hub_rows"
+    PARTS_PARAM = ", i64 parts"
 
-    def _node_loop_open(self, s: Src, G: int, xcd: int):
+    def _node_loop_open(self, s: Src, G: int, xcd: int, parts: bool = False):
         """One wave group per walk position. A position is a receiver node with its edge segment, or, for
         a node with more than ``hub_limit`` edges, one chunk of that many edges: the first chunk is the
         node's own position, the others are listed in ``hubnode`` (``hubptr[v]`` = first extra position of
@@ -1165,11 +1170,13 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         Workgroups are handed to the XCDs round-robin; with ``xcd`` > 1 (grid a multiple of it, and so is
         the number of blocks the extra positions take) block ids are remapped so that each XCD walks one
         contiguous range of nodes and neighbouring receivers share their senders' rows through that
-        XCD's L2."""
+        XCD's L2.
+        With ``parts`` the kernel has that parameter: every node's own segment is cut into that many positions
+        (for kernels whose results are per edge, so that the parts need not meet again)."""
         # ``order`` (may be NULL) lists the nodes in the order in which they are to be walked: nodes that
         # share senders next to each other, so that the blocks resident on one XCD gather from a small set
         # of sender rows (the library derives it from the graph at every index build).
-        s("const i64 walk_end = hub_units + node_count;")
+        s(f"const i64 walk_end = hub_units + node_count{' * parts' if parts else ''};")
         if xcd > 1:
             s(f"const i64 hub_blocks = hub_units / {G};")
             s(f"const i64 vper = ((i64)gridDim.x - hub_blocks) / {xcd};")
@@ -1189,25 +1196,96 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         s("if (e1 - e0 > hub_limit) e1 = e0 + hub_limit;")
         s.close()
         s.open("else")
-        s("const i64 vnode = wpos - hub_units;")
+        if parts:
+            s("int vnode = (int)(wpos - hub_units), part = 0;")
+            s("if (parts > 1) { part = vnode % (int)parts; vnode /= (int)parts; }")
+        else:
+            s("const i64 vnode = wpos - hub_units;")
         s("node = order ? order[vnode] : vnode;")
         s("e0 = oeq_pos(rowptr[node], nnz);")
         s("e1 = oeq_pos(rowptr[node + 1], nnz);")
         s("if (hub_limit > 0 && e1 - e0 > hub_limit) e1 = e0 + hub_limit;")
+        if parts:
+            s.open("if (parts > 1)")
+            s("const i64 per = ((int)(e1 - e0) + (int)parts - 1) / (int)parts;")
+            s("e0 += part * per;")
+            s("if (e0 >= e1) continue;")
+            s("if (e1 - e0 > per) e1 = e0 + per;")
+            s.close()
         s.close()
 
+    # -------------------------------------------- a node's edges dealt out to several waves of its block
+    SPLIT_WORDS = 28  # accumulator words a wave puts into LDS at a time (7 KB)
+
+    split_stride = 0  # elements of a wave's LDS slice
+
+    def _split_store(self, s: Src, si: int, rowexpr: str, split: int, segw: int, barriers: Dict[Tuple[int, int], int]):
+        """Sum of the waves' accumulators of segment ``si`` and its store. In rounds: every wave puts its values of a
+        few output blocks into its LDS slice, then each of these blocks is summed over the waves, in wave
+        order, and stored by one of them. ``barriers`` counts the block barriers per (chunk, sg)."""
+        low, limit = self.low, self.split_stride // 64
+        rounds: List[List[int]] = []
+        for io in self._out_of(self.segments[si]):
+            if not rounds or len(rounds[-1]) == split or sum(low.out[b].d for b in rounds[-1]) + low.out[io].d > limit:
+                rounds.append([])
+            rounds[-1].append(io)
+        s.open("")
+        s(f"T* const mine = s_red + wave * {self.split_stride} + lane;")
+        s(f"const T* const first = s_red + (wave - part * {self.NCH * segw}) * {self.split_stride} + lane;")
+        for rnd in rounds:
+            at = 0
+            for io in rnd:
+                for k in range(low.out[io].d):
+                    s(f"mine[{(at + k) * 64}] = a.o{io}[{k}];")
+                at += low.out[io].d
+            s("__syncthreads();")
+            at = 0
+            for n, io in enumerate(rnd):
+                s.open(f"if (part == {n})")
+                for k in range(low.out[io].d):
+                    terms = [f"first[{p * self.NCH * segw * self.split_stride + (at + k) * 64}]" for p in range(split)]
+                    s(f"a.o{io}[{k}] = {' + '.join(terms)};")
+                segments, self.segments = self.segments, list(self.segments)
+                self.segments[si] = [io]
+                try:
+                    self._store_seg(s, si, rowexpr, "r == 0" if self.R > 1 else "true")
+                finally:
+                    self.segments = segments
+                s.close()
+                at += low.out[io].d
+            s("__syncthreads();")
+        s.close()
+        for c in (range(self.NCH) if self.cur_chunk is None else [self.cur_chunk]):
+            key = (c, si % segw)
+            barriers[key] = barriers.get(key, 0) + 2 * len(rounds)
+
+    def _split_pad(self, s: Src, segw: int, barriers: Dict[Tuple[int, int], int]):
+        """Waves whose share of the outputs took fewer rounds than another's meet the remaining block barriers."""
+        most = max(barriers.values())
+        for c in range(self.NCH):
+            for sg in range(segw):
+                missing = most - barriers.get((c, sg), 0)
+                if missing:
+                    cond = " && ".join([f"chunk == {c}"] + ([f"sg == {sg}"] if segw > 1 else []))
+                    s(f"if ({cond}) for (int t = 0; t < {missing}; ++t) __syncthreads();")
+
     def emit_conv_forward(self, s: Src, G: int, deterministic: bool, pipelined: bool, waves_per_eu: int = 0,
-                          xcd: int = 1, tr_atomics: bool = True, name: str = "forward"):
+                          xcd: int = 1, tr_atomics: bool = True, name: str = "forward", split: int = 1):
+        """``split`` > 1 (receiver walk only): that many waves of a block deal the node's edges out between them and
+        add their accumulators through LDS at the end, in wave order."""
         low = self.low
+        assert split == 1 or (deterministic and G == 1 and not self.kahan and not self.use_q)
         # With several output segments the waves of a node can each own some of them (their accumulators
         # stay in registers) and walk the node's edges side by side, instead of one wave walking the edges
         # once per segment.
         segw = self.seg_waves if deterministic else 1
-        block = 64 * self.NCH * G * segw
+        block = 64 * self.NCH * G * segw * split
         R = self.R
         # weights two edges ahead: only where the loop body issues no stores or atomics (they share the
         # vector-memory counter with the loads the loop waits for by count)
         mode = self._edge_mode(pipelined if (deterministic or pipelined != 4) else 2)
+        if split > 1 and mode > 2:
+            mode = self._edge_mode(2)
         s.open(
             f'extern "C" __global__ {self._attrs(block, waves_per_eu)} void {name}(i64 node_count, i64 nnz, '
             "const T* __restrict__ L1_in, const T* __restrict__ L2_in, const T* __restrict__ W, "
@@ -1216,13 +1294,16 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
             f"{self.HUB_PARAMS}{self.HUB_ROWS_PARAM})"
         )
         self._lane_prologue(s, segw)
+        if split > 1:
+            # (the waves of a node are (chunk, sg, part) triples: what the prologue calls the node of the block)
+            s("const int part = g;")
         if self.use_q:
             self._emit_q_prologue(s, block // 64)
         if self.can_preload:
             s("E_t A, B;")
         if mode in (2, 4):
             floats = self.stage["floats"] + (self.stage["nqw"] * 256 if mode == 4 else 0)
-            s(f"__shared__ __attribute__((aligned(16))) T s_stage[{self.NCH * G}][{floats}];")
+            s(f"__shared__ __attribute__((aligned(16))) T s_stage[{self.NCH * G * split}][{floats}];")
             self._emit_stage_offsets(s)
         if mode == 3:
             for b in "AB":
@@ -1230,7 +1311,7 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
             self._emit_stage3_offsets(s)
         self.tr_atomics = (not deterministic) and tr_atomics and self._regular_wave() and not self.ir_mul
         if self.tr_atomics or (self.tr_stores & 1 and self.R == 1):
-            s(f"__shared__ T s_tr[{self.NCH * G * segw}][{64 * max(low.out[io].d for io in self.used_out)}];")
+            s(f"__shared__ T s_tr[{self.NCH * G * segw * split}][{64 * max(low.out[io].d for io in self.used_out)}];")
 
         def make_load(si):
             def load(buf, e):
@@ -1267,7 +1348,18 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
                 s.close()
 
         if deterministic:
+            if split > 1:
+                s.open("")
+                s("const int g = 0;")
+                if mode == 2:  # (the edge's staging buffers are free by then)
+                    s("T* const s_red = &s_stage[0][0];")
+                    self.split_stride = floats
+                else:
+                    widest = max(low.out[io].d for io in self.used_out)
+                    self.split_stride = max(self.SPLIT_WORDS // self.words, widest) * 64
+                    s(f"__shared__ T s_red[{block // 64 * self.split_stride}];")
             self._node_loop_open(s, G, xcd)
+            barriers: Dict[Tuple[int, int], int] = {}
             s(f"T* zrow = hubpos >= 0 ? hub_rows + hubpos * {low.L3} : L3_out + node * {low.L3};")
             for si in range(len(self.segments)):
                 s.open(f"if (sg == {si % segw})" if segw > 1 else "")
@@ -1278,7 +1370,8 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
                     s(f"A{si}_t a; zero_seg{si}(a);")
                     if kahan:
                         s(f"A{si}_t c; zero_seg{si}(c);")
-                    self._edge_loop(s, "e0 + r", "e1", make_load(si), make_compute(si), mode)
+                    self._edge_loop(s, f"e0 + part * {R} + r" if split > 1 else "e0 + r", "e1", make_load(si),
+                                    make_compute(si), mode, split=split)
                     if R > 1:
                         # fold the R lane groups (fixed order) into group 0
                         for io in self.segments[si]:
@@ -1287,12 +1380,20 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
                                 while m < 64:
                                     s(f"a.o{io}[{k}] += __shfl_xor(a.o{io}[{k}], {m});")
                                     m *= 2
-                    self._store_seg(s, si, "zrow", "r == 0" if self.R > 1 else "true")
+                    if split > 1:
+                        self._split_store(s, si, "zrow", split, segw, barriers)
+                    else:
+                        self._store_seg(s, si, "zrow", "r == 0" if self.R > 1 else "true")
 
                 self._per_chunk(s, node_body)
                 s.close()
-            self._zero_untouched_out(s, "zrow", "r == 0 && sg == 0" if segw > 1 else "r == 0")
+            if split > 1:
+                self._split_pad(s, segw, barriers)
+            first = "r == 0 && sg == 0" if segw > 1 else "r == 0"
+            self._zero_untouched_out(s, "zrow", first + " && part == 0" if split > 1 else first)
             s.close()
+            if split > 1:
+                s.close()
         else:
             # contiguous edge range per wave group; flush with atomics whenever the receiver changes
             s(f"const i64 ngrp = (i64)gridDim.x * {G};")
@@ -1912,7 +2013,7 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
             "const T* __restrict__ L3_grad, const i64* __restrict__ rows, const i64* __restrict__ cols, "
             "const i64* __restrict__ rowptr, T* __restrict__ dx_tmp, const i64* __restrict__ eperm, "
             "T* __restrict__ wpartial, const i64* __restrict__ colptr, const i64* __restrict__ sperm, "
-            f"int* __restrict__ arrivals, const i64* __restrict__ order{self.HUB_PARAMS})"
+            f"int* __restrict__ arrivals, const i64* __restrict__ order{self.HUB_PARAMS}{self.PARTS_PARAM})"
         )
         self._lane_prologue(s, SW)
         if self.use_q:
@@ -1922,7 +2023,7 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         s(f"__shared__ T s_dy[{SW * self.NCH}][{self.l2_pad}];")
         s(f"__shared__ T s_dx[{SW}][{self.NCH}][{XW}][64];")
         s("E_t A;")
-        self._node_loop_open(s, 1, xcd)
+        self._node_loop_open(s, 1, xcd, parts=True)
         for si in range(SW):
             s.open(f"if (sg == {si})")
 
@@ -2051,7 +2152,7 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
             "const T* __restrict__ L3_grad, const i64* __restrict__ rows, const i64* __restrict__ cols, "
             "const i64* __restrict__ rowptr, T* __restrict__ dx_tmp, const i64* __restrict__ eperm, "
             "T* __restrict__ wpartial, const i64* __restrict__ colptr, const i64* __restrict__ sperm, "
-            f"int* __restrict__ arrivals, const i64* __restrict__ order{self.HUB_PARAMS})"
+            f"int* __restrict__ arrivals, const i64* __restrict__ order{self.HUB_PARAMS}{self.PARTS_PARAM})"
         )
         self._lane_prologue(s)
         if self.use_q:
@@ -2145,7 +2246,7 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
             return compute
 
         if deterministic:
-            self._node_loop_open(s, G, xcd)
+            self._node_loop_open(s, G, xcd, parts=True)
 
             def node_body():
                 if resident:
@@ -2310,7 +2411,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
                     conv_segw=4, conv_split=1, conv_dd=1, dd_acc=0, dd_g=2, dd_wa=2, dd_wb=2, dd_fp=0, dd_fw=32,
                     dd_gres=-1, dd_split=1, dd_segw=4, dd_merge=0, dd_need=200, dd_ngrp=0, conv_gbud=0, conv_ngrp=0, conv_fit=300, conv_fw=0, conv_pf=0,
                     conv_dxm=-1, conv_q=0, conv_hops=2, conv_qpin=1, conv_qaf=48, conv_qab=24, tp_mask=0, tp_forms=1,
-                    conv_hub=256, conv_dxs=-1, conv_omin=32768))
+                    conv_hub=256, conv_dxs=-1, conv_omin=32768, conv_fsplit=-1, conv_fsmax=-1, conv_parts=-1))
     assert deterministic or not kahan, "kahan=True requires deterministic=True"
     # knobs somebody set: the rules below leave those alone
     user_tune = os.environ.get("OEQ_AMD_TUNE", "")
@@ -2432,6 +2533,13 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     xcd = max(1, t["conv_xcd"])
     xcd_b = 1 if (walk and low.shared_weights) else xcd  # bounded grid: one partial dW row per wave group
     blk_f = em.emit_conv_forward(s, G_f, walk, t["conv_pipe_f"], t["conv_wf"], xcd, bool(t["conv_tra"]))
+    splits: Dict[str, int] = {}  # the kernels with a node's edges dealt out to several waves: how many
+    if walk and not kahan and not q_fwd:
+        n = t["conv_fsplit"] if t["conv_fsplit"] >= 0 else split_waves(em.NCH * em.seg_waves, t["conv_wf"])
+        if n > 1:
+            splits["forward_split"] = n
+            blk_fs = em.emit_conv_forward(s, 1, True, t["conv_pipe_f"], t["conv_wf"], xcd, bool(t["conv_tra"]),
+                                          name="forward_split", split=n)
     em.use_q = q_bwd
     gres = None if t["conv_gres"] < 0 else bool(t["conv_gres"])
     dx_mode = 0
@@ -2494,6 +2602,8 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
             (rt.ROLE_CONV_BACKWARD, "backward", blk_b, G_b, compute_units * 8 if low.shared_weights else 0, xcd_b),
             (rt.ROLE_CONV_FIXUP_BACKWARD, "fixup_backward", 256, 1, 0),
         ]
+        if splits:
+            descs.append((rt.ROLE_CONV_FORWARD_SPLIT, "forward_split", blk_fs, 1, 0, xcd))
         if low.shared_weights:
             descs.append((rt.ROLE_TP_BACKWARD_WREDUCE, "oeq_wreduce", 256, 64, 0))
         if dx_mode == UvuEmitter.DX_SENDER_WALK:
@@ -2513,11 +2623,17 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
             waves_x = t["conv_wx"] if t["conv_wx"] else (-2 if words_x <= 48 else 2)
             blk_x = ex.emit_conv_forward(s, G_x, True, t["conv_pipe_f"] if pipe_x else 0, waves_x,
                                          xcd, bool(t["conv_tra"]), name="backward_dx")
-            s("}  // namespace oeq_dx")
             descs.append((rt.ROLE_CONV_BACKWARD_DX, "backward_dx", blk_x, G_x, 0, xcd))
+            n = t["conv_fsplit"] if t["conv_fsplit"] >= 0 else split_waves(ex.NCH, waves_x)
+            if n > 1 and not kahan:
+                splits["backward_dx_split"] = n
+                blk_xs = ex.emit_conv_forward(s, 1, True, t["conv_pipe_f"] if pipe_x else 0, waves_x, xcd,
+                                              bool(t["conv_tra"]), name="backward_dx_split", split=n)
+                descs.append((rt.ROLE_CONV_BACKWARD_DX_SPLIT, "backward_dx_split", blk_xs, 1, 0, xcd))
+            s("}  // namespace oeq_dx")
         from . import uvu_double
         if t["conv_dd"] and uvu_double.supported(low, conv=True):
-            descs += uvu_double.add_conv_kernels(s, low, em, t, xcd, G_b, compute_units, kahan)
+            descs += uvu_double.add_conv_kernels(s, low, em, t, xcd, G_b, compute_units, kahan, splits)
         # counting sort: of the edge indices by node (GROUPED mode) and of the nodes by cluster (walk order)
         descs += [
             (rt.ROLE_GROUP_COUNT, "oeq_group_count", 256, 256, compute_units * 16),
@@ -2581,7 +2697,53 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
             third = conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wf=3))
             if _forward_scratch(third[0]) == 0:
                 return third
+    if walk:
+        descs = _small_graph_rules(src, descs, splits, compute_units, t, low.shared_weights)
     return src, dims, descs
+
+
+def split_waves(node_waves: int, waves_per_eu: int) -> int:
+    """How many waves a node's edges are dealt out to in the small-graph form of a forward-shaped kernel with
+    ``node_waves`` waves per node: a block of eight waves (two per SIMD), four where a lane has 512 registers."""
+    return (4 if waves_per_eu == 1 else 8) // node_waves
+
+
+def _small_graph_rules(src: str, descs: List[tuple], splits: Dict[str, int], compute_units: int, t: dict,
+                       shared: bool) -> List[tuple]:
+    """Launch descriptors with what the host needs to know to run small graphs (csrc/oeq_amd.cpp: split_role,
+    backward_parts): how many walk positions of a backward-shaped kernel the device holds at once, and up to how many
+    nodes the split form of a forward-shaped kernel is the faster one. Both follow from the registers and the LDS the
+    compiler gave the kernels.
+
+    The split form (one node per block, its edges dealt out to ``n`` waves) pays while the plain kernel's waves are
+    too few to hide their latencies: up to about n * nodes = 2.5 times the nodes the plain kernel holds at once.
+    Measured with 30 edges per node, plain / split in us: mace-large (n = 4) 80 nodes 43 / 19, 500 nodes 52 / 39, 1 000
+    nodes 69 / 73; mace-medium (4) 150 nodes 27 / 13, 1 500 nodes 47 / 44, 3 000 nodes 87 / 87; nequip-lips (8) 80 nodes
+    30 / 15, 750 nodes 51 / 46, 1 000 nodes 56 / 62."""
+    from .. import runtime as rt
+    blob = rt.compile_source(src)
+    regs, res = rt.kernel_registers(blob), rt.kernel_resources(blob)
+    by_name = {d[1]: d for d in descs}
+
+    def blocks_at_once(name: str) -> int:
+        waves = by_name[name][2] // 64
+        simd = max(1, min(8, 512 // max(1, regs.get(name, 128))))
+        lds = res.get(name, (0, 0))[0]
+        return compute_units * max(1, min(4 * simd // waves, (160 * 1024) // lds if lds else 32))
+
+    out = []
+    for d in descs:
+        fill = limit = 0
+        if d[1] in splits:
+            plain = d[1].replace("_split", "")
+            limit = t["conv_fsmax"] if t["conv_fsmax"] >= 0 else int(
+                2.5 * blocks_at_once(plain) * by_name[plain][3] / splits[d[1]])
+        elif d[0] in (rt.ROLE_CONV_BACKWARD, rt.ROLE_DOUBLE_BACKWARD_B) and not shared and not t["dd_merge"]:
+            fill = -t["conv_parts"] if t["conv_parts"] >= 0 else blocks_at_once(d[1]) * d[3]
+        out.append(tuple(d[:5]) + (d[5] if len(d) > 5 else 0, fill, limit))
+    return out
+
+
 
 
 def _forward_scratch(source: str) -> int:

@@ -31,7 +31,7 @@ from typing import Dict, List, Optional, Tuple
 
 from .common import Src
 from .lower import Lowered, Path
-from .uvu import UNROLL_V_LIMIT, UvuEmitter
+from .uvu import UNROLL_V_LIMIT, UvuEmitter, split_waves
 
 
 # Convolution: above this many paths (after folding of wide rows) the kernels' register needs (two
@@ -489,22 +489,31 @@ class DoubleEmitter(UvuEmitter):
         s(f"const T* wrow = W{'' if low.shared_weights else f' + eid * {low.WN}'};")
         s(f"const T* crow = W_dgrad{'' if low.shared_weights else f' + eid * {low.WN}'};")
 
-    def emit_conv_double_a(self, s: Src, G: int, waves_per_eu: int = 0, xcd: int = 1, segw: int = 1):
+    def emit_conv_double_a(self, s: Src, G: int, waves_per_eu: int = 0, xcd: int = 1, segw: int = 1,
+                           name: str = "double_backward_A", split: int = 1):
         """Receiver-major walk: the node's accumulators stay in registers over its edges. With ``segw``
         > 1 the output segments of a node are shared between that many waves, which walk its edges side
-        by side (fewer registers per wave, more waves in flight)."""
+        by side (fewer registers per wave, more waves in flight). ``split``: as in ``emit_conv_forward``."""
         low = self.low
         segw = max(1, min(segw, len(self.segments))) if self.R == 1 else 1
-        block = 64 * self.NCH * G * segw
+        block = 64 * self.NCH * G * segw * split
+        assert split == 1 or (G == 1 and not self.kahan)
         s.open(
-            f'extern "C" __global__ {self._attrs(block, waves_per_eu)} void double_backward_A(i64 node_count, '
+            f'extern "C" __global__ {self._attrs(block, waves_per_eu)} void {name}(i64 node_count, '
             f"i64 nnz, {self._CONV_OPERANDS}T* __restrict__ L3_dgrad, const i64* __restrict__ rows, "
             "const i64* __restrict__ cols, const i64* __restrict__ rowptr, const i64* __restrict__ eperm, "
             f"const i64* __restrict__ order{self.HUB_PARAMS}{self.HUB_ROWS_PARAM})"
         )
         self._lane_prologue(s, segw)
         if self.tr_stores & 1 and self.R == 1:
-            s(f"__shared__ T s_tr[{self.NCH * G * segw}][{64 * max(low.out[io].d for io in self.used_out)}];")
+            s(f"__shared__ T s_tr[{self.NCH * G * segw * split}][{64 * max(low.out[io].d for io in self.used_out)}];")
+        if split > 1:
+            s("const int part = g;")
+            s.open("")
+            s("const int g = 0;")
+            self.split_stride = max(self.SPLIT_WORDS // self.words, max(low.out[io].d for io in self.used_out)) * 64
+            s(f"__shared__ T s_red[{block // 64 * self.split_stride}];")
+        barriers: Dict[Tuple[int, int], int] = {}
         self._node_loop_open(s, G, xcd)
         s(f"T* zrow = hubpos >= 0 ? hub_rows + hubpos * {low.L3} : L3_dgrad + node * {low.L3};")
         for si in range(len(self.segments)):
@@ -516,7 +525,8 @@ class DoubleEmitter(UvuEmitter):
                 s(f"D{si}_t a; zero_dseg{si}(a);")
                 if self.kahan:
                     s(f"D{si}_t c; zero_dseg{si}(c);")
-                s.open(f"for (i64 e = e0 + r; e < e1; e += {self.R})")
+                first = f"e0 + part * {self.R} + r" if split > 1 else "e0 + r"
+                s.open(f"for (i64 e = {first}; e < e1; e += {self.R * split})")
                 self._edge_rows(s, "e")
                 s("X_t x, xa;")
                 self._load_x(s, "xrow", self.seg_in1[si])
@@ -532,12 +542,20 @@ class DoubleEmitter(UvuEmitter):
                             while m < 64:
                                 s(f"a.o{io}[{k}] += __shfl_xor(a.o{io}[{k}], {m});")
                                 m *= 2
-                self._store_seg(s, si, "zrow", "r == 0" if self.R > 1 else "true")
+                if split > 1:
+                    self._split_store(s, si, "zrow", split, segw, barriers)
+                else:
+                    self._store_seg(s, si, "zrow", "r == 0" if self.R > 1 else "true")
 
             self._per_chunk(s, node_body)
             s.close()
-        self._zero_untouched_out(s, "zrow", "r == 0 && sg == 0" if segw > 1 else "r == 0")
+        if split > 1:
+            self._split_pad(s, segw, barriers)
+        first = "r == 0 && sg == 0" if segw > 1 else "r == 0"
+        self._zero_untouched_out(s, "zrow", first + " && part == 0" if split > 1 else first)
         s.close()
+        if split > 1:
+            s.close()
         s.close()
         return block
 
@@ -554,7 +572,8 @@ class DoubleEmitter(UvuEmitter):
             f"i64 nnz, {self._CONV_OPERANDS}const T* __restrict__ L3_grad, T* __restrict__ L2_grad, "
             "T* __restrict__ W_grad, const i64* __restrict__ rows, const i64* __restrict__ cols, "
             "const i64* __restrict__ rowptr, T* __restrict__ dx_tmp, const i64* __restrict__ eperm, "
-            f"T* __restrict__ L3_dgrad, const i64* __restrict__ order, T* __restrict__ wpartial{self.HUB_PARAMS})"
+            f"T* __restrict__ L3_dgrad, const i64* __restrict__ order, T* __restrict__ wpartial{self.HUB_PARAMS}"
+            f"{self.PARTS_PARAM})"
         )
         self._lane_prologue(s)
         shared = low.shared_weights
@@ -569,7 +588,7 @@ class DoubleEmitter(UvuEmitter):
             s(f"T dwacc[{self.n_wslots}];")
             s(f"for (int t = 0; t < {self.n_wslots}; ++t) dwacc[t] = T(0);")
         resident = self.double_b_resident() or self.merged
-        self._node_loop_open(s, G, xcd)
+        self._node_loop_open(s, G, xcd, parts=True)
 
         def node_body():
             if resident:
@@ -729,14 +748,15 @@ class DoubleEmitter(UvuEmitter):
             f"i64 nnz, {self._CONV_OPERANDS}const T* __restrict__ L3_grad, T* __restrict__ L2_grad, "
             "T* __restrict__ W_grad, const i64* __restrict__ rows, const i64* __restrict__ cols, "
             "const i64* __restrict__ rowptr, T* __restrict__ dx_tmp, const i64* __restrict__ eperm, "
-            f"T* __restrict__ L3_dgrad, const i64* __restrict__ order, T* __restrict__ wpartial{self.HUB_PARAMS})"
+            f"T* __restrict__ L3_dgrad, const i64* __restrict__ order, T* __restrict__ wpartial{self.HUB_PARAMS}"
+            f"{self.PARTS_PARAM})"
         )
         self._lane_prologue(s, SW)
         s(f"__shared__ T s_dy[{SW * self.NCH}][{self.l2_pad}];")
         s(f"__shared__ T s_dx[{SW}][{self.NCH}][{XW}][64];")
         if self.merged and self.tr_stores & 1:
             s(f"__shared__ T s_tr[{self.NCH * SW}][{64 * max(low.out[io].d for io in self.used_out)}];")
-        self._node_loop_open(s, 1, xcd)
+        self._node_loop_open(s, 1, xcd, parts=True)
         for si in range(SW):
             s.open(f"if (sg == {si})")
 
@@ -853,10 +873,12 @@ def add_tp_kernels(s: Src, low: Lowered, base: UvuEmitter, tune: dict, groups_b:
 
 
 def add_conv_kernels(s: Src, low: Lowered, base: UvuEmitter, tune: dict, xcd: int, groups_b: int = 0,
-                     compute_units: int = 256, kahan: bool = False) -> List[tuple]:
+                     compute_units: int = 256, kahan: bool = False,
+                     splits: Optional[Dict[str, int]] = None) -> List[tuple]:
     """Append the convolution double-backward kernels (receiver-major walk) to a module. Shared weights: kernel B
     runs with the first-order backward kernel's wave groups per block (``groups_b``) on a bounded grid, one
-    partial weight-gradient row per group, and is never split between waves or merged with kernel A."""
+    partial weight-gradient row per group, and is never split between waves or merged with kernel A. ``splits``
+    receives the number of waves of kernel A's small-graph form."""
     from .. import runtime as rt
 
     def kernel_a_need(e: DoubleEmitter) -> int:
@@ -917,6 +939,11 @@ def add_conv_kernels(s: Src, low: Lowered, base: UvuEmitter, tune: dict, xcd: in
             G_a = 1
         blk_a = em.emit_conv_double_a(s, G_a, tune.get("dd_wa", 2), xcd, segw)
         descs.append((rt.ROLE_DOUBLE_BACKWARD_A, "double_backward_A", blk_a, G_a, 0, xcd))
+        n = tune["conv_fsplit"] if tune["conv_fsplit"] >= 0 else split_waves(em.NCH * segw, tune.get("dd_wa", 2))
+        if n > 1 and not kahan and splits is not None:
+            splits["double_backward_A_split"] = n
+            blk_as = em.emit_conv_double_a(s, 1, tune.get("dd_wa", 2), xcd, segw, "double_backward_A_split", n)
+            descs.append((rt.ROLE_DOUBLE_BACKWARD_A_SPLIT, "double_backward_A_split", blk_as, 1, 0, xcd))
     if groups:
         blk_b = em.emit_conv_double_b_split(s, groups, tune.get("dd_wb", 2), xcd)
         G_b = 1

@@ -52,6 +52,8 @@ struct RoleInfo {
     unsigned units_per_block = 1;
     unsigned max_blocks = 0;
     unsigned grid_multiple = 0;
+    int fill_units = 0;
+    unsigned max_nodes = 0;
 };
 
 struct DeviceSlot {
@@ -72,6 +74,14 @@ struct TimedLaunch {
     int role;
     hipEvent_t start, stop;
 };
+
+// The small-graph form of a kernel is timed under the name of the kernel it stands in for.
+int timed_as(int role) {
+    return role == OEQ_ROLE_CONV_FORWARD_SPLIT        ? OEQ_ROLE_CONV_FORWARD
+           : role == OEQ_ROLE_CONV_BACKWARD_DX_SPLIT  ? OEQ_ROLE_CONV_BACKWARD_DX
+           : role == OEQ_ROLE_DOUBLE_BACKWARD_A_SPLIT ? OEQ_ROLE_DOUBLE_BACKWARD_A
+                                                      : role;
+}
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
@@ -186,7 +196,7 @@ struct oeq_kernels {
             return OEQ_OK;
         }
         // profiling mode: bracket the role's kernels with events on their own stream
-        TimedLaunch t{role, nullptr, nullptr};
+        TimedLaunch t{timed_as(role), nullptr, nullptr};
         HIP_TRY(hipEventCreate(&t.start));
         HIP_TRY(hipEventCreate(&t.stop));
         HIP_TRY(hipEventRecord(t.start, (hipStream_t)stream));
@@ -394,6 +404,8 @@ int oeq_kernels_create(const void* code, size_t code_size, const oeq_problem_dim
         r.units_per_block = d.units_per_block;
         r.max_blocks = d.max_blocks;
         r.grid_multiple = d.grid_multiple;
+        r.fill_units = d.fill_units;
+        r.max_nodes = d.max_nodes;
     }
     *out = k;
     return OEQ_OK;
@@ -551,6 +563,8 @@ int oeq_tp_backward(oeq_kernels* k, int64_t num_batch, const void* L1_in, void* 
 // fused graph convolution
 // ---------------------------------------------------------------------------
 
+static bool walk_mode(const oeq_kernels* k) { return k->dims.deterministic != OEQ_CONV_ATOMIC; }
+
 // The generated kernels force every node and edge index into range with 32-bit arithmetic.
 static int check_graph_size(const char* who, int64_t node_count, int64_t nnz) {
     if (node_count < 0 || nnz < 0) return fail(OEQ_ERR_INVALID, "%s: negative size", who);
@@ -596,6 +610,29 @@ static int64_t hub_units(const oeq_kernels* k, int role, int64_t nnz) {
     const int64_t g = std::max(1u, k->roles[role].units_per_block), m = std::max(1u, k->roles[role].grid_multiple);
     const int64_t blocks = ((cap + g - 1) / g + m - 1) / m * m;
     return blocks * g;
+}
+// The form of a forward-shaped kernel for a graph of this many nodes.
+static int split_role(const oeq_kernels* k, int role, int64_t node_count) {
+    const int split = role == OEQ_ROLE_CONV_FORWARD       ? OEQ_ROLE_CONV_FORWARD_SPLIT
+                      : role == OEQ_ROLE_CONV_BACKWARD_DX ? OEQ_ROLE_CONV_BACKWARD_DX_SPLIT
+                                                          : OEQ_ROLE_DOUBLE_BACKWARD_A_SPLIT;
+    return walk_mode(k) && k->roles[split].present && node_count <= (int64_t)k->roles[split].max_nodes ? split : role;
+}
+
+// Walk positions per node of a backward-shaped kernel (their results are per edge, so the parts of a node need not
+// meet again; each loads the node's output gradient for itself). Few nodes: as many as fill the device, of at least 4
+// edges each (30 edges a node, mace-large: 80 nodes 115 -> 28 us, 300 nodes 132 -> 61). Up to about 16 times
+// what the device holds at once, parts of 10 edges: the last ones to run then leave less of it idle (1 500 nodes 282 ->
+// 239 us, 3 000 nodes 490 -> 450, 7 000 nodes 1 034 in parts and whole, 20 000 nodes 2 890 in parts against 2 847).
+// Double precision: half of that, 15 edges (1 000 nodes 398 -> 372 us; 3 000 nodes 1 055 in parts of 10, 1 029 whole).
+static int64_t backward_parts(const oeq_kernels* k, int role, int64_t node_count, int64_t nnz) {
+    const int64_t fill = k->roles[role].fill_units;
+    if (fill < 0) return -fill;
+    if (fill == 0 || node_count <= 0) return 1;
+    const bool wide = k->dims.elem_size == 8;
+    const int64_t idle = std::min(fill / node_count, nnz / (node_count * 4));
+    const int64_t tail = std::min(((wide ? 8 : 16) * fill + node_count / 2) / node_count, nnz / (node_count * (wide ? 15 : 10)));
+    return std::max<int64_t>(1, std::max(idle, tail));
 }
 static size_t hub_rows_bytes(const oeq_kernels* k, int role, int64_t nnz) {
     return align_up((size_t)hub_units(k, role, nnz) * (size_t)k->dims.L3_dim * (size_t)k->dims.elem_size, 256);
@@ -677,7 +714,7 @@ static ScratchLayout scratch_layout(const oeq_kernels* k, int64_t node_count, in
         w.arrivals = take(align_up((size_t)node_count * (size_t)std::max(1, k->dims.n_chunks) * sizeof(int32_t), 256));
     if (terms && wpartial_role == OEQ_ROLE_CONV_BACKWARD && k->dims.dx_mode == OEQ_DX_SENDER_WALK) {
         // no terms: the sender-side walk forms the rows itself, and writes those of its extra chunks here
-        if (int64_t su = hub_units(k, OEQ_ROLE_CONV_BACKWARD_DX, nnz))
+        if (int64_t su = hub_units(k, split_role(k, OEQ_ROLE_CONV_BACKWARD_DX, node_count), nnz))
             w.shub_rows = take(align_up((size_t)su * (size_t)k->dims.L1_dim * (size_t)k->dims.elem_size, 256));
     } else if (terms) {
         w.dx_tmp = take(align_up((size_t)nnz * (size_t)k->dims.L1_dim * (size_t)k->dims.elem_size, 256));
@@ -790,8 +827,6 @@ static int build_index(oeq_kernels* k, const char* who, const IndexLayout& w, in
     return k->group_by_key(node_count, node_count, 0, 0, o, IndexSide(), stream);
 }
 
-static bool walk_mode(const oeq_kernels* k) { return k->dims.deterministic != OEQ_CONV_ATOMIC; }
-
 // L1_grad[s] = sum of the per-edge terms of sender s in sender-major order; senders with more than hub_limit
 // edges in chunks whose partial sums (shub_rows) are added in chunk order afterwards.
 static int sender_sum(oeq_kernels* k, int64_t node_count, int64_t nnz, void* dx_tmp, void* L1_grad,
@@ -844,7 +879,9 @@ int oeq_conv_index_build(oeq_kernels* k, int64_t node_count, int64_t nnz, const 
 
 size_t oeq_conv_forward_scratch_bytes(const oeq_kernels* k, int64_t node_count, int64_t nnz) {
     if (!k || !walk_mode(k) || node_count < 0 || nnz < 0) return 0;
-    return scratch_layout(k, node_count, nnz, false, false, false, OEQ_ROLE_CONV_BACKWARD, OEQ_ROLE_CONV_FORWARD).total;
+    return scratch_layout(k, node_count, nnz, false, false, false, OEQ_ROLE_CONV_BACKWARD,
+                          split_role(k, OEQ_ROLE_CONV_FORWARD, node_count))
+        .total;
 }
 
 size_t oeq_conv_forward_workspace_bytes(const oeq_kernels* k, int64_t node_count, int64_t nnz) {
@@ -866,7 +903,8 @@ size_t oeq_conv_backward_workspace_bytes(const oeq_kernels* k, int64_t node_coun
 size_t oeq_conv_double_backward_scratch_bytes(const oeq_kernels* k, int64_t node_count, int64_t nnz) {
     if (!k || !walk_mode(k)) return 0;
     return scratch_layout(k, node_count, nnz, true, false, true, OEQ_ROLE_DOUBLE_BACKWARD_B,
-                          OEQ_ROLE_DOUBLE_BACKWARD_A).total;
+                          split_role(k, OEQ_ROLE_DOUBLE_BACKWARD_A, node_count))
+        .total;
 }
 
 size_t oeq_conv_double_backward_workspace_bytes(const oeq_kernels* k, int64_t node_count, int64_t nnz) {
@@ -889,14 +927,15 @@ int oeq_conv_forward_indexed(oeq_kernels* k, int64_t node_count, int64_t nnz, co
     int rc;
     int64_t units = 0;
     void* hub_rows = nullptr;
+    const int role = split_role(k, OEQ_ROLE_CONV_FORWARD, node_count);
     if (walk_mode(k)) {
         // the forward reads the receiver side only; the caller's perm stands in where the layout wants one
         rc = bind_index(k, "oeq_conv_forward", index_layout(k, node_count, nnz, index_sender_side != 0), index,
                         index_bytes, rows, &ix);
         if (rc) return rc;
         if (ix.hub_limit) {
-            units = hub_units(k, OEQ_ROLE_CONV_FORWARD, nnz);
-            const size_t need = hub_rows_bytes(k, OEQ_ROLE_CONV_FORWARD, nnz);
+            units = hub_units(k, role, nnz);
+            const size_t need = hub_rows_bytes(k, role, nnz);
             if (!scratch || scratch_bytes < need)
                 return fail(OEQ_ERR_INVALID, "oeq_conv_forward: workspace too small (%zu < %zu bytes of scratch)",
                             scratch_bytes, need);
@@ -908,7 +947,7 @@ int oeq_conv_forward_indexed(oeq_kernels* k, int64_t node_count, int64_t nnz, co
     }
     void* args[] = {&node_count, &nnz,      &L1_in,    &L2_in,      &W,           &L3_out,       &rows,  &cols,
                     &ix.rowptr,  &ix.rperm, &ix.order, &ix.hubptr, &ix.hubnode, &ix.hub_limit, &units, &hub_rows};
-    rc = k->launch(OEQ_ROLE_CONV_FORWARD, walk_mode(k) ? node_count + units : nnz, args, stream);
+    rc = k->launch(role, walk_mode(k) ? node_count + units : nnz, args, stream);
     if (rc || !units) return rc;
     // the rows of the extra chunks, added to their nodes' rows in chunk order
     int64_t row_len = k->dims.L3_dim;
@@ -1031,21 +1070,23 @@ int oeq_conv_backward_indexed(oeq_kernels* k, int64_t node_count, int64_t nnz, c
         if (rc) return rc;
     }
     int64_t units = ix.hub_limit ? hub_units(k, OEQ_ROLE_CONV_BACKWARD, nnz) : 0;
+    int64_t parts = backward_parts(k, OEQ_ROLE_CONV_BACKWARD, node_count, nnz);
     void* args[] = {&node_count,  &nnz,      &L1_in,     &L1_grad,    &L2_in,        &L2_grad,     &W,         &W_grad,
                     &L3_grad,     &rows,     &cols,      &ix.rowptr,  &sc.dx_tmp,    &ix.rperm,    &sc.wpartial,
                     &ix.colptr,   &ix.sperm, &sc.arrivals, &ix.order, &ix.hubptr,    &ix.hubnode,  &ix.hub_limit,
-                    &units};
-    rc = k->launch(OEQ_ROLE_CONV_BACKWARD, walk_mode(k) ? node_count + units : nnz, args, stream);
+                    &units,       &parts};
+    rc = k->launch(OEQ_ROLE_CONV_BACKWARD, walk_mode(k) ? node_count * parts + units : nnz, args, stream);
     if (rc || !walk_mode(k)) return rc;
     if (dx_mode == OEQ_DX_TERMS) rc = sender_sum(k, node_count, nnz, sc.dx_tmp, L1_grad, ix, sc.shub_rows, stream);
     if (dx_mode == OEQ_DX_SENDER_WALK) {
         // The forward kernel of the adjoint problem over the sender side of the index: dZ rows of the receivers
         // for the rows of X, every sender's segment in sender-major order, long segments in chunks.
         int64_t limit = (ix.shubptr && sc.shub_rows) ? ix.hub_limit : 0;
-        int64_t xunits = limit ? hub_units(k, OEQ_ROLE_CONV_BACKWARD_DX, nnz) : 0;
+        const int xrole = split_role(k, OEQ_ROLE_CONV_BACKWARD_DX, node_count);
+        int64_t xunits = limit ? hub_units(k, xrole, nnz) : 0;
         void* xargs[] = {&node_count, &nnz,       &L3_grad,   &L2_in,     &W,           &L1_grad,      &cols,  &rows,
                          &ix.colptr,  &ix.sperm,  &ix.order,  &ix.shubptr, &ix.shubnode, &limit,        &xunits, &sc.shub_rows};
-        rc = k->launch(OEQ_ROLE_CONV_BACKWARD_DX, node_count + xunits, xargs, stream);
+        rc = k->launch(xrole, node_count + xunits, xargs, stream);
         if (!rc && xunits) {
             int64_t row_len = k->dims.L1_dim;
             void* cargs[] = {&node_count, &xunits, &ix.shubptr, &ix.shubnode, &sc.shub_rows, &L1_grad, &row_len};
@@ -1170,8 +1211,9 @@ int oeq_conv_double_backward_indexed(oeq_kernels* k, int64_t node_count, int64_t
     int rc = bind_index(k, "oeq_conv_double_backward", index_layout(k, node_count, nnz, true), index, index_bytes,
                         transpose_perm, &ix);
     if (rc) return rc;
-    const ScratchLayout w = scratch_layout(k, node_count, nnz, true, false, true, OEQ_ROLE_DOUBLE_BACKWARD_B,
-                                           OEQ_ROLE_DOUBLE_BACKWARD_A);
+    const int role_a = split_role(k, OEQ_ROLE_DOUBLE_BACKWARD_A, node_count);
+    const ScratchLayout w =
+        scratch_layout(k, node_count, nnz, true, false, true, OEQ_ROLE_DOUBLE_BACKWARD_B, role_a);
     if (!scratch || scratch_bytes < w.total)
         return fail(OEQ_ERR_INVALID, "oeq_conv_double_backward: workspace too small (%zu < %zu bytes of scratch)",
                     scratch_bytes, w.total);
@@ -1179,13 +1221,14 @@ int oeq_conv_double_backward_indexed(oeq_kernels* k, int64_t node_count, int64_t
     // shared weights: kernel B leaves one partial weight-gradient row per wave group, summed in order at the end
     void* wpartial = at_offset(scratch, w.wpartial);
     void* hub_rows = at_offset(scratch, w.hub_rows);
-    int64_t units_a = (ix.hub_limit && hub_rows) ? hub_units(k, OEQ_ROLE_DOUBLE_BACKWARD_A, nnz) : 0;
+    int64_t units_a = (ix.hub_limit && hub_rows) ? hub_units(k, role_a, nnz) : 0;
     int64_t units_b = ix.hub_limit ? hub_units(k, OEQ_ROLE_DOUBLE_BACKWARD_B, nnz) : 0;
+    int64_t parts_b = backward_parts(k, OEQ_ROLE_DOUBLE_BACKWARD_B, node_count, nnz);
     void* a[] = {&node_count, &nnz,  &L1_in,     &L1_dgrad, &L2_in,    &L2_dgrad,  &W,          &W_dgrad,      &L3_dgrad,
                  &rows,       &cols, &ix.rowptr, &ix.rperm, &ix.order, &ix.hubptr, &ix.hubnode, &ix.hub_limit, &units_a,
                  &hub_rows};
     if (k->roles[OEQ_ROLE_DOUBLE_BACKWARD_A].present) {
-        rc = k->launch(OEQ_ROLE_DOUBLE_BACKWARD_A, node_count + units_a, a, stream);
+        rc = k->launch(role_a, node_count + units_a, a, stream);
         if (rc) return rc;
         if (units_a) {
             int64_t row_len = k->dims.L3_dim;
@@ -1196,8 +1239,8 @@ int oeq_conv_double_backward_indexed(oeq_kernels* k, int64_t node_count, int64_t
     }
     void* b[] = {&node_count, &nnz,        &L1_in,      &L1_dgrad,     &L2_in,   &L2_dgrad,  &W,         &W_dgrad,
                  &L3_grad,    &L2_grad,    &W_grad,     &rows,         &cols,    &ix.rowptr, &dx_tmp,    &ix.rperm,
-                 &L3_dgrad,   &ix.order,   &wpartial,   &ix.hubptr,    &ix.hubnode, &ix.hub_limit, &units_b};
-    rc = k->launch(OEQ_ROLE_DOUBLE_BACKWARD_B, node_count + units_b, b, stream);
+                 &L3_dgrad,   &ix.order,   &wpartial,   &ix.hubptr,    &ix.hubnode, &ix.hub_limit, &units_b, &parts_b};
+    rc = k->launch(OEQ_ROLE_DOUBLE_BACKWARD_B, node_count * parts_b + units_b, b, stream);
     if (rc) return rc;
     rc = sender_sum(k, node_count, nnz, dx_tmp, L1_grad, ix, at_offset(scratch, w.shub_rows), stream);
     if (rc || !wpartial) return rc;

@@ -51,8 +51,11 @@ ROLE_DOUBLE_BACKWARD_A = 13
 ROLE_DOUBLE_BACKWARD_B = 14
 ROLE_ORDER_HOP = 15
 ROLE_INDEX_SMALL = 16
+ROLE_CONV_FORWARD_SPLIT = 17
 ROLE_CONV_FIXUP_FORWARD = 18
 ROLE_CONV_BACKWARD_DX = 19
+ROLE_CONV_BACKWARD_DX_SPLIT = 20
+ROLE_DOUBLE_BACKWARD_A_SPLIT = 21
 
 CONV_ATOMIC, CONV_SORTED, CONV_GROUPED = 0, 1, 2
 DX_TERMS, DX_ATOMIC, DX_ARRIVAL, DX_SENDER_WALK = 0, 1, 2, 3
@@ -85,6 +88,8 @@ class _KernelDesc(ctypes.Structure):
         ("units_per_block", ctypes.c_uint32),
         ("max_blocks", ctypes.c_uint32),
         ("grid_multiple", ctypes.c_uint32),
+        ("fill_units", ctypes.c_int32),
+        ("max_nodes", ctypes.c_uint32),
     ]
 
 
@@ -560,6 +565,7 @@ class KernelSet:
             slot.role, slot.kernel_name, slot.block_threads = role, enc, block
             slot.units_per_block, slot.max_blocks = upb, maxb
             slot.grid_multiple = desc[5] if len(desc) > 5 else 0
+            slot.fill_units, slot.max_nodes = desc[6:8] if len(desc) > 7 else (0, 0)
         pd = _ProblemDims(**dims)
         handle = _P()
         _check(lib.oeq_kernels_create(code, len(code), ctypes.byref(pd), arr, len(descs), ctypes.byref(handle)),

@@ -1,0 +1,82 @@
+"""Small-graph forms of the convolution kernels: a node's edges dealt out to several waves of a block (forward-shaped
+kernels, summed through LDS) or to several walk positions (backward-shaped kernels), against the plain kernels of the
+same problem, which the oracle tests cover. Degrees from none over fewer than there are waves to a segment cut into
+chunks; every kernel structure that has such a form."""
+
+import numpy as np
+import pytest
+import torch
+
+import openequivariance_amd as oeq
+from openequivariance_amd._torch import ops
+from openequivariance_amd.core import problems as P
+from openequivariance_amd.core.graph import CoordGraph
+
+pytestmark = pytest.mark.gpu
+
+
+def _f64(p):
+    p.irrep_dtype = p.weight_dtype = np.float64
+    return p
+
+
+PROBLEMS = {
+    "mace-medium": lambda: P.mace_problems()[1],          # two chunks, LDS staging
+    "mace-large-f64": lambda: _f64(P.mace_problems()[0]),  # one wave per SIMD
+    "config1": P.config1_single_uvu,                      # 64 rows to a wave
+    "config2": P.config2_nequip_uvu,                      # two rows to a wave
+    "aspirin": lambda: P.nequip_problems()[1],            # one chunk; sender gradients by the sender walk
+    "SevenNet-main": lambda: P.seven_net_problems()[1],   # folded multiplicities, waves share the output segments
+    "SevenNet-last": lambda: P.seven_net_problems()[2],   # sender walk over long rows
+    "benzene-f64": lambda: _f64(P.nequip_problems()[3]),  # several segments per wave, stores through LDS
+    "wide-ragged": lambda: P.ChannelwiseTPP("96x0e+70x1o", "0e+1o+2e", "0e+1o+2e"),
+}
+
+
+def _graph(n, seed, hub):
+    """Degrees 0, 1, 2, ... over the first nodes, random ones after that, and one node with ``hub`` edges."""
+    rng = np.random.default_rng(seed)
+    deg = np.concatenate([np.arange(min(n, 20)), rng.integers(0, 30, size=max(0, n - 20))])
+    if hub:
+        deg[-1] = hub
+    rows = np.repeat(np.arange(n), deg)
+    cols = rng.integers(0, n, size=len(rows))
+    if hub:
+        cols[rng.permutation(len(rows))[:hub]] = 1
+    return CoordGraph(np.zeros((n, 3)), rows.astype(np.int64), cols.astype(np.int64))
+
+
+def _run(problem, tune, det, g, tensors, monkeypatch):
+    monkeypatch.setenv("OEQ_AMD_TUNE", tune)
+    conv = oeq.TensorProductConv(problem, deterministic=det)
+    monkeypatch.delenv("OEQ_AMD_TUNE")
+    e = [torch.tensor(a, device="cuda") for a in (g.rows, g.cols, g.transpose_perm)]
+    x, y, w, gr, a, b, c = tensors
+    out = [ops.conv_forward(x, y, w, *e, conv.kid), *ops.conv_backward(x, y, w, gr, *e, conv.kid),
+           *ops.conv_double_backward(x, y, w, gr, a, b, c, *e, conv.kid)]
+    again = ops.conv_forward(x, y, w, *e, conv.kid)
+    assert torch.equal(again, out[0]), "the sum over the waves has a fixed order"
+    return out
+
+
+@pytest.mark.parametrize("name", list(PROBLEMS))
+@pytest.mark.parametrize("tune,n,hub", [("", 1, 5), ("", 33, 300), ("conv_fsplit=2,conv_parts=3", 40, 0),
+                                        ("conv_fsmax=100000,conv_parts=16", 700, 600)])
+def test_small_forms_match_the_plain_kernels(name, tune, n, hub, monkeypatch):
+    problem = PROBLEMS[name]()
+    det = n != 33
+    g = _graph(n, 3, hub)
+    dt = torch.float64 if problem.irrep_dtype == np.float64 else torch.float32
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    dims = (problem.irreps_in1.dim, problem.irreps_in2.dim, problem.weight_numel, problem.irreps_out.dim)
+    shapes = [(n, dims[0]), (g.nnz, dims[1]), (g.nnz, dims[2]), (n, dims[3]), (n, dims[0]), (g.nnz, dims[1]),
+              (g.nnz, dims[2])]
+    tensors = [torch.randn(*s, device="cuda", dtype=dt, generator=gen) for s in shapes]
+    plain = _run(problem, "conv_fsplit=0,conv_parts=0", det, g, tensors, monkeypatch)
+    small = _run(problem, tune, det, g, tensors, monkeypatch)
+    tol = 1e-12 if dt == torch.float64 else 1e-5
+    for i, (got, want) in enumerate(zip(small, plain)):
+        scale = max(float(want.abs().max()), 1e-30)
+        assert float((got - want).abs().max()) / scale <= tol, (name, i)
+    # results per edge do not depend on which position walks the edge
+    assert torch.equal(small[2], plain[2]) and torch.equal(small[3], plain[3])
