@@ -2624,13 +2624,17 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
             blk_x = ex.emit_conv_forward(s, G_x, True, t["conv_pipe_f"] if pipe_x else 0, waves_x,
                                          xcd, bool(t["conv_tra"]), name="backward_dx")
             descs.append((rt.ROLE_CONV_BACKWARD_DX, "backward_dx", blk_x, G_x, 0, xcd))
+            s("}  // namespace oeq_dx")
             n = t["conv_fsplit"] if t["conv_fsplit"] >= 0 else split_waves(ex.NCH, waves_x)
             if n > 1 and not kahan:
                 splits["backward_dx_split"] = n
+                s("namespace oeq_dx_split {")
+                ex.emit_structs(s)
+                ex.emit_forward_cores(s, preloaded=True)
                 blk_xs = ex.emit_conv_forward(s, 1, True, t["conv_pipe_f"] if pipe_x else 0, waves_x, xcd,
                                               bool(t["conv_tra"]), name="backward_dx_split", split=n)
+                s("}  // namespace oeq_dx_split")
                 descs.append((rt.ROLE_CONV_BACKWARD_DX_SPLIT, "backward_dx_split", blk_xs, 1, 0, xcd))
-            s("}  // namespace oeq_dx")
         from . import uvu_double
         if t["conv_dd"] and uvu_double.supported(low, conv=True):
             descs += uvu_double.add_conv_kernels(s, low, em, t, xcd, G_b, compute_units, kahan, splits)
