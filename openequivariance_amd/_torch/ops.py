@@ -1,4 +1,6 @@
-"""PyTorch custom ops over the C ABI.
+"""PyTorch custom ops over the C ABI: kernel sets by description, the index of an edge list, fake kernels, autocast and
+the second-order routes. The ops themselves, with their autograd, are in ``csrc/oeq_torch.cpp``, which calls back into
+this file for what is rare or needs the code generator.
 
 Stand in for the reference's native op library
 (openequivariance/openequivariance/extension/torch_core.hpp:274-644:
@@ -35,8 +37,28 @@ from typing import Dict, List, Optional, Tuple
 import torch
 
 from .. import runtime as rt
+from . import native
 
-_registry: Dict[int, "KernelEntry"] = {}
+_native = native.load()
+
+
+class _Registry(dict):
+    """Kernel sets by id. What leaves it leaves the native ops' table as well."""
+
+    def pop(self, kid, *default):
+        _native.forget_entry(kid)
+        return super().pop(kid, *default)
+
+    def __delitem__(self, kid):
+        _native.forget_entry(kid)
+        super().__delitem__(kid)
+
+    def clear(self):
+        for kid in list(self):
+            del self[kid]
+
+
+_registry: Dict[int, "KernelEntry"] = _Registry()
 _registry_lock = threading.RLock()
 
 
@@ -178,100 +200,48 @@ def get_entry(kid: int, spec: Optional[torch.Tensor] = None) -> KernelEntry:
     return _registry[kid]
 
 
-_DTYPE_CODE = {torch.float32: 1, torch.float64: 2, torch.int32: 3, torch.int64: 4, torch.uint8: 5}
-
-
-def check_tensor(t: torch.Tensor, shape: List[int], dtype: torch.dtype, name: str):
-    """torch_core.hpp:109-134."""
-    if t.dim() != len(shape) or any(int(a) != int(b) for a, b in zip(t.shape, shape)):
-        raise RuntimeError(
-            f"Shape mismatch for tensor '{name}'. Expected: {list(shape)}. Got: {list(t.shape)}"
-        )
-    if not t.is_cuda:
-        raise RuntimeError(f"Tensor '{name}' is not on the GPU.")
-    if t.dtype != dtype:
-        raise RuntimeError(
-            f"Dtype mismatch for tensor '{name}'. Expected: {_DTYPE_CODE.get(dtype, dtype)}. "
-            f"Got: {_DTYPE_CODE.get(t.dtype, t.dtype)}"
-        )
-
-
 def _stream() -> int:
     return torch.cuda.current_stream().cuda_stream
 
 
-def _wshape(e: KernelEntry, n: int) -> List[int]:
-    return [e.WN] if e.shared else [n, e.WN]
+def _resolve(kid: int, spec: Optional[torch.Tensor]):
+    """Called by the native ops for an id they have not seen: builds the kernel set and hands over its handle."""
+    e = get_entry(kid, spec)
+    plain = not e.factored and not e.unfused
+    dims = e.kernels().dims if plain else {}
+    walk = _walk_dims(e) if not e.unfused else {}
+    conv = "order_hops" in walk
+    atomic = conv and not e.deterministic and walk["deterministic"] == rt.CONV_ATOMIC
+    _native.register_entry(kid, dict(
+        handle=e.kernels().handle.value if plain else 0, L1=e.L1, L2=e.L2, L3=e.L3, WN=e.WN, shared=bool(e.shared),
+        deterministic=bool(e.deterministic), double=e.dtype == torch.float64, mode=dims.get("deterministic", 0),
+        dx_mode=dims.get("dx_mode", 0), native=plain, alert_forward=atomic,
+        alert_backward=atomic or (conv and not e.deterministic and walk.get("dx_mode", 0) == rt.DX_ATOMIC),
+        second_order_kid=e.second_order_kid or 0, owner=e))
 
 
 # ---------------------------------------------------------------------------
 # batch tensor product
 # ---------------------------------------------------------------------------
 
-
-@torch.library.custom_op("oeq_amd::tp_forward", mutates_args=(), device_types="cuda")
-def tp_forward(L1_in: torch.Tensor, L2_in: torch.Tensor, W: torch.Tensor, kid: int,
-               spec: Optional[torch.Tensor] = None) -> torch.Tensor:
-    e = get_entry(kid, spec)
-    n = L1_in.shape[0] if L1_in.dim() > 0 else -1
-    check_tensor(L1_in, [n, e.L1], e.dtype, "L1_in")
-    check_tensor(L2_in, [n, e.L2], e.dtype, "L2_in")
-    check_tensor(W, _wshape(e, n), e.dtype, "W")
-    x, y, w = L1_in.contiguous(), L2_in.contiguous(), W.contiguous()
-    out = x.new_empty((n, e.L3))
-    with torch.cuda.device(x.device):
-        e.kernels().tp_forward(n, x.data_ptr(), y.data_ptr(), w.data_ptr(), out.data_ptr(), _stream())
-    return out
+# (overloads, not packets: a call then goes straight to the dispatcher)
+tp_forward = torch.ops.oeq_amd.tp_forward.default
+tp_backward = torch.ops.oeq_amd.tp_backward.default
+tp_double_backward = torch.ops.oeq_amd.tp_double_backward.default
+conv_forward = torch.ops.oeq_amd.conv_forward.default
+conv_backward = torch.ops.oeq_amd.conv_backward.default
+conv_double_backward = torch.ops.oeq_amd.conv_double_backward.default
 
 
-@tp_forward.register_fake
+@torch.library.register_fake("oeq_amd::tp_forward")
 def _(L1_in, L2_in, W, kid, spec=None):
     e = get_entry(kid, spec)
     return L1_in.new_empty((L1_in.shape[0], e.L3))
 
 
-@torch.library.custom_op("oeq_amd::tp_backward", mutates_args=(), device_types="cuda")
-def tp_backward(L1_in: torch.Tensor, L2_in: torch.Tensor, W: torch.Tensor, L3_grad: torch.Tensor,
-                kid: int, spec: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    e = get_entry(kid, spec)
-    n = L1_in.shape[0] if L1_in.dim() > 0 else -1
-    check_tensor(L1_in, [n, e.L1], e.dtype, "L1_in")
-    check_tensor(L2_in, [n, e.L2], e.dtype, "L2_in")
-    check_tensor(W, _wshape(e, n), e.dtype, "W")
-    check_tensor(L3_grad, [n, e.L3], e.dtype, "L3_grad")
-    x, y, w, g = L1_in.contiguous(), L2_in.contiguous(), W.contiguous(), L3_grad.contiguous()
-    dx, dy, dw = torch.empty_like(x), torch.empty_like(y), torch.empty_like(w)
-    with torch.cuda.device(x.device):
-        ks = e.kernels()
-        nb = ks.tp_backward_workspace_bytes(n)
-        ws = torch.empty(max(nb, 1), dtype=torch.uint8, device=x.device)
-        ks.tp_backward(n, x.data_ptr(), dx.data_ptr(), y.data_ptr(), dy.data_ptr(), w.data_ptr(), dw.data_ptr(),
-                       g.data_ptr(), ws.data_ptr() if nb else 0, nb, _stream())
-    return dx, dy, dw
-
-
-@tp_backward.register_fake
+@torch.library.register_fake("oeq_amd::tp_backward")
 def _(L1_in, L2_in, W, L3_grad, kid, spec=None):
     return torch.empty_like(L1_in), torch.empty_like(L2_in), torch.empty_like(W)
-
-
-def _tp_fwd_setup(ctx, inputs, output):
-    ctx.kid, ctx.spec = inputs[3], inputs[4]
-    ctx.save_for_backward(inputs[0], inputs[1], inputs[2])
-
-
-def _tp_fwd_backward(ctx, grad):
-    x, y, w = ctx.saved_tensors
-    dx, dy, dw = tp_backward(x, y, w, grad, ctx.kid, ctx.spec)
-    return dx, dy, dw, None, None
-
-
-tp_forward.register_autograd(_tp_fwd_backward, setup_context=_tp_fwd_setup)
-
-
-def _tp_bwd_setup(ctx, inputs, output):
-    ctx.kid, ctx.spec = inputs[4], inputs[5]
-    ctx.save_for_backward(inputs[0], inputs[1], inputs[2], inputs[3])
 
 
 def _sum2(a, b):
@@ -326,53 +296,19 @@ def _zeros_if_none(t, like):
     return torch.zeros_like(like) if t is None else t
 
 
-@torch.library.custom_op("oeq_amd::tp_double_backward", mutates_args=(), device_types="cuda")
-def tp_double_backward(L1_in: torch.Tensor, L2_in: torch.Tensor, W: torch.Tensor, L3_grad: torch.Tensor,
-                       L1_dgrad: torch.Tensor, L2_dgrad: torch.Tensor, W_dgrad: torch.Tensor,
-                       kid: int, spec: Optional[torch.Tensor] = None
-                       ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
-    """(L1_grad, L2_grad, W_grad, L3_dgrad): the op of the reference's jit_tp_double_backward
-    (extension/torch_core.hpp:357-420)."""
-    e = get_entry(kid, spec)
-    n = L1_in.shape[0] if L1_in.dim() > 0 else -1
-    for t, name in ((L1_in, "L1_in"), (L1_dgrad, "L1_dgrad")):
-        check_tensor(t, [n, e.L1], e.dtype, name)
-    for t, name in ((L2_in, "L2_in"), (L2_dgrad, "L2_dgrad")):
-        check_tensor(t, [n, e.L2], e.dtype, name)
-    for t, name in ((W, "W"), (W_dgrad, "W_dgrad")):
-        check_tensor(t, _wshape(e, n), e.dtype, name)
-    check_tensor(L3_grad, [n, e.L3], e.dtype, "L3_grad")
-    x, y, w, g = L1_in.contiguous(), L2_in.contiguous(), W.contiguous(), L3_grad.contiguous()
-    a, b, c = L1_dgrad.contiguous(), L2_dgrad.contiguous(), W_dgrad.contiguous()
-    dx, dy, dw, gg = torch.empty_like(x), torch.empty_like(y), torch.empty_like(w), torch.empty_like(g)
-    with torch.cuda.device(x.device):
-        ks = e.kernels()
-        nb = ks.tp_double_backward_workspace_bytes(n)
-        ws = torch.empty(max(nb, 1), dtype=torch.uint8, device=x.device)
-        ks.tp_double_backward(n, x.data_ptr(), y.data_ptr(), w.data_ptr(), g.data_ptr(), a.data_ptr(),
-                              b.data_ptr(), c.data_ptr(), dx.data_ptr(), dy.data_ptr(), dw.data_ptr(),
-                              gg.data_ptr(), ws.data_ptr(), nb, _stream())
-    return dx, dy, dw, gg
-
-
-@tp_double_backward.register_fake
+@torch.library.register_fake("oeq_amd::tp_double_backward")
 def _(L1_in, L2_in, W, L3_grad, L1_dgrad, L2_dgrad, W_dgrad, kid, spec=None):
     return torch.empty_like(L1_in), torch.empty_like(L2_in), torch.empty_like(W), torch.empty_like(L3_grad)
 
 
-def _tp_bwd_backward(ctx, ddx, ddy, ddw):
-    x, y, w, g = ctx.saved_tensors
-    kid, spec = ctx.kid, ctx.spec
+def _tp_second_order(operands, cotangents, kid, spec):
+    """Backward of ``tp_backward``: gradients with respect to x, y, w and g."""
+    (x, y, w, g), (ddx, ddy, ddw) = operands, cotangents
     if _use_fused(kid, spec, ddx, ddy, ddw):
-        dx, dy, dw, gg = tp_double_backward(x, y, w, g, _zeros_if_none(ddx, x), _zeros_if_none(ddy, y),
-                                            _zeros_if_none(ddw, w), kid, spec)
-        return dx, dy, dw, gg, None, None
-    dx, dy, dw, gg = _second_order(lambda a, b, c: tp_forward(a, b, c, kid, spec),
-                                   lambda a, b, c, d: tp_backward(a, b, c, d, kid, spec), x, y, w, g, ddx, ddy, ddw)
-    return dx, dy, dw, gg, None, None
-
-
-tp_backward.register_autograd(_tp_bwd_backward, setup_context=_tp_bwd_setup)
+        return tp_double_backward(x, y, w, g, _zeros_if_none(ddx, x), _zeros_if_none(ddy, y),
+                                  _zeros_if_none(ddw, w), kid, spec)
+    return _second_order(lambda a, b, c: tp_forward(a, b, c, kid, spec),
+                         lambda a, b, c, d: tp_backward(a, b, c, d, kid, spec), x, y, w, g, ddx, ddy, ddw)
 
 
 # ---------------------------------------------------------------------------
@@ -421,36 +357,9 @@ def _walk_dims(e: KernelEntry) -> dict:
     return (get_entry(e.factored[0]) if e.factored else e).kernels().dims
 
 
-def _conv_checks(e: KernelEntry, L1_in, L2_in, W, rows, cols, perm, L3_grad=None):
-    nodes = L1_in.shape[0] if L1_in.dim() > 0 else -1
-    nnz = rows.shape[0] if rows.dim() > 0 else -1
-    check_tensor(L1_in, [nodes, e.L1], e.dtype, "L1_in")
-    check_tensor(L2_in, [nnz, e.L2], e.dtype, "L2_in")
-    check_tensor(W, _wshape(e, nnz), e.dtype, "W")
-    if L3_grad is not None:
-        check_tensor(L3_grad, [nodes, e.L3], e.dtype, "L3_grad")
-    check_tensor(rows, [nnz], torch.int64, "rows")
-    check_tensor(cols, [nnz], torch.int64, "cols")
-    if e.deterministic:
-        check_tensor(perm, [nnz], torch.int64, "transpose perm")
+def _check_edges(nodes, rows, cols, perm, deterministic):
     if _check_indices_enabled():
-        check_edge_list(nodes, rows, cols, perm if e.deterministic else None, bool(e.deterministic))
-    if e.deterministic:
-        pass
-    elif (torch.are_deterministic_algorithms_enabled() and not e.unfused
-          and (_walk_dims(e)["deterministic"] == rt.CONV_ATOMIC
-               or (L3_grad is not None and _walk_dims(e).get("dx_mode", 0) == rt.DX_ATOMIC))):
-        # counterpart of at::globalContext().alertNotDeterministic (torch_core.hpp:448) for the calls that
-        # use float atomics: the backward of deterministic=False (sender gradients), and both directions
-        # of the float-atomics kernels. The grouped forward sums in a fixed order and needs no alert.
-        msg = ("OpenEquivariance_conv_atomic does not have a deterministic implementation, but you set "
-               "'torch.use_deterministic_algorithms(True)'. Use TensorProductConv(..., deterministic=True).")
-        if torch.is_deterministic_algorithms_warn_only_enabled():
-            import warnings
-            warnings.warn(msg)
-        else:
-            raise RuntimeError(msg)
-    return nodes, nnz
+        check_edge_list(nodes, rows, cols, perm, deterministic)
 
 
 # ---------------------------------------------------------------------------
@@ -518,6 +427,13 @@ def _conv_index(ks, nodes: int, nnz: int, r: torch.Tensor, c: torch.Tensor, p: O
                                  "refs": (r, c, p)})
             del _index_cache[:-INDEX_CACHE_ENTRIES]
     return index, sender_side
+
+
+def _native_index(kid: int, nodes: int, nnz: int, r, c, p, need_sender_side: bool):
+    """Called by the native convolutions: the (optionally checked) edge list's index and its sender_side flag."""
+    e = _registry[kid]
+    _check_edges(nodes, r, c, p, bool(e.deterministic))
+    return _conv_index(e.kernels(), nodes, nnz, r, c, p, need_sender_side)
 
 
 def _segment_sum(ks, src: torch.Tensor, n_segments: int, keys: torch.Tensor, perm: Optional[torch.Tensor]):
@@ -608,116 +524,33 @@ def _factored_backward(e: KernelEntry, x, y, w, g, r, c, p):
     return dx, dy, dw
 
 
-@torch.library.custom_op("oeq_amd::conv_forward", mutates_args=(), device_types="cuda")
-def conv_forward(L1_in: torch.Tensor, L2_in: torch.Tensor, W: torch.Tensor, rows: torch.Tensor,
-                 cols: torch.Tensor, transpose_perm: torch.Tensor, kid: int,
-                 spec: Optional[torch.Tensor] = None) -> torch.Tensor:
-    e = get_entry(kid, spec)
-    nodes, nnz = _conv_checks(e, L1_in, L2_in, W, rows, cols, transpose_perm)
-    x, y, w = L1_in.contiguous(), L2_in.contiguous(), W.contiguous()
-    r, c = rows.contiguous(), cols.contiguous()
+# The convolutions without fused kernels, called by the native ops with checked, contiguous operands.
+
+
+def _composed_forward(x, y, w, r, c, p, kid):
+    e = _registry[kid]
+    nodes, nnz = x.shape[0], r.shape[0]
+    _check_edges(nodes, r, c, p if e.deterministic else None, bool(e.deterministic))
     if e.factored:
-        return _factored_forward(e, x, y, w, r, c, transpose_perm)
-    if e.unfused:
-        with torch.cuda.device(x.device):
-            return _unfused_forward(e, e.kernels(), x, y, w, r, c, nodes, nnz)
-    out = x.new_empty((nodes, e.L3))
+        return _factored_forward(e, x, y, w, r, c, p)
     with torch.cuda.device(x.device):
-        ks = e.kernels()
-        if ks.dims["deterministic"] == rt.CONV_ATOMIC or nodes == 0 or nnz == 0:
-            ks.conv_forward(nodes, nnz, x.data_ptr(), y.data_ptr(), w.data_ptr(), out.data_ptr(), r.data_ptr(),
-                            c.data_ptr(), 0, 0, _stream())
-        else:
-            perm = transpose_perm.contiguous() if e.deterministic else None
-            # the forward walk needs the receiver side only; where the backward pass will want the edges grouped
-            # by sender as well, both are built now, so that one index serves the whole step
-            both = ks.dims["deterministic"] == rt.CONV_GROUPED and ks.dims.get("dx_mode", 0) != rt.DX_ATOMIC
-            index, side = _conv_index(ks, nodes, nnz, r, c, perm, both)
-            nb = ks.conv_forward_scratch_bytes(nodes, nnz)
-            ws = torch.empty(max(nb, 1), dtype=torch.uint8, device=x.device)
-            ks.conv_forward_indexed(nodes, nnz, x.data_ptr(), y.data_ptr(), w.data_ptr(), out.data_ptr(), r.data_ptr(),
-                                    c.data_ptr(), index.data_ptr(), index.numel(), side, ws.data_ptr() if nb else 0, nb,
-                                    _stream())
-    return out
+        return _unfused_forward(e, e.kernels(), x, y, w, r, c, nodes, nnz)
 
 
-@conv_forward.register_fake
-def _(L1_in, L2_in, W, rows, cols, transpose_perm, kid, spec=None):
-    e = get_entry(kid, spec)
-    return L1_in.new_empty((L1_in.shape[0], e.L3))
-
-
-@torch.library.custom_op("oeq_amd::conv_backward", mutates_args=(), device_types="cuda")
-def conv_backward(L1_in: torch.Tensor, L2_in: torch.Tensor, W: torch.Tensor, L3_grad: torch.Tensor,
-                  rows: torch.Tensor, cols: torch.Tensor, transpose_perm: torch.Tensor,
-                  kid: int, spec: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    e = get_entry(kid, spec)
-    nodes, nnz = _conv_checks(e, L1_in, L2_in, W, rows, cols, transpose_perm, L3_grad)
-    x, y, w, g = L1_in.contiguous(), L2_in.contiguous(), W.contiguous(), L3_grad.contiguous()
-    r, c, p = rows.contiguous(), cols.contiguous(), transpose_perm.contiguous()
+def _composed_backward(x, y, w, g, r, c, p, kid):
+    e = _registry[kid]
+    nodes, nnz = x.shape[0], r.shape[0]
+    _check_edges(nodes, r, c, p if e.deterministic else None, bool(e.deterministic))
     if e.factored:
         return _factored_backward(e, x, y, w, g, r, c, p)
-    if e.unfused:
-        with torch.cuda.device(x.device):
-            return _unfused_backward(e, e.kernels(), x, y, w, g, r, c, p, nodes, nnz)
-    dx, dy, dw = torch.empty_like(x), torch.empty_like(y), torch.empty_like(w)
     with torch.cuda.device(x.device):
-        ks = e.kernels()
-        pp = p.data_ptr() if e.deterministic else 0
-        if ks.dims["deterministic"] == rt.CONV_ATOMIC or nodes == 0 or nnz == 0:
-            ks.conv_backward(nodes, nnz, x.data_ptr(), dx.data_ptr(), y.data_ptr(), dy.data_ptr(), w.data_ptr(),
-                             dw.data_ptr(), g.data_ptr(), r.data_ptr(), c.data_ptr(), pp, 0, 0, _stream())
-        else:
-            terms = ks.dims.get("dx_mode", 0) != rt.DX_ATOMIC
-            index, side = _conv_index(ks, nodes, nnz, r, c, p if e.deterministic else None, terms)
-            nb = ks.conv_backward_scratch_bytes(nodes, nnz)
-            ws = torch.empty(max(nb, 1), dtype=torch.uint8, device=x.device)
-            ks.conv_backward_indexed(nodes, nnz, x.data_ptr(), dx.data_ptr(), y.data_ptr(), dy.data_ptr(), w.data_ptr(),
-                                     dw.data_ptr(), g.data_ptr(), r.data_ptr(), c.data_ptr(), pp, index.data_ptr(),
-                                     index.numel(), side, ws.data_ptr() if nb else 0, nb, _stream())
-    return dx, dy, dw
+        return _unfused_backward(e, e.kernels(), x, y, w, g, r, c, p, nodes, nnz)
 
 
-@conv_backward.register_fake
-def _(L1_in, L2_in, W, L3_grad, rows, cols, transpose_perm, kid, spec=None):
-    return torch.empty_like(L1_in), torch.empty_like(L2_in), torch.empty_like(W)
-
-
-def _conv_fwd_setup(ctx, inputs, output):
-    ctx.kid, ctx.spec = inputs[6], inputs[7]
-    ctx.save_for_backward(*inputs[:6])
-
-
-def _conv_fwd_backward(ctx, grad):
-    x, y, w, rows, cols, perm = ctx.saved_tensors
-    dx, dy, dw = conv_backward(x, y, w, grad, rows, cols, perm, ctx.kid, ctx.spec)
-    return dx, dy, dw, None, None, None, None, None
-
-
-conv_forward.register_autograd(_conv_fwd_backward, setup_context=_conv_fwd_setup)
-
-
-def _conv_bwd_setup(ctx, inputs, output):
-    ctx.kid, ctx.spec = inputs[7], inputs[8]
-    ctx.save_for_backward(*inputs[:7])
-
-
-@torch.library.custom_op("oeq_amd::conv_double_backward", mutates_args=(), device_types="cuda")
-def conv_double_backward(L1_in: torch.Tensor, L2_in: torch.Tensor, W: torch.Tensor, L3_grad: torch.Tensor,
-                         L1_dgrad: torch.Tensor, L2_dgrad: torch.Tensor, W_dgrad: torch.Tensor,
-                         rows: torch.Tensor, cols: torch.Tensor, transpose_perm: torch.Tensor,
-                         kid: int, spec: Optional[torch.Tensor] = None
-                         ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
-    """(L1_grad, L2_grad, W_grad, L3_dgrad): the op of the reference's jit_conv_double_backward
-    (extension/torch_core.hpp:544-625)."""
-    e = get_entry(kid, spec)
-    if e.second_order_kid is not None:
-        e = get_entry(e.second_order_kid)
-    nodes, nnz = _conv_checks(e, L1_in, L2_in, W, rows, cols, transpose_perm, L3_grad)
-    _conv_checks(e, L1_dgrad, L2_dgrad, W_dgrad, rows, cols, transpose_perm)
-    x, y, w, g = L1_in.contiguous(), L2_in.contiguous(), W.contiguous(), L3_grad.contiguous()
-    a, b, c = L1_dgrad.contiguous(), L2_dgrad.contiguous(), W_dgrad.contiguous()
-    r, cc, p = rows.contiguous(), cols.contiguous(), transpose_perm.contiguous()
+def _composed_double_backward(x, y, w, g, a, b, c, r, cc, p, kid):
+    e = _registry[kid]
+    nodes, nnz = x.shape[0], r.shape[0]
+    _check_edges(nodes, r, cc, p if e.deterministic else None, bool(e.deterministic))
     if e.factored:
         # the map is linear in each of X, Y, W: its second-order pass is a sum of first-order calls, each of
         # them the cheap factored form (one channel mix per node)
@@ -725,58 +558,45 @@ def conv_double_backward(L1_in: torch.Tensor, L2_in: torch.Tensor, W: torch.Tens
             return _second_order(lambda p1, q1, r1: _factored_forward(e, p1, q1, r1, r, cc, p),
                                  lambda p1, q1, r1, s1: _factored_backward(e, p1, q1, r1, s1, r, cc, p),
                                  x, y, w, g, a, b, c)
-    if e.unfused:
-        with torch.cuda.device(x.device):
-            return _unfused_double_backward(e, e.kernels(), x, y, w, g, a, b, c, r, cc, p, nodes, nnz)
-    dx, dy, dw, gg = torch.empty_like(x), torch.empty_like(y), torch.empty_like(w), torch.empty_like(g)
     with torch.cuda.device(x.device):
-        ks = e.kernels()
-        pp = p.data_ptr() if e.deterministic else 0
-        if nodes == 0 or nnz == 0:
-            ks.conv_double_backward(nodes, nnz, x.data_ptr(), y.data_ptr(), w.data_ptr(), g.data_ptr(), a.data_ptr(),
-                                    b.data_ptr(), c.data_ptr(), dx.data_ptr(), dy.data_ptr(), dw.data_ptr(),
-                                    gg.data_ptr(), r.data_ptr(), cc.data_ptr(), pp, 0, 0, _stream())
-        else:
-            index, _side = _conv_index(ks, nodes, nnz, r, cc, p if e.deterministic else None, True)
-            nb = ks.conv_double_backward_scratch_bytes(nodes, nnz)
-            ws = torch.empty(max(nb, 1), dtype=torch.uint8, device=x.device)
-            ks.conv_double_backward_indexed(nodes, nnz, x.data_ptr(), y.data_ptr(), w.data_ptr(), g.data_ptr(),
-                                            a.data_ptr(), b.data_ptr(), c.data_ptr(), dx.data_ptr(), dy.data_ptr(),
-                                            dw.data_ptr(), gg.data_ptr(), r.data_ptr(), cc.data_ptr(), pp,
-                                            index.data_ptr(), index.numel(), ws.data_ptr() if nb else 0, nb, _stream())
-    return dx, dy, dw, gg
+        return _unfused_double_backward(e, e.kernels(), x, y, w, g, a, b, c, r, cc, p, nodes, nnz)
 
 
-@conv_double_backward.register_fake
+@torch.library.register_fake("oeq_amd::conv_forward")
+def _(L1_in, L2_in, W, rows, cols, transpose_perm, kid, spec=None):
+    e = get_entry(kid, spec)
+    return L1_in.new_empty((L1_in.shape[0], e.L3))
+
+
+@torch.library.register_fake("oeq_amd::conv_backward")
+def _(L1_in, L2_in, W, L3_grad, rows, cols, transpose_perm, kid, spec=None):
+    return torch.empty_like(L1_in), torch.empty_like(L2_in), torch.empty_like(W)
+
+
+@torch.library.register_fake("oeq_amd::conv_double_backward")
 def _(L1_in, L2_in, W, L3_grad, L1_dgrad, L2_dgrad, W_dgrad, rows, cols, transpose_perm, kid, spec=None):
     return torch.empty_like(L1_in), torch.empty_like(L2_in), torch.empty_like(W), torch.empty_like(L3_grad)
 
 
-def _conv_bwd_backward(ctx, ddx, ddy, ddw):
-    x, y, w, g, rows, cols, perm = ctx.saved_tensors
-    kid, spec = ctx.kid, ctx.spec
+def _conv_second_order(operands, cotangents, kid, spec):
+    """Backward of ``conv_backward``: gradients with respect to x, y, w and g."""
+    (x, y, w, g, rows, cols, perm), (ddx, ddy, ddw) = operands, cotangents
     if _use_fused(kid, spec, ddx, ddy, ddw):
-        dx, dy, dw, gg = conv_double_backward(x, y, w, g, _zeros_if_none(ddx, x), _zeros_if_none(ddy, y),
-                                              _zeros_if_none(ddw, w), rows, cols, perm, kid, spec)
-        return dx, dy, dw, gg, None, None, None, None, None
-    dx, dy, dw, gg = _second_order(lambda a, b, c: conv_forward(a, b, c, rows, cols, perm, kid, spec),
-                                   lambda a, b, c, d: conv_backward(a, b, c, d, rows, cols, perm, kid, spec),
-                                   x, y, w, g, ddx, ddy, ddw)
-    return dx, dy, dw, gg, None, None, None, None, None
+        return conv_double_backward(x, y, w, g, _zeros_if_none(ddx, x), _zeros_if_none(ddy, y),
+                                    _zeros_if_none(ddw, w), rows, cols, perm, kid, spec)
+    return _second_order(lambda a, b, c: conv_forward(a, b, c, rows, cols, perm, kid, spec),
+                         lambda a, b, c, d: conv_backward(a, b, c, d, rows, cols, perm, kid, spec),
+                         x, y, w, g, ddx, ddy, ddw)
 
 
-conv_backward.register_autograd(_conv_bwd_backward, setup_context=_conv_bwd_setup)
+_native.set_callbacks(dict(
+    resolve=_resolve, check_edges=_check_edges, conv_index=_native_index, conv_forward=_composed_forward,
+    conv_backward=_composed_backward, conv_double_backward=_composed_double_backward,
+    tp_second_order=_tp_second_order, conv_second_order=_conv_second_order, error_type=rt.OeqError))
 
 
 # Mixed precision: the kernels are compiled for one dtype; under autocast the
 # ops run in that dtype (cf. the reference's register_autocast to float32,
 # _torch/TensorProduct.py:362-374).
-def _register_autocast():
-    for op in (tp_forward, tp_backward, conv_forward, conv_backward):
-        try:
-            op.register_autocast("cuda", torch.float32)
-        except Exception:  # older/newer torch without this hook: ops still validate dtypes
-            pass
-
-
-_register_autocast()
+for _name in ("tp_forward", "tp_backward", "conv_forward", "conv_backward"):
+    torch.library.register_autocast(f"oeq_amd::{_name}", "cuda", torch.float32)
