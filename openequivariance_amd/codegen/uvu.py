@@ -37,6 +37,7 @@ from .common import Src, fixup_backward_kernel, prelude, utility_kernels
 from .lower import Lowered, Path, float_literal
 
 UNROLL_V_LIMIT = 8
+LDS_LIMIT = 160 * 1024  # bytes a block may declare
 
 
 def _pow2ceil(n: int) -> int:
@@ -1268,6 +1269,17 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
                 if missing:
                     cond = " && ".join([f"chunk == {c}"] + ([f"sg == {sg}"] if segw > 1 else []))
                     s(f"if ({cond}) for (int t = 0; t < {missing}; ++t) __syncthreads();")
+
+    def split_count(self, n: int, pipelined: int) -> int:
+        """How many waves a node's edges can be dealt out to, ``n`` or a half, a quarter ... of it: every wave has an LDS
+        buffer for an edge's operands, and a wide problem's do not all fit a CU (the sender walk of 128x{0e,1o,2e} with
+        l <= 3 harmonics: 31 KB a wave)."""
+        mode = self._edge_mode(pipelined)
+        if (self._edge_mode(2) if mode > 2 else mode) != 2:
+            return n
+        while n > 1 and self.NCH * n * self.stage["floats"] * 4 > LDS_LIMIT:
+            n //= 2
+        return n
 
     def emit_conv_forward(self, s: Src, G: int, deterministic: bool, pipelined: bool, waves_per_eu: int = 0,
                           xcd: int = 1, tr_atomics: bool = True, name: str = "forward", split: int = 1):
@@ -2536,6 +2548,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     splits: Dict[str, int] = {}  # the kernels with a node's edges dealt out to several waves: how many
     if walk and not kahan and not q_fwd:
         n = t["conv_fsplit"] if t["conv_fsplit"] >= 0 else split_waves(em.NCH * em.seg_waves, t["conv_wf"])
+        n = em.split_count(n, t["conv_pipe_f"])
         if n > 1:
             splits["forward_split"] = n
             blk_fs = em.emit_conv_forward(s, 1, True, t["conv_pipe_f"], t["conv_wf"], xcd, bool(t["conv_tra"]),
@@ -2626,6 +2639,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
             descs.append((rt.ROLE_CONV_BACKWARD_DX, "backward_dx", blk_x, G_x, 0, xcd))
             s("}  // namespace oeq_dx")
             n = t["conv_fsplit"] if t["conv_fsplit"] >= 0 else split_waves(ex.NCH, waves_x)
+            n = ex.split_count(n, t["conv_pipe_f"] if pipe_x else 0)
             if n > 1 and not kahan:
                 splits["backward_dx_split"] = n
                 s("namespace oeq_dx_split {")
