@@ -248,6 +248,218 @@ class UvwEmitter:
         s.close()
         return block
 
+    # ------------------------------------------- conv forward, packed lanes
+    # The channel mix of an edge reads its weight row once and does little with it, so its time is how many bytes the
+    # waves keep in flight. A lane per output channel and a load per input channel moves 4 B per lane and leaves the
+    # lanes beyond a narrow block idle (10 channels: 40 B an instruction), behind a chain of edge number, sender, row of
+    # X and LDS tile for every path. Here a lane takes ``vw`` neighbouring channels (16 B) and the lanes left over further
+    # input channels (10 channels: 12 of them, 480 B an instruction; 48: 5, 960 B), their partial sums meeting once per
+    # node; all paths of the segment share one pass over the LDS tile; edge numbers and senders come 64 at a time, and
+    # rows of X and the weights of the next edge are requested as soon as their registers are free.
+    # Forward with 20 edges per node, before / after: DiffDock L=1 (6 928 weights an edge) 3 000 nodes 412 / 293 us
+    # (4.0 / 5.7 TB/s of weights), 800 x 25 238 / 115, 250 x 12 82 / 24; L=2 3 000 nodes 452 / 302; e3tools 3 000 nodes
+    # 418 / 324, 400 x 10 72 / 27. Held to a quarter of a SIMD's registers the same kernel spills (DiffDock 366 us,
+    # e3tools 1 007).
+    PACK_JOBS = 24    # jobs (path, channel of the second operand, 64 input channels) a segment is unrolled for
+    PACK_LDS = 12288  # bytes of a wave's LDS tile (three blocks of four waves to a CU)
+    PACK_WORDS = 96   # 32-bit registers for an edge's weights (e3tools needs 80: with 64 its forward takes 383 us instead
+                      # of 324); segments with more weights stream them through half of that
+
+    def _pack_plan(self, io: int, wc: int):
+        """How the lanes share segment ``io``, channels ``wc`` .. : (vw, lanes per input channel, input channels per
+        instruction, jobs, words per LDS row), a job being (path, v, first input channel, input channels, first LDS row).
+        None: the plain scheme, for segments of so many jobs that their straight-line code or LDS tile would be large."""
+        low, bo = self.low, self.low.out[io]
+        nw = min(64, bo.mul - wc)
+        words = low.elem_size // 4
+        vw = next(n for n in (4, 2, 1) if n == 1 or (nw % n == 0 and n * words <= 4 and n * bo.d * words <= 32))
+        lanes = nw // vw
+        jobs, rows = [], 0
+        for p in (q for q in low.paths if q.io == io):
+            b1 = low.in1[p.i1]
+            for v in range(low.in2[p.i2].mul):
+                for uc in range(0, b1.mul, 64):
+                    jobs.append((p, v, uc, min(64, b1.mul - uc), rows))
+                    rows += bo.d
+        groups = 64 // lanes
+        stride = max([64] + [-(-nu // groups) * groups for *_, nu, _ in jobs])
+        if len(jobs) > self.PACK_JOBS or rows * stride * low.elem_size > self.PACK_LDS or low.L2 > 32:
+            return None
+        return vw, lanes, groups, jobs, stride
+
+    def _emit_packed_segment(self, s: Src, io: int, wc: int, plan, kahan: bool):
+        """The edges e0 .. e1 of a node for one segment, by one wave: see above."""
+        low, bo = self.low, self.low.out[io]
+        vw, lanes, groups, jobs, stride = plan
+        words = low.elem_size // 4
+        xs = sorted({(p.i1, uc) for p, v, uc, nu, r in jobs})
+        ys = sorted({low.in2[p.i2].off + v * low.in2[p.i2].d + j for p, v, *_ in jobs for _, j, _, _ in p.nnz})
+        steps = [(n, it) for n, job in enumerate(jobs) for it in range(-(-job[3] // groups))]
+        resident = len(steps) * vw * words <= self.PACK_WORDS
+
+        def load_x(row: str):
+            s(f"const T* xrow = L1_in + (i64){row} * {low.L1};")
+            for i1, uc in xs:
+                b1 = low.in1[i1]
+                u = "lane" if uc + 64 <= b1.mul else f"(lane < {b1.mul - uc} ? lane : {b1.mul - uc - 1})"
+                for i in range(b1.d):
+                    s(f"x{i1}_{uc}[{i}] = *oeq_at(xrow + {b1.off + uc * b1.d + i}, (unsigned){u} * {b1.d * low.elem_size}u);")
+
+        def load_y(row: str):
+            s(f"const T* yrow = L2_in + (i64){row} * {low.L2};")
+            for y in ys:
+                s(f"yv{y} = yrow[{y}];")
+
+        def load_w(k: int, first: int = 0):
+            """weights of step ``k`` into its registers (those of step ``first`` are the first)"""
+            n, it = steps[k]
+            p, v, uc, nu, _ = jobs[n]
+            mul2 = low.in2[p.i2].mul
+            base = p.woff + (uc * mul2 + v) * bo.mul + wc + it * groups * mul2 * bo.mul
+            left = nu - it * groups  # (of the last step's input channels those that are there)
+            u = "gl" if left >= groups else f"(gl < {left} ? gl : {left - 1})"
+            s(f"wr[{k - first}] = *(const oeq_wvec{vw}_any*)oeq_at(wrow + {base}, (unsigned)({u} * "
+              f"{mul2 * bo.mul} + wl) * {low.elem_size}u);")
+
+        def use_w(k: int, acc: str, first: int = 0):
+            n, it = steps[k]
+            p, v, uc, nu, r0 = jobs[n]
+            s.open("")
+            if (it + 1) * groups > nu:  # no product of a channel that is not there: the weight read in its place may be infinite
+                s(f"const bool in = {it * groups} + gl < {nu};")
+                weight = lambda q: f"(in ? wr[{k - first}][{q}] : T(0))"
+            else:
+                weight = lambda q: f"wr[{k - first}][{q}]"
+            for c in range(bo.d):
+                s(f"const T t{c} = s_row[{(r0 + c) * stride + it * groups} + gl];")
+            for q in range(vw):
+                s(f"const T w{q} = {weight(q)};")
+                for c in range(bo.d):
+                    s(f"{acc}[{q * bo.d + c}] += w{q} * t{c};")
+            s.close()
+
+        # (the lane number through an empty asm statement: the compiler would otherwise compute every segment's lane
+        # offsets before the loop over the nodes and keep them all, hundreds of registers, through each segment)
+        s("int lane = oeq_lane();")
+        s('asm volatile("" : "+v"(lane));')
+        s(f"const int gl = lane / {lanes} < {groups} ? lane / {lanes} : 0, wl = (lane % {lanes}) * {vw};")
+        s(f"T* s_row = s_t[wave];")
+        # input channels past the 64 lanes' (the last step of a job): zeros
+        if stride > 64:
+            s(f"for (int r = 0; r < {len(jobs) * bo.d}; ++r) for (int c = 64 + lane; c < {stride}; c += 64) "
+              f"s_row[r * {stride} + c] = T(0);")
+        n_acc = vw * bo.d
+        s(f"T acc[{n_acc}];")
+        s(f"for (int q = 0; q < {n_acc}; ++q) acc[q] = T(0);")
+        if kahan:
+            s(f"T comp[{n_acc}];")
+            s(f"for (int q = 0; q < {n_acc}; ++q) comp[q] = T(0);")
+        # (everything the walk carries lives inside this branch: initialised on one path only, the compiler would carry it
+        # round the loop over the nodes)
+        s.open("if (e0 < e1)")
+        for i1, uc in xs:
+            s(f"T x{i1}_{uc}[{low.in1[i1].d}];")
+        for y in ys:
+            s(f"T yv{y};")
+        if resident:
+            s(f"oeq_wvec{vw} wr[{len(steps)}];")
+        s("int el = 0, sl = 0;")  # edge number and sender of position (64-position group of pos) + lane
+        edge = f"__builtin_amdgcn_readlane(el, (int)(pos - e0) & 63)"
+        sender = f"__builtin_amdgcn_readlane(sl, (int)(pos - e0) & 63)"
+        shared = low.shared_weights
+        s.open("auto next = [&](i64 pos)")
+        s.open("if (((pos - e0) & 63) == 0)")
+        s("const i64 pl = pos + lane < e1 ? pos + lane : e1 - 1;")
+        s("el = (int)oeq_idx(OEQ_EDGE(pl), nnz);")
+        s("sl = (int)oeq_idx(cols[el], node_count);")
+        s.close()
+        s.close(";")
+        s.open("auto request_xy = [&](i64 pos)")
+        load_x(sender)
+        load_y(edge)
+        s.close(";")
+        s.open("auto request_w = [&](i64 pos)")
+        s(f"const T* wrow = W{'' if shared else f' + (i64){edge} * {low.WN}'};")
+        if resident:
+            for k in range(len(steps)):
+                load_w(k)
+        s.close(";")
+        s("next(e0);")
+        s("request_xy(e0);")
+        if resident:
+            s("request_w(e0);")
+        s.open("for (i64 pos = e0;;)")
+        if not resident:
+            s(f"const T* wrow = W{'' if shared else f' + (i64){edge} * {low.WN}'};")
+        s("oeq_wave_sync();")
+        for n, (p, v, uc, nu, r0) in enumerate(jobs):
+            b1, b2 = low.in1[p.i1], low.in2[p.i2]
+            s.open("")
+            names, started = {}, set()
+            for i, j, k, c in p.nnz:
+                key = (self.lit(abs(c)), j)
+                if key not in names:
+                    names[key] = f"q{len(names)}"
+                    s(f"const T {names[key]} = T({key[0]}) * yv{b2.off + v * b2.d + j};")
+                term = f"{names[key]} * x{p.i1}_{uc}[{i}]"
+                if k not in started:
+                    s(f"T t{k} = {'-' if c < 0 else ''}{term};")
+                    started.add(k)
+                else:
+                    s(f"t{k} {'-=' if c < 0 else '+='} {term};")
+            for k in range(bo.d):
+                val = f"t{k}" if k in started else "T(0)"
+                if nu < 64:
+                    val = f"(lane < {nu} ? {val} : T(0))"
+                s(f"s_row[{(r0 + k) * stride} + lane] = {val};")
+            s.close()
+        s("oeq_wave_sync();")
+        s("const bool more = pos + 1 < e1;")
+        s("const i64 then = more ? pos + 1 : pos;")
+        s("next(then);")
+        s("request_xy(then);")
+        acc = "acc"
+        if kahan:
+            acc = "msg"
+            s(f"T msg[{n_acc}];")
+            s(f"for (int q = 0; q < {n_acc}; ++q) msg[q] = T(0);")
+        if resident:
+            for k in range(len(steps)):
+                use_w(k, acc)
+        else:
+            per = max(1, self.PACK_WORDS // 2 // (vw * words))
+            for k0 in range(0, len(steps), per):
+                some = range(k0, min(k0 + per, len(steps)))
+                s.open("")
+                s(f"oeq_wvec{vw} wr[{len(some)}];")
+                for k in some:
+                    load_w(k, k0)
+                for k in some:
+                    use_w(k, acc, k0)
+                s.close()
+        if kahan:
+            s(f"for (int q = 0; q < {n_acc}; ++q) {{ const T y = msg[q] - comp[q]; const T t = acc[q] + y; "
+              "comp[q] = (t - acc[q]) - y; acc[q] = t; }")
+        s("if (!more) break;")
+        if resident:
+            s("request_w(then);")
+        s("pos = then;")
+        s.close()
+        s.close()
+        # the groups' partial sums, pairwise
+        step = _pow2ceil(groups) // 2
+        while step:
+            s.open("")
+            s(f"const bool in = lane / {lanes} < {step} && lane / {lanes} + {step} < {groups};")
+            s(f"for (int q = 0; q < {n_acc}; ++q) {{ const T o = __shfl(acc[q], (lane + {step * lanes}) & 63); "
+              "acc[q] += in ? o : T(0); }")
+            s.close()
+            step //= 2
+        s.open(f"if (live && lane < {lanes})")
+        s(f"for (int q = 0; q < {vw}; ++q) for (int c = 0; c < {bo.d}; ++c) "
+          f"zrow[{bo.off} + ({wc} + wl + q) * {bo.d} + c] = acc[q * {bo.d} + c];")
+        s.close()
+
     def emit_conv_forward(self, s: Src, kahan: bool = False, second: bool = False):
         """Fused convolution, forward: the waves of a block share a receiver node's output segments (64
         channels of one output block each, lanes = w) and each keeps its segments in registers over the
@@ -263,6 +475,9 @@ class UvwEmitter:
         wpn = max(1, min(WAVES_PER_BLOCK, len(segs)))  # waves per node
         G = WAVES_PER_BLOCK // wpn
         block = 64 * wpn * G
+        packed = {} if second else {seg: self._pack_plan(*seg) for seg in segs}
+        if not all(packed.values()):
+            packed = {}
         if second:
             s.open(
                 f'extern "C" __global__ __launch_bounds__({block}) void double_backward_A(i64 node_count, i64 nnz, '
@@ -280,7 +495,11 @@ class UvwEmitter:
                 "const i64* __restrict__ rowptr, const i64* __restrict__ eperm, const i64* __restrict__ order"
                 f"{HUB_PARAMS})"
             )
-        s(f"__shared__ T s_t[{wpn * G}][{self.max_d3 * (2 if second else 1)}][64];")
+        if packed:
+            tile = max(len(pl[3]) * low.out[io].d * pl[4] for (io, _), pl in packed.items())
+            s(f"__shared__ T s_t[{wpn * G}][{tile}];")
+        else:
+            s(f"__shared__ T s_t[{wpn * G}][{self.max_d3 * (2 if second else 1)}][64];")
         s("const int lane = oeq_lane();")
         s("const int wave = oeq_wave();")
         s(f"const int g = wave / {wpn}, sg = wave % {wpn};")
@@ -319,6 +538,10 @@ class UvwEmitter:
             bo = low.out[io]
             s(f"// ---- out[{io}]: {bo.mul} x l={bo.l}, channels {wc}..")
             s.open(f"if (sg == {si % wpn})")
+            if packed:
+                self._emit_packed_segment(s, io, wc, packed[(io, wc)], kahan)
+                s.close()
+                continue
             s(f"const int wc = {wc};")
             s("const int w = wc + lane;")
             s(f"T acc[{bo.d}];")
@@ -1019,6 +1242,9 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     s(prelude(low.ctype))
     s(utility_kernels(kahan))
     s("#define OEQ_EDGE(j) (eperm ? eperm[(j)] : (j))")
+    for n in (1, 2, 4):
+        s(f"typedef T oeq_wvec{n} __attribute__((ext_vector_type({n})));")
+        s(f"typedef oeq_wvec{n} oeq_wvec{n}_any __attribute__((aligned(sizeof(T))));")
     blk_f, G_f = em.emit_conv_forward(s, kahan)
     blk_b = em.emit_backward(s, conv=True)
     s(fixup_backward_kernel(low.L1, kahan, True))
