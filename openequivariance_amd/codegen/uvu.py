@@ -2601,6 +2601,12 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
             auto = 9 * low.L1 >= 2 * (low.WN + low.L2 + low.L3) and not low.shared_weights and t["conv_dxm"] < 0
             if (t["conv_dxs"] > 0) or (t["conv_dxs"] < 0 and auto):
                 dx_mode = em.DX_SENDER_WALK
+        if dx_mode == em.DX_ATOMIC and walk and low.elem_size == 4 and t["conv_wb"] == 2 and "conv_wb" not in user_tune:
+            # With the dX terms leaving as atomics a third wave per SIMD pays where the compiler finds the registers
+            # for it (of the zoo's kernels two do, at 176 registers before; step: mace-large 6 001 nodes x 32 edges
+            # 1 357 -> 1 293 us, nequip-uvu 5 000 x 30 284 -> 259; the others' code stays as it is). With the terms
+            # stored and summed in order it does not (mace-large 3 000 x 32 758 / 759 us, 600 x 32 191 / 197).
+            t["conv_wb"] = 23
         blk_b = em.emit_conv_backward(s, walk, G_b, t["conv_pipe_b"], t["conv_wb"], gres, xcd_b,
                                       bool(t["conv_tra"]), dx_mode)
         G_b = em.backward_groups_per_block
