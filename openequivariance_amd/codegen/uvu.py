@@ -2666,7 +2666,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
             (rt.ROLE_GROUP_SCATTER, "oeq_group_scatter", 256, 256, compute_units * 16),
             (rt.ROLE_GROUP_ORDER, "oeq_group_order", 256, 4, compute_units * 32),
             (rt.ROLE_ORDER_HOP, "oeq_order_hop", 256, 256, compute_units * 16),
-            (rt.ROLE_INDEX_SMALL, "oeq_index_small", 1024, 1, 2),
+            (rt.ROLE_INDEX_SMALL, "oeq_index_small", 1024, 1, 32),
             # long edge segments in chunks: the sum of the chunks' rows
             (rt.ROLE_CONV_FIXUP_FORWARD, "fixup_forward", 256, 1, compute_units * 32),
         ]

@@ -1273,7 +1273,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         (rt.ROLE_GROUP_SCATTER, "oeq_group_scatter", 256, 256, cu * 16),
         (rt.ROLE_GROUP_ORDER, "oeq_group_order", 256, 4, cu * 32),
         (rt.ROLE_ORDER_HOP, "oeq_order_hop", 256, 256, cu * 16),
-        (rt.ROLE_INDEX_SMALL, "oeq_index_small", 1024, 1, 2),
+        (rt.ROLE_INDEX_SMALL, "oeq_index_small", 1024, 1, 32),
         (rt.ROLE_CONV_FIXUP_FORWARD, "fixup_forward", 256, 1, cu * 32),
     ]
     t = em.tune

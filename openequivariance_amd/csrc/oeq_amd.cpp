@@ -796,7 +796,8 @@ static int build_index(oeq_kernels* k, const char* who, const IndexLayout& w, in
     if (nnz <= kSmallItems && node_count <= kSmallSegments && k->roles[OEQ_ROLE_INDEX_SMALL].present) {
         int64_t n = nnz, ns = node_count, lim = limit, c = cap;
         void* args[] = {&n, &ns, &lim, &c, &a, &b};
-        rc = k->launch(OEQ_ROLE_INDEX_SMALL, 0, args, stream, b.ptr ? 2u : 1u);
+        const unsigned parts = grouped ? (unsigned)((nnz + 1023) / 1024) : 1u;
+        rc = k->launch(OEQ_ROLE_INDEX_SMALL, 0, args, stream, parts * (b.ptr ? 2u : 1u));
     } else if (grouped) {
         rc = k->group_by_key(nnz, node_count, limit, cap, a, b, stream);
     } else {
