@@ -61,7 +61,11 @@ def _run(problem, tune, det, g, tensors, monkeypatch):
 
 @pytest.mark.parametrize("name", list(PROBLEMS))
 @pytest.mark.parametrize("tune,n,hub", [("", 1, 5), ("", 33, 300), ("conv_fsplit=2,conv_parts=3", 40, 0),
-                                        ("conv_fsmax=100000,conv_parts=16", 700, 600)])
+                                        ("conv_fsmax=100000,conv_parts=16", 700, 600),
+                                        # two waves a node: segments walked whole up to 512 nodes; many parallel edges: in chunks
+                                        ("conv_fsplit=2,conv_fsmax=4000", 512, 700),
+                                        ("conv_fsplit=2,conv_fsmax=4000", 513, 700),
+                                        ("", 3, 900)])
 def test_small_forms_match_the_plain_kernels(name, tune, n, hub, monkeypatch):
     problem = PROBLEMS[name]()
     det = n != 33
