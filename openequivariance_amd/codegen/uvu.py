@@ -1234,6 +1234,7 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
             if not rounds or len(rounds[-1]) == split or sum(low.out[b].d for b in rounds[-1]) + low.out[io].d > limit:
                 rounds.append([])
             rounds[-1].append(io)
+        assert all(sum(low.out[io].d for io in rnd) <= limit for rnd in rounds), "outputs wider than a wave's LDS slice"
         s.open("")
         s(f"T* const mine = s_red + wave * {self.split_stride} + lane;")
         s(f"const T* const first = s_red + (wave - part * {self.NCH * segw}) * {self.split_stride} + lane;")
@@ -1274,14 +1275,24 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
                     cond = " && ".join([f"chunk == {c}"] + ([f"sg == {sg}"] if segw > 1 else []))
                     s(f"if ({cond}) for (int t = 0; t < {missing}; ++t) __syncthreads();")
 
-    def split_count(self, n: int, pipelined: int) -> int:
-        """How many waves a node's edges can be dealt out to, ``n`` or a half, a quarter ... of it: every wave has an LDS
-        buffer for an edge's operands, and a wide problem's do not all fit a CU (the sender walk of 128x{0e,1o,2e} with
-        l <= 3 harmonics: 31 KB a wave)."""
+    def _split_mode(self, pipelined: int) -> int:
         mode = self._edge_mode(pipelined)
-        if (self._edge_mode(2) if mode > 2 else mode) != 2:
-            return n
-        while n > 1 and self.NCH * n * self.stage["floats"] * 4 > LDS_LIMIT:
+        return self._edge_mode(2) if mode > 2 else mode
+
+    def _split_slice(self, staged: bool) -> int:
+        """Elements of a wave's LDS slice for its accumulators: the wave's staging buffer where it has one, and in any
+        case the widest output block (64x0e x 1x4e -> 64x4e: 576 elements beside a staging buffer of 512)."""
+        widest = max(self.low.out[io].d for io in self.used_out)
+        return max(self.stage["floats"] if staged else self.SPLIT_WORDS // self.words * 64, widest * 64)
+
+    def split_count(self, n: int, pipelined: int, segw: int = 1) -> int:
+        """How many waves a node's edges can be dealt out to, ``n`` or a half, a quarter ... of it: every wave has an LDS
+        slice for an edge's operands and its accumulators, and a wide problem's do not all fit a CU (the sender walk of
+        128x{0e,1o,2e} with l <= 3 harmonics: 31 KB a wave)."""
+        wave = self._split_slice(self._split_mode(pipelined) == 2)
+        if self.tr_stores & 1 and self.R == 1:
+            wave += 64 * max(self.low.out[io].d for io in self.used_out)
+        while n > 1 and self.NCH * segw * n * wave * self.low.elem_size > LDS_LIMIT:
             n //= 2
         return n
 
@@ -1300,8 +1311,8 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         # weights two edges ahead: only where the loop body issues no stores or atomics (they share the
         # vector-memory counter with the loads the loop waits for by count)
         mode = self._edge_mode(pipelined if (deterministic or pipelined != 4) else 2)
-        if split > 1 and mode > 2:
-            mode = self._edge_mode(2)
+        if split > 1:
+            mode = self._split_mode(pipelined)
         s.open(
             f'extern "C" __global__ {self._attrs(block, waves_per_eu)} void {name}(i64 node_count, i64 nnz, '
             "const T* __restrict__ L1_in, const T* __restrict__ L2_in, const T* __restrict__ W, "
@@ -1319,6 +1330,8 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
             s("E_t A, B;")
         if mode in (2, 4):
             floats = self.stage["floats"] + (self.stage["nqw"] * 256 if mode == 4 else 0)
+            if split > 1:
+                floats = self._split_slice(True)
             s(f"__shared__ __attribute__((aligned(16))) T s_stage[{self.NCH * G * split}][{floats}];")
             self._emit_stage_offsets(s)
         if mode == 3:
@@ -1367,12 +1380,10 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
             if split > 1:
                 s.open("")
                 s("const int g = 0;")
+                self.split_stride = self._split_slice(mode == 2)
                 if mode == 2:  # (the edge's staging buffers are free by then)
                     s("T* const s_red = &s_stage[0][0];")
-                    self.split_stride = floats
                 else:
-                    widest = max(low.out[io].d for io in self.used_out)
-                    self.split_stride = max(self.SPLIT_WORDS // self.words, widest) * 64
                     s(f"__shared__ T s_red[{block // 64 * self.split_stride}];")
             self._node_loop_open(s, G, xcd)
             barriers: Dict[Tuple[int, int], int] = {}
@@ -2179,6 +2190,8 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
             s("E_t A, B;")
         if mode in (2, 4):
             floats = self.stage["floats"] + (self.stage["nqw"] * 256 if mode == 4 else 0)
+            if split > 1:
+                floats = self._split_slice(True)
             s(f"__shared__ __attribute__((aligned(16))) T s_stage[{self.NCH * G}][{floats}];")
             self._emit_stage_offsets(s)
         if mode == 3:
@@ -2549,7 +2562,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     splits: Dict[str, int] = {}  # the kernels with a node's edges dealt out to several waves: how many
     if walk and not kahan and not q_fwd:
         n = t["conv_fsplit"] if t["conv_fsplit"] >= 0 else split_waves(em.NCH * em.seg_waves, t["conv_wf"])
-        n = em.split_count(n, t["conv_pipe_f"])
+        n = em.split_count(n, t["conv_pipe_f"], em.seg_waves)
         if n > 1:
             splits["forward_split"] = n
             blk_fs = em.emit_conv_forward(s, 1, True, t["conv_pipe_f"], t["conv_wf"], xcd, bool(t["conv_tra"]),

@@ -511,7 +511,7 @@ class DoubleEmitter(UvuEmitter):
             s("const int part = g;")
             s.open("")
             s("const int g = 0;")
-            self.split_stride = max(self.SPLIT_WORDS // self.words, max(low.out[io].d for io in self.used_out)) * 64
+            self.split_stride = self._split_slice(False)
             s(f"__shared__ T s_red[{block // 64 * self.split_stride}];")
         barriers: Dict[Tuple[int, int], int] = {}
         self._node_loop_open(s, G, xcd)
@@ -940,6 +940,7 @@ def add_conv_kernels(s: Src, low: Lowered, base: UvuEmitter, tune: dict, xcd: in
         blk_a = em.emit_conv_double_a(s, G_a, tune.get("dd_wa", 2), xcd, segw)
         descs.append((rt.ROLE_DOUBLE_BACKWARD_A, "double_backward_A", blk_a, G_a, 0, xcd))
         n = tune["conv_fsplit"] if tune["conv_fsplit"] >= 0 else split_waves(em.NCH * segw, tune.get("dd_wa", 2))
+        n = em.split_count(n, 0, segw)
         if n > 1 and not kahan and splits is not None:
             splits["double_backward_A_split"] = n
             blk_as = em.emit_conv_double_a(s, 1, tune.get("dd_wa", 2), xcd, segw, "double_backward_A_split", n)

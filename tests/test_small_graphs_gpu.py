@@ -12,6 +12,9 @@ from openequivariance_amd._torch import ops
 from openequivariance_amd.core import problems as P
 from openequivariance_amd.core.graph import CoordGraph
 
+from gpu_util import err, to_gpu
+from oracle import e3nn_ref as R
+
 pytestmark = pytest.mark.gpu
 
 
@@ -84,3 +87,27 @@ def test_small_forms_match_the_plain_kernels(name, tune, n, hub, monkeypatch):
         assert float((got - want).abs().max()) / scale <= tol, (name, i)
     # results per edge do not depend on which position walks the edge
     assert torch.equal(small[2], plain[2]) and torch.equal(small[3], plain[3])
+
+
+@pytest.mark.parametrize("in1,in2,out", [("64x0e", "1x4e", "64x4e"), ("64x0e", "1x0e+1x2e+1x4e", "64x0e+64x2e+64x4e"),
+                                         ("128x0e", "1x4e", "128x4e"), ("64x0e+64x1o", "1x3o", "64x4e"),
+                                         ("64x4e", "1x4e", "64x0e")])
+@pytest.mark.parametrize("det", [False, True])
+def test_blocks_wider_than_the_staging_buffer(in1, in2, out, det, monkeypatch):
+    """Outputs (last problem: rows of the sender walk) whose 9 components do not fit a wave's staging buffer."""
+    problem = P.ChannelwiseTPP(in1, in2, out)
+    g = _graph(40, 3, 60)
+    rng = np.random.default_rng(1)
+    x, y, w, gr = (rng.normal(size=s).astype(np.float32) for s in (
+        (40, problem.irreps_in1.dim), (g.nnz, problem.irreps_in2.dim), (g.nnz, problem.weight_numel),
+        (40, problem.irreps_out.dim)))
+    monkeypatch.setenv("OEQ_AMD_TUNE", "conv_dxs=1" if in1 == "64x4e" else "")
+    conv = oeq.TensorProductConv(problem, deterministic=det)
+    e = [torch.tensor(a, device="cuda") for a in (g.rows, g.cols, g.transpose_perm)]
+    tx, ty, tw = to_gpu(x, y, w, requires_grad=True)
+    z = conv(tx, ty, tw, *e)
+    z.backward(torch.tensor(gr, device="cuda"))
+    ref = R.Problem.from_spec(problem)
+    want = [R.conv_forward(ref, x, y, w, g.rows, g.cols), *R.conv_backward(ref, x, y, w, gr, g.rows, g.cols)]
+    for got, exp in zip((z, tx.grad, ty.grad, tw.grad), want):
+        assert err(got, exp) <= 1e-5
