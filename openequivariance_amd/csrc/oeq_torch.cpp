@@ -491,6 +491,28 @@ struct ConvBackward : public torch::autograd::Function<ConvBackward> {
     }
 };
 
+// The fused second-order ops are not differentiated themselves: a call that records returns outputs whose backward is
+// an error (without a kernel for the Autograd key torch would warn and leave their part of the gradient out). Third
+// derivatives go through the first-order ops: _tp_second_order and _conv_second_order in _torch/ops.py.
+template <typename Sig, const char* const& name>
+struct NotDifferentiated : public torch::autograd::Function<NotDifferentiated<Sig, name>> {
+    template <typename... Args>
+    static variable_list forward(AutogradContext* ctx, const Args&... args) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        ctx->set_materialize_grads(false);
+        static const auto op = find_op<Sig>(name);
+        auto [dx, dy, dw, gg] = op.call(args...);
+        return {dx, dy, dw, gg};
+    }
+    static variable_list backward(AutogradContext*, variable_list) {
+        TORCH_CHECK(false, "Trying to backward through ", name, " but no autograd formula was registered. Differentiate ",
+                    "the first-order ops with create_graph=True instead.");
+    }
+};
+
+const char* const kTpDoubleBackward = "oeq_amd::tp_double_backward";
+const char* const kConvDoubleBackward = "oeq_amd::conv_double_backward";
+
 template <typename... Ts>
 bool records(const Ts&... ts) {
     return at::GradMode::is_enabled() && (ts.requires_grad() || ...);
@@ -524,6 +546,31 @@ Tensor3 conv_backward_autograd(const Tensor& x, const Tensor& y, const Tensor& w
     }
     at::AutoDispatchBelowADInplaceOrView below;
     return call_conv_backward(x, y, w, g, r, c, p, kid, spec);
+}
+
+Tensor4 tp_double_backward_autograd(const Tensor& x, const Tensor& y, const Tensor& w, const Tensor& g,
+                                    const Tensor& a, const Tensor& b, const Tensor& c, int64_t kid,
+                                    const OptTensor& spec) {
+    if (records(x, y, w, g, a, b, c)) {
+        const auto out =
+            NotDifferentiated<decltype(tp_double_backward_gpu), kTpDoubleBackward>::apply(x, y, w, g, a, b, c, kid, spec);
+        return {out[0], out[1], out[2], out[3]};
+    }
+    at::AutoDispatchBelowADInplaceOrView below;
+    static const auto op = find_op<decltype(tp_double_backward_gpu)>(kTpDoubleBackward);
+    return op.call(x, y, w, g, a, b, c, kid, spec);
+}
+Tensor4 conv_double_backward_autograd(const Tensor& x, const Tensor& y, const Tensor& w, const Tensor& g,
+                                      const Tensor& a, const Tensor& b, const Tensor& c, const Tensor& rows,
+                                      const Tensor& cols, const Tensor& p, int64_t kid, const OptTensor& spec) {
+    if (records(x, y, w, g, a, b, c)) {
+        const auto out = NotDifferentiated<decltype(conv_double_backward_gpu), kConvDoubleBackward>::apply(
+            x, y, w, g, a, b, c, rows, cols, p, kid, spec);
+        return {out[0], out[1], out[2], out[3]};
+    }
+    at::AutoDispatchBelowADInplaceOrView below;
+    static const auto op = find_op<decltype(conv_double_backward_gpu)>(kConvDoubleBackward);
+    return op.call(x, y, w, g, a, b, c, rows, cols, p, kid, spec);
 }
 
 }  // namespace
@@ -568,6 +615,8 @@ TORCH_LIBRARY_IMPL(oeq_amd, Autograd, m) {
     m.impl("tp_backward", tp_backward_autograd);
     m.impl("conv_forward", conv_forward_autograd);
     m.impl("conv_backward", conv_backward_autograd);
+    m.impl("tp_double_backward", tp_double_backward_autograd);
+    m.impl("conv_double_backward", conv_double_backward_autograd);
 }
 
 PYBIND11_MODULE(_oeq_torch, m) {

@@ -1,13 +1,15 @@
 """Host-side logic that needs no GPU: the description a kernel set is rebuilt from in another process
 (core/spec.py: problem_to_dict / problem_from_dict; _torch/ops.py: make_spec / spec_hash) and the factored form
-of the shared-weight 'uvw' convolution (core/problems.py: factor_shared_uvw), the latter against the oracle."""
+of the shared-weight 'uvw' convolution (core/problems.py: factor_shared_uvw), the latter against the oracle; autograd of the second-order ops."""
 
 import json
 
 import numpy as np
 import pytest
+import torch
 
 import openequivariance_amd as oeq
+from openequivariance_amd._torch import ops
 from openequivariance_amd.core import problems as P
 from openequivariance_amd.core.graph import CoordGraph
 from openequivariance_amd.core.spec import problem_from_dict, problem_to_dict
@@ -47,7 +49,6 @@ def test_problem_description_round_trip(problem):
 
 
 def test_kernel_set_id_is_a_function_of_the_description(monkeypatch):
-    from openequivariance_amd._torch import ops
     monkeypatch.setenv("OEQ_AMD_TUNE", "")
     p = P.config2_nequip_uvu()
     s1, s2 = ops.make_spec("conv", p, True, False), ops.make_spec("conv", P.config2_nequip_uvu(), True, False)
@@ -106,3 +107,26 @@ def test_factored_convolution_equals_the_per_edge_one(make):
     assert np.abs(dw - dw_ref).max() <= 1e-12 * scale(dw_ref)
     assert np.abs(dx - dx_ref).max() <= 1e-12 * scale(dx_ref)
     assert np.abs(dy - dy_ref).max() <= 1e-12 * scale(dy_ref)
+
+
+@pytest.mark.parametrize("conv", [False, True])
+def test_second_order_ops_refuse_to_be_differentiated(conv):
+    """The fused second-order ops have no derivative: differentiating through them is an error, never a gradient without
+    their part. On meta tensors, which take the dispatch of the real call."""
+    problem = P.config1_single_uvu()
+    module = oeq.TensorProductConv(problem) if conv else oeq.TensorProduct(problem)
+    n = 6
+    d1, d2, d3, wn = problem.irreps_in1.dim, problem.irreps_in2.dim, problem.irreps_out.dim, problem.weight_numel
+    x, y, w, g, a, b, c = (torch.empty(n, d, device="meta", requires_grad=True) for d in (d1, d2, wn, d3, d1, d2, wn))
+    edges = [torch.empty(n, dtype=torch.int64, device="meta") for _ in range(3)] if conv else []
+    op = ops.conv_double_backward if conv else ops.tp_double_backward
+    out = op(x, y, w, g, a, b, c, *edges, module.kid)
+    assert all(t.requires_grad for t in out)
+    for i in range(4):
+        with pytest.raises(RuntimeError, match="no autograd formula"):
+            (out[i].sum() + x.sum()).backward(retain_graph=True)
+    with torch.no_grad():
+        assert not any(t.requires_grad for t in op(x, y, w, g, a, b, c, *edges, module.kid))
+    # first-order ops as before
+    first = (ops.conv_forward if conv else ops.tp_forward)(x, y, w, *edges, module.kid)
+    assert [t.shape for t in torch.autograd.grad(first.sum(), (x, y, w))] == [x.shape, y.shape, w.shape]
