@@ -1,0 +1,37 @@
+"""Building and importing the package from states that a working tree can be in."""
+
+import os
+import shutil
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+
+
+@pytest.fixture
+def tree(tmp_path):
+    """A copy of the package's sources without anything built."""
+    for name in ("openequivariance_amd", "include"):
+        shutil.copytree(ROOT / name, tmp_path / name,
+                        ignore=shutil.ignore_patterns("*.so", "*.so.tmp*", "_kcache", "__pycache__"))
+    shutil.copy(ROOT / "__graft_entry__.py", tmp_path)
+    return tmp_path
+
+
+def _python(tree, code, **env):
+    return subprocess.run([sys.executable, "-c", code], cwd=tree, capture_output=True, text=True,
+                          env=dict(os.environ, PYTHONPATH=str(tree), **env))
+
+
+def test_build_replaces_a_library_of_another_abi(tree):
+    lib = tree / "openequivariance_amd" / "liboeq_amd.so"
+    (tree / "old.c").write_text("int oeq_abi_version(void) { return 6; }\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", str(tree / "old.c"), "-o", str(lib)], check=True)
+    res = _python(tree, "import __graft_entry__ as g\n"
+                        "rt = g.build_libraries()\n"
+                        "print(rt.load_library().oeq_abi_version() == rt.ABI_VERSION)")
+    assert res.returncode == 0, res.stderr
+    assert res.stdout.split()[-1] == "True"
