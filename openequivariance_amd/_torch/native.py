@@ -1,5 +1,5 @@
 """Loads ``_oeq_torch.so``, the torch ops over the C ABI (``csrc/oeq_torch.cpp``), and builds it where no built file
-exists. There is no other implementation of the ops: a library that cannot be loaded is an error."""
+exists. There is no other implementation of the ops: without the library every call of one is an error."""
 
 from __future__ import annotations
 

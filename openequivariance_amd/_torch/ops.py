@@ -1,5 +1,5 @@
-"""PyTorch custom ops over the C ABI: kernel sets by description, the index of an edge list, fake kernels, autocast and
-the second-order routes. The ops themselves, with their autograd, are in ``csrc/oeq_torch.cpp``, which calls back into
+"""PyTorch custom ops over the C ABI: schemas, kernel sets by description, the index of an edge list, fake kernels,
+autocast and the second-order routes. The ops themselves, with their autograd, are in ``csrc/oeq_torch.cpp``, which calls back into
 this file for what is rare or needs the code generator.
 
 Stand in for the reference's native op library
@@ -39,18 +39,44 @@ import torch
 from .. import runtime as rt
 from . import native
 
-_native = native.load()
+# Problems, layouts and generated sources are of use without a compiler or ROCm, so a library that cannot be loaded
+# does not fail the import but the first call of an op.
+try:
+    _native = native.load()
+except (rt.OeqError, OSError, ImportError) as exc:
+    _native, _native_error = None, exc
+
+_library = torch.library.Library("oeq_amd", "DEF")
+_OPERANDS = "Tensor L1_in, Tensor L2_in, Tensor W"
+_COTANGENTS = "Tensor L1_dgrad, Tensor L2_dgrad, Tensor W_dgrad"
+_EDGES = "Tensor rows, Tensor cols, Tensor transpose_perm"
+_ID = "int kid, Tensor? spec=None"
+_THREE, _FOUR = "(Tensor, Tensor, Tensor)", "(Tensor, Tensor, Tensor, Tensor)"
+for _schema in (f"tp_forward({_OPERANDS}, {_ID}) -> Tensor",
+                f"tp_backward({_OPERANDS}, Tensor L3_grad, {_ID}) -> {_THREE}",
+                f"tp_double_backward({_OPERANDS}, Tensor L3_grad, {_COTANGENTS}, {_ID}) -> {_FOUR}",
+                f"conv_forward({_OPERANDS}, {_EDGES}, {_ID}) -> Tensor",
+                f"conv_backward({_OPERANDS}, Tensor L3_grad, {_EDGES}, {_ID}) -> {_THREE}",
+                f"conv_double_backward({_OPERANDS}, Tensor L3_grad, {_COTANGENTS}, {_EDGES}, {_ID}) -> {_FOUR}"):
+    _name = _library.define(_schema, tags=(torch.Tag.pt2_compliant_tag,))
+    if _native is None:
+        def _unavailable(*_args):
+            raise rt.OeqError(f"the torch ops could not be loaded: {_native_error}") from _native_error
+
+        _library.impl(_name, _unavailable, "CUDA")
 
 
 class _Registry(dict):
     """Kernel sets by id. What leaves it leaves the native ops' table as well."""
 
     def pop(self, kid, *default):
-        _native.forget_entry(kid)
+        if _native is not None:
+            _native.forget_entry(kid)
         return super().pop(kid, *default)
 
     def __delitem__(self, kid):
-        _native.forget_entry(kid)
+        if _native is not None:
+            _native.forget_entry(kid)
         super().__delitem__(kid)
 
     def clear(self):
@@ -589,10 +615,11 @@ def _conv_second_order(operands, cotangents, kid, spec):
                          x, y, w, g, ddx, ddy, ddw)
 
 
-_native.set_callbacks(dict(
-    resolve=_resolve, check_edges=_check_edges, conv_index=_native_index, conv_forward=_composed_forward,
-    conv_backward=_composed_backward, conv_double_backward=_composed_double_backward,
-    tp_second_order=_tp_second_order, conv_second_order=_conv_second_order, error_type=rt.OeqError))
+if _native is not None:
+    _native.set_callbacks(dict(
+        resolve=_resolve, check_edges=_check_edges, conv_index=_native_index, conv_forward=_composed_forward,
+        conv_backward=_composed_backward, conv_double_backward=_composed_double_backward,
+        tp_second_order=_tp_second_order, conv_second_order=_conv_second_order, error_type=rt.OeqError))
 
 
 # Mixed precision: the kernels are compiled for one dtype; under autocast the

@@ -1,7 +1,7 @@
 // _oeq_torch.so: the torch ops over the C ABI of include/oeq_amd.h, as the Python module _torch/ops.py loads it.
 //
 // Stands in for the reference's native op library (openequivariance/openequivariance/extension/torch_core.hpp:274-644):
-// schemas, argument checks (torch_core.hpp:109-134), allocation of results and scratch memory, launches on
+// argument checks (torch_core.hpp:109-134), allocation of results and scratch memory, launches on
 // torch's current stream, and autograd. An op carries the id of its kernel set and, for processes that have not
 // seen it, the set's description; what is rare or needs the code generator stays in Python and is called from here:
 // building a kernel set, the index of an edge list (it is kept between calls there), the convolutions without a fused
@@ -575,32 +575,7 @@ Tensor4 conv_double_backward_autograd(const Tensor& x, const Tensor& y, const Te
 
 }  // namespace
 
-TORCH_LIBRARY(oeq_amd, m) {
-    const std::vector<at::Tag> tags = {at::Tag::pt2_compliant_tag};
-    m.def("tp_forward(Tensor L1_in, Tensor L2_in, Tensor W, int kid, Tensor? spec=None) -> Tensor", tags);
-    m.def(
-        "tp_backward(Tensor L1_in, Tensor L2_in, Tensor W, Tensor L3_grad, int kid, Tensor? spec=None) -> "
-        "(Tensor, Tensor, Tensor)",
-        tags);
-    m.def(
-        "tp_double_backward(Tensor L1_in, Tensor L2_in, Tensor W, Tensor L3_grad, Tensor L1_dgrad, Tensor L2_dgrad, "
-        "Tensor W_dgrad, int kid, Tensor? spec=None) -> (Tensor, Tensor, Tensor, Tensor)",
-        tags);
-    m.def(
-        "conv_forward(Tensor L1_in, Tensor L2_in, Tensor W, Tensor rows, Tensor cols, Tensor transpose_perm, int kid, "
-        "Tensor? spec=None) -> Tensor",
-        tags);
-    m.def(
-        "conv_backward(Tensor L1_in, Tensor L2_in, Tensor W, Tensor L3_grad, Tensor rows, Tensor cols, "
-        "Tensor transpose_perm, int kid, Tensor? spec=None) -> (Tensor, Tensor, Tensor)",
-        tags);
-    m.def(
-        "conv_double_backward(Tensor L1_in, Tensor L2_in, Tensor W, Tensor L3_grad, Tensor L1_dgrad, Tensor L2_dgrad, "
-        "Tensor W_dgrad, Tensor rows, Tensor cols, Tensor transpose_perm, int kid, Tensor? spec=None) -> "
-        "(Tensor, Tensor, Tensor, Tensor)",
-        tags);
-}
-
+// (schemas, fake kernels and autocast: _torch/ops.py)
 TORCH_LIBRARY_IMPL(oeq_amd, CUDA, m) {
     m.impl("tp_forward", tp_forward_gpu);
     m.impl("tp_backward", tp_backward_gpu);

@@ -35,3 +35,24 @@ def test_build_replaces_a_library_of_another_abi(tree):
                         "print(rt.load_library().oeq_abi_version() == rt.ABI_VERSION)")
     assert res.returncode == 0, res.stderr
     assert res.stdout.split()[-1] == "True"
+
+
+def test_import_needs_neither_built_libraries_nor_compilers(tree):
+    """Problems and modules can be made with torch alone, meta tensors traced; a call of an op says what is missing."""
+    (tree / "none").mkdir()
+    res = _python(tree, """
+import torch
+import openequivariance_amd as oeq
+from openequivariance_amd._torch import ops
+p = oeq.TPProblem("4x1e", "1x1e", "4x0e", [(0, 0, 0, "uvu", True)], shared_weights=False, internal_weights=False)
+tp = oeq.TensorProduct(p)
+x, y, w = (torch.empty(3, n, device="meta") for n in (12, 3, 4))
+assert ops.tp_forward(x, y, w, tp.kid).shape == (3, 4)
+try:
+    torch.ops.oeq_amd.tp_forward.default.redispatch(torch._C.DispatchKeySet(torch._C.DispatchKey.CUDA), x, y, w, tp.kid)
+except oeq.runtime.OeqError as exc:
+    assert "could not be loaded" in str(exc) and "hipcc" in str(exc), exc
+    print("refused")
+""", PATH=str(tree / "none"))
+    assert res.returncode == 0, res.stderr
+    assert res.stdout.split()[-1] == "refused"
