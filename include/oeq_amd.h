@@ -21,6 +21,9 @@
 #include <stddef.h>
 #include <stdint.h>
 
+/* Changes with every change of a struct, an argument list or an enumerator below. */
+#define OEQ_ABI_VERSION 7
+
 #ifdef __cplusplus
 extern "C" {
 #endif
@@ -363,7 +366,7 @@ int oeq_kernel_timing_collect(oeq_kernels* k, int role, double* total_ms, int64_
 
 /* ---- diagnostics -------------------------------------------------------- */
 const char* oeq_last_error(void);
-int oeq_abi_version(void);
+int oeq_abi_version(void); /* OEQ_ABI_VERSION of the header the library was compiled with */
 
 #ifdef __cplusplus
 }

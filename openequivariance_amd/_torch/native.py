@@ -1,4 +1,4 @@
-"""Loads ``_oeq_torch.so``, the torch ops over the C ABI (``csrc/oeq_torch.cpp``), and builds it where no built file
+"""Loads ``_oeq_torch-*.so``, the torch ops over the C ABI (``csrc/oeq_torch.cpp``), and builds it where no built file
 exists. There is no other implementation of the ops: without the library every call of one is an error."""
 
 from __future__ import annotations
@@ -7,6 +7,7 @@ import importlib.machinery
 import importlib.util
 import os
 import subprocess
+import sys
 import sysconfig
 import threading
 from pathlib import Path
@@ -15,7 +16,9 @@ import torch
 
 from .. import runtime as rt
 
-_SO_PATH = rt._PKG_DIR / "_oeq_torch.so"
+# The file is bound to the torch it was compiled against (its C++ interface changes between releases), to this Python
+# and to the C ABI: what was built for others has another name and is not loaded.
+_SO_PATH = rt._PKG_DIR / f"_oeq_torch-{torch.__version__}-{sys.implementation.cache_tag}-abi{rt.ABI_VERSION}.so"
 _SRC_PATH = rt._PKG_DIR / "csrc" / "oeq_torch.cpp"
 _lock = threading.Lock()
 _module = None
@@ -47,6 +50,10 @@ def _stale() -> bool:
     return any(src.exists() and src.stat().st_mtime > built for src in (_SRC_PATH, rt._INCLUDE_DIR / "oeq_amd.h"))
 
 
+def so_path() -> Path:
+    return _SO_PATH
+
+
 def load():
     """The extension module; loading it registers the ops ``torch.ops.oeq_amd.*``."""
     global _module
@@ -60,6 +67,7 @@ def load():
             module = importlib.util.module_from_spec(spec)
             loader.exec_module(module)
             if module.abi_version() != rt.ABI_VERSION:
-                raise rt.OeqError(f"{_SO_PATH} was built against another liboeq_amd.so: rebuild it")
+                raise rt.OeqError(f"{_SO_PATH} was compiled for C ABI {module.abi_version()}, this package has "
+                                  f"{rt.ABI_VERSION}: rebuild it")
             _module = module
     return _module

@@ -1,4 +1,4 @@
-// _oeq_torch.so: the torch ops over the C ABI of include/oeq_amd.h, as the Python module _torch/ops.py loads it.
+// _oeq_torch-*.so: the torch ops over the C ABI of include/oeq_amd.h, as the Python module _torch/ops.py loads it.
 //
 // Stands in for the reference's native op library (openequivariance/openequivariance/extension/torch_core.hpp:274-644):
 // argument checks (torch_core.hpp:109-134), allocation of results and scratch memory, launches on
@@ -595,7 +595,7 @@ TORCH_LIBRARY_IMPL(oeq_amd, Autograd, m) {
 }
 
 PYBIND11_MODULE(_oeq_torch, m) {
-    m.def("abi_version", [] { return oeq_abi_version(); });
+    m.def("abi_version", [] { return OEQ_ABI_VERSION; });
     m.def("set_callbacks", [](py::dict fns) {
         auto* c = new Callbacks();
         c->resolve = fns["resolve"];

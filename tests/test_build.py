@@ -56,3 +56,19 @@ except oeq.runtime.OeqError as exc:
 """, PATH=str(tree / "none"))
     assert res.returncode == 0, res.stderr
     assert res.stdout.split()[-1] == "refused"
+
+
+def test_ops_built_for_another_torch_are_not_loaded(tree):
+    from openequivariance_amd import runtime as rt
+    from openequivariance_amd._torch import native
+    assert native.load().abi_version() == rt.ABI_VERSION
+    pkg = tree / "openequivariance_amd"
+    shutil.copy(rt.lib_path(), pkg)
+    built = native.so_path()
+    for other in ("_oeq_torch.so", built.name.replace("torch-", "torch-1."), built.name.replace("-abi", "-abi1")):
+        shutil.copy(built, pkg / other)
+    (tree / "none").mkdir()
+    code = "from openequivariance_amd._torch import ops; print(ops._native is None)"
+    assert _python(tree, code, PATH=str(tree / "none")).stdout.split() == ["True"]
+    shutil.copy(built, pkg)
+    assert _python(tree, code, PATH=str(tree / "none")).stdout.split() == ["False"]
