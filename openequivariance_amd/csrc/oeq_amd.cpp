@@ -601,25 +601,15 @@ static int64_t hub_capacity(const oeq_kernels* k, int64_t nnz) {
     const int64_t limit = hub_limit_of(k);
     return limit ? nnz / limit : 0;
 }
-// The small-graph form of a kernel deals a node's edges out to n waves, so it needs no chunks while the waves have no
-// more than hub_limit edges each. A node has fewer edges than there are nodes unless edges are parallel, which makes
-// that n * hub_limit nodes. Edges are parallel in small periodic cells, whose nodes have much the same number of them:
-// there half of hub_limit on average means none is long. Spares the launch that adds the chunks' rows, 3.4 us on the
-// device and about as much on the host: one of them in forward and backward of 192 nodes x 32 edges, three in a
-// training step on forces of 16 molecules (285 -> 271 us with what the launch costs the host).
-static bool whole_segments(const oeq_kernels* k, int role, int64_t node_count, int64_t nnz) {
-    const int plain = timed_as(role);
-    if (plain == role || !k->roles[role].present || !k->roles[plain].block) return false;
-    const RoleInfo &split = k->roles[role], &whole = k->roles[plain];
-    const int64_t limit = hub_limit_of(k), waves = split.block * whole.units_per_block / whole.block;
-    return node_count <= limit * waves && nnz <= limit / 2 * node_count;
-}
 // Walk positions that the kernel of `role` reserves for the extra chunks, at the front of its grid: the
 // capacity rounded up to whole blocks and to the grid multiple of the role, so that the blocks behind them
 // still divide evenly among the XCDs.
-static int64_t hub_units(const oeq_kernels* k, int role, int64_t node_count, int64_t nnz) {
+// Small-graph forms included, though an even graph's step then pays the launch that adds the chunks' rows (3.4 us) for
+// nothing: how many edges one node holds is not known here, and walked whole by one block 1 000 edges at one node take
+// mace-medium's forward 162 us instead of 45, 8 000 edges 1 313 instead of 49.
+static int64_t hub_units(const oeq_kernels* k, int role, int64_t nnz) {
     const int64_t cap = hub_capacity(k, nnz);
-    if (!cap || !k->roles[role].present || whole_segments(k, role, node_count, nnz)) return 0;
+    if (!cap || !k->roles[role].present) return 0;
     const int64_t g = std::max(1u, k->roles[role].units_per_block), m = std::max(1u, k->roles[role].grid_multiple);
     const int64_t blocks = ((cap + g - 1) / g + m - 1) / m * m;
     return blocks * g;
@@ -647,8 +637,8 @@ static int64_t backward_parts(const oeq_kernels* k, int role, int64_t node_count
     const int64_t tail = std::min(((wide ? 8 : 16) * fill + node_count / 2) / node_count, nnz / (node_count * (wide ? 15 : 10)));
     return std::max<int64_t>(1, std::max(idle, tail));
 }
-static size_t hub_rows_bytes(const oeq_kernels* k, int role, int64_t node_count, int64_t nnz) {
-    return align_up((size_t)hub_units(k, role, node_count, nnz) * (size_t)k->dims.L3_dim * (size_t)k->dims.elem_size, 256);
+static size_t hub_rows_bytes(const oeq_kernels* k, int role, int64_t nnz) {
+    return align_up((size_t)hub_units(k, role, nnz) * (size_t)k->dims.L3_dim * (size_t)k->dims.elem_size, 256);
 }
 
 // The index of an edge list: what the walk kernels derive from (rows, cols) alone. Receiver side: CSR
@@ -722,22 +712,22 @@ static ScratchLayout scratch_layout(const oeq_kernels* k, int64_t node_count, in
     auto take = [&w](size_t bytes) { size_t at = w.total; w.total += bytes; return at; };
     // rows that the extra chunks of long segments write (forward-shaped kernels)
     if (hub_rows_role >= 0)
-        if (size_t hb = hub_rows_bytes(k, hub_rows_role, node_count, nnz)) w.hub_rows = take(hb);
+        if (size_t hb = hub_rows_bytes(k, hub_rows_role, nnz)) w.hub_rows = take(hb);
     if (arrivals)
         w.arrivals = take(align_up((size_t)node_count * (size_t)std::max(1, k->dims.n_chunks) * sizeof(int32_t), 256));
     if (terms && wpartial_role == OEQ_ROLE_CONV_BACKWARD && k->dims.dx_mode == OEQ_DX_SENDER_WALK) {
         // no terms: the sender-side walk forms the rows itself, and writes those of its extra chunks here
-        if (int64_t su = hub_units(k, split_role(k, OEQ_ROLE_CONV_BACKWARD_DX, node_count), node_count, nnz))
+        if (int64_t su = hub_units(k, split_role(k, OEQ_ROLE_CONV_BACKWARD_DX, node_count), nnz))
             w.shub_rows = take(align_up((size_t)su * (size_t)k->dims.L1_dim * (size_t)k->dims.elem_size, 256));
     } else if (terms) {
         w.dx_tmp = take(align_up((size_t)nnz * (size_t)k->dims.L1_dim * (size_t)k->dims.elem_size, 256));
         // partial sums of the senders whose terms fixup_backward sums in chunks
         if (!arrivals)
-            if (int64_t su = hub_units(k, OEQ_ROLE_CONV_FIXUP_BACKWARD, node_count, nnz))
+            if (int64_t su = hub_units(k, OEQ_ROLE_CONV_FIXUP_BACKWARD, nnz))
                 w.shub_rows = take(align_up((size_t)su * (size_t)k->dims.L1_dim * (size_t)k->dims.elem_size, 256));
     }
     if (wpartial)
-        if (size_t wp = conv_wpartial_bytes(k, node_count + hub_units(k, wpartial_role, node_count, nnz), wpartial_role))
+        if (size_t wp = conv_wpartial_bytes(k, node_count + hub_units(k, wpartial_role, nnz), wpartial_role))
             w.wpartial = take(wp);
     return w;
 }
@@ -846,7 +836,7 @@ static int build_index(oeq_kernels* k, const char* who, const IndexLayout& w, in
 static int sender_sum(oeq_kernels* k, int64_t node_count, int64_t nnz, void* dx_tmp, void* L1_grad,
                       const WalkIndex& ix, void* shub_rows, void* stream) {
     int64_t limit = (ix.shubptr && shub_rows) ? ix.hub_limit : 0;
-    int64_t units = limit ? hub_units(k, OEQ_ROLE_CONV_FIXUP_BACKWARD, node_count, nnz) : 0;
+    int64_t units = limit ? hub_units(k, OEQ_ROLE_CONV_FIXUP_BACKWARD, nnz) : 0;
     void* fargs[] = {&node_count, &nnz,         &dx_tmp, &L1_grad, (void*)&ix.sperm, (void*)&ix.colptr,
                      (void*)&ix.shubptr, (void*)&ix.shubnode, &limit, &units, &shub_rows};
     int rc = k->launch(OEQ_ROLE_CONV_FIXUP_BACKWARD, node_count + units, fargs, stream);
@@ -947,10 +937,9 @@ int oeq_conv_forward_indexed(oeq_kernels* k, int64_t node_count, int64_t nnz, co
         rc = bind_index(k, "oeq_conv_forward", index_layout(k, node_count, nnz, index_sender_side != 0), index,
                         index_bytes, rows, &ix);
         if (rc) return rc;
-        units = ix.hub_limit ? hub_units(k, role, node_count, nnz) : 0;
-        if (!units) ix.hub_limit = 0;
-        if (units) {
-            const size_t need = hub_rows_bytes(k, role, node_count, nnz);
+        if (ix.hub_limit) {
+            units = hub_units(k, role, nnz);
+            const size_t need = hub_rows_bytes(k, role, nnz);
             if (!scratch || scratch_bytes < need)
                 return fail(OEQ_ERR_INVALID, "oeq_conv_forward: workspace too small (%zu < %zu bytes of scratch)",
                             scratch_bytes, need);
@@ -1084,7 +1073,7 @@ int oeq_conv_backward_indexed(oeq_kernels* k, int64_t node_count, int64_t nnz, c
                           stream);
         if (rc) return rc;
     }
-    int64_t units = ix.hub_limit ? hub_units(k, OEQ_ROLE_CONV_BACKWARD, node_count, nnz) : 0;
+    int64_t units = ix.hub_limit ? hub_units(k, OEQ_ROLE_CONV_BACKWARD, nnz) : 0;
     int64_t parts = backward_parts(k, OEQ_ROLE_CONV_BACKWARD, node_count, nnz);
     void* args[] = {&node_count,  &nnz,      &L1_in,     &L1_grad,    &L2_in,        &L2_grad,     &W,         &W_grad,
                     &L3_grad,     &rows,     &cols,      &ix.rowptr,  &sc.dx_tmp,    &ix.rperm,    &sc.wpartial,
@@ -1098,8 +1087,7 @@ int oeq_conv_backward_indexed(oeq_kernels* k, int64_t node_count, int64_t nnz, c
         // for the rows of X, every sender's segment in sender-major order, long segments in chunks.
         int64_t limit = (ix.shubptr && sc.shub_rows) ? ix.hub_limit : 0;
         const int xrole = split_role(k, OEQ_ROLE_CONV_BACKWARD_DX, node_count);
-        int64_t xunits = limit ? hub_units(k, xrole, node_count, nnz) : 0;
-        if (!xunits) limit = 0;
+        int64_t xunits = limit ? hub_units(k, xrole, nnz) : 0;
         void* xargs[] = {&node_count, &nnz,       &L3_grad,   &L2_in,     &W,           &L1_grad,      &cols,  &rows,
                          &ix.colptr,  &ix.sperm,  &ix.order,  &ix.shubptr, &ix.shubnode, &limit,        &xunits, &sc.shub_rows};
         rc = k->launch(xrole, node_count + xunits, xargs, stream);
@@ -1237,12 +1225,11 @@ int oeq_conv_double_backward_indexed(oeq_kernels* k, int64_t node_count, int64_t
     // shared weights: kernel B leaves one partial weight-gradient row per wave group, summed in order at the end
     void* wpartial = at_offset(scratch, w.wpartial);
     void* hub_rows = at_offset(scratch, w.hub_rows);
-    int64_t units_a = (ix.hub_limit && hub_rows) ? hub_units(k, role_a, node_count, nnz) : 0;
-    int64_t limit_a = units_a ? ix.hub_limit : 0;
-    int64_t units_b = ix.hub_limit ? hub_units(k, OEQ_ROLE_DOUBLE_BACKWARD_B, node_count, nnz) : 0;
+    int64_t units_a = (ix.hub_limit && hub_rows) ? hub_units(k, role_a, nnz) : 0;
+    int64_t units_b = ix.hub_limit ? hub_units(k, OEQ_ROLE_DOUBLE_BACKWARD_B, nnz) : 0;
     int64_t parts_b = backward_parts(k, OEQ_ROLE_DOUBLE_BACKWARD_B, node_count, nnz);
     void* a[] = {&node_count, &nnz,  &L1_in,     &L1_dgrad, &L2_in,    &L2_dgrad,  &W,          &W_dgrad,      &L3_dgrad,
-                 &rows,       &cols, &ix.rowptr, &ix.rperm, &ix.order, &ix.hubptr, &ix.hubnode, &limit_a,      &units_a,
+                 &rows,       &cols, &ix.rowptr, &ix.rperm, &ix.order, &ix.hubptr, &ix.hubnode, &ix.hub_limit, &units_a,
                  &hub_rows};
     if (k->roles[OEQ_ROLE_DOUBLE_BACKWARD_A].present) {
         rc = k->launch(role_a, node_count + units_a, a, stream);

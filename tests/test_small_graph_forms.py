@@ -1,14 +1,16 @@
 """Where the small-graph form of the forward kernel puts its waves' accumulators: every value inside the slice of the
-wave that writes it, every read inside a slice, and the whole inside the array that the kernel declares."""
+wave that writes it, every read inside a slice, and the whole inside the array that the kernel declares. And that such
+forms keep to chunks where a node has many edges."""
 
 import re
 
 import numpy as np
 import pytest
 
+from openequivariance_amd import runtime as rt
 from openequivariance_amd.codegen.common import Src
 from openequivariance_amd.codegen.lower import adjoint, lower
-from openequivariance_amd.codegen.uvu import LDS_LIMIT, UvuEmitter, split_waves
+from openequivariance_amd.codegen.uvu import LDS_LIMIT, UvuEmitter, conv_module, split_waves
 from openequivariance_amd.core import problems as P
 
 
@@ -57,3 +59,15 @@ def test_slices_of_the_waves_do_not_overlap(name):
     reads = {int(v) for v in re.findall(r"first\[(\d+)\]", text)}
     assert writes and max(writes) + 64 <= stride
     assert reads == {p * em.NCH * stride + v for p in range(n) for v in writes}
+
+
+def test_small_graph_forms_walk_long_segments_in_chunks():
+    """A node may hold nearly all edges of a small graph (a virtual node, parallel edges, the padding of an edge list): the
+    small-graph form leaves room for the rows of its extra chunks as the plain one does."""
+    low = lower(P.nequip_problems()[1])
+    src, dims, descs = conv_module(low, True)
+    ks = rt.KernelSet(b"\x7fELFxxxx", dims, descs)
+    roles = {d[0]: d for d in descs}
+    for nodes, edges in ((200, 20000), (1000, 1500), (32, 600)):
+        assert nodes <= roles[rt.ROLE_CONV_FORWARD_SPLIT][7]
+        assert ks.conv_forward_scratch_bytes(nodes, edges) >= edges // dims["hub_limit"] * low.L3 * 4
