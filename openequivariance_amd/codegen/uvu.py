@@ -31,7 +31,7 @@ from __future__ import annotations
 
 import os
 import re
-from typing import Callable, Dict, List, Optional, Sequence, Tuple
+from typing import Callable, Dict, List, NamedTuple, Optional, Sequence, Tuple
 
 from .common import Src, fixup_backward_kernel, prelude, utility_kernels
 from .lower import Lowered, Path, float_literal
@@ -2437,7 +2437,8 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
                     conv_segw=4, conv_split=1, conv_dd=1, dd_acc=0, dd_g=2, dd_wa=2, dd_wb=2, dd_fp=0, dd_fw=32,
                     dd_gres=-1, dd_split=1, dd_segw=4, dd_merge=0, dd_need=200, dd_ngrp=0, conv_gbud=0, conv_ngrp=0, conv_fit=300, conv_fw=0, conv_pf=0,
                     conv_dxm=-1, conv_q=0, conv_hops=2, conv_qpin=1, conv_qaf=48, conv_qab=24, tp_mask=0, tp_forms=1,
-                    conv_hub=256, conv_dxs=-1, conv_omin=32768, conv_fsplit=-1, conv_fsmax=-1, conv_parts=-1))
+                    conv_hub=256, conv_dxs=-1, conv_omin=32768, conv_fsplit=-1, conv_fsplit_f=-1, conv_fsplit_x=-1, conv_fsplit_a=-1,
+                    conv_fsmax=-1, conv_parts=-1))
     assert deterministic or not kahan, "kahan=True requires deterministic=True"
     # knobs somebody set: the rules below leave those alone
     user_tune = os.environ.get("OEQ_AMD_TUNE", "")
@@ -2559,12 +2560,12 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     xcd = max(1, t["conv_xcd"])
     xcd_b = 1 if (walk and low.shared_weights) else xcd  # bounded grid: one partial dW row per wave group
     blk_f = em.emit_conv_forward(s, G_f, walk, t["conv_pipe_f"], t["conv_wf"], xcd, bool(t["conv_tra"]))
-    splits: Dict[str, int] = {}  # the kernels with a node's edges dealt out to several waves: how many
+    splits: Dict[str, Split] = {}  # the kernels with a node's edges dealt out to several waves
     if walk and not kahan and not q_fwd:
-        n = t["conv_fsplit"] if t["conv_fsplit"] >= 0 else split_waves(em.NCH * em.seg_waves, t["conv_wf"])
+        n = split_waves(t, "conv_fsplit_f", em, em.seg_waves, t["conv_wf"])
         n = em.split_count(n, t["conv_pipe_f"], em.seg_waves)
         if n > 1:
-            splits["forward_split"] = n
+            splits["forward_split"] = Split("conv_fsplit_f", n, em.R, em.seg_waves)
             blk_fs = em.emit_conv_forward(s, 1, True, t["conv_pipe_f"], t["conv_wf"], xcd, bool(t["conv_tra"]),
                                           name="forward_split", split=n)
     em.use_q = q_bwd
@@ -2658,10 +2659,10 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
                                          xcd, bool(t["conv_tra"]), name="backward_dx")
             descs.append((rt.ROLE_CONV_BACKWARD_DX, "backward_dx", blk_x, G_x, 0, xcd))
             s("}  // namespace oeq_dx")
-            n = t["conv_fsplit"] if t["conv_fsplit"] >= 0 else split_waves(ex.NCH, waves_x)
+            n = split_waves(t, "conv_fsplit_x", ex, 1, waves_x)
             n = ex.split_count(n, t["conv_pipe_f"] if pipe_x else 0)
             if n > 1 and not kahan:
-                splits["backward_dx_split"] = n
+                splits["backward_dx_split"] = Split("conv_fsplit_x", n, ex.R, 1)
                 s("namespace oeq_dx_split {")
                 ex.emit_structs(s)
                 ex.emit_forward_cores(s, preloaded=True)
@@ -2736,18 +2737,52 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
             if _forward_scratch(third[0]) == 0:
                 return third
     if walk:
-        descs = _small_graph_rules(src, descs, splits, compute_units, t, low.shared_weights)
+        # A small-graph form that needs scratch memory where the plain kernel does not: half as many waves leave each of
+        # them twice the registers (toluene, fp32, 640 nodes x 30 edges: plain 59 us, eight waves with 48 B of scratch
+        # 79, four without 46; 40 nodes 49 / 18 / 19). Not where that does not help either (nequip-uvu, fp64, second
+        # order: 12 B with two waves to eight, and faster than plain all the same).
+        res = rt.kernel_resources(rt.compile_source(src))
+        fewer = {sp.knob: sp.waves // 2 for name, sp in splits.items()
+                 if res[name][1] > res[name.replace("_split", "")][1] == 0 and t[sp.knob] < 0 and t["conv_fsplit"] < 0}
+        if fewer:
+            half = conv_module(low, deterministic, compute_units, kahan, dict(override or {}, **fewer))
+            res = rt.kernel_resources(rt.compile_source(half[0]))
+            if all(res.get(name, (0, 0))[1] == 0 for name, sp in splits.items() if sp.knob in fewer):
+                return half
+        descs = _small_graph_rules(src, descs, splits, compute_units, t, low.shared_weights, em.R)
     return src, dims, descs
 
 
-def split_waves(node_waves: int, waves_per_eu: int) -> int:
-    """How many waves a node's edges are dealt out to in the small-graph form of a forward-shaped kernel with
-    ``node_waves`` waves per node: a block of eight waves (two per SIMD), four where a lane has 512 registers."""
-    return (4 if waves_per_eu == 1 else 8) // node_waves
+class Split(NamedTuple):
+    """Small-graph form of a forward-shaped kernel: the knob with its number of waves, that number, the rows a wave
+    walks side by side and the waves that share a node's output segments."""
+    knob: str
+    waves: int
+    rows: int
+    seg_waves: int
 
 
-def _small_graph_rules(src: str, descs: List[tuple], splits: Dict[str, int], compute_units: int, t: dict,
-                       shared: bool) -> List[tuple]:
+def split_waves(t: dict, knob: str, em: UvuEmitter, seg_waves: int, waves_per_eu: int) -> int:
+    """How many waves a node's edges are dealt out to in the small-graph form of a forward-shaped kernel: a block of
+    eight waves (two per SIMD), four where a lane has 512 registers.
+
+    Waves that walk R edges side by side: no more than 16 edges to a round of the block, or most lanes have none (blocks
+    of equal channels, l <= 2, fp32, 300 nodes x 12 edges, plain / 8 / 4 / 2 waves: 16 channels, R = 4: 8.6 / 10.8 / 7.9
+    / 7.9 us; 8 channels, R = 8: 7.4 / 11.7 / 8.6 / 7.5; 4 channels, R = 16: 7.4 / 13.2 / 8.8 / 7.6).
+    None where the waves of a node own different output segments and several each: every round of the sum over the parts
+    is a barrier of the whole block, at which the waves wait for each other's segments (400 nodes x 30 edges, plain /
+    small-graph form: SevenNet's main layers in fp64 108 / 162 us, second order 193 / 272; nequip-benzene in fp64 280 /
+    428, second order in fp32 210 / 335)."""
+    for name in (knob, "conv_fsplit"):
+        if t[name] >= 0:
+            return t[name]
+    if seg_waves > 1 and len(em.segments) > seg_waves:
+        return 1
+    return min((4 if waves_per_eu == 1 else 8) // (em.NCH * seg_waves), 16 // em.R)
+
+
+def _small_graph_rules(src: str, descs: List[tuple], splits: Dict[str, Split], compute_units: int, t: dict,
+                       shared: bool, rows: int) -> List[tuple]:
     """Launch descriptors with what the host needs to know to run small graphs (csrc/oeq_amd.cpp: split_role,
     backward_parts): how many walk positions of a backward-shaped kernel the device holds at once, and up to how many
     nodes the split form of a forward-shaped kernel is the faster one. Both follow from the registers and the LDS the
@@ -2757,7 +2792,16 @@ def _small_graph_rules(src: str, descs: List[tuple], splits: Dict[str, int], com
     too few to hide their latencies: up to about n * nodes = 2.5 times the nodes the plain kernel holds at once.
     Measured with 30 edges per node, plain / split in us: mace-large (n = 4) 80 nodes 43 / 19, 500 nodes 52 / 39, 1 000
     nodes 69 / 73; mace-medium (4) 150 nodes 27 / 13, 1 500 nodes 47 / 44, 3 000 nodes 87 / 87; nequip-lips (8) 80 nodes
-    30 / 15, 750 nodes 51 / 46, 1 000 nodes 56 / 62."""
+    30 / 15, 750 nodes 51 / 46, 1 000 nodes 56 / 62. And up to three times the nodes the split form holds itself
+    (12 edges per node: NequiX's main layers 640 nodes 0.83 of the plain time, 960 nodes 1.15; its first layer 1 500
+    nodes 0.90, 2 240 nodes 1.12), twice where its registers or LDS leave it less than half of the plain kernel's waves
+    (SevenNet's first layer, fp64, 88 and 176 registers: 400 nodes 0.96, 640 nodes 1.06, 800 nodes 1.28). Six waves to a
+    CU where the waves of a node own different output segments (three: SevenNet's main layers, fp32, 400 nodes 1.00, 640
+    nodes 1.10, 1 280 nodes 1.44; two: NequiX's main layers as above), two and a half nodes to a CU where a wave walks
+    four edges side by side or more (16 channels: 640 nodes 0.97, 1 280 nodes 1.23).
+
+    Backward-shaped kernels whose waves walk 64 edges side by side get no parts: a part of ten edges leaves most lanes
+    idle (a single path of one channel, second order, 2 560 nodes x 30 edges: 7.7 us whole, 11.4 in parts)."""
     from .. import runtime as rt
     blob = rt.compile_source(src)
     regs, res = rt.kernel_registers(blob), rt.kernel_resources(blob)
@@ -2769,19 +2813,27 @@ def _small_graph_rules(src: str, descs: List[tuple], splits: Dict[str, int], com
         lds = res.get(name, (0, 0))[0]
         return compute_units * max(1, min(4 * simd // waves, (160 * 1024) // lds if lds else 32))
 
+    def largest(name: str) -> int:
+        if t["conv_fsmax"] >= 0:
+            return t["conv_fsmax"]
+        sp, plain = splits[name], name.replace("_split", "")
+        nodes, own = blocks_at_once(plain) * by_name[plain][3], blocks_at_once(name)
+        limit = min(2.5 * nodes / sp.waves, (2 if 2 * own * sp.waves < nodes else 3) * own)
+        if sp.seg_waves > 1:
+            limit = min(limit, 6 * compute_units / sp.seg_waves)
+        if sp.rows >= 4:
+            limit = min(limit, 2.5 * compute_units)
+        return int(limit)
+
     out = []
     for d in descs:
         fill = limit = 0
         if d[1] in splits:
-            plain = d[1].replace("_split", "")
-            limit = t["conv_fsmax"] if t["conv_fsmax"] >= 0 else int(
-                2.5 * blocks_at_once(plain) * by_name[plain][3] / splits[d[1]])
+            limit = largest(d[1])
         elif d[0] in (rt.ROLE_CONV_BACKWARD, rt.ROLE_DOUBLE_BACKWARD_B) and not shared and not t["dd_merge"]:
-            fill = -t["conv_parts"] if t["conv_parts"] >= 0 else blocks_at_once(d[1]) * d[3]
+            fill = -t["conv_parts"] if t["conv_parts"] >= 0 else (blocks_at_once(d[1]) * d[3] if rows < 64 else 0)
         out.append(tuple(d[:5]) + (d[5] if len(d) > 5 else 0, fill, limit))
     return out
-
-
 
 
 def _forward_scratch(source: str) -> int:

@@ -31,7 +31,7 @@ from typing import Dict, List, Optional, Tuple
 
 from .common import Src
 from .lower import Lowered, Path
-from .uvu import UNROLL_V_LIMIT, UvuEmitter, split_waves
+from .uvu import UNROLL_V_LIMIT, Split, UvuEmitter, split_waves
 
 
 # Convolution: above this many paths (after folding of wide rows) the kernels' register needs (two
@@ -874,11 +874,11 @@ def add_tp_kernels(s: Src, low: Lowered, base: UvuEmitter, tune: dict, groups_b:
 
 def add_conv_kernels(s: Src, low: Lowered, base: UvuEmitter, tune: dict, xcd: int, groups_b: int = 0,
                      compute_units: int = 256, kahan: bool = False,
-                     splits: Optional[Dict[str, int]] = None) -> List[tuple]:
+                     splits: Optional[Dict[str, Split]] = None) -> List[tuple]:
     """Append the convolution double-backward kernels (receiver-major walk) to a module. Shared weights: kernel B
     runs with the first-order backward kernel's wave groups per block (``groups_b``) on a bounded grid, one
     partial weight-gradient row per group, and is never split between waves or merged with kernel A. ``splits``
-    receives the number of waves of kernel A's small-graph form."""
+    receives kernel A's small-graph form."""
     from .. import runtime as rt
 
     def kernel_a_need(e: DoubleEmitter) -> int:
@@ -939,10 +939,10 @@ def add_conv_kernels(s: Src, low: Lowered, base: UvuEmitter, tune: dict, xcd: in
             G_a = 1
         blk_a = em.emit_conv_double_a(s, G_a, tune.get("dd_wa", 2), xcd, segw)
         descs.append((rt.ROLE_DOUBLE_BACKWARD_A, "double_backward_A", blk_a, G_a, 0, xcd))
-        n = tune["conv_fsplit"] if tune["conv_fsplit"] >= 0 else split_waves(em.NCH * segw, tune.get("dd_wa", 2))
+        n = split_waves(tune, "conv_fsplit_a", em, segw, tune.get("dd_wa", 2))
         n = em.split_count(n, 0, segw)
         if n > 1 and not kahan and splits is not None:
-            splits["double_backward_A_split"] = n
+            splits["double_backward_A_split"] = Split("conv_fsplit_a", n, em.R, segw)
             blk_as = em.emit_conv_double_a(s, 1, tune.get("dd_wa", 2), xcd, segw, "double_backward_A_split", n)
             descs.append((rt.ROLE_DOUBLE_BACKWARD_A_SPLIT, "double_backward_A_split", blk_as, 1, 0, xcd))
     if groups:

@@ -42,7 +42,7 @@ def test_slices_of_the_waves_do_not_overlap(name):
     low = lower(PROBLEMS[name]())
     em = UvuEmitter(adjoint(low) if "sender walk" in name else low, acc_budget_words=128)
     em.tr_stores = 3 if em.low.elem_size == 8 else 0  # (as conv_module sets it)
-    n = em.split_count(split_waves(em.NCH, 2), 2)
+    n = em.split_count(split_waves({"conv_fsplit": -1}, "conv_fsplit", em, 1, 2), 2)
     assert n > 1
     s = Src()
     block = em.emit_conv_forward(s, 1, True, 2, 2, 8, name="forward_split", split=n)
@@ -71,3 +71,23 @@ def test_small_graph_forms_walk_long_segments_in_chunks():
     for nodes, edges in ((200, 20000), (1000, 1500), (32, 600)):
         assert nodes <= roles[rt.ROLE_CONV_FORWARD_SPLIT][7]
         assert ks.conv_forward_scratch_bytes(nodes, edges) >= edges // dims["hub_limit"] * low.L3 * 4
+
+
+def _forms(problem):
+    src, _dims, descs = conv_module(lower(problem), True)
+    scratch = {name: r[1] for name, r in rt.kernel_resources(rt.compile_source(src)).items()}
+    return {d[1]: d for d in descs}, scratch
+
+
+def test_small_graph_forms_only_where_they_pay():
+    toluene, scratch = _forms(P.nequip_problems()[2])
+    assert toluene["forward_split"][2] == 64 * 4 and scratch["forward_split"] == scratch["forward"] == 0
+    assert toluene["double_backward_A_split"][2] == 64 * 8
+    several_segments, _ = _forms(_f64(P.seven_net_problems()[1]))
+    assert "forward_split" not in several_segments and "double_backward_A_split" not in several_segments
+    assert several_segments["backward"][6] > 0
+    many_rows, _ = _forms(P.config1_single_uvu())  # 64 edges to a wave
+    assert not any("split" in name for name in many_rows)
+    assert many_rows["backward"][6] == many_rows["double_backward_B"][6] == 0
+    four_rows, _ = _forms(P.ChannelwiseTPP("16x0e+16x1o", "0e+1o", "16x0e+16x1o"))
+    assert four_rows["forward_split"][2] == 64 * 4 and four_rows["forward_split"][7] <= 640
