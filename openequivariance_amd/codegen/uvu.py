@@ -2412,7 +2412,7 @@ def _forward_plan(low: Lowered, first_budget: int) -> Tuple[UvuEmitter, bool]:
 
 
 def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kahan: bool = False,
-                override: Optional[Dict[str, int]] = None):
+                override: Optional[Dict[str, int]] = None, draft: bool = False):
     """Source + launch descriptors for the fused convolution (forward, backward).
 
     ``deterministic``: the caller passes receiver-sorted edges and the sender-major permutation; the
@@ -2427,7 +2427,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     reference (templates/loop_unroll_conv_det.cuh:70-94, 135-160, 227-271).
 
     ``override``: knob values that take precedence over ``OEQ_AMD_TUNE`` (the function's own second attempt,
-    see the end)."""
+    see the end). ``draft``: for a look at the source, without the rules for small graphs, which compile it."""
     from .. import runtime as rt
 
     assert not (deterministic and low.shared_weights), "deterministic convolution needs per-edge weights"
@@ -2706,7 +2706,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         # (forced on shapes beyond the rule, adjoint kernels with 200 - 320 B of scratch ran 3x slower than the terms)
         _lds, scratch = rt.kernel_resources(rt.compile_source(src)).get("backward_dx", (0, 0))
         if scratch > 64:
-            return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_dxs=0))
+            return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_dxs=0), draft)
     if em.seg_waves > 1 and "conv_segw" not in user_tune:
         # Waves that share a node's output segments: with two operand sets in flight and three or more segments
         # the compiler has been seen to need more registers for the kernel that selects a wave's segments by
@@ -2715,7 +2715,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         # The code object says so (compiled here, cached like any other): then one wave owns the node.
         _lds, scratch = rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))
         if scratch > 64:
-            return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_segw=0))
+            return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_segw=0), draft)
     if wide64_forward:
         # fp64 with a node's whole output row in one wave's 512 registers: the estimate that admits this plan is
         # optimistic for rows of 96 channels (two waves' lanes, the second half empty). With scratch memory the
@@ -2723,7 +2723,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         # 25.9 against 8.3 ms; 228 B, 15.4 / 8.7; 96x{0e,1o,2e}: 196 B, 11.3 / 6.8).
         _lds, scratch = rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))
         if scratch > 64:
-            return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wf=2))
+            return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wf=2), draft)
     if walk and t["conv_wf"] == 23 and "conv_wf" not in user_tune and low.elem_size == 4:
         # A forward kernel that the compiler gave more than a third of a SIMD's registers runs two waves there.
         # Held to a third it runs three, which pays where the compiler manages that without scratch memory (fp32,
@@ -2733,10 +2733,10 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         # The code objects say which it is (compiled here, cached like any other; of the second form only the
         # forward kernel).
         if rt.kernel_registers(rt.compile_source(src)).get("forward", 0) > 168:
-            third = conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wf=3))
-            if _forward_scratch(third[0]) == 0:
-                return third
-    if walk:
+            third = dict(override or {}, conv_wf=3)
+            if _forward_scratch(conv_module(low, deterministic, compute_units, kahan, third, draft=True)[0]) == 0:
+                return conv_module(low, deterministic, compute_units, kahan, third, draft)
+    if walk and not draft:
         # A small-graph form that needs scratch memory where the plain kernel does not: half as many waves leave each of
         # them twice the registers (toluene, fp32, 640 nodes x 30 edges: plain 59 us, eight waves with 48 B of scratch
         # 79, four without 46; 40 nodes 49 / 18 / 19). Not where that does not help either (nequip-uvu, fp64, second
