@@ -85,7 +85,7 @@ int timed_as(int role) {
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
-// Entries of the long-segment list that oeq_group_scan leaves behind a cursor array (the kernels in
+// Entries of the long-segment list that oeq_group_scan leaves behind the segment starts (the kernels in
 // codegen/common.py use the same number).
 constexpr int64_t OEQ_LONG_LIST = 126;
 
@@ -98,8 +98,8 @@ struct IndexSide {
 
 // Segments per tile of oeq_group_scan, and the blocks it gets per side (each sums what lies before its range).
 constexpr int64_t kScanTile = 1024, kScanBlocks = 32;
-// Largest edge list that oeq_index_small takes (its LDS; beyond it one block is also slower than the whole device:
-// 80 000 edges would be 80 per thread).
+// Largest edge list that oeq_index_small takes: its LDS arrays, of which every block holds histogram and item list of
+// the whole side (the blocks share out only the placing, so that their number squared is what a side costs).
 constexpr int64_t kSmallItems = 16384, kSmallSegments = 4096;
 
 }  // namespace
@@ -574,14 +574,14 @@ static int check_graph_size(const char* who, int64_t node_count, int64_t nnz) {
     return OEQ_OK;
 }
 
-// Shared weights, walk kernels: one partial weight-gradient row per wave group of the backward grid.
-// A segment-pointer (or cursor) array: n + 1 entries, and behind them the list of long segments that
-// oeq_group_scan leaves for oeq_group_order (a count and up to OEQ_LONG_LIST entries).
+// A segment-pointer array: n + 1 entries, and behind them the list of long segments that oeq_group_scan leaves for
+// oeq_group_order (a count and up to OEQ_LONG_LIST entries).
 static size_t ptr_bytes_of(int64_t node_count) {
     return align_up((size_t)(node_count + 1 + 1 + OEQ_LONG_LIST) * sizeof(int64_t), 256);
 }
 static size_t perm_bytes_of(int64_t nnz) { return align_up((size_t)nnz * sizeof(int64_t), 256); }
 
+// Shared weights, walk kernels: one partial weight-gradient row per wave group of the backward grid.
 static size_t conv_wpartial_bytes(const oeq_kernels* k, int64_t walk_positions, int role = OEQ_ROLE_CONV_BACKWARD) {
     if (!k->dims.shared_weights || !k->dims.wpartial_per_block || !k->roles[role].present) return 0;
     size_t rows = (size_t)k->grid_for(role, walk_positions) * (size_t)k->dims.wpartial_per_block;

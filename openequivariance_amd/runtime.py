@@ -622,9 +622,6 @@ class KernelSet:
     def conv_backward_workspace_bytes(self, nodes, nnz) -> int:
         return self._lib.oeq_conv_backward_workspace_bytes(self.handle, nodes, nnz)
 
-    def conv_double_backward_workspace_bytes(self, nodes, nnz) -> int:
-        return self._lib.oeq_conv_double_backward_workspace_bytes(self.handle, nodes, nnz)
-
     def conv_forward(self, nodes, nnz, x, y, w, out, rows, cols, ws, ws_bytes, stream):
         _check(self._lib.oeq_conv_forward(self.handle, nodes, nnz, x, y, w, out, rows, cols, ws, ws_bytes, stream),
                "oeq_conv_forward")
@@ -655,30 +652,6 @@ class KernelSet:
     def conv_forward_scratch_bytes(self, nodes, nnz) -> int:
         return self._lib.oeq_conv_forward_scratch_bytes(self.handle, nodes, nnz)
 
-    def conv_forward_indexed(self, nodes, nnz, x, y, w, out, rows, cols, index, index_bytes, sender_side, scratch,
-                             scratch_bytes, stream):
-        _check(self._lib.oeq_conv_forward_indexed(self.handle, nodes, nnz, x, y, w, out, rows, cols, index, index_bytes,
-                                                  int(sender_side), scratch, scratch_bytes, stream),
-               "oeq_conv_forward_indexed")
-
-    def conv_backward_scratch_bytes(self, nodes, nnz) -> int:
-        return self._lib.oeq_conv_backward_scratch_bytes(self.handle, nodes, nnz)
-
-    def conv_backward_indexed(self, nodes, nnz, x, dx, y, dy, w, dw, g, rows, cols, perm, index, index_bytes,
-                              sender_side, scratch, scratch_bytes, stream):
-        _check(self._lib.oeq_conv_backward_indexed(self.handle, nodes, nnz, x, dx, y, dy, w, dw, g, rows, cols, perm,
-                                                   index, index_bytes, int(sender_side), scratch, scratch_bytes,
-                                                   stream), "oeq_conv_backward_indexed")
-
-    def conv_double_backward_scratch_bytes(self, nodes, nnz) -> int:
-        return self._lib.oeq_conv_double_backward_scratch_bytes(self.handle, nodes, nnz)
-
-    def conv_double_backward_indexed(self, nodes, nnz, x, y, w, g, ddx, ddy, ddw, dx, dy, dw, gg, rows, cols, perm,
-                                     index, index_bytes, scratch, scratch_bytes, stream):
-        _check(self._lib.oeq_conv_double_backward_indexed(self.handle, nodes, nnz, x, y, w, g, ddx, ddy, ddw, dx, dy, dw,
-                                                          gg, rows, cols, perm, index, index_bytes, scratch,
-                                                          scratch_bytes, stream), "oeq_conv_double_backward_indexed")
-
     def has_double_backward(self) -> bool:
         return bool(self._lib.oeq_has_double_backward(self.handle))
 
@@ -688,15 +661,6 @@ class KernelSet:
     def tp_double_backward(self, n, x, y, w, g, ddx, ddy, ddw, dx, dy, dw, gg, ws, ws_bytes, stream):
         _check(self._lib.oeq_tp_double_backward(self.handle, n, x, y, w, g, ddx, ddy, ddw, dx, dy, dw, gg, ws,
                                                 ws_bytes, stream), "oeq_tp_double_backward")
-
-    def conv_double_backward(self, nodes, nnz, x, y, w, g, ddx, ddy, ddw, dx, dy, dw, gg, rows, cols, perm, ws,
-                             ws_bytes, stream):
-        _check(self._lib.oeq_conv_double_backward(self.handle, nodes, nnz, x, y, w, g, ddx, ddy, ddw, dx, dy, dw, gg,
-                                                  rows, cols, perm, ws, ws_bytes, stream), "oeq_conv_double_backward")
-
-    def conv_backward(self, nodes, nnz, x, dx, y, dy, w, dw, g, rows, cols, perm, ws, ws_bytes, stream):
-        _check(self._lib.oeq_conv_backward(self.handle, nodes, nnz, x, dx, y, dy, w, dw, g, rows, cols, perm, ws,
-                                           ws_bytes, stream), "oeq_conv_backward")
 
 
 _kernel_cache: Dict[str, KernelSet] = {}
