@@ -220,7 +220,9 @@ GraphSize conv_checks(const Entry& e, const Tensor& L1_in, const Tensor& L2_in, 
             "OpenEquivariance_conv_atomic does not have a deterministic implementation, but you set "
             "'torch.use_deterministic_algorithms(True)'. Use TensorProductConv(..., deterministic=True).";
         TORCH_CHECK(at::globalContext().deterministicAlgorithmsWarnOnly(), msg);
-        TORCH_WARN(msg);
+        // (a Python warning: TORCH_WARN from an op called directly would only print)
+        py::gil_scoped_acquire gil;
+        if (PyErr_WarnEx(PyExc_UserWarning, msg, 1) < 0) throw py::error_already_set();
     }
     return {nodes, nnz};
 }

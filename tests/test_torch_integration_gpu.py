@@ -244,3 +244,25 @@ def test_conv_under_inference_mode():
             z2 = conv(tX, tY, tW, tr, tc, tp if det else None)
         assert err(z, z_ref) <= 1e-5 and torch.equal(z, z2)
         assert not ops._index_cache, "nothing is kept for tensors whose changes cannot be seen"
+
+
+def test_nondeterministic_calls_warn_or_raise(monkeypatch):
+    """torch.use_deterministic_algorithms: calls that use float atomics are errors, or Python warnings with warn_only,
+    in both directions."""
+    monkeypatch.setenv("OEQ_AMD_TUNE", "conv_sort=0")
+    problem = P.config1_single_uvu()
+    conv = oeq.TensorProductConv(problem, deterministic=False)
+    x, y, w = (torch.randn(4, n, device="cuda", requires_grad=True)
+               for n in (problem.irreps_in1.dim, problem.irreps_in2.dim, problem.weight_numel))
+    edges = [torch.tensor([0, 1, 2, 3], device="cuda") for _ in range(2)]
+    try:
+        torch.use_deterministic_algorithms(True, warn_only=True)
+        with pytest.warns(UserWarning, match="deterministic implementation"):
+            z = conv(x, y, w, *edges)
+        with pytest.warns(UserWarning, match="deterministic implementation"):
+            z.sum().backward()
+        torch.use_deterministic_algorithms(True)
+        with pytest.raises(RuntimeError, match="deterministic implementation"):
+            conv(x, y, w, *edges)
+    finally:
+        torch.use_deterministic_algorithms(False)
