@@ -1,6 +1,6 @@
 """Small-graph forms of the convolution kernels: a node's edges dealt out to several waves of a block (forward-shaped
 kernels, summed through LDS) or to several walk positions (backward-shaped kernels), against the plain kernels of the
-same problem, which the oracle tests cover. Degrees from none over fewer than there are waves to a segment cut into
+same problem and, on the smallest graphs, the oracle. Degrees from none over fewer than there are waves to a segment cut into
 chunks; every kernel structure that has such a form."""
 
 import numpy as np
@@ -14,6 +14,7 @@ from openequivariance_amd.core.graph import CoordGraph
 
 from gpu_util import err, to_gpu
 from oracle import e3nn_ref as R
+from oracle.torch_ref import TorchConv
 
 pytestmark = pytest.mark.gpu
 
@@ -45,7 +46,7 @@ def _graph(n, seed, hub):
     rows = np.repeat(np.arange(n), deg)
     cols = rng.integers(0, n, size=len(rows))
     if hub:
-        cols[rng.permutation(len(rows))[:hub]] = 1
+        cols[rng.permutation(len(rows))[:hub]] = min(1, n - 1)
     return CoordGraph(np.zeros((n, 3)), rows.astype(np.int64), cols.astype(np.int64))
 
 
@@ -79,7 +80,8 @@ def test_small_forms_match_the_plain_kernels(name, tune, n, hub, monkeypatch):
     shapes = [(n, dims[0]), (g.nnz, dims[1]), (g.nnz, dims[2]), (n, dims[3]), (n, dims[0]), (g.nnz, dims[1]),
               (g.nnz, dims[2])]
     tensors = [torch.randn(*s, device="cuda", dtype=dt, generator=gen) for s in shapes]
-    plain = _run(problem, "conv_fsplit=0,conv_parts=0", det, g, tensors, monkeypatch)
+    # (the same source as the default knobs': one compilation for both)
+    plain = _run(problem, "conv_fsmax=0,conv_parts=0", det, g, tensors, monkeypatch)
     small = _run(problem, tune, det, g, tensors, monkeypatch)
     tol = 1e-12 if dt == torch.float64 else 1e-5
     for i, (got, want) in enumerate(zip(small, plain)):
@@ -87,6 +89,14 @@ def test_small_forms_match_the_plain_kernels(name, tune, n, hub, monkeypatch):
         assert float((got - want).abs().max()) / scale <= tol, (name, i)
     # results per edge do not depend on which position walks the edge
     assert torch.equal(small[2], plain[2]) and torch.equal(small[3], plain[3])
+    if n <= 40 and g.nnz < 1000:
+        x, y, w, gr, a, b, c = (t.double().cpu() for t in tensors)
+        leaves = [t.requires_grad_() for t in (x, y, w)]
+        z = TorchConv(R.Problem.from_spec(problem), torch.float64)(*leaves, torch.tensor(g.rows), torch.tensor(g.cols))
+        first = torch.autograd.grad(z, leaves, gr.requires_grad_(), create_graph=True)
+        second = torch.autograd.grad(first, [*leaves, gr], [a, b, c], allow_unused=True)
+        for i, (got, want) in enumerate(zip(small, (z, *first, *second))):
+            assert err(got, want.detach().numpy()) <= tol, (name, i)
 
 
 @pytest.mark.parametrize("in1,in2,out", [("64x0e", "1x4e", "64x4e"), ("64x0e", "1x0e+1x2e+1x4e", "64x0e+64x2e+64x4e"),
