@@ -2190,8 +2190,6 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
             s("E_t A, B;")
         if mode in (2, 4):
             floats = self.stage["floats"] + (self.stage["nqw"] * 256 if mode == 4 else 0)
-            if split > 1:
-                floats = self._split_slice(True)
             s(f"__shared__ __attribute__((aligned(16))) T s_stage[{self.NCH * G}][{floats}];")
             self._emit_stage_offsets(s)
         if mode == 3:
