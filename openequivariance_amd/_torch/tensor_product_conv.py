@@ -50,7 +50,7 @@ def build_conv_module(problem: TPProblem, deterministic: bool, kahan: bool = Fal
     # segment sum scatters the result, like the reference's unfused convolution
     # (core/ConvolutionBase.py:292-301, _torch/TensorProductConv.py:595-640).
     cu = compute_units()
-    src, dims, descs = uvw.tp_module(low, cu, kahan)
+    src, dims, descs = uvw.tp_module(low, cu, kahan, edge_lists=True)
     descs = list(descs) + [(rt.ROLE_SEGMENT_PTR, "oeq_segment_ptr", 256, 256, cu * 16),
                            (rt.ROLE_SEGMENT_SUM, "oeq_segment_sum", 256, 1, cu * 32),
                            (rt.ROLE_GROUP_COUNT, "oeq_group_count", 256, 256, cu * 16),

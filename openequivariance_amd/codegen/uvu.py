@@ -2358,7 +2358,7 @@ def tp_module(low: Lowered, compute_units: int = 256):
     em.tr_stores = t["tp_trs"]
     s = Src()
     s(prelude(low.ctype))
-    s(utility_kernels())
+    s(utility_kernels(edge_lists=False))
     em.emit_structs(s)
     em.emit_forward_cores(s, preloaded=False)
     G_f, G_b = t["tp_gf"], (1 if em.NCH > 1 else t["tp_gb"])
@@ -2526,7 +2526,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     em.prefetch_runs = bool(t["conv_pf"])
     s = Src()
     s(prelude(low.ctype))
-    s(utility_kernels(kahan))
+    s(utility_kernels(kahan, sorted_lists=deterministic))
     # position in the walk -> edge index: through the library's grouping when there is one
     s("#define OEQ_EDGE(j) (eperm ? eperm[(j)] : (j))")
     em.emit_structs(s)

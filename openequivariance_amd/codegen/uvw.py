@@ -1240,7 +1240,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     em = UvwEmitter(low)
     s = Src()
     s(prelude(low.ctype))
-    s(utility_kernels(kahan))
+    s(utility_kernels(kahan, sorted_lists=deterministic))
     s("#define OEQ_EDGE(j) (eperm ? eperm[(j)] : (j))")
     for n in (1, 2, 4):
         s(f"typedef T oeq_wvec{n} __attribute__((ext_vector_type({n})));")
@@ -1286,19 +1286,20 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     return s.text(), dims, descs
 
 
-def tp_module(low: Lowered, compute_units: int = 256, kahan: bool = False):
-    """``kahan`` only affects the ordered segment sum used by the unfused convolution."""
+def tp_module(low: Lowered, compute_units: int = 256, kahan: bool = False, edge_lists: bool = False):
+    """``edge_lists``: with the kernels that the unfused convolution adds; ``kahan`` only affects its ordered segment
+    sum."""
     from .. import runtime as rt
 
     if low.shared_weights and not kahan:
         from . import uvw_mfma
         from .uvu import tuning
         if uvw_mfma.supported(low) and tuning(dict(uvw_mfma=1))["uvw_mfma"]:
-            return uvw_mfma.tp_module(low, compute_units)
+            return uvw_mfma.tp_module(low, compute_units, edge_lists)
     em = UvwEmitter(low)
     s = Src()
     s(prelude(low.ctype))
-    s(utility_kernels(kahan))
+    s(utility_kernels(kahan, edge_lists))
     blk_f = em.emit_forward(s)
     blk_b = em.emit_backward(s)
     max_blocks_b = compute_units * (3 if em.shared_lds else 2)

@@ -1211,7 +1211,7 @@ class MfmaEmitter:
         return names_a, names_b
 
 
-def tp_module(low: Lowered, compute_units: int = 256):
+def tp_module(low: Lowered, compute_units: int = 256, edge_lists: bool = False):
     from .. import runtime as rt
 
     em = MfmaEmitter(low)
@@ -1246,7 +1246,7 @@ def tp_module(low: Lowered, compute_units: int = 256):
     # quad_perm otherwise)
     s("template <int CTRL> OEQ_DEV float oeq_dpp(float v) { return __builtin_bit_cast(float, "
       "__builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true)); }")
-    s(utility_kernels())
+    s(utility_kernels(edge_lists=edge_lists))
     em._emit_path_fns(s)
     fwd_names = em.emit_forward(s)
     bwd_names = em.emit_backward(s)
