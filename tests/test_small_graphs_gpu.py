@@ -66,7 +66,7 @@ def _run(problem, tune, det, g, tensors, monkeypatch):
 @pytest.mark.parametrize("name", list(PROBLEMS))
 @pytest.mark.parametrize("tune,n,hub", [("", 1, 5), ("", 33, 300), ("conv_fsplit=2,conv_parts=3", 40, 0),
                                         ("conv_fsmax=100000,conv_parts=16", 700, 600),
-                                        # two waves a node: segments walked whole up to 512 nodes; many parallel edges: in chunks
+                                        # two waves a node, a node that is walked in chunks, walk positions before and past a block
                                         ("conv_fsplit=2,conv_fsmax=4000", 512, 700),
                                         ("conv_fsplit=2,conv_fsmax=4000", 513, 700),
                                         ("", 3, 900)])
