@@ -33,7 +33,7 @@ import os
 import re
 from typing import Callable, Dict, List, NamedTuple, Optional, Sequence, Tuple
 
-from .common import Src, fixup_backward_kernel, prelude, utility_kernels
+from .common import LOOK_AHEAD, Src, fixup_backward_kernel, prelude, utility_kernels
 from .lower import Lowered, Path, float_literal
 
 UNROLL_V_LIMIT = 8
@@ -143,6 +143,7 @@ class UvuEmitter:
         self.q_slot: Dict[Tuple[int, int, str, int], int] = {}  # (path, v, |c| literal, j) -> slot
         self.stage = self._stage_layout()
         self.stage3 = self._stage3_layout()
+        self.rows_stage = self._rows_stage_layout()
 
     def _stage_layout(self):
         """Layout of one wave's LDS staging buffer for the operands of an edge
@@ -249,6 +250,74 @@ class UvuEmitter:
         else:
             for j in range(low.L2):
                 s(f"{buf}.y[{j}] = yn[{j}];")
+
+    # ---- staging of whole rows: several edges to a wave --------------------------------
+    def _rows_stage_layout(self):
+        """Layout of one wave's LDS staging buffer where a wave walks two edges side by side (blocks of 17 to 32
+        channels): the rows of X[sender] and W[edge] of its edges, each row from an instruction boundary on, and their Y
+        rows. None where rows are no multiple of 16 bytes.
+
+        Loaded by the lanes, a pair of edges takes a 4-byte load per value (NequIP lips: 57 of them, the 63 that a wave
+        can have outstanding), and two operand sets beside 102 accumulators do not fit the registers, so that the
+        outputs were walked in two passes over X. 16-byte loads into LDS are 14 for the same rows and need no second
+        operand set. What is left is the W stream: NequIP lips, 5 000 nodes x 28 edges, ir_mul, forward 165 -> 138 us
+        (5.3 TB/s of W while a node's edges are walked, and 11 us per node until the first edge has arrived and the row
+        is stored); 3 000 x 28 127 / 96, 700 x 40 69 / 38; nequip-uvu 20 000 x 30 346 / 273; water 1 500 x 35 34 / 26,
+        50 000 x 20 336 / 325; the same in double precision, nequip-uvu 3 000 x 30 110 / 89."""
+        low, es = self.low, self.low.elem_size
+        if not (self.R == 2 and self.can_preload and len(self.segments) == 1 and not low.shared_weights):
+            return None
+        if low.L2 > self.LPR or low.L1 * es % 16 or low.WN * es % 16:
+            return None
+        nqx, nqw = -(-low.L1 * es // 1024), -(-low.WN * es // 1024)
+        y = -(-low.L2 // 4) * 4
+        XF, row = nqx * 1024 // es, (nqx + nqw) * 1024 // es
+        return dict(nqx=nqx, nqw=nqw, XF=XF, row=row, y=y, floats=self.R * (row + y))
+
+    def _emit_rows_issue(self, s: Src, e: str, last: str, step: int):
+        """Request the operands of the wave's next R edges, positions ``e`` .. ``e`` + R - 1 of the walk. Their numbers
+        and senders come from the lanes, which hold those of 64 edges of the wave."""
+        low, st, R, es = self.low, self.rows_stage, self.R, self.low.elem_size
+        s.open("")
+        s(f"if ((handed & 63) == 0) oeq_look_ahead(ahead, {e} + (i64)(lane / {R}) * {step} + lane % {R}, {last}, "
+          "eperm, cols, node_count);")
+        s("const int at = handed & 63;")
+        def request(r: int, index: str, row: str, n: int, numel: int, lds: int, aux: int):
+            s.open(f"if ({e} + {r} < {last})" if r else "")
+            s(f"const T* row = {row} + (i64)__builtin_amdgcn_readlane(ahead.{index}, at + {r}) * {numel};")
+            for q in range(n):
+                # (lanes beyond the row repeat its last 16 bytes into the padding)
+                end = numel * es - 16 - q * 1024
+                off = "lane * 16u" if end >= 63 * 16 else f"(lane * 16u < {end}u ? lane * 16u : {end}u)"
+                s(f"__builtin_amdgcn_global_load_lds((const OEQ_GPTR)oeq_at(row + {q * 1024 // es}, {off}), "
+                  f"(OEQ_LPTR)(&s_stage[wave][{r * st['row'] + lds + q * 1024 // es}]), 16, 0, {aux});")
+            s.close()
+
+        # (weights and Y first: their addresses need the edge's number only, the senders are a load behind it)
+        for r in range(R):
+            request(r, "eid", "W", st["nqw"], low.WN, st["XF"], 2 if self.nt & 1 else 0)
+        s(f"yn = L2_in[(i64)__shfl(ahead.eid, at + r) * {low.L2} + (ul < {low.L2} ? ul : {low.L2 - 1})];")
+        for r in range(R):
+            request(r, "sender", "L1_in", st["nqx"], low.L1, 0, 0)
+        s(f"handed += {R};")
+        s.close()
+
+    def _emit_rows_read(self, s: Src, buf: str):
+        low, st = self.low, self.rows_stage
+        s(f"T* const sr = &s_stage[wave][0] + r * {st['row']};")
+        s(f"T* const sy = &s_stage[wave][{self.R * st['row']}] + r * {st['y']};")
+        s(f"if (ul < {low.L2}) sy[ul] = yn;")
+        for b in self.used_in1:
+            (off, ls), cs = self._lane_ptr(low.in1[b])
+            for i in range(low.in1[b].d):
+                s(f"{buf}.x.b{b}[{i}] = sr[{off + i * cs} + ul * {ls}];")
+        for p in low.paths:
+            V = low.in2[p.i2].mul
+            for v in range(V):
+                s(f"{buf}.w[{self.wslot[p.index] + v}] = sr[{st['XF'] + p.woff + v} + ul * {V}];")
+        s("oeq_wave_sync();")
+        for j in range(low.L2):
+            s(f"{buf}.y[{j}] = sy[{j}];")
 
     # ---- double-buffered staging: X, W and Y of an edge live only in LDS ------------
     def _stage3_layout(self):
@@ -655,6 +724,8 @@ class UvuEmitter:
     # ------------------------------------------------------- shared structs
     def emit_structs(self, s: Src):
         low = self.low
+        if self.rows_stage is not None:
+            s(LOOK_AHEAD)
         s("struct X_t {")
         for b in self.used_in1:
             s(f"    T b{b}[{low.in1[b].d}];")
@@ -913,6 +984,52 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
                     s(f"zp[{k * st}] = a.o{io}[{k}];")
             s.close()
 
+    def _fold_store(self, s: Src, si: int, rowexpr: str):
+        """Sum of the R lane groups' accumulators of segment ``si`` and its store, R values at a time: every step of the
+        sum halves what a lane still holds, so each lane group ends up with one of the values and stores it (a lane
+        exchange and a store for R values; the terms are added in the order of the lane groups, as by a butterfly of
+        every value)."""
+        low = self.low
+        vals = [(io, k) for io in self._out_of(self.segments[si]) for k in range(low.out[io].d)]
+        # (opaque copies: the compiler would otherwise form every store's offset before the edge loop and keep it)
+        s("int fr = r, fu = u;")
+        s('asm volatile("" : "+v"(fr), "+v"(fu));')
+        for n in range(0, len(vals), self.R):
+            group = vals[n:n + self.R]
+            s.open("")
+            names = []
+            for q in range(self.R):
+                names.append(f"v{q}")
+                io, k = group[min(q, len(group) - 1)]
+                s(f"T v{q} = a.o{io}[{k}];")
+            m = self.LPR
+            while m < 64:
+                half = len(names) // 2
+                s.open("")
+                s(f"const bool hi = (lane & {m}) != 0;")
+                # (lane group bit m chooses between neighbouring values: group r is left with value r)
+                for q in range(half):
+                    s(f"{{ const T keep = hi ? v{2 * q + 1} : v{2 * q}, send = hi ? v{2 * q} : v{2 * q + 1}; "
+                      f"v{q} = keep + __shfl_xor(send, {m}); }}")
+                s.close()
+                names = names[:half]
+                m *= 2
+            off, cond = None, None
+            for q in range(len(group) - 1, -1, -1):
+                io, k = group[q]
+                (o, ls), cs = self._lane_ptr(low.out[io])
+                code, c = f"{o + k * cs} + fu * {ls}", self._store_cond(low.out[io].mul) or "true"
+                off = code if off is None else f"fr == {q} ? {code} : ({off})"
+                cond = c if cond is None or cond == c else f"(fr == {q} ? {c} : {cond})"
+            if len(group) < self.R:
+                cond = f"fr < {len(group)}" if cond == "true" else f"fr < {len(group)} && {cond}"
+            s('asm volatile("" : "+v"(v0));')
+            s.open(f"if ({cond})" if cond != "true" else "")
+            s(f"T* zp = {rowexpr} + ({off});")
+            s("__builtin_nontemporal_store(v0, zp);" if self.nt & 8 else "*zp = v0;")
+            s.close()
+            s.close()
+
     def _zero_untouched_out(self, s: Src, rowexpr: str, guard: str):
         """Output blocks no instruction writes are still part of the row."""
         low = self.low
@@ -1009,7 +1126,7 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         two operand sets (A, B); the next edge's loads are issued before the current edge is
         computed. ``load(buf, e)`` / ``compute(buf, e)`` emit code."""
         R = self.R * split
-        assert split == 1 or pipelined <= 2
+        assert split == 1 or pipelined in (0, 1, 2, 5)
         # The compiler takes a direct global->LDS load to write only the bytes at the pointer it is given,
         # not the 64 lanes' worth behind it, so it would move reads of the staging buffer across the load
         # or across the wait for it. The empty asm statements pin them: no memory access crosses one.
@@ -1089,6 +1206,25 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
             s("++e; wpar ^= 1;")
             s.close()
             return
+        if pipelined == 5:
+            # rows of R edges: one LDS buffer per wave, copied to registers before the next rows are requested
+            s("oeq_ahead ahead; int handed = 0;")
+            s("T yn = T(0);")
+            s(f"i64 e = {first};")
+            s(f"if (e < {last})")
+            self._emit_rows_issue(s, "e", last, R)
+            s.open(f"while (e < {last})")
+            s(vmcnt(0))
+            self._emit_rows_read(s, "A")
+            s(lgkm0)
+            s(f"if (e + {R} < {last})")
+            self._emit_rows_issue(s, f"(e + {R})", last, R)
+            s.open(f"if (e + r < {last})")
+            compute("A", "e")
+            s.close()
+            s(f"e += {R};")
+            s.close()
+            return
         if pipelined == 2:
             # one LDS buffer per wave, copied to registers before the next edge's loads are issued
             s(f"T yn[{self.q_slabs if self.use_q else self.low.L2}];")
@@ -1141,15 +1277,18 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         s(f"e += {2 * R};")
         s.close()
 
-    def _edge_mode(self, pipelined: int) -> int:
+    def _edge_mode(self, pipelined: int, rows: bool = False) -> int:
         """0: load, then compute; 1: next edge's operands prefetched into a second register set;
-        2: next edge's operands prefetched into the wave's LDS staging buffer."""
+        2: next edge's operands prefetched into the wave's LDS staging buffer; 5: likewise where a wave walks several
+        edges side by side (``rows``: by kernels that can)."""
         if pipelined == 3 and self.stage3 is not None and not self.use_q:
             return 3
         if pipelined == 4 and self.stage is not None and self.R == 1:
             return 4
         if pipelined >= 2 and self.stage is not None:
             return 2
+        if pipelined >= 2 and rows and self.rows_stage is not None:
+            return 5
         if pipelined and self.can_preload:
             return 1
         return 0
@@ -1276,20 +1415,31 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
                     s(f"if ({cond}) for (int t = 0; t < {missing}; ++t) __syncthreads();")
 
     def _split_mode(self, pipelined: int) -> int:
-        mode = self._edge_mode(pipelined)
-        return self._edge_mode(2) if mode > 2 else mode
+        """Edge mode of a small-graph form. Its waves have an edge or two each, so what counts is the latency of the
+        first: rows by way of LDS only where two operand sets do not fit the registers beside the accumulators
+        (several edges to a wave; plain loads / staged rows: NequIP water, 1 000 nodes x 20 edges, sender walk 15 / 22
+        us, forward 500 x 20 12 / 14; lips, whose outputs plain loads take two passes for, 400 x 20 28 / 19)."""
+        mode = self._edge_mode(pipelined, rows=self.operand_words(2) > 170)
+        return self._edge_mode(2) if mode in (3, 4) else mode
+
+    def operand_words(self, sets: int) -> int:
+        """Registers of a forward kernel's accumulators and ``sets`` operand sets of an edge."""
+        low = self.low
+        return self.words * (sum(low.out[io].d for io in self.used_out)
+                             + sets * (sum(low.in1[b].d for b in self.used_in1) + low.L2 + self.n_wslots))
 
     def _split_slice(self, staged: bool) -> int:
         """Elements of a wave's LDS slice for its accumulators: the wave's staging buffer where it has one, and in any
         case the widest output block (64x0e x 1x4e -> 64x4e: 576 elements beside a staging buffer of 512)."""
         widest = max(self.low.out[io].d for io in self.used_out)
-        return max(self.stage["floats"] if staged else self.SPLIT_WORDS // self.words * 64, widest * 64)
+        buffer = (self.stage or self.rows_stage)["floats"] if staged else self.SPLIT_WORDS // self.words * 64
+        return max(buffer, widest * 64)
 
     def split_count(self, n: int, pipelined: int, segw: int = 1) -> int:
         """How many waves a node's edges can be dealt out to, ``n`` or a half, a quarter ... of it: every wave has an LDS
         slice for an edge's operands and its accumulators, and a wide problem's do not all fit a CU (the sender walk of
         128x{0e,1o,2e} with l <= 3 harmonics: 31 KB a wave)."""
-        wave = self._split_slice(self._split_mode(pipelined) == 2)
+        wave = self._split_slice(self._split_mode(pipelined) in (2, 5))
         if self.tr_stores & 1 and self.R == 1:
             wave += 64 * max(self.low.out[io].d for io in self.used_out)
         while n > 1 and self.NCH * segw * n * wave * self.low.elem_size > LDS_LIMIT:
@@ -1310,7 +1460,7 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         R = self.R
         # weights two edges ahead: only where the loop body issues no stores or atomics (they share the
         # vector-memory counter with the loads the loop waits for by count)
-        mode = self._edge_mode(pipelined if (deterministic or pipelined != 4) else 2)
+        mode = self._edge_mode(pipelined if (deterministic or pipelined != 4) else 2, rows=deterministic)
         if split > 1:
             mode = self._split_mode(pipelined)
         s.open(
@@ -1334,6 +1484,9 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
                 floats = self._split_slice(True)
             s(f"__shared__ __attribute__((aligned(16))) T s_stage[{self.NCH * G * split}][{floats}];")
             self._emit_stage_offsets(s)
+        if mode == 5:
+            floats = self._split_slice(True) if split > 1 else self.rows_stage["floats"]
+            s(f"__shared__ __attribute__((aligned(16))) T s_stage[{G * split}][{floats}];")
         if mode == 3:
             for b in "AB":
                 s(f"__shared__ __attribute__((aligned(16))) T s_stage{b}[{self.NCH * G}][{self.stage3['floats']}];")
@@ -1380,8 +1533,8 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
             if split > 1:
                 s.open("")
                 s("const int g = 0;")
-                self.split_stride = self._split_slice(mode == 2)
-                if mode == 2:  # (the edge's staging buffers are free by then)
+                self.split_stride = self._split_slice(mode in (2, 5))
+                if mode in (2, 5):  # (the edge's staging buffers are free by then)
                     s("T* const s_red = &s_stage[0][0];")
                 else:
                     s(f"__shared__ T s_red[{block // 64 * self.split_stride}];")
@@ -1397,8 +1550,12 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
                     s(f"A{si}_t a; zero_seg{si}(a);")
                     if kahan:
                         s(f"A{si}_t c; zero_seg{si}(c);")
-                    self._edge_loop(s, f"e0 + part * {R} + r" if split > 1 else "e0 + r", "e1", make_load(si),
+                    first = f"e0 + part * {R}" if split > 1 else "e0"
+                    self._edge_loop(s, first if mode == 5 else first + " + r", "e1", make_load(si),
                                     make_compute(si), mode, split=split)
+                    if R > 1 and split == 1:
+                        self._fold_store(s, si, "zrow")
+                        return
                     if R > 1:
                         # fold the R lane groups (fixed order) into group 0
                         for io in self.segments[si]:
@@ -2395,7 +2552,7 @@ def _forward_plan(low: Lowered, first_budget: int) -> Tuple[UvuEmitter, bool]:
         return e, need + (40 if e.ragged() else 0)
 
     e = UvuEmitter(low, acc_budget_words=first_budget)
-    if e.stage is not None or not e.can_preload:
+    if e.stage is not None or e.rows_stage is not None or not e.can_preload:
         return e, True
     budgets = (first_budget, 96, 64, 48)
     for budget in budgets:
@@ -2474,7 +2631,8 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     if wide64 and not any(k in user_tune for k in ("conv_wb", "conv_gres", "conv_split")):
         if 240 < em.backward_words(True) <= 480:
             t["conv_wb"], t["conv_gres"], t["conv_split"] = 1, 1, 0
-    if em.stage is None and em.can_preload and "conv_acc" not in user_tune and t["conv_acc"] < (1 << 20):
+    if (em.stage is None and em.rows_stage is None and em.can_preload and "conv_acc" not in user_tune
+            and t["conv_acc"] < (1 << 20)):
         # Forward without LDS staging keeps two operand sets of an edge (X blocks, the weights of the
         # output segment's paths, Y) beside the accumulators: shrink the segments until that fits, and
         # give up the prefetch when even 48-word segments do not.
@@ -2498,6 +2656,11 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
                 em, need = plan(budget, 1)
                 if need <= 190:
                     break
+    if walk and em.rows_stage is not None:
+        # (one node per block and two waves per SIMD, what the registers and 6 to 14 KB of LDS per wave leave room for)
+        for knob, value in (("conv_wf", 2), ("conv_gf", 1)):
+            if knob not in user_tune:
+                t[knob] = value
     em.nt = t["conv_nt"]
     em.mask_loads = bool(t["tp_mask"])
     em.forms = bool(t["tp_forms"])
@@ -2651,8 +2814,10 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
             ex.emit_structs(s)
             ex.use_q = False
             ex.emit_forward_cores(s, preloaded=True)
-            G_x = max(1, 4 // low_x.n_chunks)
-            waves_x = t["conv_wx"] if t["conv_wx"] else (-2 if words_x <= 48 else 2)
+            G_x = 1 if ex.rows_stage is not None else max(1, 4 // low_x.n_chunks)
+            # (rows staged in LDS: one operand set in registers, so that a fourth wave per SIMD costs nothing)
+            small = -4 if ex.rows_stage is not None else -2
+            waves_x = t["conv_wx"] if t["conv_wx"] else (small if words_x <= 48 else 2)
             blk_x = ex.emit_conv_forward(s, G_x, True, t["conv_pipe_f"] if pipe_x else 0, waves_x,
                                          xcd, bool(t["conv_tra"]), name="backward_dx")
             descs.append((rt.ROLE_CONV_BACKWARD_DX, "backward_dx", blk_x, G_x, 0, xcd))

@@ -1,0 +1,70 @@
+"""Convolution kernels whose waves walk two edges side by side with the edges' rows staged in LDS, against the oracle:
+rows of less than an instruction's 1 024 bytes, of whole instructions and with a rest, blocks without a channel for every
+lane, several channels in the second operand; segments without an edge, with odd and even numbers, on either side of the
+64 edges whose numbers a wave holds, and cut into chunks."""
+
+import numpy as np
+import pytest
+
+import openequivariance_amd as oeq
+from openequivariance_amd.codegen.lower import lower
+from openequivariance_amd.codegen.uvu import UvuEmitter
+from openequivariance_amd.core import problems as P
+from openequivariance_amd.core.graph import CoordGraph
+from openequivariance_amd.core.layout import transpose_irrep_layout
+
+from gpu_util import err, to_gpu, tol_of
+from oracle import e3nn_ref as R
+
+PROBLEMS = {
+    "short": ("32x0e", "0e+1o", "0e+1o"),                            # 128 and 256 bytes
+    "whole": ("32x0e+32x1o+32x0o+32x1e", "0e+1o", "0e+1o+1e"),       # X: one instruction
+    "rest": ("32x0e+32x1o+32x2e", "0e+1o+2e", "0e+1o+2e"),
+    "ragged": ("20x0e+32x1o+4x2e", "0e+1o", "0e+1o+2e"),
+    "channels": ("32x0e+32x1o", "2x0e+3x1o", "0e+1o"),
+    "lips": None,
+}
+DEGREES = [0, 1, 2, 3, 31, 63, 64, 65, 0, 128, 129, 300, 5, 0]
+
+
+def _problem(name, dtype, layout):
+    p = P.nequip_problems()[0] if name == "lips" else P.ChannelwiseTPP(*PROBLEMS[name])
+    p.irrep_dtype = p.weight_dtype = dtype
+    p.layout = layout
+    return p
+
+
+@pytest.mark.parametrize("name", ["rest", "ragged", "channels", "lips"])
+def test_these_problems_stage_their_rows(name):
+    assert UvuEmitter(lower(_problem(name, np.float32, "mul_ir"))).rows_stage is not None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(PROBLEMS))
+@pytest.mark.parametrize("dtype,layout,det,tune", [
+    (np.float32, "mul_ir", True, "conv_fsmax=0"), (np.float32, "ir_mul", False, "conv_fsmax=0,conv_dxs=1"),
+    (np.float64, "mul_ir", False, "conv_fsmax=0,conv_dxs=1"), (np.float32, "mul_ir", False, "conv_fsplit=4")])
+def test_against_the_oracle(name, dtype, layout, det, tune, monkeypatch):
+    problem = _problem(name, dtype, layout)
+    n = len(DEGREES)
+    rng = np.random.default_rng(7)
+    rows = np.repeat(np.arange(n), DEGREES)
+    cols = np.where(rng.random(len(rows)) < 0.3, 4, rng.integers(0, n, size=len(rows)))
+    g = CoordGraph(np.zeros((n, 3)), rows.astype(np.int64), cols.astype(np.int64))
+    x, y, w, gz = (rng.normal(size=s).astype(dtype) for s in (
+        (n, problem.irreps_in1.dim), (g.nnz, problem.irreps_in2.dim), (g.nnz, problem.weight_numel),
+        (n, problem.irreps_out.dim)))
+    ref = R.Problem.from_spec(_problem(name, dtype, "mul_ir"))  # (the oracle works in mul_ir)
+    ref_z = R.conv_forward(ref, x, y, w, g.rows, g.cols)
+    ref_dx, ref_dy, ref_dw = R.conv_backward(ref, x, y, w, gz, g.rows, g.cols)
+    i1, i2, io = problem.irreps_in1, problem.irreps_in2, problem.irreps_out
+    x, y, gz, ref_z, ref_dx, ref_dy = (transpose_irrep_layout(a, irreps, "mul_ir", layout) for a, irreps in (
+        (x, i1), (y, i2), (gz, io), (ref_z, io), (ref_dx, i1), (ref_dy, i2)))
+    monkeypatch.setenv("OEQ_AMD_TUNE", tune)
+    conv = oeq.TensorProductConv(problem, deterministic=det)
+    tx, ty, tw = to_gpu(x, y, w, requires_grad=True)
+    r, c, perm, tg = to_gpu(g.rows, g.cols, g.transpose_perm, gz)
+    z = conv(tx, ty, tw, r, c, perm) if det else conv(tx, ty, tw, r, c)
+    z.backward(tg)
+    for got, want in ((z, ref_z), (tx.grad, ref_dx), (ty.grad, ref_dy), (tw.grad, ref_dw)):
+        assert err(got, want) <= tol_of(problem)
