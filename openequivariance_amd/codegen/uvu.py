@@ -58,7 +58,7 @@ def tuning(defaults: dict) -> dict:
 
 class UvuEmitter:
     def __init__(self, low: Lowered, *, acc_budget_words: int = 128, g_resident_words: int = 128,
-                 kahan: bool = False):
+                 kahan: bool = False, stage_segments: bool = False):
         assert low.mode == "uvu"
         assert low.n_chunks <= 16, "blocks of more than 1024 channels are cut into pieces by codegen.lower"
         self.low = low
@@ -89,6 +89,8 @@ class UvuEmitter:
         self.tr_stores = 0
         self.T = low.ctype
         self.words = 1 if low.elem_size == 4 else 2
+        self.unit = 16 // low.elem_size  # elements of a 16-byte load; 2 ** unit_bits of these are 64 elements
+        self.unit_bits = (64 // self.unit).bit_length() - 1
         self.LPR = low.lanes_per_row
         self.R = low.rows_per_wave
         self.NCH = low.n_chunks
@@ -141,43 +143,51 @@ class UvuEmitter:
         self.q_ahead = (64, 64)  # multiply-adds between the request of a path's products and their use (fwd, bwd)
         self.q_entries: List[Tuple[int, float]] = []  # table slot -> (index into the Y row, coefficient)
         self.q_slot: Dict[Tuple[int, int, str, int], int] = {}  # (path, v, |c| literal, j) -> slot
-        self.stage = self._stage_layout()
+        # one layout per output segment (the waves that share a node's segments stage what theirs need)
+        self.stages = self._stage_layouts(stage_segments)
+        self.stage = self.stages[0] if self.stages else None
         self.stage3 = self._stage3_layout()
         self.rows_stage = self._rows_stage_layout()
 
-    def _stage_layout(self):
+    def _stage_layouts(self, several: bool):
         """Layout of one wave's LDS staging buffer for the operands of an edge
-        (the wave's 64-channel slice of X[sender] and of W[edge]), filled by
-        direct global->LDS loads of 16 B per lane. None when the problem does not
+        (the wave's 64-channel slice of X[sender] and of W[edge], as far as an output segment needs them), filled by
+        direct global->LDS loads of 16 B per lane; per segment. None when the problem does not
         have the regular shape this needs."""
         low = self.low
-        if not (self.R == 1 and self.can_preload and self.words == 1 and len(self.segments) == 1
+        if not (self.R == 1 and self.can_preload and (several or len(self.segments) == 1)
                 and not low.shared_weights):
             return None
-        U = 64 * self.NCH
-        if any(low.in1[b].mul != U or low.in1[b].off % 4 for b in self.used_in1):
+        U, n = 64 * self.NCH, self.unit
+        if any(low.in1[b].mul != U or low.in1[b].off % n for b in self.used_in1):
             return None
         if any(low.in2[p.i2].mul != 1 or p.woff != p.index * U for p in low.paths):
             return None
-        if low.L1 % 4 or low.WN % 4:
+        if low.L1 % n or low.WN % n:
             return None
-        xl, units = {}, 0
-        for b in self.used_in1:
-            xl[b] = units * 4
-            units += 16 * low.in1[b].d
-        nqx = (units + 63) // 64
-        nuw = 16 * len(low.paths)
-        nqw = (nuw + 63) // 64
-        return dict(U=U, xl=xl, nux=units, nqx=nqx, nuw=nuw, nqw=nqw, XF=nqx * 256, floats=(nqx + nqw) * 256)
+        stages = []
+        for seg, in1 in zip(self.segments, self.seg_in1):
+            xl, units = {}, 0
+            for b in in1:
+                xl[b] = units * n
+                units += 64 // n * low.in1[b].d
+            paths = [p for p in low.paths if p.io in seg]
+            nqx = (units + 63) // 64
+            nuw = 64 // n * len(paths)
+            nqw = (nuw + 63) // 64
+            stages.append(dict(U=U, xl=xl, nux=units, nqx=nqx, nuw=nuw, nqw=nqw, XF=nqx * 64 * n,
+                               floats=(nqx + nqw) * 64 * n, in1=in1, paths=paths))
+        return stages
 
     def _stage_src(self, blk, first_unit: int) -> str:
         """Row offset of the 16-byte unit ``t`` of the wave's slice of a block (units in LDS order)."""
+        n = self.unit
         if self.ir_mul:
-            # component i = 16 units of 4 channels each; the components of a piece of a folded block lie the
+            # component i = 64 / n units of n channels each; the components of a piece of a folded block lie the
             # whole block's multiplicity apart
-            return (f"{blk.off} + ((t - {first_unit}) >> 4) * {blk.cstride or blk.mul} + chunk * 64 + "
-                    f"((t - {first_unit}) & 15) * 4")
-        return f"{blk.off} + chunk * {64 * blk.d} + (t - {first_unit}) * 4"
+            return (f"{blk.off} + ((t - {first_unit}) >> {self.unit_bits}) * {blk.cstride or blk.mul} + chunk * 64 + "
+                    f"((t - {first_unit}) & {64 // n - 1}) * {n}")
+        return f"{blk.off} + chunk * {64 * blk.d} + (t - {first_unit}) * {n}"
 
     def _stage_x(self, blk, base: int, i: int) -> str:
         """Index of (lane's channel, component i) in a staged block starting at ``base``."""
@@ -192,9 +202,9 @@ class UvuEmitter:
             s(f"int t = {q * 64} + lane; if (t > {st['nux'] - 1}) t = {st['nux'] - 1};")
             expr, pu = None, 0
             terms = []
-            for b in self.used_in1:
+            for b in st["in1"]:
                 blk = low.in1[b]
-                n = 16 * blk.d
+                n = 64 // self.unit * blk.d
                 terms.append((pu, pu + n, self._stage_src(blk, pu)))
                 pu += n
             code = terms[-1][2]
@@ -206,7 +216,17 @@ class UvuEmitter:
             s(f"int woff{q};")
             s.open("")
             s(f"int t = {q * 64} + lane; if (t > {st['nuw'] - 1}) t = {st['nuw'] - 1};")
-            s(f"woff{q} = (t >> 4) * {st['U']} + chunk * 64 + (t & 15) * 4;")
+            path = f"(t >> {self.unit_bits})"
+            if len(st["paths"]) < len(low.paths):  # (the rows of a segment's paths: runs of consecutive ones)
+                runs = []
+                for n, p in enumerate(st["paths"]):
+                    if not runs or p.index - n != runs[-1][1]:
+                        runs.append((n, p.index - n))
+                skip = str(runs[0][1])
+                for n, by in runs[1:]:
+                    skip = f"({path} >= {n} ? {by} : {skip})"
+                path = f"({path} + {skip})"
+            s(f"woff{q} = {path} * {st['U']} + chunk * 64 + (t & {64 // self.unit - 1}) * {self.unit};")
             s.close()
 
     def _emit_stage_issue(self, s: Src, e: str, x: bool = True, w: bool = True, wbuf: Optional[str] = None):
@@ -220,7 +240,7 @@ class UvuEmitter:
             s(f"const T* sx = L1_in + oeq_idx(cols[eid], node_count) * {low.L1};")
             for q in range(st["nqx"]):
                 s(f"__builtin_amdgcn_global_load_lds((const OEQ_GPTR)(sx + xoff{q}), "
-                  f"(OEQ_LPTR)(&s_stage[wave][{q * 256}]), 16, 0, 0);")
+                  f"(OEQ_LPTR)(&s_stage[wave][{q * 64 * self.unit}]), 16, 0, 0);")
             if self.use_q:
                 for r in range(self.q_slabs):
                     s(f"yn[{r}] = L2_in[eid * {low.L2} + qt.j[{r}]];")
@@ -229,21 +249,21 @@ class UvuEmitter:
                     s(f"yn[{j}] = L2_in[eid * {low.L2} + {j}];")
         if w:
             s(f"const T* sw = W + eid * {low.WN};")
-            base = f"{st['XF']}" if wbuf is None else f"{st['XF']} + ({wbuf}) * {st['nqw'] * 256}"
+            base = f"{st['XF']}" if wbuf is None else f"{st['XF']} + ({wbuf}) * {st['nqw'] * 64 * self.unit}"
             for q in range(st["nqw"]):
                 s(f"__builtin_amdgcn_global_load_lds((const OEQ_GPTR)(sw + woff{q}), "
-                  f"(OEQ_LPTR)(&s_stage[wave][{base} + {q * 256}]), 16, 0, {2 if self.nt & 1 else 0});")
+                  f"(OEQ_LPTR)(&s_stage[wave][{base} + {q * 64 * self.unit}]), 16, 0, {2 if self.nt & 1 else 0});")
         s.close()
 
     def _emit_stage_read(self, s: Src, buf: str, wbuf: Optional[str] = None):
         low, st = self.low, self.stage
-        wbase = f"{st['XF']}" if wbuf is None else f"{st['XF']} + ({wbuf}) * {st['nqw'] * 256}"
-        for b in self.used_in1:
+        wbase = f"{st['XF']}" if wbuf is None else f"{st['XF']} + ({wbuf}) * {st['nqw'] * 64 * self.unit}"
+        for b in st["in1"]:
             blk = low.in1[b]
             for i in range(blk.d):
                 s(f"{buf}.x.b{b}[{i}] = s_stage[wave][{self._stage_x(blk, st['xl'][b], i)}];")
-        for p in low.paths:
-            s(f"{buf}.w[{self.wslot[p.index]}] = s_stage[wave][{wbase} + {p.index * 64} + ul];")
+        for n, p in enumerate(st["paths"]):
+            s(f"{buf}.w[{self.wslot[p.index]}] = s_stage[wave][{wbase} + {n * 64} + ul];")
         if self.use_q:
             for r in range(self.q_slabs):
                 s(f"{buf}.yq[{r}] = yn[{r}];")
@@ -324,7 +344,7 @@ class UvuEmitter:
         """Two LDS buffers per wave (separate arrays, so that reads of one do not
         wait for loads into the other); the contraction reads its operands from
         LDS where it uses them, so no register copy of an edge's operands exists."""
-        if self.stage is None or self.low.L2 % 4:
+        if self.stage is None or len(self.segments) > 1 or self.words > 1 or self.low.L2 % 4:
             return None
         st = dict(self.stage)
         npaths = len(self.low.paths)
@@ -1277,15 +1297,17 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         s(f"e += {2 * R};")
         s.close()
 
-    def _edge_mode(self, pipelined: int, rows: bool = False) -> int:
+    def _edge_mode(self, pipelined: int, rows: bool = False, all_paths: bool = False) -> int:
         """0: load, then compute; 1: next edge's operands prefetched into a second register set;
         2: next edge's operands prefetched into the wave's LDS staging buffer; 5: likewise where a wave walks several
-        edges side by side (``rows``: by kernels that can)."""
+        edges side by side (``rows``: by kernels that can). ``all_paths``: for a kernel that does not walk one output
+        segment at a time."""
+        stage = None if all_paths and len(self.segments) > 1 else self.stage
         if pipelined == 3 and self.stage3 is not None and not self.use_q:
             return 3
-        if pipelined == 4 and self.stage is not None and self.R == 1:
+        if pipelined == 4 and stage is not None and len(self.segments) == 1:
             return 4
-        if pipelined >= 2 and self.stage is not None:
+        if pipelined >= 2 and stage is not None:
             return 2
         if pipelined >= 2 and rows and self.rows_stage is not None:
             return 5
@@ -1422,6 +1444,10 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         mode = self._edge_mode(pipelined, rows=self.operand_words(2) > 170)
         return self._edge_mode(2) if mode in (3, 4) else mode
 
+    def _stage_floats(self) -> int:
+        """Elements of a wave's LDS buffer for an edge's operands (the widest of the output segments')."""
+        return max(st["floats"] for st in self.stages) if self.stages else self.rows_stage["floats"]
+
     def operand_words(self, sets: int) -> int:
         """Registers of a forward kernel's accumulators and ``sets`` operand sets of an edge."""
         low = self.low
@@ -1432,7 +1458,7 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         """Elements of a wave's LDS slice for its accumulators: the wave's staging buffer where it has one, and in any
         case the widest output block (64x0e x 1x4e -> 64x4e: 576 elements beside a staging buffer of 512)."""
         widest = max(self.low.out[io].d for io in self.used_out)
-        buffer = (self.stage or self.rows_stage)["floats"] if staged else self.SPLIT_WORDS // self.words * 64
+        buffer = self._stage_floats() if staged else self.SPLIT_WORDS // self.words * 64
         return max(buffer, widest * 64)
 
     def split_count(self, n: int, pipelined: int, segw: int = 1) -> int:
@@ -1479,11 +1505,12 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         if self.can_preload:
             s("E_t A, B;")
         if mode in (2, 4):
-            floats = self.stage["floats"] + (self.stage["nqw"] * 256 if mode == 4 else 0)
+            floats = self._stage_floats() + (self.stage["nqw"] * 64 * self.unit if mode == 4 else 0)
             if split > 1:
                 floats = self._split_slice(True)
-            s(f"__shared__ __attribute__((aligned(16))) T s_stage[{self.NCH * G * split}][{floats}];")
-            self._emit_stage_offsets(s)
+            s(f"__shared__ __attribute__((aligned(16))) T s_stage[{block // 64}][{floats}];")
+            if len(self.segments) == 1:
+                self._emit_stage_offsets(s)
         if mode == 5:
             floats = self._split_slice(True) if split > 1 else self.rows_stage["floats"]
             s(f"__shared__ __attribute__((aligned(16))) T s_stage[{G * split}][{floats}];")
@@ -1547,6 +1574,9 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
                 def node_body(si=si):
                     if self.cur_chunk is not None and not self._out_of(self.segments[si]):
                         return  # this chunk has no channel of the segment's blocks
+                    if mode == 2 and len(self.segments) > 1:
+                        self.stage = self.stages[si]
+                        self._emit_stage_offsets(s)
                     s(f"A{si}_t a; zero_seg{si}(a);")
                     if kahan:
                         s(f"A{si}_t c; zero_seg{si}(c);")
@@ -2320,7 +2350,7 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         if self.NCH > 1:
             G = 1  # one node (or edge range) per block: the per-edge dY reduction uses block barriers
         block = 64 * self.NCH * G
-        mode = self._edge_mode(2 if pipelined == 4 else pipelined)  # the body stores: see emit_conv_forward
+        mode = self._edge_mode(2 if pipelined == 4 else pipelined, all_paths=True)  # the body stores: see emit_conv_forward
         if self.can_preload:
             self._emit_load_edge(s, "load_edge_b", self.used_in1, low.paths)
             if self.chunk_split and deterministic:
@@ -2346,7 +2376,7 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         if self.can_preload:
             s("E_t A, B;")
         if mode in (2, 4):
-            floats = self.stage["floats"] + (self.stage["nqw"] * 256 if mode == 4 else 0)
+            floats = self.stage["floats"] + (self.stage["nqw"] * 64 * self.unit if mode == 4 else 0)
             s(f"__shared__ __attribute__((aligned(16))) T s_stage[{self.NCH * G}][{floats}];")
             self._emit_stage_offsets(s)
         if mode == 3:
@@ -2552,6 +2582,8 @@ def _forward_plan(low: Lowered, first_budget: int) -> Tuple[UvuEmitter, bool]:
         return e, need + (40 if e.ragged() else 0)
 
     e = UvuEmitter(low, acc_budget_words=first_budget)
+    if e.words == 2 and e.operand_words(1) > 200:
+        e.stage = e.stages = None  # (an operand set copied from LDS and the accumulators: more than half a SIMD's registers)
     if e.stage is not None or e.rows_stage is not None or not e.can_preload:
         return e, True
     budgets = (first_budget, 96, 64, 48)
@@ -2564,6 +2596,34 @@ def _forward_plan(low: Lowered, first_budget: int) -> Tuple[UvuEmitter, bool]:
         if need <= 190:
             break
     return e, False
+
+
+def _staged_segments(low: Lowered, max_segments: int) -> Optional[UvuEmitter]:
+    """Double precision: the forward kernel with a node's outputs shared out between as few waves (1, 2, 4) as leave each
+    wave a register estimate for two waves per SIMD, each with its own LDS staging buffer; None for problems that cannot
+    be staged. With all outputs in one wave's 512 registers, two operand sets and one wave per SIMD, an edge's chain of
+    loads (2 us) and its arithmetic (1 us) came one after the other. Staging alone gains 11 % of that (mace-large,
+    1 500 nodes x 32 edges, 272 -> 241 us), the second wave per SIMD another 8 % although both waves of a pair read X;
+    three waves (estimate 176) take 294. Forward, before / now, 500 x 30, 1 500 x 32 and 4 000 x 30: mace-large 100 / 85,
+    272 / 225, 600 / 509; toluene 88 / 74, 250 / 191, 530 / 470 (four waves that an estimate of 204 would take: 81, 225,
+    518); mace-medium 41 / 36, 105 / 98, 239 / 232. A kernel that needs scratch memory all the same goes back to one
+    wave, staged (mace-uvu: two waves with 36 B 148, 422, 978; one 130, 382, 896; before 165, 430, 943)."""
+    for n in (1, 2, 4):
+        if n > max_segments:
+            break
+        words = low.elem_size // 4
+        budget = -(-words * sum(low.out[io].d for io in {p.io for p in low.paths}) // n)
+        e = UvuEmitter(low, acc_budget_words=budget, stage_segments=True)
+        while len(e.segments) > n:
+            budget += words
+            e = UvuEmitter(low, acc_budget_words=budget, stage_segments=True)
+        if not e.stages:
+            return None
+        need = 40 + words * max(sum(low.out[io].d for io in seg) + sum(low.in1[b].d for b in st["in1"]) + len(st["paths"])
+                                for seg, st in zip(e.segments, e.stages))
+        if need <= 230:
+            return e
+    return None
 
 
 def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kahan: bool = False,
@@ -2593,7 +2653,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
                     dd_gres=-1, dd_split=1, dd_segw=4, dd_merge=0, dd_need=200, dd_ngrp=0, conv_gbud=0, conv_ngrp=0, conv_fit=300, conv_fw=0, conv_pf=0,
                     conv_dxm=-1, conv_q=0, conv_hops=2, conv_qpin=1, conv_qaf=48, conv_qab=24, tp_mask=0, tp_forms=1,
                     conv_hub=256, conv_dxs=-1, conv_omin=32768, conv_fsplit=-1, conv_fsplit_f=-1, conv_fsplit_x=-1, conv_fsplit_a=-1,
-                    conv_fsmax=-1, conv_parts=-1))
+                    conv_fsmax=-1, conv_parts=-1, conv_stg=1))
     assert deterministic or not kahan, "kahan=True requires deterministic=True"
     # knobs somebody set: the rules below leave those alone
     user_tune = os.environ.get("OEQ_AMD_TUNE", "")
@@ -2620,7 +2680,11 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         # 128x{0e,1o,2e} with l <= 3 harmonics, 216 registers, 10.5 against 5.4 ms; 128x{0e..3o} 12.9 / 7.5 and
         # 36.2 / 19.4); the zoo's eleven fp64 kernels of this kind are within -4.3 % .. +1.4 % either way.
         t["conv_wf"] = 2
-    if wide64 and "conv_acc" not in user_tune and "conv_wf" not in user_tune:
+    own_forward = wide64 and "conv_acc" not in user_tune and "conv_wf" not in user_tune
+    staged64 = _staged_segments(low, max(1, 8 // low.n_chunks)) if own_forward and t["conv_stg"] else None
+    if staged64:
+        em = staged64
+    elif own_forward:
         x_all = sum(low.in1[b].d for b in em.used_in1)
         need_f = 2 * (sum(low.out[io].d for io in em.used_out) + x_all + em.n_wslots + low.L2) + 40
         if len(em.segments) > 1 and need_f <= 480:
@@ -2672,7 +2736,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         em.q_pin = bool(t["conv_qpin"])
         em.q_ahead = (t["conv_qaf"], t["conv_qab"])
         em.build_q_table()
-    if walk and len(em.segments) > 1 and t["conv_segw"] and em.stage is None and em.R == 1:
+    if walk and len(em.segments) > 1 and t["conv_segw"] and em.R == 1:
         em.seg_waves = max(1, min(len(em.segments), t["conv_segw"], max(1, 8 // em.NCH)))
         t["conv_gf"] = max(1, min(t["conv_gf"], 8 // (em.NCH * em.seg_waves)))
     if walk and (len(em.segments) > 1 or low.elem_size == 8) and "conv_gf" not in user_tune:
@@ -2870,6 +2934,8 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         _lds, scratch = rt.kernel_resources(rt.compile_source(src)).get("backward_dx", (0, 0))
         if scratch > 64:
             return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_dxs=0), draft)
+    if staged64 and len(em.segments) > 1 and rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))[1] > 0:
+        return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_stg=0), draft)
     if em.seg_waves > 1 and "conv_segw" not in user_tune:
         # Waves that share a node's output segments: with two operand sets in flight and three or more segments
         # the compiler has been seen to need more registers for the kernel that selects a wave's segments by

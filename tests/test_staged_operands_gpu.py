@@ -1,14 +1,15 @@
-"""Convolution kernels whose waves walk two edges side by side with the edges' rows staged in LDS, against the oracle:
+"""Convolution kernels with an edge's operands staged in LDS, against the oracle. Waves that walk two edges side by side:
 rows of less than an instruction's 1 024 bytes, of whole instructions and with a rest, blocks without a channel for every
 lane, several channels in the second operand; segments without an edge, with odd and even numbers, on either side of the
-64 edges whose numbers a wave holds, and cut into chunks."""
+64 edges whose numbers a wave holds, and cut into chunks. Double precision, a node's outputs shared out between waves that
+stage what theirs need: one, two and four of them, paths in and out of the order of their outputs."""
 
 import numpy as np
 import pytest
 
 import openequivariance_amd as oeq
 from openequivariance_amd.codegen.lower import lower
-from openequivariance_amd.codegen.uvu import UvuEmitter
+from openequivariance_amd.codegen.uvu import UvuEmitter, _staged_segments
 from openequivariance_amd.core import problems as P
 from openequivariance_amd.core.graph import CoordGraph
 from openequivariance_amd.core.layout import transpose_irrep_layout
@@ -24,6 +25,9 @@ PROBLEMS = {
     "channels": ("32x0e+32x1o", "2x0e+3x1o", "0e+1o"),
     "lips": None,
 }
+# channels, largest l of the first operand and of the harmonics, paths and their order
+SHARED = {"one": (128, 1, 2, range(9)), "two": (128, 2, 2, range(18)), "two-shuffled": (128, 2, 2, [k * 7 % 18 for k in range(18)]),
+          "four-shuffled": (64, 3, 3, [k * 5 % 34 for k in range(34)])}
 DEGREES = [0, 1, 2, 3, 31, 63, 64, 65, 0, 128, 129, 300, 5, 0]
 
 
@@ -34,9 +38,27 @@ def _problem(name, dtype, layout):
     return p
 
 
+def _shared(name, layout):
+    mul, lx, ly, order = SHARED[name]
+    paths = [(l1, l2, l3) for l1 in range(lx + 1) for l2 in range(ly + 1) for l3 in range(abs(l1 - l2), min(3, l1 + l2) + 1)]
+    in1, in2 = [f"{mul}x{l}e" for l in range(lx + 1)], [f"1x{l}e" for l in range(ly + 1)]
+    outs = [f"{mul}x{l3}e" for _, _, l3 in paths[:len(order)]]
+    p = oeq.TPProblem("+".join(in1), "+".join(in2), "+".join(outs),
+                      [(paths[k][0], paths[k][1], k, "uvu", True) for k in order], shared_weights=False,
+                      internal_weights=False, label=f"shared-{name}", irrep_dtype=np.float64, weight_dtype=np.float64)
+    p.layout = layout
+    return p
+
+
 @pytest.mark.parametrize("name", ["rest", "ragged", "channels", "lips"])
 def test_these_problems_stage_their_rows(name):
     assert UvuEmitter(lower(_problem(name, np.float32, "mul_ir"))).rows_stage is not None
+
+
+@pytest.mark.parametrize("name,waves", [("one", 1), ("two", 2), ("two-shuffled", 2), ("four-shuffled", 4)])
+def test_waves_that_share_the_outputs(name, waves):
+    em = _staged_segments(lower(_shared(name, "mul_ir")), 8)
+    assert len(em.segments) == len(em.stages) == waves
 
 
 @pytest.mark.gpu
@@ -45,7 +67,20 @@ def test_these_problems_stage_their_rows(name):
     (np.float32, "mul_ir", True, "conv_fsmax=0"), (np.float32, "ir_mul", False, "conv_fsmax=0,conv_dxs=1"),
     (np.float64, "mul_ir", False, "conv_fsmax=0,conv_dxs=1"), (np.float32, "mul_ir", False, "conv_fsplit=4")])
 def test_against_the_oracle(name, dtype, layout, det, tune, monkeypatch):
-    problem = _problem(name, dtype, layout)
+    _check(_problem(name, dtype, layout), _problem(name, dtype, "mul_ir"), det, tune, monkeypatch)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(SHARED))
+@pytest.mark.parametrize("layout,det,tune", [("mul_ir", True, "conv_fsmax=0"), ("ir_mul", False, "conv_fsmax=0"),
+                                             ("mul_ir", False, "conv_fsplit=2")])
+def test_shared_outputs_against_the_oracle(name, layout, det, tune, monkeypatch):
+    _check(_shared(name, layout), _shared(name, "mul_ir"), det, tune, monkeypatch)
+
+
+def _check(problem, plain, det, tune, monkeypatch):
+    """Forward and backward of ``problem``, whose ``mul_ir`` form, what the oracle works in, is ``plain``."""
+    dtype, layout = problem.irrep_dtype, problem.layout
     n = len(DEGREES)
     rng = np.random.default_rng(7)
     rows = np.repeat(np.arange(n), DEGREES)
@@ -54,7 +89,7 @@ def test_against_the_oracle(name, dtype, layout, det, tune, monkeypatch):
     x, y, w, gz = (rng.normal(size=s).astype(dtype) for s in (
         (n, problem.irreps_in1.dim), (g.nnz, problem.irreps_in2.dim), (g.nnz, problem.weight_numel),
         (n, problem.irreps_out.dim)))
-    ref = R.Problem.from_spec(_problem(name, dtype, "mul_ir"))  # (the oracle works in mul_ir)
+    ref = R.Problem.from_spec(plain)
     ref_z = R.conv_forward(ref, x, y, w, g.rows, g.cols)
     ref_dx, ref_dy, ref_dw = R.conv_backward(ref, x, y, w, gz, g.rows, g.cols)
     i1, i2, io = problem.irreps_in1, problem.irreps_in2, problem.irreps_out
