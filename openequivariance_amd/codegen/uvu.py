@@ -759,6 +759,7 @@ class UvuEmitter:
             # what lanes without a channel read in place of an output-gradient block (see _gptr)
             extent = max((b.d - 1) * self._lane_ptr(b)[1] + 1 for b in partial)
             s(f"__device__ const T oeq_zero_row[{extent}] = {{}};")
+        self._emit_lane_swaps(s)
         # where lanes (or rows) that must not store point their store inside a chain of paths (see _dump_unless)
         s("__device__ T oeq_dump[4096];")
         if self.can_preload and self.q_entries:
@@ -1024,15 +1025,9 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
                 s(f"T v{q} = a.o{io}[{k}];")
             m = self.LPR
             while m < 64:
-                half = len(names) // 2
-                s.open("")
-                s(f"const bool hi = (lane & {m}) != 0;")
                 # (lane group bit m chooses between neighbouring values: group r is left with value r)
-                for q in range(half):
-                    s(f"{{ const T keep = hi ? v{2 * q + 1} : v{2 * q}, send = hi ? v{2 * q} : v{2 * q + 1}; "
-                      f"v{q} = keep + __shfl_xor(send, {m}); }}")
-                s.close()
-                names = names[:half]
+                self._halve(s, names[::2], names[1::2], m)
+                names = names[::2]
                 m *= 2
             off, cond = None, None
             for q in range(len(group) - 1, -1, -1):
@@ -1870,19 +1865,68 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         while m >= 1:
             if cur > 1:
                 half = cur // 2
-                s.open("")
-                s(f"const bool hi = (ul & {m}) != 0;")
-                for j in range(half):
-                    s(f"{{ const T keep = hi ? rv[{j + half}] : rv[{j}]; const T send = hi ? rv[{j}] : rv[{j + half}]; "
-                      f"rv[{j}] = keep + __shfl_xor(send, {m}); }}")
-                s(f"dyidx += hi ? {half} : 0;")
-                s.close()
+                self._halve(s, [f"rv[{j}]" for j in range(half)], [f"rv[{j + half}]" for j in range(half)], m, mirror=True)
+                s(f"dyidx += (ul & {m}) ? {half} : 0;")
                 cur = half
             else:
-                s(f"rv[0] += __shfl_xor(rv[0], {m});")
+                s(f"{{ T a = rv[0], b = rv[0]; oeq_swap{m}(a, b); rv[0] = a + b; }}" if m >= 16
+                  else f"rv[0] += oeq_swap{m}(rv[0]);")
                 dup |= m
             m //= 2
         return cur, dup
+
+    @staticmethod
+    def _halve(s: Src, first: List[str], second: List[str], m: int, mirror: bool = False):
+        """One step of a sum over lanes that halves what a lane holds: lanes with bit ``m`` clear are left with the sums
+        of ``first``, the others with those of ``second``, over the pairs of lanes that differ in that bit (with
+        ``mirror``, for m = 4, in the two below it as well: for sums that these lanes all go into and have not been
+        halved over yet). Left in ``first``. In the vector unit: by way of
+        LDS (``__shfl_xor``) the six steps of a row's dY were six LDS latencies, and 17 LDS instructions, one after
+        the other for every edge."""
+        if m >= 16:
+            for a, b in zip(first, second):
+                s(f"oeq_swap{m}({a}, {b}); {a} += {b};")
+            return
+        s.open("")
+        s(f"const bool hi = (lane & {m}) != 0;")
+        for a, b in zip(first, second):
+            other = "__shfl_xor(send, 4)" if m == 4 and not mirror else f"oeq_swap{m}(send)"
+            s(f"{{ const T keep = hi ? {b} : {a}, send = hi ? {a} : {b}; {a} = keep + {other}; }}")
+        s.close()
+
+    def _emit_lane_swaps(self, s: Src):
+        """oeq_swap<m>, what the sums over lanes exchange values with. m = 32, 16: the lanes with bit m set of ``a`` and
+        the others of ``b`` change places. m = 8, 4, 2, 1: the value of the lane that differs in bit m (m = 4: in the
+        three lowest bits)."""
+        double = self.low.elem_size == 8
+        for m in (32, 16):
+            s.open(f"OEQ_DEV void oeq_swap{m}(T& a, T& b)")
+            if double:
+                s("const unsigned long long x = __builtin_bit_cast(unsigned long long, a), "
+                  "y = __builtin_bit_cast(unsigned long long, b);")
+                s(f"const auto lo = __builtin_amdgcn_permlane{m}_swap((unsigned)x, (unsigned)y, false, false);")
+                s(f"const auto hi = __builtin_amdgcn_permlane{m}_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);")
+                for v, q in (("a", 0), ("b", 1)):
+                    s(f"{v} = __builtin_bit_cast(T, ((unsigned long long)hi[{q}] << 32) | lo[{q}]);")
+            else:
+                s(f"const auto r = __builtin_amdgcn_permlane{m}_swap(__builtin_bit_cast(unsigned, a), "
+                  "__builtin_bit_cast(unsigned, b), false, false);")
+                # (by way of variables: of an element of a vector __builtin_bit_cast takes the first, whichever it is)
+                s("const unsigned x = r[0], y = r[1];")
+                s("a = __builtin_bit_cast(T, x); b = __builtin_bit_cast(T, y);")
+            s.close()
+        # (row rotation by 8, mirror of half rows, quad permutations)
+        for m, ctrl in ((8, 0x128), (4, 0x141), (2, 0x4E), (1, 0xB1)):
+            s.open(f"OEQ_DEV T oeq_swap{m}(T v)")
+            if double:
+                s("const unsigned long long x = __builtin_bit_cast(unsigned long long, v);")
+                for part, bits in (("lo", "(int)x"), ("hi", "(int)(x >> 32)")):
+                    s(f"const unsigned {part} = (unsigned)__builtin_amdgcn_update_dpp(0, {bits}, {ctrl}, 0xf, 0xf, true);")
+                s("return __builtin_bit_cast(T, ((unsigned long long)hi << 32) | lo);")
+            else:
+                s("return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), "
+                  f"{ctrl}, 0xf, 0xf, true));")
+            s.close()
 
     def _dy_finish(self, s: Src, dst_row: str, live: str):
         """Cross-lane (and cross-chunk) reduction of dy, then write of the row."""
@@ -1909,6 +1953,57 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
             s.close()
             s.close()
             s("__syncthreads();")
+        s.close()
+
+    def _dy_batch(self) -> int:
+        """Edges whose dY the waves of a node with several chunks collect in LDS before they add them up."""
+        n = 8
+        while n > 1 and 2 * n * self.NCH * self.l2_pad * self.low.elem_size > 8192:
+            n //= 2
+        return n
+
+    def _dy_declare(self, s: Src):
+        if self.NCH > 1:
+            s(f"__shared__ T s_dy[{2 * self._dy_batch()}][{self.NCH}][{self.l2_pad}];")
+            s("int dyc = 0;  // edges collected, from a batch boundary on at every node")
+
+    def _dy_edge(self, s: Src, pos: str, last: str, eid: str):
+        """dY of the edge at position ``pos`` of a walk (number ``eid``) that ends before ``last``. With several chunks
+        their waves' partial sums meet in LDS: a batch of consecutive edges at a time, so that the waves of a node wait
+        for each other once per batch, at its end, and the threads of the block write the batch's rows together. Two
+        batches take turns in LDS: a wave gets to the second batch after this one only when all have written this
+        one's rows (they meet at the end of the next). A barrier before and one after the sum for every edge cost, with
+        the lane exchanges by way of LDS, 13 % of the fp64 kernel's time at one wave per SIMD and 2 to 5 % of the fp32
+        ones'."""
+        low, n = self.low, self._dy_batch()
+        if self.NCH == 1:
+            self._dy_finish(s, f"L2_grad + {eid} * {low.L2}", "true")
+            return
+        assert self.R == 1
+        s.open("")
+        cur, dup = self._dy_reduce(s)
+        s.open(f"if ((ul & {dup}) == 0)")
+        for j in range(cur):
+            s(f"s_dy[dyc & {2 * n - 1}][chunk][dyidx + {j}] = rv[{j}];")
+        s.close()
+        s("++dyc;")
+        s.open(f"if ((dyc & {n - 1}) == 0 || {pos} + 1 == {last})")
+        s("__syncthreads();")
+        s(f"const int count = ((dyc - 1) & {n - 1}) + 1, begin = dyc - count;")
+        # (opaque: what follows from the thread's number would otherwise be formed before the edge loop and kept)
+        s("int first = (int)threadIdx.x;")
+        s('asm volatile("" : "+v"(first));')
+        s.open(f"for (int t = first; t < count * {self.l2_pad}; t += {64 * self.NCH})")
+        s(f"const int k = t / {self.l2_pad}, j = t % {self.l2_pad};")
+        if self.l2_pad != low.L2:
+            s(f"if (j >= {low.L2}) continue;")
+        s(f"const T* part = &s_dy[(begin + k) & {2 * n - 1}][0][j];")
+        s(f"T tot = part[0];")
+        s(f"for (int cc = 1; cc < {self.NCH}; ++cc) tot += part[cc * {self.l2_pad}];")
+        s(f"L2_grad[OEQ_EDGE({pos} + 1 - count + k) * {low.L2} + j] = tot;")
+        s.close()
+        s(f"dyc = (dyc + {n - 1}) & ~{n - 1};")
+        s.close()
         s.close()
 
     def _store_dx(self, s: Src, rowexpr: str, guard: str, atomic: bool = False, nt: bool = False):
@@ -2368,8 +2463,7 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         self._lane_prologue(s)
         if self.use_q:
             self._emit_q_prologue(s, block // 64)
-        if self.NCH > 1:
-            s(f"__shared__ T s_dy[{G}][{self.NCH}][{self.l2_pad}];")
+        self._dy_declare(s)
         if shared:
             s(f"T dwacc[{self.n_wslots}];")
             s(f"for (int t = 0; t < {self.n_wslots}; ++t) dwacc[t] = T(0);")
@@ -2452,7 +2546,7 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
                 else:
                     s(f"T* dxrow = L1_grad + oeq_idx(cols[{e}], node_count) * {low.L1};")
                     self._store_dx(s, "dxrow", "true", atomic=True)
-                self._dy_finish(s, f"L2_grad + {e} * {low.L2}", "true")
+                self._dy_edge(s, pos, "e1" if deterministic else "ee", e)
                 s.close()
             return compute
 

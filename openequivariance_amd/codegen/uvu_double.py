@@ -578,8 +578,7 @@ class DoubleEmitter(UvuEmitter):
         self._lane_prologue(s)
         shared = low.shared_weights
         assert not (shared and self.merged)
-        if self.NCH > 1:
-            s(f"__shared__ T s_dy[{G}][{self.NCH}][{self.l2_pad}];")
+        self._dy_declare(s)
         if (self.tr_stores & 2 or (self.merged and self.tr_stores & 1)) and self.R == 1:
             dmax = max([low.in1[b].d for b in self.used_in1] + [low.out[io].d for io in self.used_out])
             s(f"__shared__ T s_tr[{self.NCH * G}][{64 * dmax}];")
@@ -628,7 +627,7 @@ class DoubleEmitter(UvuEmitter):
             s(f"T* dxrow = dx_tmp + eid * {low.L1};")
             self._store_dx(s, "dxrow", "true", nt=bool(self.nt & 2))
             self._zero_untouched_in1(s, "dxrow", "true")
-            self._dy_finish(s, f"L2_grad + eid * {low.L2}", "true")
+            self._dy_edge(s, "e", "e1", "eid")
             s.close()
             if self.merged:
                 if self.R > 1:  # fold the lane groups of packed rows (fixed order) into group 0

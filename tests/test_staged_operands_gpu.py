@@ -24,11 +24,13 @@ PROBLEMS = {
     "ragged": ("20x0e+32x1o+4x2e", "0e+1o", "0e+1o+2e"),
     "channels": ("32x0e+32x1o", "2x0e+3x1o", "0e+1o"),
     "lips": None,
+    "chunks": ("128x0e+128x1o", "0e+1o+2e", "0e+1o+2e"),  # two waves to a node: dY of eight edges at a time
+    "ragged-chunks": ("200x0e+100x1o", "0e+1o", "0e+1o+2e"),
 }
 # channels, largest l of the first operand and of the harmonics, paths and their order
 SHARED = {"one": (128, 1, 2, range(9)), "two": (128, 2, 2, range(18)), "two-shuffled": (128, 2, 2, [k * 7 % 18 for k in range(18)]),
           "four-shuffled": (64, 3, 3, [k * 5 % 34 for k in range(34)])}
-DEGREES = [0, 1, 2, 3, 31, 63, 64, 65, 0, 128, 129, 300, 5, 0]
+DEGREES = [0, 1, 2, 3, 7, 8, 9, 16, 17, 31, 63, 64, 65, 0, 128, 129, 300, 5, 0]
 
 
 def _problem(name, dtype, layout):
@@ -76,6 +78,26 @@ def test_against_the_oracle(name, dtype, layout, det, tune, monkeypatch):
                                              ("mul_ir", False, "conv_fsplit=2")])
 def test_shared_outputs_against_the_oracle(name, layout, det, tune, monkeypatch):
     _check(_shared(name, layout), _shared(name, "mul_ir"), det, tune, monkeypatch)
+
+
+@pytest.mark.gpu
+def test_gradients_of_harmonics_where_blocks_take_several_nodes():
+    """Shared weights: a bounded grid whose blocks walk one node after the other."""
+    problem = oeq.TPProblem("128x0e+128x1o", "1x0e+1x1o", "128x0e+128x1o+128x1o",
+                            [(0, 0, 0, "uvu", True), (0, 1, 1, "uvu", True), (1, 0, 2, "uvu", True)], shared_weights=True,
+                            internal_weights=False, label="shared-chunks")
+    n, rng = 5000, np.random.default_rng(3)
+    rows = np.repeat(np.arange(n), rng.integers(0, 20, size=n))
+    cols = rng.integers(0, n, size=len(rows))
+    x, y, w, gz = (rng.normal(size=s).astype(np.float32) for s in (
+        (n, problem.irreps_in1.dim), (len(rows), 4), (problem.weight_numel,), (n, problem.irreps_out.dim)))
+    conv = oeq.TensorProductConv(problem)
+    tx, ty, tw = to_gpu(x, y, w, requires_grad=True)
+    r, c, tg = to_gpu(rows, cols, gz)
+    conv(tx, ty, tw, r, c).backward(tg)
+    dx, dy, dw = R.conv_backward(R.Problem.from_spec(problem), x, y, w, gz, rows, cols)
+    for got, want in ((tx.grad, dx), (ty.grad, dy), (tw.grad, dw)):
+        assert err(got, want) <= tol_of(problem)
 
 
 def _check(problem, plain, det, tune, monkeypatch):
