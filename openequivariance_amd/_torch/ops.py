@@ -31,7 +31,9 @@ import contextlib
 import hashlib
 import json
 import os
+import sys
 import threading
+import types
 from typing import Dict, List, Optional, Tuple
 
 import torch
@@ -238,7 +240,9 @@ def _resolve(kid: int, spec: Optional[torch.Tensor]):
     walk = _walk_dims(e) if not e.unfused else {}
     conv = "order_hops" in walk
     atomic = conv and not e.deterministic and walk["deterministic"] == rt.CONV_ATOMIC
+    order = tuple(dims.get(k, 0) for k in ("order_hops", "order_min_nodes", "hub_limit"))
     _native.register_entry(kid, dict(
+        index_dims=order, fused_second_order=plain and not e.second_order_kid and e.kernels().has_double_backward(),
         handle=e.kernels().handle.value if plain else 0, L1=e.L1, L2=e.L2, L3=e.L3, WN=e.WN, shared=bool(e.shared),
         deterministic=bool(e.deterministic), double=e.dtype == torch.float64, mode=dims.get("deterministic", 0),
         dx_mode=dims.get("dx_mode", 0), native=plain, alert_forward=atomic,
@@ -374,7 +378,8 @@ def check_edge_list(nodes: int, rows: torch.Tensor, cols: torch.Tensor, perm: Op
 
 
 def _check_indices_enabled() -> bool:
-    import os
+    if _native is not None:
+        return _native.check_indices()
     return CHECK_INDICES or os.environ.get("OEQ_AMD_CHECK_INDICES", "0") not in ("", "0")
 
 
@@ -392,74 +397,47 @@ def _check_edges(nodes, rows, cols, perm, deterministic):
 # index of an edge list, kept between calls
 # ---------------------------------------------------------------------------
 
-# A walk-mode convolution first derives an index from the edge list (CSR pointers, edge grouping, walk
-# order; include/oeq_amd.h, oeq_conv_index_build). The layers of a model, and the forward and backward of
-# each, usually run over the same edge tensors, so the ops keep the last few indices and reuse one when a
-# call brings the same tensors (same storage, same version counters, i.e. not written to since), on the same
-# stream, for a kernel set that indexes the same way. The cache holds references to the edge tensors, so
-# their memory cannot be handed to different data while an entry exists. 0 switches the cache off.
+# The ops keep the last few indices and use one again when a call brings the same edge tensors (csrc/oeq_torch.cpp:
+# IndexQuery). 0 switches that off.
 INDEX_CACHE_ENTRIES = 4
-_index_cache: List[dict] = []
-_index_cache_lock = threading.Lock()
+
+
+class _IndexCache:
+    """The kept indices, as far as Python sees them: how many there are."""
+
+    def __len__(self):
+        return _native.index_cache_size() if _native is not None else 0
+
+
+_index_cache = _IndexCache()
 
 
 def clear_index_cache():
-    with _index_cache_lock:
-        _index_cache.clear()
-
-
-def _version_of(t: torch.Tensor) -> Optional[int]:
-    """Version counter of a tensor, None where there is none (tensors made under
-    ``torch.inference_mode()`` do not track one: reading it raises)."""
-    if t.is_inference():
-        return None
-    try:
-        return t._version
-    except RuntimeError:
-        return None
+    if _native is not None:
+        _native.clear_index_cache()
 
 
 def _conv_index(ks, nodes: int, nnz: int, r: torch.Tensor, c: torch.Tensor, p: Optional[torch.Tensor],
                 need_sender_side: bool):
-    """(index tensor, sender_side flag) for the edge list; built now unless a valid one is cached."""
+    """(index tensor, sender_side flag) for the edge list; built now unless a valid one is kept."""
     dims = ks.dims
-    stream = _stream()
     grouped = dims["deterministic"] == rt.CONV_GROUPED
-    # the sender side is cheap to add when the caller brings the sender-major permutation, costly when the
-    # library has to group the edges by sender itself: then only the calls that need it build it
-    sender_side = need_sender_side or (not grouped and p is not None and p.numel() == nnz)
-    key = (dims["deterministic"], dims.get("order_hops", 0), dims.get("order_min_nodes", 0), dims.get("hub_limit", 0),
-           nodes, nnz, r.data_ptr(), c.data_ptr(),
-           p.data_ptr() if (p is not None and not grouped) else 0, stream, r.device.index)
-    versions = (_version_of(r), _version_of(c), _version_of(p) if (p is not None and not grouped) else 0)
-    # an edge tensor without a version counter could be rewritten unnoticed: such a call builds its index
-    # and keeps nothing
-    caching = (INDEX_CACHE_ENTRIES > 0 and not torch.cuda.is_current_stream_capturing()
-               and None not in versions)
-    if caching:
-        with _index_cache_lock:
-            for i, ent in enumerate(_index_cache):
-                if ent["key"] == key and ent["versions"] == versions and (ent["sender_side"] or not sender_side):
-                    _index_cache.append(_index_cache.pop(i))
-                    return ent["index"], ent["sender_side"]
-    nb = ks.conv_index_bytes(nodes, nnz, sender_side)
-    index = torch.empty(max(nb, 1), dtype=torch.uint8, device=r.device)
-    ks.conv_index_build(nodes, nnz, r.data_ptr(), c.data_ptr(), p.data_ptr() if (p is not None and not grouped) else 0,
-                        sender_side, index.data_ptr(), nb, stream)
-    if caching:
-        with _index_cache_lock:
-            _index_cache[:] = [ent for ent in _index_cache if ent["key"] != key]
-            _index_cache.append({"key": key, "versions": versions, "sender_side": sender_side, "index": index,
-                                 "refs": (r, c, p)})
-            del _index_cache[:-INDEX_CACHE_ENTRIES]
-    return index, sender_side
+
+    def build(sender_side):
+        nb = ks.conv_index_bytes(nodes, nnz, sender_side)
+        index = torch.empty(max(nb, 1), dtype=torch.uint8, device=r.device)
+        ks.conv_index_build(nodes, nnz, r.data_ptr(), c.data_ptr(),
+                            p.data_ptr() if (p is not None and not grouped) else 0, sender_side, index.data_ptr(), nb,
+                            _stream())
+        return index
+
+    order = tuple(dims.get(k, 0) for k in ("order_hops", "order_min_nodes", "hub_limit"))
+    return _native.kept_index(dims["deterministic"], order, nodes, nnz, r, c, p, need_sender_side, build)
 
 
-def _native_index(kid: int, nodes: int, nnz: int, r, c, p, need_sender_side: bool):
-    """Called by the native convolutions: the (optionally checked) edge list's index and its sender_side flag."""
-    e = _registry[kid]
-    _check_edges(nodes, r, c, p, bool(e.deterministic))
-    return _conv_index(e.kernels(), nodes, nnz, r, c, p, need_sender_side)
+def _build_index(kid: int, *args):
+    """Called by the native convolutions for an edge list whose index is not kept."""
+    _registry[kid].kernels().conv_index_build(*args)
 
 
 def _segment_sum(ks, src: torch.Tensor, n_segments: int, keys: torch.Tensor, perm: Optional[torch.Tensor]):
@@ -617,9 +595,21 @@ def _conv_second_order(operands, cotangents, kid, spec):
 
 if _native is not None:
     _native.set_callbacks(dict(
-        resolve=_resolve, check_edges=_check_edges, conv_index=_native_index, conv_forward=_composed_forward,
+        resolve=_resolve, check_edges=_check_edges, build_index=_build_index, conv_forward=_composed_forward,
         conv_backward=_composed_backward, conv_double_backward=_composed_double_backward,
         tp_second_order=_tp_second_order, conv_second_order=_conv_second_order, error_type=rt.OeqError))
+
+
+class _Module(types.ModuleType):
+    """This module: the native ops read what a program sets here."""
+
+    def __setattr__(self, name, value):
+        super().__setattr__(name, value)
+        if name in ("CHECK_INDICES", "FUSED_DOUBLE_BACKWARD", "INDEX_CACHE_ENTRIES") and _native is not None:
+            getattr(_native, "set_" + name.lower())(value)
+
+
+sys.modules[__name__].__class__ = _Module
 
 
 # Mixed precision: the kernels are compiled for one dtype; under autocast the

@@ -4,11 +4,14 @@
 // argument checks (torch_core.hpp:109-134), allocation of results and scratch memory, launches on
 // torch's current stream, and autograd. An op carries the id of its kernel set and, for processes that have not
 // seen it, the set's description; what is rare or needs the code generator stays in Python and is called from here:
-// building a kernel set, the index of an edge list (it is kept between calls there), the convolutions without a fused
-// kernel, and the second-order route.
+// building a kernel set, building the index of an edge list that is not kept from an earlier call, the convolutions
+// without a fused kernel, and the second-order routes by composition.
 //
 // The host side of a call is what a small product or graph costs: forward and backward of 777 rows take 8 us on the
-// GPU and took 111 to 196 us, by machine, through Python ops (64 to 67 now).
+// GPU and took 111 to 196 us, by machine, through Python ops (64 to 67 now). What runs in the backward pass matters
+// most: it runs in the autograd engine's thread, where Python code finds neither its interpreter state nor its data in
+// the caches. Looking up the kept index and choosing the second-order route in Python cost, per pass, before / now:
+// MACE-medium, 192 nodes, new edges, forward and backward 157 / 96 us; 16 molecules with second order 281 / 192.
 #include "oeq_amd.h"
 
 #include <ATen/ATen.h>
@@ -22,11 +25,16 @@
 #include <torch/csrc/utils/pybind.h>
 #include <torch/library.h>
 
+#include <algorithm>
+#include <array>
+#include <atomic>
+#include <cstdlib>
 #include <memory>
 #include <mutex>
 #include <shared_mutex>
 #include <tuple>
 #include <unordered_map>
+#include <vector>
 
 namespace py = pybind11;
 using at::Tensor;
@@ -42,8 +50,10 @@ struct Entry {
     bool shared = false, deterministic = false;
     at::ScalarType dtype = at::kFloat;
     int mode = 0, dx_mode = 0;  // oeq_conv_mode, oeq_dx_mode
+    std::array<int64_t, 3> index_dims{};  // what an index depends on besides the mode: order_hops, order_min_nodes, hub_limit
     bool native = true;         // false: a convolution without fused kernels, see Callbacks::conv_*
     bool alert_forward = false, alert_backward = false;  // uses float atomics
+    bool fused_second_order = false;  // has the second-order kernels (of its own: not second_order_kid's)
     int64_t second_order_kid = 0;
     py::object owner;  // keeps the kernel set alive
 };
@@ -55,7 +65,7 @@ std::shared_mutex g_entries_mu;
 
 // Python functions of _torch/ops.py; held until the process ends (no destructor runs after the interpreter's).
 struct Callbacks {
-    py::object resolve, check_edges, conv_index, conv_forward, conv_backward, conv_double_backward, tp_second_order,
+    py::object resolve, check_edges, build_index, conv_forward, conv_backward, conv_double_backward, tp_second_order,
         conv_second_order, error_type;
 };
 Callbacks* g_py = nullptr;
@@ -227,7 +237,18 @@ GraphSize conv_checks(const Entry& e, const Tensor& L1_in, const Tensor& L2_in, 
     return {nodes, nnz};
 }
 
+// What _torch/ops.py lets a program set (its module attributes of these names).
+std::atomic<bool> g_check_indices{false}, g_fused_double_backward{true};
+std::atomic<int64_t> g_index_cache_entries{4};
+
+bool check_indices() {
+    if (g_check_indices) return true;
+    const char* env = std::getenv("OEQ_AMD_CHECK_INDICES");
+    return env && *env && !(env[0] == '0' && !env[1]);
+}
+
 void check_edges(const Entry& e, GraphSize n, const Tensor& rows, const Tensor& cols, const Tensor& perm) {
+    if (!check_indices()) return;
     py::gil_scoped_acquire gil;
     g_py->check_edges(n.nodes, rows, cols, e.deterministic ? py::cast(perm) : py::object(py::none()), e.deterministic);
 }
@@ -237,14 +258,98 @@ struct Index {
     bool sender_side = false;
 };
 
-// The index of the edge list, built now or kept from an earlier call over the same tensors (_torch/ops.py), after the
+// A walk-mode convolution first derives an index from the edge list (CSR pointers, edge grouping, walk order;
+// oeq_conv_index_build). The layers of a model, and the forward and backward of each, usually run over the same edge
+// tensors, so the last few indices are kept and one is used again when a call brings the same tensors (same storage,
+// same version counters, i.e. not written to since), on the same stream, for a kernel set that indexes the same way.
+// The list holds references to the edge tensors, so their memory cannot be handed to different data while an entry
+// exists.
+struct IndexKey {
+    std::array<int64_t, 13> v{};
+    bool operator==(const IndexKey& o) const { return v == o.v; }
+};
+
+struct KeptIndex {
+    IndexKey key;
+    std::array<uint32_t, 3> versions;
+    Index index;
+    Tensor rows, cols, perm;
+};
+
+auto& g_indices = *new std::vector<KeptIndex>();  // least recently used first
+std::mutex g_indices_mu;
+
+struct IndexQuery {
+    IndexKey key;
+    std::array<uint32_t, 3> versions{};
+    bool sender_side, keep;
+
+    // perm is undefined where the caller's edges are not sorted
+    IndexQuery(int mode, const std::array<int64_t, 3>& dims, GraphSize n, const Tensor& rows, const Tensor& cols,
+               const Tensor& perm, bool need_sender_side) {
+        const bool sorted = perm.defined() && mode != OEQ_CONV_GROUPED;
+        // the sender side is cheap to add when the caller brings the sender-major permutation, costly when the
+        // library has to group the edges by sender itself: then only the calls that need it build it
+        sender_side = need_sender_side || (sorted && perm.numel() == n.edges);
+        const auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA();
+        key.v = {mode, dims[0], dims[1], dims[2], n.nodes, n.edges, (int64_t)rows.data_ptr(), (int64_t)cols.data_ptr(),
+                 sorted ? (int64_t)perm.data_ptr() : 0, (int64_t)(hipStream_t)stream, rows.device().index(), sorted, 0};
+        // an edge tensor without a version counter could be rewritten unnoticed: such a call builds its index and
+        // keeps nothing. Nor does one that is being captured.
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        keep = g_index_cache_entries > 0 && !rows.is_inference() && !cols.is_inference() &&
+               !(sorted && perm.is_inference()) &&
+               hipStreamIsCapturing((hipStream_t)stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
+        if (keep) versions = {(uint32_t)rows._version(), (uint32_t)cols._version(), sorted ? (uint32_t)perm._version() : 0u};
+    }
+
+    int64_t stream() const { return key.v[9]; }
+
+    std::optional<Index> find() const {
+        if (!keep) return std::nullopt;
+        std::lock_guard<std::mutex> lock(g_indices_mu);
+        for (auto it = g_indices.begin(); it != g_indices.end(); ++it) {
+            if (!(it->key == key) || it->versions != versions || (sender_side && !it->index.sender_side)) continue;
+            std::rotate(it, it + 1, g_indices.end());
+            return g_indices.back().index;
+        }
+        return std::nullopt;
+    }
+
+    void store(const Tensor& data, const Tensor& rows, const Tensor& cols, const Tensor& perm) const {
+        if (!keep) return;
+        std::vector<KeptIndex> gone;  // (freed after the lock is released)
+        std::lock_guard<std::mutex> lock(g_indices_mu);
+        std::vector<KeptIndex> kept;
+        for (auto& k : g_indices) (k.key == key ? gone : kept).push_back(std::move(k));
+        kept.push_back({key, versions, {data, sender_side}, rows, cols, perm});
+        const size_t limit = (size_t)std::max<int64_t>(1, g_index_cache_entries);
+        while (kept.size() > limit) {
+            gone.push_back(std::move(kept.front()));
+            kept.erase(kept.begin());
+        }
+        g_indices.swap(kept);
+    }
+};
+
+// The index of the edge list, kept from an earlier call over the same tensors or built now (_torch/ops.py), after the
 // opt-in check of the list itself.
 Index conv_index(const Entry& e, int64_t kid, GraphSize n, const Tensor& rows, const Tensor& cols, const Tensor& perm,
                  bool sender_side) {
-    py::gil_scoped_acquire gil;
-    py::tuple got = g_py->conv_index(kid, n.nodes, n.edges, rows, cols,
-                                     e.deterministic ? py::cast(perm) : py::object(py::none()), sender_side);
-    return {py::cast<Tensor>(got[0]), py::cast<bool>(got[1])};
+    const Tensor order = e.deterministic ? perm : Tensor();
+    check_edges(e, n, rows, cols, order);
+    const IndexQuery q(e.mode, e.index_dims, n, rows, cols, order, sender_side);
+    if (auto kept = q.find()) return *kept;
+    const size_t nb = oeq_conv_index_bytes(e.k, n.nodes, n.edges, q.sender_side);
+    const Tensor data = scratch(rows, nb);
+    {
+        py::gil_scoped_acquire gil;
+        const int64_t list = order.defined() && e.mode != OEQ_CONV_GROUPED ? (int64_t)order.data_ptr() : 0;
+        g_py->build_index(kid, n.nodes, n.edges, (int64_t)rows.data_ptr(), (int64_t)cols.data_ptr(), list, q.sender_side,
+                          (int64_t)data.data_ptr(), nb, q.stream());
+    }
+    q.store(data, rows, cols, order);
+    return {data, q.sender_side};
 }
 
 py::object none_or(const OptTensor& t) { return t.has_value() ? py::cast(*t) : py::object(py::none()); }
@@ -384,6 +489,17 @@ Tensor3 call_tp_backward(const Tensor& x, const Tensor& y, const Tensor& w, cons
     static const auto op = find_op<decltype(tp_backward_gpu)>("oeq_amd::tp_backward");
     return op.call(x, y, w, g, kid, spec);
 }
+Tensor4 call_tp_double_backward(const Tensor& x, const Tensor& y, const Tensor& w, const Tensor& g, const Tensor& a,
+                                const Tensor& b, const Tensor& c, int64_t kid, const OptTensor& spec) {
+    static const auto op = find_op<decltype(tp_double_backward_gpu)>("oeq_amd::tp_double_backward");
+    return op.call(x, y, w, g, a, b, c, kid, spec);
+}
+Tensor4 call_conv_double_backward(const Tensor& x, const Tensor& y, const Tensor& w, const Tensor& g, const Tensor& a,
+                                  const Tensor& b, const Tensor& c, const Tensor& rows, const Tensor& cols,
+                                  const Tensor& p, int64_t kid, const OptTensor& spec) {
+    static const auto op = find_op<decltype(conv_double_backward_gpu)>("oeq_amd::conv_double_backward");
+    return op.call(x, y, w, g, a, b, c, rows, cols, p, kid, spec);
+}
 Tensor call_conv_forward(const Tensor& x, const Tensor& y, const Tensor& w, const Tensor& r, const Tensor& c,
                          const Tensor& p, int64_t kid, const OptTensor& spec) {
     static const auto op = find_op<decltype(conv_forward_gpu)>("oeq_amd::conv_forward");
@@ -411,11 +527,25 @@ OptTensor spec_of(AutogradContext* ctx) {
 py::object defined_or_none(const Tensor& t) { return t.defined() ? py::cast(t) : py::object(py::none()); }
 Tensor tensor_or_none(py::handle h) { return h.is_none() ? Tensor() : py::cast<Tensor>(h); }
 
-// The backward of a backward op, in Python: the fused second-order op or a composition of first-order ones.
+// The backward of a backward op. The fused second-order op, called here, is for calls that record nothing for a third
+// derivative (then the composition of differentiable first-order ops is needed) and bring at least two of the three
+// cotangents (a missing one is passed as zeros; with a single one the two first-order calls of the composition read
+// less). The compositions, and kernel sets that borrow another's second-order kernels, are in Python.
 variable_list second_order(const py::object& fn, const variable_list& saved, const variable_list& grads, int64_t kid,
                            const OptTensor& spec, size_t n_inputs) {
     variable_list out(n_inputs);
-    if (!grads[0].defined() && !grads[1].defined() && !grads[2].defined()) return out;
+    const int present = (int)grads[0].defined() + (int)grads[1].defined() + (int)grads[2].defined();
+    if (!present) return out;
+    if (present >= 2 && g_fused_double_backward && !at::GradMode::is_enabled() && entry_of(kid, spec)->fused_second_order) {
+        std::array<Tensor, 3> d;
+        for (size_t i = 0; i < 3; ++i) d[i] = grads[i].defined() ? grads[i] : at::zeros_like(saved[i]);
+        const Tensor4 got = saved.size() == 4
+            ? call_tp_double_backward(saved[0], saved[1], saved[2], saved[3], d[0], d[1], d[2], kid, spec)
+            : call_conv_double_backward(saved[0], saved[1], saved[2], saved[3], d[0], d[1], d[2], saved[4], saved[5],
+                                        saved[6], kid, spec);
+        std::tie(out[0], out[1], out[2], out[3]) = got;
+        return out;
+    }
     py::gil_scoped_acquire gil;
     py::tuple ts(saved.size()), gs(3);
     for (size_t i = 0; i < saved.size(); ++i) ts[i] = py::cast(saved[i]);
@@ -559,8 +689,7 @@ Tensor4 tp_double_backward_autograd(const Tensor& x, const Tensor& y, const Tens
         return {out[0], out[1], out[2], out[3]};
     }
     at::AutoDispatchBelowADInplaceOrView below;
-    static const auto op = find_op<decltype(tp_double_backward_gpu)>(kTpDoubleBackward);
-    return op.call(x, y, w, g, a, b, c, kid, spec);
+    return call_tp_double_backward(x, y, w, g, a, b, c, kid, spec);
 }
 Tensor4 conv_double_backward_autograd(const Tensor& x, const Tensor& y, const Tensor& w, const Tensor& g,
                                       const Tensor& a, const Tensor& b, const Tensor& c, const Tensor& rows,
@@ -571,8 +700,7 @@ Tensor4 conv_double_backward_autograd(const Tensor& x, const Tensor& y, const Te
         return {out[0], out[1], out[2], out[3]};
     }
     at::AutoDispatchBelowADInplaceOrView below;
-    static const auto op = find_op<decltype(conv_double_backward_gpu)>(kConvDoubleBackward);
-    return op.call(x, y, w, g, a, b, c, rows, cols, p, kid, spec);
+    return call_conv_double_backward(x, y, w, g, a, b, c, rows, cols, p, kid, spec);
 }
 
 }  // namespace
@@ -602,7 +730,7 @@ PYBIND11_MODULE(_oeq_torch, m) {
         auto* c = new Callbacks();
         c->resolve = fns["resolve"];
         c->check_edges = fns["check_edges"];
-        c->conv_index = fns["conv_index"];
+        c->build_index = fns["build_index"];
         c->conv_forward = fns["conv_forward"];
         c->conv_backward = fns["conv_backward"];
         c->conv_double_backward = fns["conv_double_backward"];
@@ -626,6 +754,8 @@ PYBIND11_MODULE(_oeq_torch, m) {
         e->dtype = d["double"].cast<bool>() ? at::kDouble : at::kFloat;
         e->mode = d["mode"].cast<int>();
         e->dx_mode = d["dx_mode"].cast<int>();
+        e->index_dims = d["index_dims"].cast<std::array<int64_t, 3>>();
+        e->fused_second_order = d["fused_second_order"].cast<bool>();
         e->native = d["native"].cast<bool>();
         e->alert_forward = d["alert_forward"].cast<bool>();
         e->alert_backward = d["alert_backward"].cast<bool>();
@@ -634,6 +764,29 @@ PYBIND11_MODULE(_oeq_torch, m) {
         EntryRef old = std::move(e);  // (what it replaces, if anything, goes after the lock is released)
         std::unique_lock<std::shared_mutex> lock(g_entries_mu);
         std::swap(g_entries[kid], old);
+    });
+    m.def("set_check_indices", [](bool on) { g_check_indices = on; });
+    m.def("set_fused_double_backward", [](bool on) { g_fused_double_backward = on; });
+    m.def("set_index_cache_entries", [](int64_t n) { g_index_cache_entries = n; });
+    m.def("check_indices", check_indices);
+    m.def("index_cache_size", [] {
+        std::lock_guard<std::mutex> lock(g_indices_mu);
+        return g_indices.size();
+    });
+    m.def("clear_index_cache", [] {
+        std::vector<KeptIndex> gone;
+        std::lock_guard<std::mutex> lock(g_indices_mu);
+        gone.swap(g_indices);
+    });
+    // (index, sender_side) of the edge list: the kept one, or what build(sender_side) returns, which is kept if it may be
+    m.def("kept_index", [](int mode, std::array<int64_t, 3> dims, int64_t nodes, int64_t edges, const Tensor& rows,
+                           const Tensor& cols, const OptTensor& perm, bool need_sender_side, py::function build) {
+        const Tensor order = perm.has_value() ? *perm : Tensor();
+        const IndexQuery q(mode, dims, {nodes, edges}, rows, cols, order, need_sender_side);
+        if (auto kept = q.find()) return std::make_pair(kept->data, kept->sender_side);
+        const Tensor data = py::cast<Tensor>(build(q.sender_side));
+        q.store(data, rows, cols, order);
+        return std::make_pair(data, q.sender_side);
     });
     m.def("forget_entry", [](int64_t kid) {
         EntryRef old;

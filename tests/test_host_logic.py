@@ -3,6 +3,7 @@
 of the shared-weight 'uvw' convolution (core/problems.py: factor_shared_uvw), the latter against the oracle; autograd of the second-order ops."""
 
 import json
+import types
 
 import numpy as np
 import pytest
@@ -130,3 +131,20 @@ def test_second_order_ops_refuse_to_be_differentiated(conv):
     # first-order ops as before
     first = (ops.conv_forward if conv else ops.tp_forward)(x, y, w, *edges, module.kid)
     assert [t.shape for t in torch.autograd.grad(first.sum(), (x, y, w))] == [x.shape, y.shape, w.shape]
+
+
+def test_switches_reach_the_native_ops(monkeypatch):
+    """What a program sets on the ops module is read without Python: the check of edge lists also follows the environment."""
+    assert not ops._native.check_indices()
+    monkeypatch.setattr(ops, "CHECK_INDICES", True)
+    assert ops._native.check_indices()
+    monkeypatch.setattr(ops, "CHECK_INDICES", False)
+    for value, on in (("1", True), ("0", False), ("", False), ("yes", True)):
+        monkeypatch.setenv("OEQ_AMD_CHECK_INDICES", value)
+        assert ops._native.check_indices() == on == ops._check_indices_enabled()
+    calls = []
+    monkeypatch.setattr(ops, "_native", types.SimpleNamespace(
+        set_index_cache_entries=lambda n: calls.append(n), set_fused_double_backward=lambda on: calls.append(on)))
+    ops.INDEX_CACHE_ENTRIES, ops.FUSED_DOUBLE_BACKWARD = 2, False
+    ops.INDEX_CACHE_ENTRIES, ops.FUSED_DOUBLE_BACKWARD = 4, True
+    assert calls == [2, False, 4, True]
