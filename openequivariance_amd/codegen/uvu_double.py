@@ -928,6 +928,25 @@ def add_conv_kernels(s: Src, low: Lowered, base: UvuEmitter, tune: dict, xcd: in
     if em.merged and not groups and not em.merged_fits_one_wave():
         em.merged = False
         groups = em.plan_double_groups(max(1, 8 // em.NCH)) if tune.get("dd_split", 1) else None
+    # Kernels of few words per lane run as many waves as their registers allow instead of two per SIMD, as the
+    # first-order ones do (conv_module): they read an edge's operands where they use them, and only other waves hide
+    # that. Kernel A, up to 96 words (accumulators, X and A, W and C; 3 000 nodes x 32 edges and 9 000 x 20): SevenNet's first
+    # layer (26 words) 116 / 87 us and 198 / 168, NequiX's first 89 / 78 and 146 / 141, water (58) 77 / 64 and 132 / 122,
+    # MACE-medium (50) 198 / 187 and 344 / 342, aspirin (58) 125 / 124, nequip-uvu (87) 106 / 89 and 180 / 164; a third
+    # wave only where X outweighs the accumulators (SevenNet's last layer 90 / 97 without a limit, 93 with three; 700 x 30
+    # 44 / 23 and 25); from 123 words on (mace-large) nothing gains. Staging the operands in LDS gives no more than the
+    # waves do (MACE-medium 188, aspirin 123; mace-large 414 / 428).
+    # Kernel B, a third wave up to 80 words: SevenNet's first layer 162 / 136 and 297 / 243, water 110 / 105 and 197 / 188,
+    # MACE-medium 294 / 284 and 536 / 514; not where a row has nearly as many terms of d/dX as weights, unless two edges
+    # share the wave (aspirin 196 / 199 and 359 / 362), nor above (nequip-uvu, 112: 158 / 163 and 302 / 308).
+    waves_a, waves_b = tune.get("dd_wa", 2), tune.get("dd_wb", 2)
+    user_tune = os.environ.get("OEQ_AMD_TUNE", "")
+    x_all, acc = sum(low.in1[b].d for b in em.used_in1), sum(low.out[io].d for io in em.used_out)
+    if low.elem_size == 4 and not kahan and "dd_wa" not in user_tune and kernel_a_need(em) <= 96:
+        waves_a = -2 if acc >= x_all else 23
+    if (low.elem_size == 4 and not shared and not em.merged and "dd_wb" not in user_tune
+            and acc + 3 * x_all + em.l2_pad + 2 * em.n_wslots <= 80 and (em.R > 1 or 3 * x_all <= 2 * em.n_wslots)):
+        waves_b = 23
     descs = []
     if not em.merged:
         segw = min(len(em.segments), max(1, tune.get("dd_segw", 4)), max(1, 8 // em.NCH)) if em.R == 1 else 1
@@ -936,23 +955,23 @@ def add_conv_kernels(s: Src, low: Lowered, base: UvuEmitter, tune: dict, xcd: in
             # several output segments: one node per block, as in the first-order forward kernel (second-order op:
             # SevenNet main layer -4 %, three more mixed-multiplicity shapes -2 % .. -3 %, nothing slower)
             G_a = 1
-        blk_a = em.emit_conv_double_a(s, G_a, tune.get("dd_wa", 2), xcd, segw)
+        blk_a = em.emit_conv_double_a(s, G_a, waves_a, xcd, segw)
         descs.append((rt.ROLE_DOUBLE_BACKWARD_A, "double_backward_A", blk_a, G_a, 0, xcd))
-        n = split_waves(tune, "conv_fsplit_a", em, segw, tune.get("dd_wa", 2))
+        n = split_waves(tune, "conv_fsplit_a", em, segw, waves_a)
         n = em.split_count(n, 0, segw)
         if n > 1 and not kahan and splits is not None:
             splits["double_backward_A_split"] = Split("conv_fsplit_a", n, em.R, segw)
-            blk_as = em.emit_conv_double_a(s, 1, tune.get("dd_wa", 2), xcd, segw, "double_backward_A_split", n)
+            blk_as = em.emit_conv_double_a(s, 1, waves_a, xcd, segw, "double_backward_A_split", n)
             descs.append((rt.ROLE_DOUBLE_BACKWARD_A_SPLIT, "double_backward_A_split", blk_as, 1, 0, xcd))
     if groups:
-        blk_b = em.emit_conv_double_b_split(s, groups, tune.get("dd_wb", 2), xcd)
+        blk_b = em.emit_conv_double_b_split(s, groups, waves_b, xcd)
         G_b = 1
     elif shared:
         G_b = 1 if em.NCH > 1 else groups_b
-        blk_b = em.emit_conv_double_b(s, G_b, tune.get("dd_wb", 2), 1)
+        blk_b = em.emit_conv_double_b(s, G_b, waves_b, 1)
         return descs + [(rt.ROLE_DOUBLE_BACKWARD_B, "double_backward_B", blk_b, G_b, compute_units * 8, 1)]
     else:
-        blk_b = em.emit_conv_double_b(s, G, tune.get("dd_wb", 2), xcd)
+        blk_b = em.emit_conv_double_b(s, G, waves_b, xcd)
         G_b = 1 if em.NCH > 1 else G
     return descs + [(rt.ROLE_DOUBLE_BACKWARD_B, "double_backward_B", blk_b, G_b, 0, xcd)]
 
