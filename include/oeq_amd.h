@@ -22,7 +22,7 @@
 #include <stdint.h>
 
 /* Changes with every change of a struct, an argument list or an enumerator below. */
-#define OEQ_ABI_VERSION 7
+#define OEQ_ABI_VERSION 8
 
 #ifdef __cplusplus
 extern "C" {
@@ -93,7 +93,10 @@ typedef enum {
                                        receivers for the senders and the sender-side index) */
     OEQ_ROLE_CONV_BACKWARD_DX_SPLIT = 20,  /* the same for OEQ_ROLE_CONV_BACKWARD_DX */
     OEQ_ROLE_DOUBLE_BACKWARD_A_SPLIT = 21, /* and for OEQ_ROLE_DOUBLE_BACKWARD_A */
-    OEQ_ROLE_COUNT = 22
+    OEQ_ROLE_SLICE_COUNT = 22,      /* grouping a list of moderate size slice by slice: a histogram per slice, */
+    OEQ_ROLE_SLICE_SCAN = 23,       /*   first position of every slice's items of a segment, and the segment starts, */
+    OEQ_ROLE_SLICE_PLACE = 24,      /*   every item to its place, and the table of extra walk positions */
+    OEQ_ROLE_COUNT = 25
 } oeq_role;
 
 /* How the convolution kernels of a set find the edges of a node (oeq_problem_dims.deterministic):

@@ -33,7 +33,7 @@ import os
 import re
 from typing import Callable, Dict, List, NamedTuple, Optional, Sequence, Tuple
 
-from .common import LOOK_AHEAD, Src, fixup_backward_kernel, prelude, utility_kernels
+from .common import LOOK_AHEAD, SLICE_DESCS, Src, fixup_backward_kernel, prelude, utility_kernels
 from .lower import Lowered, Path, float_literal
 
 UNROLL_V_LIMIT = 8
@@ -3004,6 +3004,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
             (rt.ROLE_GROUP_ORDER, "oeq_group_order", 256, 4, compute_units * 32),
             (rt.ROLE_ORDER_HOP, "oeq_order_hop", 256, 256, compute_units * 16),
             (rt.ROLE_INDEX_SMALL, "oeq_index_small", 1024, 1, 32),
+            *([] if deterministic else SLICE_DESCS),
             # long edge segments in chunks: the sum of the chunks' rows
             (rt.ROLE_CONV_FIXUP_FORWARD, "fixup_forward", 256, 1, compute_units * 32),
         ]

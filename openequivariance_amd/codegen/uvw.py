@@ -1233,7 +1233,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     sum for the backward pass. ``deterministic``: the caller brings receiver-sorted edges and the
     sender-major permutation; otherwise the library groups the edge ids on the device first."""
     from .. import runtime as rt
-    from .common import fixup_backward_kernel
+    from .common import SLICE_DESCS, fixup_backward_kernel
 
     assert conv_supported(low)
     shared = low.shared_weights
@@ -1274,6 +1274,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         (rt.ROLE_GROUP_ORDER, "oeq_group_order", 256, 4, cu * 32),
         (rt.ROLE_ORDER_HOP, "oeq_order_hop", 256, 256, cu * 16),
         (rt.ROLE_INDEX_SMALL, "oeq_index_small", 1024, 1, 32),
+        *([] if deterministic else SLICE_DESCS),
         (rt.ROLE_CONV_FIXUP_FORWARD, "fixup_forward", 256, 1, cu * 32),
     ]
     t = em.tune

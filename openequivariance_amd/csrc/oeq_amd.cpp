@@ -101,6 +101,12 @@ constexpr int64_t kScanTile = 1024, kScanBlocks = 32;
 // Largest edge list that oeq_index_small takes: its LDS arrays, of which every block holds histogram and item list of
 // the whole side (the blocks share out only the placing, so that their number squared is what a side costs).
 constexpr int64_t kSmallItems = 16384, kSmallSegments = 4096;
+// Caller-sorted lists: one block per side reads a cache line for every key of the senders' list, 12 us for 7 800 edges and
+// 23 for 15 500; the two launches over the whole grid take 9 us and the gap between them.
+constexpr int64_t kSmallSorted = 8192;
+// Largest edge list that is grouped slice by slice (oeq_slice_count / scan / place): the scan keeps the counts of all
+// slices of a segment in registers, the placing blocks have two LDS entries per segment.
+constexpr int64_t kSlice = 4096, kSlices = 64, kSliceSegments = 16384;
 
 }  // namespace
 
@@ -228,6 +234,21 @@ struct oeq_kernels {
         void* args[] = {&n_items, &n_segments, &limit, &capacity, &a, &b};
         const int64_t per_side = std::min<int64_t>(kScanBlocks, (n_segments + kScanTile) / kScanTile);
         return launch(OEQ_ROLE_GROUP_SCAN, 0, args, stream, (unsigned)(per_side * (b.ptr ? 2 : 1)));
+    }
+
+    // What group_by_key does, for lists that fit (grouped_in_slices); the histograms lie in the sides' slots.
+    int group_in_slices(int64_t n_items, int64_t n_segments, int64_t limit, int64_t capacity, IndexSide a, IndexSide b,
+                        void* stream) {
+        const int64_t sides = b.ptr ? 2 : 1;
+        int64_t parts = (n_items + kSlice - 1) / kSlice;
+        int64_t hub_blocks = a.hubptr ? std::min<int64_t>(kScanBlocks, (n_segments + kScanTile) / kScanTile) : 0;
+        void* cargs[] = {&n_items, &n_segments, &parts, &a, &b};
+        int rc = launch(OEQ_ROLE_SLICE_COUNT, 0, cargs, stream, (unsigned)(parts * sides));
+        void* sargs[] = {&n_segments, &parts, &a, &b};
+        if (!rc) rc = launch(OEQ_ROLE_SLICE_SCAN, 0, sargs, stream, (unsigned)((n_segments + 64) / 64 * sides));
+        void* pargs[] = {&n_items, &n_segments, &parts, &hub_blocks, &limit, &capacity, &a, &b};
+        if (!rc) rc = launch(OEQ_ROLE_SLICE_PLACE, 0, pargs, stream, (unsigned)((parts + hub_blocks) * sides));
+        return rc;
     }
 
     // Counting sort of the item indices 0..n_items-1 by key, for one or two key lists: ptr[0..n_segments] =
@@ -641,6 +662,22 @@ static size_t hub_rows_bytes(const oeq_kernels* k, int role, int64_t nnz) {
     return align_up((size_t)hub_units(k, role, nnz) * (size_t)k->dims.L3_dim * (size_t)k->dims.elem_size, 256);
 }
 
+// Grouping slice by slice, and the histograms it leaves in a side's scratch: a row per slice, and the sums over 64
+// segments.
+static bool grouped_in_slices(const oeq_kernels* k, int64_t node_count, int64_t nnz) {
+    return k->dims.deterministic == OEQ_CONV_GROUPED && nnz <= kSlice * kSlices && node_count <= kSliceSegments &&
+           k->roles[OEQ_ROLE_SLICE_COUNT].present && k->roles[OEQ_ROLE_SLICE_SCAN].present &&
+           k->roles[OEQ_ROLE_SLICE_PLACE].present;
+}
+static size_t group_scratch_bytes(const oeq_kernels* k, int64_t node_count, int64_t nnz) {
+    size_t bytes = perm_bytes_of(nnz);  // (number and place of every item, 32 bits each)
+    if (grouped_in_slices(k, node_count, nnz)) {
+        const size_t parts = (size_t)((nnz + kSlice - 1) / kSlice), row = (size_t)(node_count + (node_count + 63) / 64);
+        bytes = std::max(bytes, align_up(parts * row * sizeof(uint32_t), 256));
+    }
+    return bytes;
+}
+
 // The index of an edge list: what the walk kernels derive from (rows, cols) alone. Receiver side: CSR
 // pointers, in GROUPED mode the edge ids grouped by receiver, and the walk order of the nodes. Sender side
 // (for the calls that reduce per-edge dX terms): CSR pointers over senders and, in GROUPED mode, the edge ids
@@ -685,8 +722,9 @@ static IndexLayout index_layout(const oeq_kernels* k, int64_t node_count, int64_
     w.keep = w.total;
     if (grouped) {
         w.counts = take(pb);  // (32 bits per node and side)
-        w.scratch = take(qb);
-        if (sender_side) w.scratch2 = take(qb);
+        const size_t sb = group_scratch_bytes(k, node_count, nnz);
+        w.scratch = take(sb);
+        if (sender_side) w.scratch2 = take(sb);
     }
     if (ordered) {
         w.key_a = take(pb);
@@ -796,11 +834,13 @@ static int build_index(oeq_kernels* k, const char* who, const IndexLayout& w, in
     } else {
         b.list = transpose_perm;
     }
-    if (nnz <= kSmallItems && node_count <= kSmallSegments && k->roles[OEQ_ROLE_INDEX_SMALL].present) {
+    if (nnz <= (grouped ? kSmallItems : kSmallSorted) && node_count <= kSmallSegments && k->roles[OEQ_ROLE_INDEX_SMALL].present) {
         int64_t n = nnz, ns = node_count, lim = limit, c = cap;
         void* args[] = {&n, &ns, &lim, &c, &a, &b};
         const unsigned parts = grouped ? (unsigned)((nnz + 1023) / 1024) : 1u;
         rc = k->launch(OEQ_ROLE_INDEX_SMALL, 0, args, stream, parts * (b.ptr ? 2u : 1u));
+    } else if (grouped && grouped_in_slices(k, node_count, nnz)) {
+        rc = k->group_in_slices(nnz, node_count, limit, cap, a, b, stream);
     } else if (grouped) {
         rc = k->group_by_key(nnz, node_count, limit, cap, a, b, stream);
     } else {

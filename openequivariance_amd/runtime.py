@@ -56,10 +56,13 @@ ROLE_CONV_FIXUP_FORWARD = 18
 ROLE_CONV_BACKWARD_DX = 19
 ROLE_CONV_BACKWARD_DX_SPLIT = 20
 ROLE_DOUBLE_BACKWARD_A_SPLIT = 21
+ROLE_SLICE_COUNT = 22
+ROLE_SLICE_SCAN = 23
+ROLE_SLICE_PLACE = 24
 
 CONV_ATOMIC, CONV_SORTED, CONV_GROUPED = 0, 1, 2
 DX_TERMS, DX_ATOMIC, DX_ARRIVAL, DX_SENDER_WALK = 0, 1, 2, 3
-ABI_VERSION = 7
+ABI_VERSION = 8
 
 
 class OeqError(RuntimeError):

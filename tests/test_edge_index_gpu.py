@@ -1,6 +1,6 @@
 """The index of an edge list (segment starts, grouped edge ids, table of extra walk positions, walk order) against
-numpy, at the sizes where its kernels hand over to each other: one-launch build up to 16 384 edges and 4 096 nodes,
-scan tiles of 1 024 segments, segments ranked by a wave / through a bitmap / by the whole grid."""
+numpy, at the sizes where its kernels hand over to each other: one-launch build up to 16 384 edges (sorted lists: 8 192) and 4 096 nodes,
+grouping slice by slice up to 262 144 edges and 16 384 nodes, scan tiles of 1 024 segments, segments ranked by a wave / through a bitmap / by the whole grid."""
 
 import numpy as np
 import pytest
@@ -33,6 +33,11 @@ SIZES = [
     (1, 1, (0, 0)), (3, 700, (400, 500)), (64, 1024, (0, 257)), (192, 6144, (0, 0)),
     (4096, 16384, (256, 16384)), (4096, 16384, (5000, 0)), (4097, 16384, (300, 1025)), (100, 16385, (0, 1024)),
     (1023, 20000, (2000, 3000)), (1024, 20000, (0, 0)), (8191, 50001, (0, 1030)), (8192, 40000, (255, 512)), (140001, 150000, (4000, 10)),
+    # grouped slice by slice: up to 64 slices of 4 096 edges and 16 384 nodes, more than 256 edges of a node in a slice
+    # through a bitmap
+    (1, 20480, (0, 0)), (5000, 24576, (1536, 1542)), (16384, 262144, (262144, 70000)), (300, 262144, (0, 0)),
+    (300, 262145, (0, 0)), (16385, 20000, (300, 0)), (255, 16385, (16385, 256)), (256, 69633, (0, 4097)),
+    (300, 8192, (257, 0)), (300, 8193, (0, 257)),
 ]
 
 
