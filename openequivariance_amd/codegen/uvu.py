@@ -31,6 +31,7 @@ from __future__ import annotations
 
 import os
 import re
+from dataclasses import replace
 from typing import Callable, Dict, List, NamedTuple, Optional, Sequence, Tuple
 
 from .common import LOOK_AHEAD, SLICE_DESCS, Src, fixup_backward_kernel, prelude, utility_kernels
@@ -789,18 +790,19 @@ class UvuEmitter:
                         s(f"{{ const T y = c.{e}; const T t = a.{e} + y; c.{e} = y - (t - a.{e}); a.{e} = t; }}")
                 s.close()
 
-    def _emit_load_edge(self, s: Src, name: str, in1_blocks: List[int], paths: List[Path]):
+    def _emit_load_edge(self, s: Src, name: str, in1_blocks: List[int], paths: List[Path], sender: bool = False):
         """load_edge: fetch X[cols[e]] (the listed blocks), the weights of the
-        listed paths and the edge's Y into an E_t."""
+        listed paths and the edge's Y into an E_t. ``sender``: the caller has cols[e]."""
         low = self.low
         paths = self._paths(paths)
         s.open(
-            f"OEQ_DEV void {name}{self._sfx()}(E_t& d, const i64 e, const T* __restrict__ L1_in, "
+            f"OEQ_DEV void {name}{self._sfx()}(E_t& d, const i64 e, {'const i64 c, ' if sender else ''}const T* __restrict__ L1_in, "
             "const T* __restrict__ L2_in, "
 f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, const int u"
             f"{', const Q_t& qt' if self.use_q else ''})"
         )
-        s("const i64 c = oeq_idx(cols[e], node_count);")
+        if not sender:
+            s("const i64 c = oeq_idx(cols[e], node_count);")
         s(f"const T* xrow = L1_in + c * {low.L1};")
         s(f"const T* yrow = L2_in + e * {low.L2};")
         s(f"const T* wrow = W{'' if low.shared_weights else f' + e * {low.WN}'};")
@@ -2426,6 +2428,163 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         s.close()
         return block
 
+    GROUP_BATCH = 8  # edges whose dY the waves of a node collect before they add them up
+
+    def plan_width_groups(self) -> Optional[List["UvuEmitter"]]:
+        """Groups of paths for the backward kernel of rows with blocks of different widths: an emitter per width, the
+        blocks of up to 64 channels first, which run one edge to a wave, then those of up to 32, 16, ... channels, two,
+        four, ... edges side by side. Every input and output block belongs to one group. None where that saves less
+        than a quarter of the multiply-adds that lanes without a channel take part in, and where a group's gradient
+        slice does not fit its wave's registers.
+
+        One wave per edge leaves half the lanes idle in blocks of 32 channels, which have three quarters of the
+        multiply-adds of SevenNet's main layer, and the waves that shared its outputs summed dX through LDS, two
+        barriers for every edge. In groups a wave has its rows of dX to itself and meets the others once in eight edges.
+        Whole passes, us, before / in groups: SevenNet's main layer 2 003 nodes x 40 edges 707 / 564, 8 000 x 30
+        1 896 / 1 532, 600 x 20 195 / 157, ir_mul 3 000 x 30 803 / 622; NequiX's main layer (one wave before) 600 x 20
+        126 / 123, 3 000 x 30 513 / 495, 9 000 x 24 1 110 / 1 054. The wide blocks and the two narrow ones in three waves of 168 registers
+        each: 594, of which 48 B scratch memory."""
+        low = self.low
+        if self.R != 1 or self.NCH != 1 or low.shared_weights or not self.can_preload or low.elem_size != 4:
+            return None
+        lanes: Dict[int, int] = {}
+        for p in low.paths:
+            n = _pow2ceil(low.in1[p.i1].mul)
+            if _pow2ceil(low.out[p.io].mul) != n or lanes.setdefault(p.io, n) != n or n * self.GROUP_BATCH < 64:
+                return None
+        idle = sum(len(p.nnz) * (64 - lanes[p.io]) for p in low.paths)
+        if 4 * idle < 64 * sum(len(p.nnz) for p in low.paths):
+            return None
+        groups = []
+        for n in sorted(set(lanes.values()), reverse=True):
+            em = UvuEmitter(replace(low, paths=[p for p in low.paths if lanes[p.io] == n], lanes_per_row=n,
+                                    rows_per_wave=64 // n))
+            em.nt, em.mask_loads, em.forms = self.nt, self.mask_loads, self.forms
+            em.rows_stage = None  # (the forward's)
+            groups.append(em)
+        if len(groups) < 2 or any(em.backward_words(True) > 285 for em in groups):
+            return None
+        return groups
+
+    def emit_conv_backward_groups(self, s: Src, ems: List["UvuEmitter"], waves_per_eu: int, xcd: int) -> int:
+        """Backward of rows with blocks of different widths (``plan_width_groups``): every wave of a block walks the
+        edges of one node for its own group of paths, whose rows of dX and dW are its own as well; the waves meet
+        once in ``GROUP_BATCH`` edges, to add up their partial sums of dY."""
+        low, W, n = self.low, len(ems), self.GROUP_BATCH
+        block = 64 * W
+        operands = ("i64 node_count, i64 nnz, const T* __restrict__ L1_in, const T* __restrict__ L2_in, "
+                    "T* __restrict__ L2_grad, const T* __restrict__ W, T* __restrict__ W_grad, "
+                    "const T* __restrict__ L3_grad, const i64* __restrict__ cols, T* __restrict__ dx_tmp, "
+                    "const i64* __restrict__ eperm, ")
+        s(LOOK_AHEAD)
+        for gi, em in enumerate(ems):
+            # the next edges' operands in a second set of registers, where they fit
+            ahead = (em.backward_words(True) + sum(low.in1[b].d for b in em.used_in1) + em.n_wslots
+                     + (low.L2 if em.R > 1 else 0)) <= 240
+            s(f"namespace oeq_group{gi} {{")
+            em.emit_structs(s)
+            em._emit_load_edge(s, "load_edge_b", em.used_in1, em.low.paths, sender=True)
+            s.open(f"OEQ_DEV void walk({operands}const i64 node, const i64 e0, const i64 e1, "
+                   f"T (*s_dy)[{W}][{self.l2_pad}])")
+            em._lane_prologue(s)
+            s("G_t gr;")
+            em._load_g(s, f"L3_grad + node * {low.L3}", em.used_out)
+            s("int batch = 0;")
+            # The lanes hold the numbers and senders of the next 64 edges. (Read by lane number: an exchange through LDS
+            # would not see what lanes hold that have no edge left.)
+            s("oeq_ahead ahead;")
+
+            def of(field, k):
+                lanes = [f"__builtin_amdgcn_readlane(ahead.{field}, ({k} + {q}) & 63)" for q in range(em.R)]
+                value = lanes[-1]
+                for q in range(em.R - 2, -1, -1):
+                    value = f"(r == {q} ? {lanes[q]} : {value})"
+                return value
+
+            def load(buf, k):
+                s(f"const i64 eid_{buf} = {of('eid', k)}, sender_{buf} = {of('sender', k)};")
+                s(f"load_edge_b({buf}, eid_{buf}, sender_{buf}, L1_in, L2_in, W, cols, node_count, u);")
+
+            if ahead:
+                s("E_t B;")
+                s.open("if (e0 < e1)")
+                s("oeq_look_ahead(ahead, e0 + lane, e1, eperm, cols, node_count);")
+                load("B", "0")
+                s.close()
+            s.open(f"for (i64 eb = e0; eb < e1; eb += {n}, batch ^= {n})")
+            s(f"const int count = e1 - eb < {n} ? (int)(e1 - eb) : {n}, done = (int)(eb - e0);")
+            if not ahead:
+                s("if ((done & 63) == 0) oeq_look_ahead(ahead, eb + lane, e1, eperm, cols, node_count);")
+            s.open(f"for (int k0 = 0; k0 < count; k0 += {em.R})")
+            s("const int k = k0 + r;")
+            s("E_t A;")
+            if ahead:
+                s(f"const i64 eid = {of('eid', '(done + k0)')};")
+                s("A = B;")
+                s(f"const int next = done + k0 + {em.R};")
+                s.open(f"if (next < (int)(e1 - e0))")
+                s("if ((next & 63) == 0) oeq_look_ahead(ahead, e0 + next + lane, e1, eperm, cols, node_count);")
+                load("B", "next")
+                s.close()
+            else:
+                load("A", "(done + k0)")
+                s("const i64 eid = eid_A;")
+            # (No lane drops out: lanes past the last edge do that edge again, store what its own lanes store, and
+            # leave dY where no sum looks.)
+            yacc, wacc = em._acc_preloaded("A")
+            s(f"T* dwrow = W_grad + eid * {low.WN};")
+            s("X_t dx;")
+            em._zero_x(s, "dx")
+            s(f"T dy[{self.l2_pad}];")
+            s(f"for (int t = 0; t < {self.l2_pad}; ++t) dy[t] = T(0);")
+            deferred = em._dw_deferred(None)
+            if deferred:
+                s(f"T dwkeep[{em.n_wslots}];")
+            em._bwd_paths(s, xname="A.x", yacc=yacc, wacc=wacc, dw_mode="store")
+            em._pin_gradients(s, em.used_in1, deferred)
+            if deferred:
+                em._flush_dwkeep(s, None)
+            s(f"T* dxrow = dx_tmp + eid * {low.L1};")
+            em._store_dx(s, "dxrow", "true", nt=bool(self.nt & 2))
+            if gi == 0:
+                self._zero_untouched_in1(s, "dxrow", "true")
+            cur, dup = em._dy_reduce(s)
+            s.open(f"if ((ul & {dup}) == 0)")
+            for j in range(cur):
+                s(f"s_dy[batch + k][{gi}][dyidx + {j}] = rv[{j}];")
+            s.close()
+            s.close()
+            # (two batches take turns in LDS: a wave gets to the one after the next only when all have read this one)
+            s("__syncthreads();")
+            s.open(f"for (int t = (int)threadIdx.x; t < count * {self.l2_pad}; t += {block})")
+            s(f"const int k = t / {self.l2_pad}, j = t % {self.l2_pad};")
+            if self.l2_pad != low.L2:
+                s(f"if (j >= {low.L2}) continue;")
+            terms = " + ".join(f"s_dy[batch + k][{c}][j]" for c in range(W))
+            s(f"L2_grad[OEQ_EDGE(eb + k) * {low.L2} + j] = {terms};")
+            s.close()
+            s.close()
+            s.close()
+            s(f"}}  // namespace oeq_group{gi}")
+        s.open(
+            f'extern "C" __global__ {self._attrs(block, waves_per_eu)} void backward(i64 node_count, i64 nnz, '
+            "const T* __restrict__ L1_in, T* __restrict__ L1_grad, const T* __restrict__ L2_in, "
+            "T* __restrict__ L2_grad, const T* __restrict__ W, T* __restrict__ W_grad, "
+            "const T* __restrict__ L3_grad, const i64* __restrict__ rows, const i64* __restrict__ cols, "
+            "const i64* __restrict__ rowptr, T* __restrict__ dx_tmp, const i64* __restrict__ eperm, "
+            "T* __restrict__ wpartial, const i64* __restrict__ colptr, const i64* __restrict__ sperm, "
+            f"int* __restrict__ arrivals, const i64* __restrict__ order{self.HUB_PARAMS}{self.PARTS_PARAM})"
+        )
+        self._lane_prologue(s, W)
+        s(f"__shared__ T s_dy[{2 * n}][{W}][{self.l2_pad}];")
+        self._node_loop_open(s, 1, xcd, parts=True)
+        for gi in range(W):
+            s(f"{'else ' if gi else ''}if (sg == {gi}) oeq_group{gi}::walk(node_count, nnz, L1_in, L2_in, L2_grad, W, "
+              "W_grad, L3_grad, cols, dx_tmp, eperm, node, e0, e1, s_dy);")
+        s.close()
+        s.close()
+        return block
+
     DX_TERMS, DX_ATOMIC, DX_ARRIVAL, DX_SENDER_WALK = 0, 1, 2, 3
 
     def emit_conv_backward(self, s: Src, deterministic: bool, G: int, pipelined: bool, waves_per_eu: int = 0,
@@ -2749,7 +2908,8 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
                     dd_gres=-1, dd_split=1, dd_segw=4, dd_merge=0, dd_need=200, dd_ngrp=0, conv_gbud=0, conv_ngrp=0, conv_fit=300, conv_fw=0, conv_pf=0,
                     conv_dxm=-1, conv_q=0, conv_hops=2, conv_qpin=1, conv_qaf=48, conv_qab=24, tp_mask=0, tp_forms=1,
                     conv_hub=256, conv_dxs=-1, conv_omin=32768, conv_fsplit=-1, conv_fsplit_f=-1, conv_fsplit_x=-1, conv_fsplit_a=-1,
-                    conv_fsmax=-1, conv_parts=-1, conv_stg=1))
+                    conv_fsmax=-1, conv_parts=-1, conv_stg=1,
+                    conv_wgrp=1))
     assert deterministic or not kahan, "kahan=True requires deterministic=True"
     # knobs somebody set: the rules below leave those alone
     user_tune = os.environ.get("OEQ_AMD_TUNE", "")
@@ -2896,7 +3056,15 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     em.fit_words = t["conv_fit"]
     em.group_count = t["conv_ngrp"]
     em.bwd_groups = em.plan_backward_groups(max(1, 8 // em.NCH)) if (walk and t["conv_split"] and gres is None) else None
-    if em.bwd_groups:
+    sender_walk = (9 * low.L1 >= 2 * (low.WN + low.L2 + low.L3) and not low.shared_weights and t["conv_dxm"] < 0
+                   and t["conv_dxs"] < 0) or t["conv_dxs"] > 0
+    width_groups = None
+    if walk and t["conv_wgrp"] and t["conv_split"] and gres is None and t["conv_dxm"] <= 0 and not sender_walk and per_lane > 48:
+        width_groups = em.plan_width_groups()
+    if width_groups:
+        G_b, dx_mode = 1, em.DX_TERMS
+        blk_b = em.emit_conv_backward_groups(s, width_groups, t["conv_wb"], xcd)
+    elif em.bwd_groups:
         G_b = 1
         wpb = em.NCH * len(em.bwd_groups)
         if 8 % wpb and 12 % wpb == 0 and "conv_wb" not in user_tune:
@@ -3031,6 +3199,10 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         _lds, scratch = rt.kernel_resources(rt.compile_source(src)).get("backward_dx", (0, 0))
         if scratch > 64:
             return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_dxs=0), draft)
+    if width_groups and rt.kernel_resources(rt.compile_source(src)).get("backward", (0, 0))[1] > 0:
+        # never with scratch memory: slower, and with the next edges' operands spilled (NequiX's main layer held to 168 registers,
+        # 240 B) the X values of an edge came back as another's
+        return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wgrp=0), draft)
     if staged64 and len(em.segments) > 1 and rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))[1] > 0:
         return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_stg=0), draft)
     if em.seg_waves > 1 and "conv_segw" not in user_tune:
