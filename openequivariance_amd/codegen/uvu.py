@@ -3059,8 +3059,20 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     sender_walk = (9 * low.L1 >= 2 * (low.WN + low.L2 + low.L3) and not low.shared_weights and t["conv_dxm"] < 0
                    and t["conv_dxs"] < 0) or t["conv_dxs"] > 0
     width_groups = None
-    if walk and t["conv_wgrp"] and t["conv_split"] and gres is None and t["conv_dxm"] <= 0 and not sender_walk and per_lane > 48:
+    # A wave per width pays where the row of all widths is much for one wave. Backward: two widths, whose waves wait for each
+    # other least, and more than the smallest rows (step, us, one wave / a wave per width, by the estimate of that one
+    # wave's registers, 3 000 nodes x 30 edges: 178 (64x0e+64x1o+8x2e+8x1e) 266 / 274,
+    # 195 (64x0e+64x1o+32x2e+32x3o) 333 / 325, 215 (96x{0e,1o,2e}) 410 / 403, 275 (NequiX's main layer) 512 / 495; above it is two
+    # waves that lose: SevenNet's main layer (2 003 x 40) 711 / 566, 96x{0e..3o} 1 026 / 879, 64x0e+64x1o+16x2e+16x3o
+    # 453 / 400). Three and four widths lose: 64x0e+32x1o+16x2e 224 / 273, 64x0e+64x1o+32x2e+16x3o 468 / 516,
+    # 128x0e+64x1o+32x2e+8x3o 359 / 422. Not where blocks leave lanes of their own width without a channel
+    # (100x0e+40x1o+20x2e+9x1e: 304 / 470). (conv_wgrp: bit 1 on, 4 regardless of this)
+    forced = bool(t["conv_wgrp"] & 4)
+    if (walk and t["conv_wgrp"] & 1 and t["conv_split"] and gres is None and t["conv_dxm"] <= 0 and not sender_walk
+            and (forced or (per_lane > 48 and em.backward_words(True) > 180))):
         width_groups = em.plan_width_groups()
+        if width_groups and not forced and (len(width_groups) > 2 or any(g.ragged() for g in width_groups)):
+            width_groups = None
     if width_groups:
         G_b, dx_mode = 1, em.DX_TERMS
         blk_b = em.emit_conv_backward_groups(s, width_groups, t["conv_wb"], xcd)

@@ -77,7 +77,7 @@ def test_a_wave_for_every_width(name, rows):
 @pytest.mark.parametrize("layout,det,tune", [("mul_ir", True, "conv_parts=1"), ("ir_mul", False, "conv_parts=3"),
                                              ("mul_ir", False, "conv_hub=40")])
 def test_widths_against_the_oracle(name, layout, det, tune, monkeypatch):
-    _check(_problem(name, np.float32, layout), _problem(name, np.float32, "mul_ir"), det, tune, monkeypatch)
+    _check(_problem(name, np.float32, layout), _problem(name, np.float32, "mul_ir"), det, "conv_wgrp=7," + tune, monkeypatch)
 
 
 @pytest.mark.gpu
