@@ -790,9 +790,10 @@ class UvuEmitter:
                         s(f"{{ const T y = c.{e}; const T t = a.{e} + y; c.{e} = y - (t - a.{e}); a.{e} = t; }}")
                 s.close()
 
-    def _emit_load_edge(self, s: Src, name: str, in1_blocks: List[int], paths: List[Path], sender: bool = False):
+    def _emit_load_edge(self, s: Src, name: str, in1_blocks: List[int], paths: List[Path], sender: bool = False,
+                        y: bool = True):
         """load_edge: fetch X[cols[e]] (the listed blocks), the weights of the
-        listed paths and the edge's Y into an E_t. ``sender``: the caller has cols[e]."""
+        listed paths and (``y``) the edge's Y into an E_t. ``sender``: the caller has cols[e]."""
         low = self.low
         paths = self._paths(paths)
         s.open(
@@ -814,7 +815,7 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         if self.use_q:
             for r in range(self.q_slabs):
                 s(f"d.yq[{r}] = yrow[qt.j[{r}]];")
-        else:
+        elif y:
             for j in range(low.L2):
                 s(f"d.y[{j}] = yrow[{j}];")
         s.close()
@@ -1057,10 +1058,16 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
               f"({rowexpr})[{bo.off} + t] = T(0);")
             s.close()
 
-    def _lane_prologue(self, s: Src, seg_waves: int = 1):
+    def _lane_prologue(self, s: Src, seg_waves: int = 1, own: bool = False):
         """``seg_waves`` > 1: the waves of a node are (chunk, sg) pairs, ``sg`` naming the output segments
-        the wave owns."""
-        s("const int lane = oeq_lane();")
+        the wave owns. ``own``: for one of several branches of a kernel, whose lane offsets the compiler is not to form
+        before it branches (SevenNet's main layer, forward with three of them: 184 registers, each by itself 136 to 160)."""
+        if own:
+            s("int own_lane = oeq_lane();")
+            s('asm volatile("" : "+v"(own_lane));')
+            s("const int lane = own_lane;")
+        else:
+            s("const int lane = oeq_lane();")
         s("const int wave = oeq_wave();")
         s(f"const int chunk = wave % {self.NCH};")
         if seg_waves > 1:
@@ -2444,6 +2451,11 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         1 896 / 1 532, 600 x 20 195 / 157, ir_mul 3 000 x 30 803 / 622; NequiX's main layer (one wave before) 600 x 20
         126 / 123, 3 000 x 30 513 / 495, 9 000 x 24 1 110 / 1 054. The wide blocks and the two narrow ones in three waves of 168 registers
         each: 594, of which 48 B scratch memory."""
+        groups = self.width_groups()
+        return groups if groups and all(em.backward_words(True) <= 285 for em in groups) else None
+
+    def width_groups(self) -> Optional[List["UvuEmitter"]]:
+        """The paths by the width of their blocks, see ``plan_width_groups``."""
         low = self.low
         if self.R != 1 or self.NCH != 1 or low.shared_weights or not self.can_preload or low.elem_size != 4:
             return None
@@ -2458,13 +2470,128 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         groups = []
         for n in sorted(set(lanes.values()), reverse=True):
             em = UvuEmitter(replace(low, paths=[p for p in low.paths if lanes[p.io] == n], lanes_per_row=n,
-                                    rows_per_wave=64 // n))
+                                    rows_per_wave=64 // n), acc_budget_words=1 << 20)
             em.nt, em.mask_loads, em.forms = self.nt, self.mask_loads, self.forms
-            em.rows_stage = None  # (the forward's)
+            em.rows_stage = None  # (it brings whole rows: of the other groups as well)
             groups.append(em)
-        if len(groups) < 2 or any(em.backward_words(True) > 285 for em in groups):
-            return None
-        return groups
+        return groups if len(groups) > 1 else None
+
+    def _group_operands(self, s: Src, name: str):
+        """For the walk of a group: what requests the operands of its R edges from position ``k`` of the walk on into
+        ``buf``, and the edges' numbers. The lanes hold numbers and senders of the next 64 edges. (Read by lane number:
+        an exchange through LDS would not see what lanes hold that have no edge left.)"""
+        s("oeq_ahead ahead;")
+
+        def of(field: str, k: str) -> str:
+            lanes = [f"__builtin_amdgcn_readlane(ahead.{field}, ({k} + {q}) & 63)" for q in range(self.R)]
+            value = lanes[-1]
+            for q in range(self.R - 2, -1, -1):
+                value = f"(r == {q} ? {lanes[q]} : {value})"
+            return value
+
+        def load(buf: str, k: str):
+            s(f"const i64 eid_{buf} = {of('eid', k)}, sender_{buf} = {of('sender', k)};")
+            s(f"{name}({buf}, eid_{buf}, sender_{buf}, L1_in, L2_in, W, cols, node_count, u);")
+
+        return of, load
+
+    def plan_forward_groups(self) -> Optional[List["UvuEmitter"]]:
+        """Groups of paths for the forward kernel (``emit_conv_forward_groups``): those of ``width_groups``, halved
+        by output blocks where accumulators and two operand sets of an edge do not fit the registers of a third of a
+        SIMD. None where the halves do not either."""
+        groups = []
+        for em in self.width_groups() or []:
+            if em.operand_words(2) <= 150:
+                groups.append(em)
+                continue
+            halves: List[List[Path]] = [[], []]
+            by_out = {io: [p for p in em.low.paths if p.io == io] for io in em.used_out}
+            for io in sorted(by_out, key=lambda io: -sum(len(p.nnz) for p in by_out[io])):
+                min(halves, key=lambda h: sum(len(p.nnz) for p in h)).extend(by_out[io])
+            for half in halves:
+                paths = [p for p in em.low.paths if p in half]
+                part = UvuEmitter(replace(em.low, paths=paths), acc_budget_words=1 << 20)
+                part.nt, part.mask_loads, part.forms, part.rows_stage = em.nt, em.mask_loads, em.forms, None
+                groups.append(part)
+        return groups if groups and len(groups) <= 8 and all(em.operand_words(2) <= 150 for em in groups) else None
+
+    def emit_conv_forward_groups(self, s: Src, ems: List["UvuEmitter"], waves_per_eu: int, xcd: int) -> int:
+        """Forward of rows with blocks of different widths: every wave of a block walks the edges of one node for its
+        own group of paths (``width_groups``), several edges side by side where its blocks are narrow, and stores the
+        blocks of the node's row that its paths go to. The waves do not meet.
+
+        With one edge to a wave half of the lanes were idle in blocks of 32 channels, and the waves that shared the outputs
+        by segments read the rows of X two or three times. Three waves per SIMD; two of them with 250 registers and the
+        narrow blocks of SevenNet's main layer in one wave: 600 x 20 57 us, 8 000 x 30 449. Now bound by W (8 000 x 30:
+        1.7 GB at 4.1 TB/s) and, at fewer nodes, by the latencies of an edge's chain of number, sender and row. Whole forward
+        passes, us, waves by segment / by width: SevenNet's main layer 600 nodes x 20 edges 69 / 55, 2 003 x 40 211 / 173,
+        8 000 x 30 520 / 459, ir_mul 3 000 x 30 223 / 189; NequiX's 600 x 20 53 / 49, 3 000 x 30 163 / 153, 9 000 x 24
+        340 / 333, ir_mul 1 500 x 20 86 / 71."""
+        low, W = self.low, len(ems)
+        block = 64 * W
+        operands = ("i64 node_count, const T* __restrict__ L1_in, const T* __restrict__ L2_in, "
+                    "const T* __restrict__ W, const i64* __restrict__ cols, const i64* __restrict__ eperm, ")
+        for gi, em in enumerate(ems):
+            s(f"namespace oeq_forward_group{gi} {{")
+            em.emit_structs(s)
+            # Y rows of several edges: a value a lane, and from there by way of LDS (rows of 16 values in every lane,
+            # twice, are registers that SevenNet's main layer does not have); of one edge: in scalar registers
+            lds_y = em.R > 1 and low.L2 <= em.LPR
+            em._emit_load_edge(s, "load_edge_f0", em.used_in1, em.low.paths, sender=True, y=not lds_y)
+            em._emit_fwd_seg(s, 0, True)
+            s.open(f"OEQ_DEV void walk({operands}const i64 e0, const i64 e1, T* __restrict__ zrow)")
+            em._lane_prologue(s, own=True)
+            s("A0_t a; zero_seg0(a);")
+            _, load_edge = em._group_operands(s, "load_edge_f0")
+            s("E_t B;")
+            if lds_y:
+                s(f"__shared__ T s_y[{em.R}][{low.L2}];")
+                s("T yn = T(0);")
+
+            def load(buf, k):
+                load_edge(buf, k)
+                if lds_y:
+                    s(f"yn = L2_in[eid_{buf} * {low.L2} + (ul < {low.L2} ? ul : {low.L2 - 1})];")
+
+            s("const int count = (int)(e1 - e0);")
+            s.open("if (count > 0)")
+            s("oeq_look_ahead(ahead, e0 + lane, e1, eperm, cols, node_count);")
+            load("B", "0")
+            s.close()
+            s.open(f"for (int done = 0; done < count; done += {em.R})")
+            s("E_t A = B;")
+            if lds_y:
+                s(f"if (ul < {low.L2}) s_y[r][ul] = yn;")
+                s("oeq_wave_sync();")
+                for j in range(low.L2):
+                    s(f"A.y[{j}] = s_y[r][{j}];")
+            s(f"const int next = done + {em.R};")
+            s.open("if (next < count)")
+            s("if ((next & 63) == 0) oeq_look_ahead(ahead, e0 + next + lane, e1, eperm, cols, node_count);")
+            load("B", "next")
+            s.close()
+            s("if (done + r < count) fwd_seg0_pre(A, a);" if em.R > 1 else "fwd_seg0_pre(A, a);")
+            s.close()
+            em._fold_store(s, 0, "zrow")
+            s.close()
+            s(f"}}  // namespace oeq_forward_group{gi}")
+        s.open(
+            f'extern "C" __global__ {self._attrs(block, waves_per_eu)} void forward(i64 node_count, i64 nnz, '
+            "const T* __restrict__ L1_in, const T* __restrict__ L2_in, const T* __restrict__ W, "
+            "T* __restrict__ L3_out, const i64* __restrict__ rows, const i64* __restrict__ cols, "
+            f"const i64* __restrict__ rowptr, const i64* __restrict__ eperm, const i64* __restrict__ order"
+            f"{self.HUB_PARAMS}{self.HUB_ROWS_PARAM})"
+        )
+        self._lane_prologue(s, W)
+        self._node_loop_open(s, 1, xcd)
+        s(f"T* zrow = hubpos >= 0 ? hub_rows + hubpos * {low.L3} : L3_out + node * {low.L3};")
+        for gi in range(W):
+            s(f"{'else ' if gi else ''}if (sg == {gi}) oeq_forward_group{gi}::walk(node_count, L1_in, L2_in, W, cols, "
+              "eperm, e0, e1, zrow);")
+        self._zero_untouched_out(s, "zrow", "sg == 0")
+        s.close()
+        s.close()
+        return block
 
     def emit_conv_backward_groups(self, s: Src, ems: List["UvuEmitter"], waves_per_eu: int, xcd: int) -> int:
         """Backward of rows with blocks of different widths (``plan_width_groups``): every wave of a block walks the
@@ -2476,7 +2603,6 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
                     "T* __restrict__ L2_grad, const T* __restrict__ W, T* __restrict__ W_grad, "
                     "const T* __restrict__ L3_grad, const i64* __restrict__ cols, T* __restrict__ dx_tmp, "
                     "const i64* __restrict__ eperm, ")
-        s(LOOK_AHEAD)
         for gi, em in enumerate(ems):
             # the next edges' operands in a second set of registers, where they fit
             ahead = (em.backward_words(True) + sum(low.in1[b].d for b in em.used_in1) + em.n_wslots
@@ -2490,21 +2616,7 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
             s("G_t gr;")
             em._load_g(s, f"L3_grad + node * {low.L3}", em.used_out)
             s("int batch = 0;")
-            # The lanes hold the numbers and senders of the next 64 edges. (Read by lane number: an exchange through LDS
-            # would not see what lanes hold that have no edge left.)
-            s("oeq_ahead ahead;")
-
-            def of(field, k):
-                lanes = [f"__builtin_amdgcn_readlane(ahead.{field}, ({k} + {q}) & 63)" for q in range(em.R)]
-                value = lanes[-1]
-                for q in range(em.R - 2, -1, -1):
-                    value = f"(r == {q} ? {lanes[q]} : {value})"
-                return value
-
-            def load(buf, k):
-                s(f"const i64 eid_{buf} = {of('eid', k)}, sender_{buf} = {of('sender', k)};")
-                s(f"load_edge_b({buf}, eid_{buf}, sender_{buf}, L1_in, L2_in, W, cols, node_count, u);")
-
+            of, load = em._group_operands(s, "load_edge_b")
             if ahead:
                 s("E_t B;")
                 s.open("if (e0 < e1)")
@@ -2909,7 +3021,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
                     conv_dxm=-1, conv_q=0, conv_hops=2, conv_qpin=1, conv_qaf=48, conv_qab=24, tp_mask=0, tp_forms=1,
                     conv_hub=256, conv_dxs=-1, conv_omin=32768, conv_fsplit=-1, conv_fsplit_f=-1, conv_fsplit_x=-1, conv_fsplit_a=-1,
                     conv_fsmax=-1, conv_parts=-1, conv_stg=1,
-                    conv_wgrp=1))
+                    conv_wgrp=3))
     assert deterministic or not kahan, "kahan=True requires deterministic=True"
     # knobs somebody set: the rules below leave those alone
     user_tune = os.environ.get("OEQ_AMD_TUNE", "")
@@ -3040,7 +3152,38 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     G_b = 1 if em.NCH > 1 else t["conv_gb"]
     xcd = max(1, t["conv_xcd"])
     xcd_b = 1 if (walk and low.shared_weights) else xcd  # bounded grid: one partial dW row per wave group
-    blk_f = em.emit_conv_forward(s, G_f, walk, t["conv_pipe_f"], t["conv_wf"], xcd, bool(t["conv_tra"]))
+    gres = None if t["conv_gres"] < 0 else bool(t["conv_gres"])
+    sender_walk = (9 * low.L1 >= 2 * (low.WN + low.L2 + low.L3) and not low.shared_weights and t["conv_dxm"] < 0
+                   and t["conv_dxs"] < 0) or t["conv_dxs"] > 0
+    forward_groups = width_groups = None
+    # A wave per width pays where the row of all widths is much for one wave. Backward: two widths, whose waves wait for each
+    # other least, and more than the smallest rows (step, us, one wave / a wave per width, by the estimate of that one
+    # wave's registers, 3 000 nodes x 30 edges: 178 (64x0e+64x1o+8x2e+8x1e) 266 / 274,
+    # 195 (64x0e+64x1o+32x2e+32x3o) 333 / 325, 215 (96x{0e,1o,2e}) 410 / 403, 275 (NequiX's main layer) 512 / 495; above it is two
+    # waves that lose: SevenNet's main layer (2 003 x 40) 711 / 566, 96x{0e..3o} 1 026 / 879, 64x0e+64x1o+16x2e+16x3o
+    # 453 / 400). Three and four widths lose: 64x0e+32x1o+16x2e 224 / 273, 64x0e+64x1o+32x2e+16x3o 468 / 516,
+    # 128x0e+64x1o+32x2e+8x3o 359 / 422. Forward, whose waves do not meet: where the outputs would be walked in several
+    # segments (64x0e+64x1o+32x2e+16x3o 177 / 124, 64x1o+32x2e+32x3o+32x1e 378 / 120, 96x{0e..3o} 275 / 260, and the figures
+    # at emit_conv_forward_groups; one segment: 64x0e+32x1o+16x2e 69 / 86, 96x{0e,1o,2e} 115 / 119), with blocks of eight
+    # channels not (64x0e+64x1o+8x2e+8x1e, 9 000 x 24: 177 / 184). Neither where blocks leave lanes of their own width
+    # without a channel (100x0e+40x1o+20x2e+9x1e: forward 98 / 109, step 304 / 470).
+    # (conv_wgrp: bit 1 backward, 2 forward, 4 regardless of this)
+    forced = bool(t["conv_wgrp"] & 4)
+    apart = em.width_groups() if walk and t["conv_wgrp"] & 3 and (forced or per_lane > 48) else None
+    if apart and (forced or not any(g.ragged() for g in apart)):
+        if (t["conv_wgrp"] & 2 and not kahan and not q_fwd and "conv_wf" not in user_tune
+                and (forced or (len(em.segments) > 1 and all(g.R <= 4 for g in apart)))):
+            forward_groups = em.plan_forward_groups()
+        if (t["conv_wgrp"] & 1 and t["conv_split"] and gres is None and t["conv_dxm"] <= 0 and not sender_walk
+                and (forced or (len(apart) == 2 and em.backward_words(True) > 180))):
+            width_groups = em.plan_width_groups()
+    if forward_groups or width_groups:
+        s(LOOK_AHEAD)
+    if forward_groups:
+        G_f = 1
+        blk_f = em.emit_conv_forward_groups(s, forward_groups, 3, xcd)
+    else:
+        blk_f = em.emit_conv_forward(s, G_f, walk, t["conv_pipe_f"], t["conv_wf"], xcd, bool(t["conv_tra"]))
     splits: Dict[str, Split] = {}  # the kernels with a node's edges dealt out to several waves
     if walk and not kahan and not q_fwd:
         n = split_waves(t, "conv_fsplit_f", em, em.seg_waves, t["conv_wf"])
@@ -3050,29 +3193,11 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
             blk_fs = em.emit_conv_forward(s, 1, True, t["conv_pipe_f"], t["conv_wf"], xcd, bool(t["conv_tra"]),
                                           name="forward_split", split=n)
     em.use_q = q_bwd
-    gres = None if t["conv_gres"] < 0 else bool(t["conv_gres"])
     dx_mode = 0
     em.group_budget = t["conv_gbud"]
     em.fit_words = t["conv_fit"]
     em.group_count = t["conv_ngrp"]
     em.bwd_groups = em.plan_backward_groups(max(1, 8 // em.NCH)) if (walk and t["conv_split"] and gres is None) else None
-    sender_walk = (9 * low.L1 >= 2 * (low.WN + low.L2 + low.L3) and not low.shared_weights and t["conv_dxm"] < 0
-                   and t["conv_dxs"] < 0) or t["conv_dxs"] > 0
-    width_groups = None
-    # A wave per width pays where the row of all widths is much for one wave. Backward: two widths, whose waves wait for each
-    # other least, and more than the smallest rows (step, us, one wave / a wave per width, by the estimate of that one
-    # wave's registers, 3 000 nodes x 30 edges: 178 (64x0e+64x1o+8x2e+8x1e) 266 / 274,
-    # 195 (64x0e+64x1o+32x2e+32x3o) 333 / 325, 215 (96x{0e,1o,2e}) 410 / 403, 275 (NequiX's main layer) 512 / 495; above it is two
-    # waves that lose: SevenNet's main layer (2 003 x 40) 711 / 566, 96x{0e..3o} 1 026 / 879, 64x0e+64x1o+16x2e+16x3o
-    # 453 / 400). Three and four widths lose: 64x0e+32x1o+16x2e 224 / 273, 64x0e+64x1o+32x2e+16x3o 468 / 516,
-    # 128x0e+64x1o+32x2e+8x3o 359 / 422. Not where blocks leave lanes of their own width without a channel
-    # (100x0e+40x1o+20x2e+9x1e: 304 / 470). (conv_wgrp: bit 1 on, 4 regardless of this)
-    forced = bool(t["conv_wgrp"] & 4)
-    if (walk and t["conv_wgrp"] & 1 and t["conv_split"] and gres is None and t["conv_dxm"] <= 0 and not sender_walk
-            and (forced or (per_lane > 48 and em.backward_words(True) > 180))):
-        width_groups = em.plan_width_groups()
-        if width_groups and not forced and (len(width_groups) > 2 or any(g.ragged() for g in width_groups)):
-            width_groups = None
     if width_groups:
         G_b, dx_mode = 1, em.DX_TERMS
         blk_b = em.emit_conv_backward_groups(s, width_groups, t["conv_wb"], xcd)
@@ -3214,7 +3339,9 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     if width_groups and rt.kernel_resources(rt.compile_source(src)).get("backward", (0, 0))[1] > 0:
         # never with scratch memory: slower, and with the next edges' operands spilled (NequiX's main layer held to 168 registers,
         # 240 B) the X values of an edge came back as another's
-        return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wgrp=0), draft)
+        return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wgrp=t["conv_wgrp"] & ~1), draft)
+    if forward_groups and rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))[1] > 0:
+        return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wgrp=t["conv_wgrp"] & ~2), draft)
     if staged64 and len(em.segments) > 1 and rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))[1] > 0:
         return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_stg=0), draft)
     if em.seg_waves > 1 and "conv_segw" not in user_tune:
@@ -3234,7 +3361,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         _lds, scratch = rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))
         if scratch > 64:
             return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wf=2), draft)
-    if walk and t["conv_wf"] == 23 and "conv_wf" not in user_tune and low.elem_size == 4:
+    if walk and t["conv_wf"] == 23 and "conv_wf" not in user_tune and low.elem_size == 4 and not forward_groups:
         # A forward kernel that the compiler gave more than a third of a SIMD's registers runs two waves there.
         # Held to a third it runs three, which pays where the compiler manages that without scratch memory (fp32,
         # config-5 graph, forward: 96 channels of l <= 3 with l <= 3 harmonics 176 -> 168 registers, -18 %; 64
@@ -3259,7 +3386,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
             res = rt.kernel_resources(rt.compile_source(half[0]))
             if all(res.get(name, (0, 0))[1] == 0 for name, sp in splits.items() if sp.knob in fewer):
                 return half
-        descs = _small_graph_rules(src, descs, splits, compute_units, t, low.shared_weights, em.R)
+        descs = _small_graph_rules(src, descs, splits, compute_units, t, low.shared_weights, em.R, bool(forward_groups))
     return src, dims, descs
 
 
@@ -3292,7 +3419,7 @@ def split_waves(t: dict, knob: str, em: UvuEmitter, seg_waves: int, waves_per_eu
 
 
 def _small_graph_rules(src: str, descs: List[tuple], splits: Dict[str, Split], compute_units: int, t: dict,
-                       shared: bool, rows: int) -> List[tuple]:
+                       shared: bool, rows: int, groups: bool = False) -> List[tuple]:
     """Launch descriptors with what the host needs to know to run small graphs (csrc/oeq_amd.cpp: split_role,
     backward_parts): how many walk positions of a backward-shaped kernel the device holds at once, and up to how many
     nodes the split form of a forward-shaped kernel is the faster one. Both follow from the registers and the LDS the
@@ -3308,7 +3435,10 @@ def _small_graph_rules(src: str, descs: List[tuple], splits: Dict[str, Split], c
     (SevenNet's first layer, fp64, 88 and 176 registers: 400 nodes 0.96, 640 nodes 1.06, 800 nodes 1.28). Six waves to a
     CU where the waves of a node own different output segments (three: SevenNet's main layers, fp32, 400 nodes 1.00, 640
     nodes 1.10, 1 280 nodes 1.44; two: NequiX's main layers as above), two and a half nodes to a CU where a wave walks
-    four edges side by side or more (16 channels: 640 nodes 0.97, 1 280 nodes 1.23).
+    four edges side by side or more (16 channels: 640 nodes 0.97, 1 280 nodes 1.23). Where the plain forward has a wave
+    per width (``groups``), a node to a CU per two waves that the edges are dealt out to (split / plain, us: SevenNet's
+    main layer, two waves, 96 nodes x 12 17 / 19, 256 x 30 36 / 36, 320 x 30 54 / 39; NequiX's, four, 500 x 20 30 / 32,
+    630 x 12 29 / 25).
 
     Backward-shaped kernels whose waves walk 64 edges side by side get no parts: a part of ten edges leaves most lanes
     idle (a single path of one channel, second order, 2 560 nodes x 30 edges: 7.7 us whole, 11.4 in parts)."""
@@ -3331,6 +3461,8 @@ def _small_graph_rules(src: str, descs: List[tuple], splits: Dict[str, Split], c
         limit = min(2.5 * nodes / sp.waves, (2 if 2 * own * sp.waves < nodes else 3) * own)
         if sp.seg_waves > 1:
             limit = min(limit, 6 * compute_units / sp.seg_waves)
+        if groups and name == "forward_split":
+            limit = min(limit, compute_units * sp.waves / 2)
         if sp.rows >= 4:
             limit = min(limit, 2.5 * compute_units)
         return int(limit)

@@ -2,7 +2,7 @@
 rows of less than an instruction's 1 024 bytes, of whole instructions and with a rest, blocks without a channel for every
 lane, several channels in the second operand; segments without an edge, with odd and even numbers, on either side of the
 64 edges whose numbers a wave holds, and cut into chunks. Double precision, a node's outputs shared out between waves that
-stage what theirs need: one, two and four of them, paths in and out of the order of their outputs. Backward, blocks of different
+stage what theirs need: one, two and four of them, paths in and out of the order of their outputs. Blocks of different
 widths: a wave per width, one to eight edges side by side."""
 
 import numpy as np
@@ -31,8 +31,9 @@ PROBLEMS = {
 # channels, largest l of the first operand and of the harmonics, paths and their order
 SHARED = {"one": (128, 1, 2, range(9)), "two": (128, 2, 2, range(18)), "two-shuffled": (128, 2, 2, [k * 7 % 18 for k in range(18)]),
           "four-shuffled": (64, 3, 3, [k * 5 % 34 for k in range(34)])}
-# blocks of different widths: a wave per width in the backward kernel
+# blocks of different widths: a wave per width
 WIDTHS = {"two": ("64x0e+64x1o+32x2e+32x3o", "0e+1o+2e+3o", "0e+1o+2e"), "three": ("64x0e+32x1o+16x2e", "0e+1o+2e", "0e+1o+2e+3o"),
+          "halved": ("64x1o+32x2e+32x3o+32x1e", "0e+1o+2e+3o", "0e+1o+2e+3o"),
           "eighth": ("64x0e+64x1o+8x2e+8x1e", "0e+1o+2e", "0e+1o+2e+1e"), "ragged-widths": ("100x0e+40x1o+20x2e+9x1e", "0e+1o+2e", "0e+1o+2e+1e")}
 DEGREES = [0, 1, 2, 3, 7, 8, 9, 16, 17, 31, 63, 64, 65, 0, 128, 129, 300, 5, 0]
 
@@ -67,15 +68,20 @@ def test_waves_that_share_the_outputs(name, waves):
     assert len(em.segments) == len(em.stages) == waves
 
 
-@pytest.mark.parametrize("name,rows", [("two", [1, 2]), ("three", [1, 2, 4]), ("eighth", [1, 8]), ("ragged-widths", [1, 2, 4])])
+@pytest.mark.parametrize("name,rows", [("two", [1, 2]), ("three", [1, 2, 4]), ("halved", [1, 2]), ("eighth", [1, 8]),
+                                       ("ragged-widths", [1, 2, 4])])
 def test_a_wave_for_every_width(name, rows):
-    assert [em.R for em in UvuEmitter(lower(_problem(name, np.float32, "mul_ir"))).plan_width_groups()] == rows
+    em = UvuEmitter(lower(_problem(name, np.float32, "mul_ir")))
+    assert [g.R for g in em.plan_width_groups()] == rows
+    # (forward: a third of the registers, so that a group with many outputs is halved)
+    assert [g.R for g in em.plan_forward_groups()] == ([1, 2, 2] if name == "halved" else rows)
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", list(WIDTHS))
 @pytest.mark.parametrize("layout,det,tune", [("mul_ir", True, "conv_parts=1"), ("ir_mul", False, "conv_parts=3"),
-                                             ("mul_ir", False, "conv_hub=40")])
+                                             ("mul_ir", False, "conv_hub=40"), ("mul_ir", True, "conv_fsmax=0"),
+                                             ("ir_mul", False, "conv_fsmax=0,conv_hub=40")])
 def test_widths_against_the_oracle(name, layout, det, tune, monkeypatch):
     _check(_problem(name, np.float32, layout), _problem(name, np.float32, "mul_ir"), det, "conv_wgrp=7," + tune, monkeypatch)
 
