@@ -2479,15 +2479,13 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
     def _group_operands(self, s: Src, name: str):
         """For the walk of a group: what requests the operands of its R edges from position ``k`` of the walk on into
         ``buf``, and the edges' numbers. The lanes hold numbers and senders of the next 64 edges. (Read by lane number:
-        an exchange through LDS would not see what lanes hold that have no edge left.)"""
+        an exchange through LDS would not see what lanes hold that have no edge left.) Such reads never stand in a
+        branch of some lanes only, see ``oeq_held``: they did, and a kernel with ``ahead`` in scratch memory (NequiX's main
+        layer held to 168 registers, backward) took other edges' senders."""
         s("oeq_ahead ahead;")
 
         def of(field: str, k: str) -> str:
-            lanes = [f"__builtin_amdgcn_readlane(ahead.{field}, ({k} + {q}) & 63)" for q in range(self.R)]
-            value = lanes[-1]
-            for q in range(self.R - 2, -1, -1):
-                value = f"(r == {q} ? {lanes[q]} : {value})"
-            return value
+            return f"oeq_held<{self.R}>(ahead.{field}, {k}, r)"
 
         def load(buf: str, k: str):
             s(f"const i64 eid_{buf} = {of('eid', k)}, sender_{buf} = {of('sender', k)};")
@@ -3167,7 +3165,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     # at emit_conv_forward_groups; one segment: 64x0e+32x1o+16x2e 69 / 86, 96x{0e,1o,2e} 115 / 119), with blocks of eight
     # channels not (64x0e+64x1o+8x2e+8x1e, 9 000 x 24: 177 / 184). Neither where blocks leave lanes of their own width
     # without a channel (100x0e+40x1o+20x2e+9x1e: forward 98 / 109, step 304 / 470).
-    # (conv_wgrp: bit 1 backward, 2 forward, 4 regardless of this)
+    # (conv_wgrp: bit 1 backward, 2 forward, 4 regardless of this and of scratch memory)
     forced = bool(t["conv_wgrp"] & 4)
     apart = em.width_groups() if walk and t["conv_wgrp"] & 3 and (forced or per_lane > 48) else None
     if apart and (forced or not any(g.ragged() for g in apart)):
@@ -3336,11 +3334,10 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         _lds, scratch = rt.kernel_resources(rt.compile_source(src)).get("backward_dx", (0, 0))
         if scratch > 64:
             return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_dxs=0), draft)
-    if width_groups and rt.kernel_resources(rt.compile_source(src)).get("backward", (0, 0))[1] > 0:
-        # never with scratch memory: slower, and with the next edges' operands spilled (NequiX's main layer held to 168 registers,
-        # 240 B) the X values of an edge came back as another's
+    # A wave per width not with scratch memory, which is slower, unless asked for regardless.
+    if width_groups and not forced and rt.kernel_resources(rt.compile_source(src)).get("backward", (0, 0))[1] > 0:
         return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wgrp=t["conv_wgrp"] & ~1), draft)
-    if forward_groups and rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))[1] > 0:
+    if forward_groups and not forced and rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))[1] > 0:
         return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wgrp=t["conv_wgrp"] & ~2), draft)
     if staged64 and len(em.segments) > 1 and rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))[1] > 0:
         return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_stg=0), draft)

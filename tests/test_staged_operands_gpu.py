@@ -5,12 +5,15 @@ lane, several channels in the second operand; segments without an edge, with odd
 stage what theirs need: one, two and four of them, paths in and out of the order of their outputs. Blocks of different
 widths: a wave per width, one to eight edges side by side."""
 
+import re
+
 import numpy as np
 import pytest
 
 import openequivariance_amd as oeq
+from openequivariance_amd import runtime as rt
 from openequivariance_amd.codegen.lower import lower
-from openequivariance_amd.codegen.uvu import UvuEmitter, _staged_segments
+from openequivariance_amd.codegen.uvu import UvuEmitter, _staged_segments, conv_module
 from openequivariance_amd.core import problems as P
 from openequivariance_amd.core.graph import CoordGraph
 from openequivariance_amd.core.layout import transpose_irrep_layout
@@ -39,7 +42,7 @@ DEGREES = [0, 1, 2, 3, 7, 8, 9, 16, 17, 31, 63, 64, 65, 0, 128, 129, 300, 5, 0]
 
 
 def _problem(name, dtype, layout):
-    p = P.nequip_problems()[0] if name == "lips" else P.ChannelwiseTPP(*{**PROBLEMS, **WIDTHS}[name])
+    p = P.nequip_problems()[0] if name == "lips" else P.nequix_problems()[1] if name == "nequix" else P.ChannelwiseTPP(*{**PROBLEMS, **WIDTHS}[name])
     p.irrep_dtype = p.weight_dtype = dtype
     p.layout = layout
     return p
@@ -75,6 +78,37 @@ def test_a_wave_for_every_width(name, rows):
     assert [g.R for g in em.plan_width_groups()] == rows
     # (forward: a third of the registers, so that a group with many outputs is halved)
     assert [g.R for g in em.plan_forward_groups()] == ([1, 2, 2] if name == "halved" else rows)
+
+
+def _module(name, layout, det, tune, monkeypatch):
+    monkeypatch.setenv("OEQ_AMD_TUNE", tune)
+    src = conv_module(lower(_problem(name, np.float32, layout)), det)[0]
+    return src, rt.kernel_resources(rt.compile_source(src))
+
+
+@pytest.mark.parametrize("name", list(WIDTHS))
+@pytest.mark.parametrize("layout,det", [("mul_ir", True), ("ir_mul", False)])
+def test_the_module_has_a_wave_for_every_width(name, layout, det, monkeypatch):
+    """The kernels that the oracle tests below are about: not others that the generator went back to."""
+    src, resources = _module(name, layout, det, "conv_wgrp=7", monkeypatch)
+    assert "namespace oeq_group0" in src and "namespace oeq_forward_group0" in src
+    assert (resources["backward"][1] > 0) == (name == "halved")
+
+
+@pytest.mark.parametrize("layout,det", [("mul_ir", True), ("ir_mul", False)])
+def test_lanes_are_read_outside_of_branches(layout, det, monkeypatch):
+    """A lane's value (numbers and senders of the edges ahead) is read by the whole wave, before lanes choose: a spilled
+    register is reloaded for the lanes of a branch only. NequiX's main layer held to 168 registers has spilled ones."""
+    src, resources = _module("nequix", layout, det, "conv_wgrp=7,conv_wb=3", monkeypatch)
+    assert "namespace oeq_group1" in src and resources["backward"][1] > 0
+    assert not re.search(r"\?[^;\n]*__builtin_amdgcn_readlane", src)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout,det", [("mul_ir", True), ("ir_mul", False)])
+def test_spilled_operands_against_the_oracle(layout, det, monkeypatch):
+    _check(_problem("nequix", np.float32, layout), _problem("nequix", np.float32, "mul_ir"), det, "conv_wgrp=7,conv_wb=3",
+           monkeypatch)
 
 
 @pytest.mark.gpu
