@@ -3334,10 +3334,15 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         _lds, scratch = rt.kernel_resources(rt.compile_source(src)).get("backward_dx", (0, 0))
         if scratch > 64:
             return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_dxs=0), draft)
-    # A wave per width not with scratch memory, which is slower, unless asked for regardless.
+    # A wave per width: not a backward with scratch memory unless asked for regardless (NequiX's main layer held to 168
+    # registers, 236 B: step of 3 000 nodes x 30 edges 753 us against 448; the wide blocks and the narrow ones of SevenNet's
+    # main layer in three waves, 48 B: 594 / 564). The forward may have a few bytes: of those seen, written
+    # once and read once per node (us, by segment / by width: SevenNet's main layer, ir_mul, 8 B, 600 nodes x 20 edges 68 / 53, 2 003 x 40 196 / 166,
+    # 8 000 x 30 498 / 418; with 12 B 96x{0e..3o} 272 / 253 at 3 000 x 30, 64x0e+64x1o+32x2e+32x3o 176 / 122,
+    # 64x0e+64x1o+16x2e+16x3o 172 / 116); more than 12 was not seen.
     if width_groups and not forced and rt.kernel_resources(rt.compile_source(src)).get("backward", (0, 0))[1] > 0:
         return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wgrp=t["conv_wgrp"] & ~1), draft)
-    if forward_groups and not forced and rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))[1] > 0:
+    if forward_groups and not forced and rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))[1] > 16:
         return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wgrp=t["conv_wgrp"] & ~2), draft)
     if staged64 and len(em.segments) > 1 and rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))[1] > 0:
         return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_stg=0), draft)

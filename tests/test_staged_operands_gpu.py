@@ -37,6 +37,7 @@ SHARED = {"one": (128, 1, 2, range(9)), "two": (128, 2, 2, range(18)), "two-shuf
 # blocks of different widths: a wave per width
 WIDTHS = {"two": ("64x0e+64x1o+32x2e+32x3o", "0e+1o+2e+3o", "0e+1o+2e"), "three": ("64x0e+32x1o+16x2e", "0e+1o+2e", "0e+1o+2e+3o"),
           "halved": ("64x1o+32x2e+32x3o+32x1e", "0e+1o+2e+3o", "0e+1o+2e+3o"),
+          "few-spilled": ("64x0e+64x1o+32x2e+32x3o", "0e+1o+2e+3o", "0e+1o+2e+3o"),
           "eighth": ("64x0e+64x1o+8x2e+8x1e", "0e+1o+2e", "0e+1o+2e+1e"), "ragged-widths": ("100x0e+40x1o+20x2e+9x1e", "0e+1o+2e", "0e+1o+2e+1e")}
 DEGREES = [0, 1, 2, 3, 7, 8, 9, 16, 17, 31, 63, 64, 65, 0, 128, 129, 300, 5, 0]
 
@@ -93,6 +94,12 @@ def test_the_module_has_a_wave_for_every_width(name, layout, det, monkeypatch):
     src, resources = _module(name, layout, det, "conv_wgrp=7", monkeypatch)
     assert "namespace oeq_group0" in src and "namespace oeq_forward_group0" in src
     assert (resources["backward"][1] > 0) == (name == "halved")
+
+
+@pytest.mark.parametrize("tune", ["", "conv_wgrp=7"])
+def test_a_forward_by_width_may_spill_a_few_bytes(tune, monkeypatch):
+    src, resources = _module("few-spilled", "mul_ir", True, tune, monkeypatch)
+    assert "namespace oeq_forward_group0" in src and 0 < resources["forward"][1] <= 16
 
 
 @pytest.mark.parametrize("layout,det", [("mul_ir", True), ("ir_mul", False)])
