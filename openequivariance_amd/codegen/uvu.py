@@ -178,7 +178,21 @@ class UvuEmitter:
             nqw = (nuw + 63) // 64
             stages.append(dict(U=U, xl=xl, nux=units, nqx=nqx, nuw=nuw, nqw=nqw, XF=nqx * 64 * n,
                                floats=(nqx + nqw) * 64 * n, in1=in1, paths=paths))
-        return stages
+        # (the waves of a node, one or more per segment, have to fit a block)
+        waves = self.NCH * min(len(stages), max(1, 8 // self.NCH))
+        return stages if waves * self._wave_lds(max(st["floats"] for st in stages)) <= LDS_LIMIT else None
+
+    def _wave_lds(self, floats: int) -> int:
+        """Bytes of LDS of a wave that stages ``floats`` elements, with the buffer that fp64 rows are stored through."""
+        widest = max(self.low.out[io].d for io in self.used_out) if self.words == 2 and self.R == 1 else 0
+        return (floats + 64 * widest) * self.low.elem_size
+
+    def groups_that_fit(self, G: int) -> int:
+        """How many nodes a block of a forward kernel that stages an edge's operands can take, ``G`` or fewer."""
+        staged = self.stages or self.rows_stage
+        while G > 1 and staged and G * self.NCH * self.seg_waves * self._wave_lds(self._stage_floats()) > LDS_LIMIT:
+            G //= 2
+        return G
 
     def _stage_src(self, blk, first_unit: int) -> str:
         """Row offset of the 16-byte unit ``t`` of the wave's slice of a block (units in LDS order)."""
@@ -293,6 +307,8 @@ class UvuEmitter:
         nqx, nqw = -(-low.L1 * es // 1024), -(-low.WN * es // 1024)
         y = -(-low.L2 // 4) * 4
         XF, row = nqx * 1024 // es, (nqx + nqw) * 1024 // es
+        if self.R * (row + y) * es > LDS_LIMIT:
+            return None
         return dict(nqx=nqx, nqw=nqw, XF=XF, row=row, y=y, floats=self.R * (row + y))
 
     def _emit_rows_issue(self, s: Src, e: str, last: str, step: int):
@@ -3146,7 +3162,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         # fp32: -8 % .. +0.3 %, mean -1.7 %; NequiX main layer 6.13 -> 5.77 ms; small kernels: up to +1.4 %; 18
         # problems in fp64: -8 % .. +1 %)
         t["conv_gb"] = 1
-    G_f = t["conv_gf"]
+    G_f = em.groups_that_fit(t["conv_gf"])
     G_b = 1 if em.NCH > 1 else t["conv_gb"]
     xcd = max(1, t["conv_xcd"])
     xcd_b = 1 if (walk and low.shared_weights) else xcd  # bounded grid: one partial dW row per wave group
@@ -3277,7 +3293,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
             ex.emit_structs(s)
             ex.use_q = False
             ex.emit_forward_cores(s, preloaded=True)
-            G_x = 1 if ex.rows_stage is not None else max(1, 4 // low_x.n_chunks)
+            G_x = 1 if ex.rows_stage is not None else ex.groups_that_fit(max(1, 4 // low_x.n_chunks))
             # (rows staged in LDS: one operand set in registers, so that a fourth wave per SIMD costs nothing)
             small = -4 if ex.rows_stage is not None else -2
             waves_x = t["conv_wx"] if t["conv_wx"] else (small if words_x <= 48 else 2)

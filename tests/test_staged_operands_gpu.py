@@ -34,6 +34,10 @@ PROBLEMS = {
 # channels, largest l of the first operand and of the harmonics, paths and their order
 SHARED = {"one": (128, 1, 2, range(9)), "two": (128, 2, 2, range(18)), "two-shuffled": (128, 2, 2, [k * 7 % 18 for k in range(18)]),
           "four-shuffled": (64, 3, 3, [k * 5 % 34 for k in range(34)])}
+# double precision, more than the LDS of a block holds: staged for sixteen waves (with the buffer the rows are stored
+# through), two segments of two chunks, more nodes to a block of the sender walk
+WIDE = {"sixteen-waves": ("1024x0e+1024x1o+1024x2e+1024x3o", "0e", "0e+1o+2e+3o"),
+        "two-segments": ("128x0e+128x1o+128x2e+128x3o", "0e+1o+2e+3o", "0e+0o+1o+1e+2e+2o+3o+3e+4e+4o")}
 # blocks of different widths: a wave per width
 WIDTHS = {"two": ("64x0e+64x1o+32x2e+32x3o", "0e+1o+2e+3o", "0e+1o+2e"), "three": ("64x0e+32x1o+16x2e", "0e+1o+2e", "0e+1o+2e+3o"),
           "halved": ("64x1o+32x2e+32x3o+32x1e", "0e+1o+2e+3o", "0e+1o+2e+3o"),
@@ -43,7 +47,7 @@ DEGREES = [0, 1, 2, 3, 7, 8, 9, 16, 17, 31, 63, 64, 65, 0, 128, 129, 300, 5, 0]
 
 
 def _problem(name, dtype, layout):
-    p = P.nequip_problems()[0] if name == "lips" else P.nequix_problems()[1] if name == "nequix" else P.ChannelwiseTPP(*{**PROBLEMS, **WIDTHS}[name])
+    p = P.nequip_problems()[0] if name == "lips" else P.nequix_problems()[1] if name == "nequix" else P.ChannelwiseTPP(*{**PROBLEMS, **WIDTHS, **WIDE}[name])
     p.irrep_dtype = p.weight_dtype = dtype
     p.layout = layout
     return p
@@ -70,6 +74,20 @@ def test_these_problems_stage_their_rows(name):
 def test_waves_that_share_the_outputs(name, waves):
     em = _staged_segments(lower(_shared(name, "mul_ir")), 8)
     assert len(em.segments) == len(em.stages) == waves
+
+
+@pytest.mark.parametrize("name", list(WIDE))
+def test_staging_leaves_a_block_its_lds(name, monkeypatch):
+    monkeypatch.delenv("OEQ_AMD_TUNE", raising=False)
+    src = conv_module(lower(_problem(name, np.float64, "mul_ir")), True)[0]
+    assert rt.kernel_resources(rt.compile_source(src))["forward"][0] <= 160 * 1024
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(WIDE))
+@pytest.mark.parametrize("layout,det", [("mul_ir", True), ("ir_mul", False)])
+def test_rows_too_wide_for_staging_against_the_oracle(name, layout, det, monkeypatch):
+    _check(_problem(name, np.float64, layout), _problem(name, np.float64, "mul_ir"), det, "conv_fsmax=0", monkeypatch)
 
 
 @pytest.mark.parametrize("name,rows", [("two", [1, 2]), ("three", [1, 2, 4]), ("halved", [1, 2]), ("eighth", [1, 8]),
