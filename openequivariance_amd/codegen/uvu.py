@@ -1981,16 +1981,19 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         s.close()
 
     def _dy_batch(self) -> int:
-        """Edges whose dY the waves of a node with several chunks collect in LDS before they add them up."""
+        """Edges whose dY the waves of a node with several chunks collect in LDS before they add them up; 0: the waves
+        meet twice an edge, over one set of rows (second operands of hundreds of components: two sets of 16 waves'
+        288 doubles are 128 KB)."""
         n = 8
         while n > 1 and 2 * n * self.NCH * self.l2_pad * self.low.elem_size > 8192:
             n //= 2
-        return n
+        return n if 2 * n * self.NCH * self.l2_pad * self.low.elem_size <= 16384 else 0
 
     def _dy_declare(self, s: Src):
         if self.NCH > 1:
-            s(f"__shared__ T s_dy[{2 * self._dy_batch()}][{self.NCH}][{self.l2_pad}];")
-            s("int dyc = 0;  // edges collected, from a batch boundary on at every node")
+            s(f"__shared__ T s_dy[{max(1, 2 * self._dy_batch())}][{self.NCH}][{self.l2_pad}];")
+            if self._dy_batch():
+                s("int dyc = 0;  // edges collected, from a batch boundary on at every node")
 
     def _dy_edge(self, s: Src, pos: str, last: str, eid: str):
         """dY of the edge at position ``pos`` of a walk (number ``eid``) that ends before ``last``. With several chunks
@@ -2003,7 +2006,7 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         470, SevenNet's main layer 2 003 x 40 516 / 496; second order, kernel B, mace-large 708 / 685 / 670, mace-medium
         6 000 x 32 609 / 560, toluene 3 000 x 30 580 / 560."""
         low, n = self.low, self._dy_batch()
-        if self.NCH == 1:
+        if self.NCH == 1 or not n:
             self._dy_finish(s, f"L2_grad + {eid} * {low.L2}", "true")
             return
         assert self.R == 1

@@ -90,6 +90,26 @@ def test_rows_too_wide_for_staging_against_the_oracle(name, layout, det, monkeyp
     _check(_problem(name, np.float64, layout), _problem(name, np.float64, "mul_ir"), det, "conv_fsmax=0", monkeypatch)
 
 
+def _long_harmonics(in2):
+    """Sixteen waves to a node, and more components of the second operand than these have room to collect."""
+    return oeq.TPProblem("1024x0e", in2, "1024x0e", [(0, 0, 0, "uvu", True)], shared_weights=False, internal_weights=False,
+                         label="long-harmonics", irrep_dtype=np.float64, weight_dtype=np.float64)
+
+
+@pytest.mark.parametrize("in2", ["1x0e+10x4e", "1x0e+80x3o"])
+def test_gradients_of_long_harmonics_leave_a_block_its_lds(in2, monkeypatch):
+    monkeypatch.delenv("OEQ_AMD_TUNE", raising=False)
+    resources = rt.kernel_resources(rt.compile_source(conv_module(lower(_long_harmonics(in2)), True)[0]))
+    assert max(lds for lds, _ in resources.values()) <= 160 * 1024
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("det", [True, False])
+def test_gradients_of_long_harmonics_against_the_oracle(det, monkeypatch):
+    problem = _long_harmonics("1x0e+10x4e")
+    _check(problem, problem, det, "conv_fsmax=0", monkeypatch)
+
+
 @pytest.mark.parametrize("name,rows", [("two", [1, 2]), ("three", [1, 2, 4]), ("halved", [1, 2]), ("eighth", [1, 8]),
                                        ("ragged-widths", [1, 2, 4])])
 def test_a_wave_for_every_width(name, rows):
