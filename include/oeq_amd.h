@@ -181,6 +181,9 @@ int oeq_kernels_create(const void* code, size_t code_size,
                        oeq_kernels** out);
 void oeq_kernels_destroy(oeq_kernels* k);
 
+/* The calls below take the operands and results of floating point (L1_in, L2_in, W, L3_grad, gradients, cotangents) at
+ * addresses that are multiples of 16 bytes, and so are workspace, scratch and index: kernels move 16 bytes at a time. */
+
 /* ---- batched tensor product ------------------------------------------- */
 /* Replaces JITTPImpl::exec_tensor_product (extension/tensorproducts.hpp:75-85)
  * as called by jit_tp_forward (extension/torch_core.hpp:274-310).

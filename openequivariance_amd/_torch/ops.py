@@ -107,6 +107,7 @@ class KernelEntry:
         # Float-atomics convolution kernels (conv_sort=0) have no second-order pair of their own: id of the
         # grouped-walk kernel set of the same problem, whose fused pair takes the edges in any order as well.
         self.second_order_kid: Optional[int] = None
+        self.direct_loads = False  # the kernels read operands 16 bytes at a time into LDS (known once they are there)
         self._ks: Optional[rt.KernelSet] = None
         self._lock = threading.Lock()
 
@@ -115,6 +116,7 @@ class KernelEntry:
             with self._lock:
                 if self._ks is None:
                     src, dims, descs = self.build_fn()
+                    self.direct_loads = "global_load_lds" in src
                     self._ks = rt.get_kernel_set(src, dims, descs)
         return self._ks
 
@@ -243,7 +245,7 @@ def _resolve(kid: int, spec: Optional[torch.Tensor]):
     order = tuple(dims.get(k, 0) for k in ("order_hops", "order_min_nodes", "hub_limit"))
     _native.register_entry(kid, dict(
         index_dims=order, fused_second_order=plain and not e.second_order_kid and e.kernels().has_double_backward(),
-        handle=e.kernels().handle.value if plain else 0, L1=e.L1, L2=e.L2, L3=e.L3, WN=e.WN, shared=bool(e.shared),
+        handle=e.kernels().handle.value if plain else 0, direct_loads=plain and e.direct_loads, L1=e.L1, L2=e.L2, L3=e.L3, WN=e.WN, shared=bool(e.shared),
         deterministic=bool(e.deterministic), double=e.dtype == torch.float64, mode=dims.get("deterministic", 0),
         dx_mode=dims.get("dx_mode", 0), native=plain, alert_forward=atomic,
         alert_backward=atomic or (conv and not e.deterministic and walk.get("dx_mode", 0) == rt.DX_ATOMIC),

@@ -53,6 +53,7 @@ struct Entry {
     std::array<int64_t, 3> index_dims{};  // what an index depends on besides the mode: order_hops, order_min_nodes, hub_limit
     bool native = true;         // false: a convolution without fused kernels, see Callbacks::conv_*
     bool alert_forward = false, alert_backward = false;  // uses float atomics
+    bool direct_loads = false;  // has kernels that bring operands into LDS 16 bytes at a time, see operand()
     bool fused_second_order = false;  // has the second-order kernels (of its own: not second_order_kid's)
     int64_t second_order_kid = 0;
     py::object owner;  // keeps the kernel set alive
@@ -139,6 +140,14 @@ Tensor scratch(const Tensor& like, size_t bytes) {
     return at::empty({(int64_t)(bytes ? bytes : 1)}, like.options().dtype(at::kByte));
 }
 
+// An operand as the kernels read it: its rows one after the other and, where they are brought into LDS 16 bytes at a time,
+// from a multiple of 16 on. A view into a larger tensor can begin anywhere (plain loads of any width want no more than
+// the alignment of an element).
+Tensor operand(const Entry& e, const Tensor& t) {
+    const Tensor c = t.contiguous();
+    return e.direct_loads && ((uintptr_t)c.data_ptr() & 15) ? c.clone() : c;
+}
+
 // ---------------------------------------------------------------------------
 // batch tensor product
 // ---------------------------------------------------------------------------
@@ -150,7 +159,7 @@ Tensor tp_forward_gpu(const Tensor& L1_in, const Tensor& L2_in, const Tensor& W,
     check_tensor(L1_in, {n, e.L1}, e.dtype, "L1_in");
     check_tensor(L2_in, {n, e.L2}, e.dtype, "L2_in");
     check_weights(e, W, n, "W");
-    const Tensor x = L1_in.contiguous(), y = L2_in.contiguous(), w = W.contiguous();
+    const Tensor x = operand(e, L1_in), y = operand(e, L2_in), w = operand(e, W);
     OnDevice dev(x);
     Tensor out = at::empty({n, e.L3}, x.options());
     check(oeq_tp_forward(e.k, n, x.data_ptr(), y.data_ptr(), w.data_ptr(), out.data_ptr(), dev.stream), "oeq_tp_forward");
@@ -166,7 +175,7 @@ Tensor3 tp_backward_gpu(const Tensor& L1_in, const Tensor& L2_in, const Tensor& 
     check_tensor(L2_in, {n, e.L2}, e.dtype, "L2_in");
     check_weights(e, W, n, "W");
     check_tensor(L3_grad, {n, e.L3}, e.dtype, "L3_grad");
-    const Tensor x = L1_in.contiguous(), y = L2_in.contiguous(), w = W.contiguous(), g = L3_grad.contiguous();
+    const Tensor x = operand(e, L1_in), y = operand(e, L2_in), w = operand(e, W), g = operand(e, L3_grad);
     OnDevice dev(x);
     Tensor dx = at::empty_like(x), dy = at::empty_like(y), dw = at::empty_like(w);
     const size_t nb = oeq_tp_backward_workspace_bytes(e.k, n);
@@ -191,8 +200,8 @@ Tensor4 tp_double_backward_gpu(const Tensor& L1_in, const Tensor& L2_in, const T
     check_weights(e, W, n, "W");
     check_weights(e, W_dgrad, n, "W_dgrad");
     check_tensor(L3_grad, {n, e.L3}, e.dtype, "L3_grad");
-    const Tensor x = L1_in.contiguous(), y = L2_in.contiguous(), w = W.contiguous(), g = L3_grad.contiguous();
-    const Tensor a = L1_dgrad.contiguous(), b = L2_dgrad.contiguous(), c = W_dgrad.contiguous();
+    const Tensor x = operand(e, L1_in), y = operand(e, L2_in), w = operand(e, W), g = operand(e, L3_grad);
+    const Tensor a = operand(e, L1_dgrad), b = operand(e, L2_dgrad), c = operand(e, W_dgrad);
     OnDevice dev(x);
     Tensor dx = at::empty_like(x), dy = at::empty_like(y), dw = at::empty_like(w), gg = at::empty_like(g);
     const size_t nb = oeq_tp_double_backward_workspace_bytes(e.k, n);
@@ -359,7 +368,7 @@ Tensor conv_forward_gpu(const Tensor& L1_in, const Tensor& L2_in, const Tensor& 
     const EntryRef ref = entry_of(kid, spec);
     const Entry& e = *ref;
     const GraphSize n = conv_checks(e, L1_in, L2_in, W, rows, cols, transpose_perm, nullptr);
-    const Tensor x = L1_in.contiguous(), y = L2_in.contiguous(), w = W.contiguous();
+    const Tensor x = operand(e, L1_in), y = operand(e, L2_in), w = operand(e, W);
     const Tensor r = rows.contiguous(), c = cols.contiguous();
     if (!e.native) {
         py::gil_scoped_acquire gil;
@@ -395,7 +404,7 @@ Tensor3 conv_backward_gpu(const Tensor& L1_in, const Tensor& L2_in, const Tensor
     const EntryRef ref = entry_of(kid, spec);
     const Entry& e = *ref;
     const GraphSize n = conv_checks(e, L1_in, L2_in, W, rows, cols, transpose_perm, &L3_grad);
-    const Tensor x = L1_in.contiguous(), y = L2_in.contiguous(), w = W.contiguous(), g = L3_grad.contiguous();
+    const Tensor x = operand(e, L1_in), y = operand(e, L2_in), w = operand(e, W), g = operand(e, L3_grad);
     const Tensor r = rows.contiguous(), c = cols.contiguous(), p = transpose_perm.contiguous();
     if (!e.native) {
         py::gil_scoped_acquire gil;
@@ -439,8 +448,8 @@ Tensor4 conv_double_backward_gpu(const Tensor& L1_in, const Tensor& L2_in, const
     check_tensor(L1_dgrad, {n.nodes, e.L1}, e.dtype, "L1_in");
     check_tensor(L2_dgrad, {n.edges, e.L2}, e.dtype, "L2_in");
     check_weights(e, W_dgrad, n.edges, "W");
-    const Tensor x = L1_in.contiguous(), y = L2_in.contiguous(), w = W.contiguous(), g = L3_grad.contiguous();
-    const Tensor a = L1_dgrad.contiguous(), b = L2_dgrad.contiguous(), c = W_dgrad.contiguous();
+    const Tensor x = operand(e, L1_in), y = operand(e, L2_in), w = operand(e, W), g = operand(e, L3_grad);
+    const Tensor a = operand(e, L1_dgrad), b = operand(e, L2_dgrad), c = operand(e, W_dgrad);
     const Tensor r = rows.contiguous(), cc = cols.contiguous(), p = transpose_perm.contiguous();
     if (!e.native) {
         py::gil_scoped_acquire gil;
@@ -755,6 +764,7 @@ PYBIND11_MODULE(_oeq_torch, m) {
         e->mode = d["mode"].cast<int>();
         e->dx_mode = d["dx_mode"].cast<int>();
         e->index_dims = d["index_dims"].cast<std::array<int64_t, 3>>();
+        e->direct_loads = d["direct_loads"].cast<bool>();
         e->fused_second_order = d["fused_second_order"].cast<bool>();
         e->native = d["native"].cast<bool>();
         e->alert_forward = d["alert_forward"].cast<bool>();

@@ -9,9 +9,11 @@ import re
 
 import numpy as np
 import pytest
+import torch
 
 import openequivariance_amd as oeq
 from openequivariance_amd import runtime as rt
+from openequivariance_amd._torch import ops
 from openequivariance_amd.codegen.lower import lower
 from openequivariance_amd.codegen.uvu import UvuEmitter, _staged_segments, conv_module
 from openequivariance_amd.core import problems as P
@@ -200,6 +202,43 @@ def test_gradients_of_harmonics_where_blocks_take_several_nodes():
     dx, dy, dw = R.conv_backward(R.Problem.from_spec(problem), x, y, w, gz, rows, cols)
     for got, want in ((tx.grad, dx), (ty.grad, dy), (tw.grad, dw)):
         assert err(got, want) <= tol_of(problem)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,dtype", [("lips", np.float32), ("chunks", np.float32), ("chunks", np.float64),
+                                        ("shared-weights", np.float32)])
+def test_operands_that_begin_anywhere(name, dtype):
+    """Contiguous views one element into a larger tensor, for kernels that bring operands into LDS 16 bytes at a time:
+    the same kernels on the same values, so the same bits."""
+    n, edges = len(DEGREES), []
+    if name == "shared-weights":
+        problem = P.FCTPP("128x0e+128x1o", "1x0e+1x1o", "128x0e+128x1o", shared_weights=True, internal_weights=False)
+        module, e, weights = oeq.TensorProduct(problem), n, (problem.weight_numel,)
+    else:
+        problem = _problem(name, dtype, "mul_ir")
+        rows = np.repeat(np.arange(n), DEGREES)
+        graph = CoordGraph(np.zeros((n, 3)), rows, np.random.default_rng(3).integers(0, n, size=len(rows)))
+        edges = to_gpu(graph.rows, graph.cols, graph.transpose_perm)
+        module, e = oeq.TensorProductConv(problem, deterministic=True), len(rows)
+        weights = (e, problem.weight_numel)
+    rng = np.random.default_rng(5)
+    values = to_gpu(*(rng.normal(size=s).astype(dtype) for s in (
+        (n, problem.irreps_in1.dim), (e, problem.irreps_in2.dim), weights, (n, problem.irreps_out.dim))))
+
+    def passes(place):
+        x, y, w, g = (place(t).requires_grad_(True) for t in values)
+        z = module(x, y, w, *edges)
+        first = torch.autograd.grad(z, (x, y, w), g, create_graph=True)
+        second = torch.autograd.grad(first, (x, y, w, g), [place(2 * t.detach()) for t in first])
+        return [t.detach() for t in (z, *first, *second)]
+
+    def inside(t):
+        view = t.new_empty(t.numel() + 1)[1:].view(t.shape).copy_(t).detach()
+        assert view.is_contiguous() and view.data_ptr() % 16
+        return view
+
+    assert all(torch.equal(p, q) for p, q in zip(passes(torch.clone), passes(inside)))
+    assert ops.get_entry(module.kid).direct_loads
 
 
 def _check(problem, plain, det, tune, monkeypatch):
