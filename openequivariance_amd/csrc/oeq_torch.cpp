@@ -252,6 +252,8 @@ std::atomic<int64_t> g_index_cache_entries{4};
 
 bool check_indices() {
     if (g_check_indices) return true;
+    // (Python's os.environ writes the environment under the interpreter lock, and may move it)
+    py::gil_scoped_acquire gil;
     const char* env = std::getenv("OEQ_AMD_CHECK_INDICES");
     return env && *env && !(env[0] == '0' && !env[1]);
 }
