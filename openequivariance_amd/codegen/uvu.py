@@ -2628,11 +2628,10 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
             em.emit_structs(s)
             em._emit_load_edge(s, "load_edge_b", em.used_in1, em.low.paths, sender=True)
             s.open(f"OEQ_DEV void walk({operands}const i64 node, const i64 e0, const i64 e1, "
-                   f"T (*s_dy)[{W}][{self.l2_pad}])")
+                   f"T (*s_dy)[{W}][{self.l2_pad}], int& batch)")
             em._lane_prologue(s)
             s("G_t gr;")
             em._load_g(s, f"L3_grad + node * {low.L3}", em.used_out)
-            s("int batch = 0;")
             of, load = em._group_operands(s, "load_edge_b")
             if ahead:
                 s("E_t B;")
@@ -2706,10 +2705,11 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
         )
         self._lane_prologue(s, W)
         s(f"__shared__ T s_dy[{2 * n}][{W}][{self.l2_pad}];")
+        s("int batch = 0;  // the half of s_dy that the next batch goes to, also where a block walks several positions")
         self._node_loop_open(s, 1, xcd, parts=True)
         for gi in range(W):
             s(f"{'else ' if gi else ''}if (sg == {gi}) oeq_group{gi}::walk(node_count, nnz, L1_in, L2_in, L2_grad, W, "
-              "W_grad, L3_grad, cols, dx_tmp, eperm, node, e0, e1, s_dy);")
+              "W_grad, L3_grad, cols, dx_tmp, eperm, node, e0, e1, s_dy, batch);")
         s.close()
         s.close()
         return block

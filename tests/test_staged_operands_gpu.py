@@ -151,6 +151,17 @@ def test_lanes_are_read_outside_of_branches(layout, det, monkeypatch):
     assert not re.search(r"\?[^;\n]*__builtin_amdgcn_readlane", src)
 
 
+@pytest.mark.parametrize("xcd", [1, 8])
+def test_batches_take_turns_across_positions(xcd, monkeypatch):
+    """The half of the dY buffer that is next belongs to the block, whatever number of batches a walk position has: with it
+    begun anew at every position, a block that walks two could overwrite rows that a slower wave still adds up."""
+    src, _ = _module("two", "mul_ir", True, f"conv_wgrp=7,conv_xcd={xcd}", monkeypatch)
+    kernel = src[src.index("void backward(i64 node_count"):]
+    assert kernel.index("int batch = 0;") < kernel.index("for (i64 wpos")
+    walks = src[src.index("namespace oeq_group0"):src.index("void backward(i64 node_count")]
+    assert walks.count("int& batch)") == 2 and "int batch" not in walks
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("layout,det", [("mul_ir", True), ("ir_mul", False)])
 def test_spilled_operands_against_the_oracle(layout, det, monkeypatch):
