@@ -38,6 +38,8 @@ SIZES = [
     (1, 20480, (0, 0)), (5000, 24576, (1536, 1542)), (16384, 262144, (262144, 70000)), (300, 262144, (0, 0)),
     (300, 262145, (0, 0)), (16385, 20000, (300, 0)), (255, 16385, (16385, 256)), (256, 69633, (0, 4097)),
     (300, 8192, (257, 0)), (300, 8193, (0, 257)),
+    # beyond the slices, with segments that the whole grid ranks on both sides
+    (16385, 40000, (2000, 3000)), (1000, 270000, (1025, 5000)),
 ]
 
 
@@ -82,10 +84,11 @@ def test_index_pieces(nodes, edges, hubs, det, monkeypatch):
 
 
 def test_indices_out_of_range_stay_out_of_the_grouping():
-    """Keys that name no node are left out; nothing is read or written outside the buffers (both builds)."""
+    """Keys that name no node are left out; nothing is read or written outside the buffers (one launch, slice by
+    slice, and the five launches beyond)."""
     src, dims, descs = build_conv_module(P.config1_single_uvu(), False)
     ks = rt.get_kernel_set(src, dims, descs)
-    for nodes, edges in ((50, 900), (5000, 20000)):
+    for nodes, edges in ((50, 900), (5000, 20000), (16385, 20000), (1000, 270000)):
         rows, cols = _edges(nodes, edges, (0, 0), seed=1)
         rows[::7], cols[::5] = nodes, -3
         tr, tc = torch.tensor(rows, device="cuda"), torch.tensor(cols, device="cuda")

@@ -29,6 +29,7 @@ PROBLEMS = {
     "mace-large-f64": lambda: _f64(P.mace_problems()[0]),  # one wave per SIMD
     "config1": P.config1_single_uvu,                      # 64 rows to a wave
     "config2": P.config2_nequip_uvu,                      # two rows to a wave
+    "config2-f64": lambda: _f64(P.config2_nequip_uvu()),  # two rows to a wave, staged: lanes hold the edges ahead
     "aspirin": lambda: P.nequip_problems()[1],            # one chunk; sender gradients by the sender walk
     "SevenNet-main": lambda: P.seven_net_problems()[1],   # folded multiplicities, waves share the output segments
     "SevenNet-last": lambda: P.seven_net_problems()[2],   # sender walk over long rows
