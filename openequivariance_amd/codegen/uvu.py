@@ -2532,10 +2532,12 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
                 groups.append(part)
         return groups if groups and len(groups) <= 8 and all(em.operand_words(2) <= 150 for em in groups) else None
 
-    def emit_conv_forward_groups(self, s: Src, ems: List["UvuEmitter"], waves_per_eu: int, xcd: int) -> int:
+    def emit_conv_forward_groups(self, s: Src, ems: List["UvuEmitter"], waves_per_eu: int, xcd: int, whole: bool) -> int:
         """Forward of rows with blocks of different widths: every wave of a block walks the edges of one node for its
         own group of paths (``width_groups``), several edges side by side where its blocks are narrow, and stores the
-        blocks of the node's row that its paths go to. The waves do not meet.
+        blocks of the node's row that its paths go to. The waves do not meet. ``whole``: lane groups past a node's last
+        edge add zeros instead of standing aside, for kernels with scratch memory: no register is then spilled in a branch
+        of some lanes, and reloaded by all of them.
 
         With one edge to a wave half of the lanes were idle in blocks of 32 channels, and the waves that shared the outputs
         by segments read the rows of X two or three times. Three waves per SIMD; two of them with 250 registers and the
@@ -2587,7 +2589,14 @@ f"const T* __restrict__ W, const i64* __restrict__ cols, const i64 node_count, c
             s("if ((next & 63) == 0) oeq_look_ahead(ahead, e0 + next + lane, e1, eperm, cols, node_count);")
             load("B", "next")
             s.close()
-            s("if (done + r < count) fwd_seg0_pre(A, a);" if em.R > 1 else "fwd_seg0_pre(A, a);")
+            if em.R > 1 and whole:
+                s.open(f"if (done + {em.R} > count)")
+                s("const bool live = done + r < count;")
+                for v in ([f"A.x.b{b}[{i}]" for b in em.used_in1 for i in range(low.in1[b].d)]
+                          + [f"A.w[{k}]" for k in range(em.n_wslots)] + [f"A.y[{j}]" for j in range(low.L2)]):
+                    s(f"{v} = oeq_sel(live, {v});")
+                s.close()
+            s("fwd_seg0_pre(A, a);" if em.R == 1 or whole else "if (done + r < count) fwd_seg0_pre(A, a);")
             s.close()
             em._fold_store(s, 0, "zrow")
             s.close()
@@ -3038,7 +3047,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
                     conv_dxm=-1, conv_q=0, conv_hops=2, conv_qpin=1, conv_qaf=48, conv_qab=24, tp_mask=0, tp_forms=1,
                     conv_hub=256, conv_dxs=-1, conv_omin=32768, conv_fsplit=-1, conv_fsplit_f=-1, conv_fsplit_x=-1, conv_fsplit_a=-1,
                     conv_fsmax=-1, conv_parts=-1, conv_stg=1,
-                    conv_wgrp=3))
+                    conv_wgrp=3, conv_wtail=0))
     assert deterministic or not kahan, "kahan=True requires deterministic=True"
     # knobs somebody set: the rules below leave those alone
     user_tune = os.environ.get("OEQ_AMD_TUNE", "")
@@ -3198,7 +3207,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         s(LOOK_AHEAD)
     if forward_groups:
         G_f = 1
-        blk_f = em.emit_conv_forward_groups(s, forward_groups, 3, xcd)
+        blk_f = em.emit_conv_forward_groups(s, forward_groups, 3, xcd, bool(t["conv_wtail"]))
     else:
         blk_f = em.emit_conv_forward(s, G_f, walk, t["conv_pipe_f"], t["conv_wf"], xcd, bool(t["conv_tra"]))
     splits: Dict[str, Split] = {}  # the kernels with a node's edges dealt out to several waves
@@ -3361,7 +3370,10 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     # 64x0e+64x1o+16x2e+16x3o 172 / 116); more than 12 was not seen.
     if width_groups and not forced and rt.kernel_resources(rt.compile_source(src)).get("backward", (0, 0))[1] > 0:
         return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wgrp=t["conv_wgrp"] & ~1), draft)
-    if forward_groups and not forced and rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))[1] > 16:
+    spilled = rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))[1] if forward_groups else 0
+    if spilled and not t["conv_wtail"]:
+        return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wtail=1), draft)
+    if spilled > 16 and not forced:
         return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wgrp=t["conv_wgrp"] & ~2), draft)
     if staged64 and len(em.segments) > 1 and rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))[1] > 0:
         return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_stg=0), draft)

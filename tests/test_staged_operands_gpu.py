@@ -140,6 +140,8 @@ def test_the_module_has_a_wave_for_every_width(name, layout, det, monkeypatch):
 def test_a_forward_by_width_may_spill_a_few_bytes(tune, monkeypatch):
     src, resources = _module("few-spilled", "mul_ir", True, tune, monkeypatch)
     assert "namespace oeq_forward_group0" in src and resources["forward"][1] <= 16
+    # then no lane group stands aside at a node's last edges (what a branch spills, it spills for its own lanes)
+    assert ("if (done + r < count)" in src) == (resources["forward"][1] == 0)
 
 
 @pytest.mark.parametrize("layout,det", [("mul_ir", True), ("ir_mul", False)])
