@@ -3366,14 +3366,15 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     # registers, 236 B: step of 3 000 nodes x 30 edges 753 us against 448; the wide blocks and the narrow ones of SevenNet's
     # main layer in three waves, 48 B: 594 / 564). The forward may have a few bytes: of those seen, written
     # once and read once per node (us, by segment / by width: SevenNet's main layer, ir_mul, 8 B, 600 nodes x 20 edges 68 / 53, 2 003 x 40 196 / 166,
-    # 8 000 x 30 498 / 418; with 12 B 96x{0e..3o} 272 / 253 at 3 000 x 30, 64x0e+64x1o+32x2e+32x3o 176 / 122,
-    # 64x0e+64x1o+16x2e+16x3o 172 / 116); more than 12 was not seen.
+    # 8 000 x 30 498 / 418; with 12 B, 3 000 x 30, 64x0e+64x1o+32x2e+32x3o 176 / 122, 64x0e+64x1o+16x2e+16x3o 172 / 116);
+    # more than 12 was not seen. None where every width takes two waves: they read X twice, as waves by segment do, which
+    # then leave less to gain (96x{0e..3o}, 12 B, 272 / 253) and run a third wave per SIMD without scratch memory.
     if width_groups and not forced and rt.kernel_resources(rt.compile_source(src)).get("backward", (0, 0))[1] > 0:
         return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wgrp=t["conv_wgrp"] & ~1), draft)
     spilled = rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))[1] if forward_groups else 0
     if spilled and not t["conv_wtail"]:
         return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wtail=1), draft)
-    if spilled > 16 and not forced:
+    if spilled > (16 if len(forward_groups or ()) < 2 * len(apart or ()) else 0) and not forced:
         return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_wgrp=t["conv_wgrp"] & ~2), draft)
     if staged64 and len(em.segments) > 1 and rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))[1] > 0:
         return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_stg=0), draft)
