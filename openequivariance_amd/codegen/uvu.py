@@ -3189,7 +3189,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     # waves that lose: SevenNet's main layer (2 003 x 40) 711 / 566, 96x{0e..3o} 1 026 / 879, 64x0e+64x1o+16x2e+16x3o
     # 453 / 400). Three and four widths lose: 64x0e+32x1o+16x2e 224 / 273, 64x0e+64x1o+32x2e+16x3o 468 / 516,
     # 128x0e+64x1o+32x2e+8x3o 359 / 422. Forward, whose waves do not meet: where the outputs would be walked in several
-    # segments (64x0e+64x1o+32x2e+16x3o 177 / 124, 64x1o+32x2e+32x3o+32x1e 378 / 120, 96x{0e..3o} 275 / 260, and the figures
+    # segments (64x0e+64x1o+32x2e+16x3o 177 / 124, 64x1o+32x2e+32x3o+32x1e 378 / 120, and the figures
     # at emit_conv_forward_groups; one segment: 64x0e+32x1o+16x2e 69 / 86, 96x{0e,1o,2e} 115 / 119), with blocks of eight
     # channels not (64x0e+64x1o+8x2e+8x1e, 9 000 x 24: 177 / 184). Neither where blocks leave lanes of their own width
     # without a channel (100x0e+40x1o+20x2e+9x1e: forward 98 / 109, step 304 / 470).
