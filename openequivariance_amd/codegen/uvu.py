@@ -298,18 +298,32 @@ class UvuEmitter:
         operand set. What is left is the W stream: NequIP lips, 5 000 nodes x 28 edges, ir_mul, forward 165 -> 138 us
         (5.3 TB/s of W while a node's edges are walked, and 11 us per node until the first edge has arrived and the row
         is stored); 3 000 x 28 127 / 96, 700 x 40 69 / 38; nequip-uvu 20 000 x 30 346 / 273; water 1 500 x 35 34 / 26,
-        50 000 x 20 336 / 325; the same in double precision, nequip-uvu 3 000 x 30 110 / 89."""
+        50 000 x 20 336 / 325; the same in double precision, nequip-uvu 3 000 x 30 110 / 89.
+
+        Of an X row what lies between the first and the last value that a path reads (us, loaded by the lanes / whole rows
+        staged / now: 32x0e+32x1o+32x2e with a scalar second operand, of which the scalars are read, 20 000 x 20, 45 / 68 / 43,
+        fp64 43 / 135 / 51; two thirds read, 32 channels down to 8, 10 800 x 20, 98 / 103 / 90)."""
         low, es = self.low, self.low.elem_size
         if not (self.R == 2 and self.can_preload and len(self.segments) == 1 and not low.shared_weights):
             return None
         if low.L2 > self.LPR or low.L1 * es % 16 or low.WN * es % 16:
             return None
-        nqx, nqw = -(-low.L1 * es // 1024), -(-low.WN * es // 1024)
+        def end(b: int, lanes: int) -> int:
+            (off, ls), cs = self._lane_ptr(low.in1[b])
+            return off + (low.in1[b].d - 1) * cs + (lanes - 1) * ls + 1
+
+        x0 = min(low.in1[b].off for b in self.used_in1) // self.unit * self.unit
+        xn = -(-(max(end(b, low.in1[b].mul) for b in self.used_in1) - x0) // self.unit) * self.unit
+        nqx, nqw = -(-xn * es // 1024), -(-low.WN * es // 1024)
         y = -(-low.L2 // 4) * 4
         XF, row = nqx * 1024 // es, (nqx + nqw) * 1024 // es
-        if self.R * (row + y) * es > LDS_LIMIT:
+        # (lanes without a channel read on behind their block, and drop what they find: within the buffer)
+        reach = max([end(b, self.LPR) - x0 for b in self.used_in1]
+                    + [XF + p.woff + self.LPR * low.in2[p.i2].mul for p in low.paths])
+        floats = -(-max(self.R * (row + y), (self.R - 1) * row + reach) // self.unit) * self.unit
+        if floats * es > LDS_LIMIT:
             return None
-        return dict(nqx=nqx, nqw=nqw, XF=XF, row=row, y=y, floats=self.R * (row + y))
+        return dict(nqx=nqx, nqw=nqw, XF=XF, row=row, y=y, x0=x0, xn=xn, floats=floats)
 
     def _emit_rows_issue(self, s: Src, e: str, last: str, step: int):
         """Request the operands of the wave's next R edges, positions ``e`` .. ``e`` + R - 1 of the walk. Their numbers
@@ -319,9 +333,9 @@ class UvuEmitter:
         s(f"if ((handed & 63) == 0) oeq_look_ahead(ahead, {e} + (i64)(lane / {R}) * {step} + lane % {R}, {last}, "
           "eperm, cols, node_count);")
         s("const int at = handed & 63;")
-        def request(r: int, index: str, row: str, n: int, numel: int, lds: int, aux: int):
+        def request(r: int, index: str, row: str, n: int, stride: int, numel: int, lds: int, aux: int):
             s.open(f"if ({e} + {r} < {last})" if r else "")
-            s(f"const T* row = {row} + (i64)__builtin_amdgcn_readlane(ahead.{index}, at + {r}) * {numel};")
+            s(f"const T* row = {row} + (i64)__builtin_amdgcn_readlane(ahead.{index}, at + {r}) * {stride};")
             for q in range(n):
                 # (lanes beyond the row repeat its last 16 bytes into the padding)
                 end = numel * es - 16 - q * 1024
@@ -332,10 +346,10 @@ class UvuEmitter:
 
         # (weights and Y first: their addresses need the edge's number only, the senders are a load behind it)
         for r in range(R):
-            request(r, "eid", "W", st["nqw"], low.WN, st["XF"], 2 if self.nt & 1 else 0)
+            request(r, "eid", "W", st["nqw"], low.WN, low.WN, st["XF"], 2 if self.nt & 1 else 0)
         s(f"yn = L2_in[(i64)__shfl(ahead.eid, at + r) * {low.L2} + (ul < {low.L2} ? ul : {low.L2 - 1})];")
         for r in range(R):
-            request(r, "sender", "L1_in", st["nqx"], low.L1, 0, 0)
+            request(r, "sender", f"L1_in + {st['x0']}" if st["x0"] else "L1_in", st["nqx"], low.L1, st["xn"], 0, 0)
         s(f"handed += {R};")
         s.close()
 
@@ -347,7 +361,7 @@ class UvuEmitter:
         for b in self.used_in1:
             (off, ls), cs = self._lane_ptr(low.in1[b])
             for i in range(low.in1[b].d):
-                s(f"{buf}.x.b{b}[{i}] = sr[{off + i * cs} + ul * {ls}];")
+                s(f"{buf}.x.b{b}[{i}] = sr[{off - st['x0'] + i * cs} + ul * {ls}];")
         for p in low.paths:
             V = low.in2[p.i2].mul
             for v in range(V):

@@ -30,6 +30,8 @@ PROBLEMS = {
     "ragged": ("20x0e+32x1o+4x2e", "0e+1o", "0e+1o+2e"),
     "channels": ("32x0e+32x1o", "2x0e+3x1o", "0e+1o"),
     "lips": None,
+    "middle": ("32x0e+32x1o+32x2e", "1o", "0e"),          # paths read one block of X, not the first
+    "ragged-middle": ("30x0e+20x1o+24x2e+2x3o", "1o", "0e+3o"),  # two of the four, the first one off a 16-byte boundary
     "chunks": ("128x0e+128x1o", "0e+1o+2e", "0e+1o+2e"),  # two waves to a node: dY of eight edges at a time
     "ragged-chunks": ("200x0e+100x1o", "0e+1o", "0e+1o+2e"),
 }
@@ -70,6 +72,13 @@ def _shared(name, layout):
 @pytest.mark.parametrize("name", ["rest", "ragged", "channels", "lips"])
 def test_these_problems_stage_their_rows(name):
     assert UvuEmitter(lower(_problem(name, np.float32, "mul_ir"))).rows_stage is not None
+
+
+@pytest.mark.parametrize("name,dtype,first,count", [("middle", np.float32, 32, 96), ("middle", np.float64, 32, 96),
+                                                    ("ragged-middle", np.float32, 28, 184), ("ragged-middle", np.float64, 30, 180)])
+def test_rows_are_staged_as_far_as_paths_read_them(name, dtype, first, count):
+    stage = UvuEmitter(lower(_problem(name, dtype, "mul_ir"))).rows_stage
+    assert (stage["x0"], stage["xn"]) == (first, count)
 
 
 @pytest.mark.parametrize("name,waves", [("one", 1), ("two", 2), ("two-shuffled", 2), ("four-shuffled", 4)])
