@@ -157,7 +157,7 @@ class UvuEmitter:
         have the regular shape this needs."""
         low = self.low
         if not (self.R == 1 and self.can_preload and (several or len(self.segments) == 1)
-                and not low.shared_weights):
+                and not low.shared_weights) or self._one_load_each():
             return None
         U, n = 64 * self.NCH, self.unit
         if any(low.in1[b].mul != U or low.in1[b].off % n for b in self.used_in1):
@@ -181,6 +181,15 @@ class UvuEmitter:
         # (the waves of a node, one or more per segment, have to fit a block)
         waves = self.NCH * min(len(stages), max(1, 8 // self.NCH))
         return stages if waves * self._wave_lds(max(st["floats"] for st in stages)) <= LDS_LIMIT else None
+
+    def _one_load_each(self) -> bool:
+        """Double precision with one value of X and one weight to a lane and edge: two loads, which staging does not make fewer,
+        and a wave instruction of them moves 512 bytes as it is. Loaded by the lanes they do without the LDS on their way. Forward,
+        us, staged / not: 64x0e 20 000 nodes x 20 edges 66.7 / 60.0, 128x0e+128x1o+128x2e -> 128x0e 5 278 x 20 40.7 / 34.4, 256x0e
+        7 512 x 20 88.5 / 84.6, two edges to a wave 32x0e 20 000 x 20 50.7 / 42.9. From two values of X or two weights on staging
+        is level or gains (64x0e+64x1o, three values a lane and two paths up, 12 207 x 20 103.4 / 103.1, 1 831 x 20 17.4 / 19.2), and in single precision
+        it gains with two values as well (32x0e 20 000 x 20 43.6 / 45.6)."""
+        return self.words == 2 and sum(self.low.in1[b].d for b in self.used_in1) + self.n_wslots <= 2
 
     def _wave_lds(self, floats: int) -> int:
         """Bytes of LDS of a wave that stages ``floats`` elements, with the buffer that fp64 rows are stored through."""
@@ -304,7 +313,7 @@ class UvuEmitter:
         staged / now: 32x0e+32x1o+32x2e with a scalar second operand, of which the scalars are read, 20 000 x 20, 45 / 68 / 43,
         fp64 43 / 135 / 51; two thirds read, 32 channels down to 8, 10 800 x 20, 98 / 103 / 90)."""
         low, es = self.low, self.low.elem_size
-        if not (self.R == 2 and self.can_preload and len(self.segments) == 1 and not low.shared_weights):
+        if not (self.R == 2 and self.can_preload and len(self.segments) == 1 and not low.shared_weights) or self._one_load_each():
             return None
         if low.L2 > self.LPR or low.L1 * es % 16 or low.WN * es % 16:
             return None

@@ -81,6 +81,15 @@ def test_rows_are_staged_as_far_as_paths_read_them(name, dtype, first, count):
     assert (stage["x0"], stage["xn"]) == (first, count)
 
 
+@pytest.mark.parametrize("mul", [32, 64, 128])
+def test_single_values_in_double_precision_are_not_staged(mul):
+    for dtype, in2, staged in ((np.float64, "0e", False), (np.float64, "0e+1o", True), (np.float32, "0e", True)):
+        p = P.ChannelwiseTPP(f"{mul}x0e", in2, "0e+1o")
+        p.irrep_dtype = p.weight_dtype = dtype
+        em = UvuEmitter(lower(p))
+        assert ((em.rows_stage if mul == 32 else em.stage) is not None) == staged
+
+
 @pytest.mark.parametrize("name,waves", [("one", 1), ("two", 2), ("two-shuffled", 2), ("four-shuffled", 4)])
 def test_waves_that_share_the_outputs(name, waves):
     em = _staged_segments(lower(_shared(name, "mul_ir")), 8)
