@@ -2983,21 +2983,24 @@ def tp_module(low: Lowered, compute_units: int = 256):
     return s.text(), dims, descs
 
 
-def _forward_plan(low: Lowered, first_budget: int) -> Tuple[UvuEmitter, bool]:
+def _forward_plan(low: Lowered, first_budget: int, rows: bool) -> Tuple[UvuEmitter, bool]:
     """(emitter, two operand sets in flight?) for a walk kernel without LDS staging: the accumulators of an output
     segment, the edge's operands (X blocks, the weights of the segment's paths, Y) once or twice, within the registers
     of two waves per SIMD. The segment budget shrinks until that fits; the prefetch goes when 48-word segments do
-    not fit with it."""
+    not fit with it. ``rows``: rows of two edges may be staged."""
     words = 1 if low.elem_size == 4 else 2
 
     def plan(budget, sets):
         e = UvuEmitter(low, acc_budget_words=budget)
+        e.rows_stage = None
         need = max(sets * words * (sum(low.in1[b].d for b in e.seg_in1[si]) + low.L2 +
                                    sum(low.in2[p.i2].mul for p in low.paths if p.io in seg))
                    + words * sum(low.out[io].d for io in seg) for si, seg in enumerate(e.segments))
         return e, need + (40 if e.ragged() else 0)
 
     e = UvuEmitter(low, acc_budget_words=first_budget)
+    if not rows:
+        e.rows_stage = None
     if e.words == 2 and e.operand_words(1) > 200:
         e.stage = e.stages = None  # (an operand set copied from LDS and the accumulators: more than half a SIMD's registers)
     if e.stage is not None or e.rows_stage is not None or not e.can_preload:
@@ -3070,7 +3073,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
                     conv_dxm=-1, conv_q=0, conv_hops=2, conv_qpin=1, conv_qaf=48, conv_qab=24, tp_mask=0, tp_forms=1,
                     conv_hub=256, conv_dxs=-1, conv_omin=32768, conv_fsplit=-1, conv_fsplit_f=-1, conv_fsplit_x=-1, conv_fsplit_a=-1,
                     conv_fsmax=-1, conv_parts=-1, conv_stg=1,
-                    conv_wgrp=3, conv_wtail=0))
+                    conv_wgrp=3, conv_wtail=0, conv_rows=3))
     assert deterministic or not kahan, "kahan=True requires deterministic=True"
     # knobs somebody set: the rules below leave those alone
     user_tune = os.environ.get("OEQ_AMD_TUNE", "")
@@ -3085,6 +3088,9 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         mode = rt.CONV_GROUPED if t["conv_sort"] else rt.CONV_ATOMIC
     walk = mode != rt.CONV_ATOMIC  # kernels walk per-node edge segments
     em = UvuEmitter(low, acc_budget_words=t["conv_acc"], kahan=kahan)
+    # (conv_rows: rows of two edges staged in LDS, bit 1 forward, 2 sender walk)
+    if not t["conv_rows"] & 1:
+        em.rows_stage = None
     # fp64 with rows that fill the wave: when everything a node needs (accumulators or gradient slice, one
     # operand set) fits the 512 registers a lane has at one wave per SIMD, that beats walking the edges once
     # per output segment / sharing the node between waves (MACE shape, fp64: forward 18.4 -> 12.5 ms,
@@ -3121,6 +3127,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
 
         def plan(budget, sets):
             e = UvuEmitter(low, acc_budget_words=budget, kahan=kahan)
+            e.rows_stage = None
             need = max(sets * words * (sum(low.in1[b].d for b in e.seg_in1[si]) + low.L2 +
                                        sum(low.in2[p.i2].mul for p in low.paths if p.io in seg))
                        + words * sum(low.out[io].d for io in seg) for si, seg in enumerate(e.segments))
@@ -3318,7 +3325,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         if dx_mode == UvuEmitter.DX_SENDER_WALK:
             from .lower import adjoint
             low_x = adjoint(low)
-            ex, pipe_x = _forward_plan(low_x, t["conv_acc"])
+            ex, pipe_x = _forward_plan(low_x, t["conv_acc"], bool(t["conv_rows"] & 2))
             ex.nt, ex.mask_loads, ex.forms, ex.tr_stores = t["conv_nt"], bool(t["tp_mask"]), bool(t["tp_forms"]), t["conv_trs"]
             words_x = (1 if low.elem_size == 4 else 2) * (
                 max(sum(low_x.out[io].d for io in seg) for seg in ex.segments)
@@ -3384,7 +3391,17 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         # (forced on shapes beyond the rule, adjoint kernels with 200 - 320 B of scratch ran 3x slower than the terms)
         _lds, scratch = rt.kernel_resources(rt.compile_source(src)).get("backward_dx", (0, 0))
         if scratch > 64:
-            return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_dxs=0), draft)
+            other = dict(conv_dxs=0) if ex.rows_stage is None else dict(conv_rows=t["conv_rows"] & ~2)
+            return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, **other), draft)
+    if walk and em.rows_stage is not None and "conv_rows" not in user_tune:
+        # Rows of two edges staged for all outputs in one pass, with an operand set beside the accumulators: not where that takes
+        # much scratch memory (forward, us, rows loaded by the lanes in several passes / staged, by the scratch memory of the latter:
+        # 52 B 32x{0e,0o,1e,1o} with 1x0e+2x1o+1x2e+2x3o 3 367 nodes x 20 137 / 114; 72 B 24x0e+24x1o in fp64 192 / 138,
+        # 8x0e+32x1o 168 / 157; 80 B 24x{0e,1o,2e} 225 / 157; 100 B 32x0e+32x1o 146 / 174; 116 B 32x{0e,1o,2e} 138 / 184; 164 to
+        # 352 B 119 to 193 / 201 to 259; at less than 400 nodes these, whose small-graph form does without scratch memory, gain
+        # by staging, 29 to 50 / 25 to 35, but both forms are of one plan)
+        if rt.kernel_resources(rt.compile_source(src)).get("forward", (0, 0))[1] > 80:
+            return conv_module(low, deterministic, compute_units, kahan, dict(override or {}, conv_rows=t["conv_rows"] & ~1), draft)
     # A wave per width: not a backward with scratch memory unless asked for regardless (NequiX's main layer held to 168
     # registers, 236 B: step of 3 000 nodes x 30 edges 753 us against 448; the wide blocks and the narrow ones of SevenNet's
     # main layer in three waves, 48 B: 594 / 564). The forward may have a few bytes: of those seen, written

@@ -81,6 +81,16 @@ def test_rows_are_staged_as_far_as_paths_read_them(name, dtype, first, count):
     assert (stage["x0"], stage["xn"]) == (first, count)
 
 
+@pytest.mark.parametrize("problem", [("32x0e+32x1o+32x2e", "0e+1o+2e+3o", "0e+0o+1e+1o+2e+2o"),
+                                     ("32x0e+32x0o+32x1e+32x1o", "3x0e+3x1o+2x2e", "0e+0o+1e+1o+2e+2o")])
+def test_rows_are_staged_where_that_takes_little_scratch_memory(problem, monkeypatch):
+    monkeypatch.delenv("OEQ_AMD_TUNE", raising=False)
+    p = P.ChannelwiseTPP(*problem)
+    p.irrep_dtype = p.weight_dtype = np.float64
+    assert UvuEmitter(lower(p)).rows_stage is not None  # (in one pass with 116 and 352 bytes)
+    assert rt.kernel_resources(rt.compile_source(conv_module(lower(p), True)[0]))["forward"][1] <= 80
+
+
 @pytest.mark.parametrize("mul", [32, 64, 128])
 def test_single_values_in_double_precision_are_not_staged(mul):
     for dtype, in2, staged in ((np.float64, "0e", False), (np.float64, "0e+1o", True), (np.float32, "0e", True)):
