@@ -309,7 +309,7 @@ class UvuEmitter:
         is stored); 3 000 x 28 127 / 96, 700 x 40 69 / 38; nequip-uvu 20 000 x 30 346 / 273; water 1 500 x 35 34 / 26,
         50 000 x 20 336 / 325; the same in double precision, nequip-uvu 3 000 x 30 110 / 89.
 
-        Of an X row what lies between the first and the last value that a path reads (us, loaded by the lanes / whole rows
+        Of an X row the blocks that paths read, one after the other in LDS (us, loaded by the lanes / whole rows
         staged / now: 32x0e+32x1o+32x2e with a scalar second operand, of which the scalars are read, 20 000 x 20, 45 / 68 / 43,
         fp64 43 / 135 / 51; two thirds read, 32 channels down to 8, 10 800 x 20, 98 / 103 / 90)."""
         low, es = self.low, self.low.elem_size
@@ -321,18 +321,28 @@ class UvuEmitter:
             (off, ls), cs = self._lane_ptr(low.in1[b])
             return off + (low.in1[b].d - 1) * cs + (lanes - 1) * ls + 1
 
-        x0 = min(low.in1[b].off for b in self.used_in1) // self.unit * self.unit
-        xn = -(-(max(end(b, low.in1[b].mul) for b in self.used_in1) - x0) // self.unit) * self.unit
+        # what is read, in whole 16-byte units: [first, end) in the row, first in LDS
+        runs: List[List[int]] = []
+        xn = 0
+        for b in sorted(self.used_in1, key=lambda b: low.in1[b].off):
+            first = low.in1[b].off // self.unit * self.unit
+            last = -(-end(b, low.in1[b].mul) // self.unit) * self.unit
+            if runs and first <= runs[-1][1]:
+                runs[-1][1] = max(last, runs[-1][1])
+            else:
+                runs.append([first, last, xn])
+            xn = runs[-1][2] + runs[-1][1] - runs[-1][0]
+        xl = {b: next(at + low.in1[b].off - a for a, z, at in runs if a <= low.in1[b].off < z) for b in self.used_in1}
         nqx, nqw = -(-xn * es // 1024), -(-low.WN * es // 1024)
         y = -(-low.L2 // 4) * 4
         XF, row = nqx * 1024 // es, (nqx + nqw) * 1024 // es
         # (lanes without a channel read on behind their block, and drop what they find: within the buffer)
-        reach = max([end(b, self.LPR) - x0 for b in self.used_in1]
+        reach = max([end(b, self.LPR) - low.in1[b].off + xl[b] for b in self.used_in1]
                     + [XF + p.woff + self.LPR * low.in2[p.i2].mul for p in low.paths])
         floats = -(-max(self.R * (row + y), (self.R - 1) * row + reach) // self.unit) * self.unit
         if floats * es > LDS_LIMIT:
             return None
-        return dict(nqx=nqx, nqw=nqw, XF=XF, row=row, y=y, x0=x0, xn=xn, floats=floats)
+        return dict(nqx=nqx, nqw=nqw, XF=XF, row=row, y=y, runs=runs, xl=xl, xn=xn, floats=floats)
 
     def _emit_rows_issue(self, s: Src, e: str, last: str, step: int):
         """Request the operands of the wave's next R edges, positions ``e`` .. ``e`` + R - 1 of the walk. Their numbers
@@ -342,23 +352,30 @@ class UvuEmitter:
         s(f"if ((handed & 63) == 0) oeq_look_ahead(ahead, {e} + (i64)(lane / {R}) * {step} + lane % {R}, {last}, "
           "eperm, cols, node_count);")
         s("const int at = handed & 63;")
-        def request(r: int, index: str, row: str, n: int, stride: int, numel: int, lds: int, aux: int):
+        def request(r: int, index: str, row: str, n: int, stride: int, runs, numel: int, lds: int, aux: int):
             s.open(f"if ({e} + {r} < {last})" if r else "")
             s(f"const T* row = {row} + (i64)__builtin_amdgcn_readlane(ahead.{index}, at + {r}) * {stride};")
             for q in range(n):
                 # (lanes beyond the row repeat its last 16 bytes into the padding)
                 end = numel * es - 16 - q * 1024
                 off = "lane * 16u" if end >= 63 * 16 else f"(lane * 16u < {end}u ? lane * 16u : {end}u)"
-                s(f"__builtin_amdgcn_global_load_lds((const OEQ_GPTR)oeq_at(row + {q * 1024 // es}, {off}), "
+                at = q * 1024 // es + runs[0][0]
+                for before, run in zip(runs, runs[1:]):
+                    unit, gap = run[2] // self.unit - q * 64, run[0] - before[1]
+                    if unit <= 0:
+                        at += gap
+                    elif unit < 64:
+                        off += f" + (lane >= {unit} ? {gap * es}u : 0u)"
+                s(f"__builtin_amdgcn_global_load_lds((const OEQ_GPTR)oeq_at(row + {at}, {off}), "
                   f"(OEQ_LPTR)(&s_stage[wave][{r * st['row'] + lds + q * 1024 // es}]), 16, 0, {aux});")
             s.close()
 
         # (weights and Y first: their addresses need the edge's number only, the senders are a load behind it)
         for r in range(R):
-            request(r, "eid", "W", st["nqw"], low.WN, low.WN, st["XF"], 2 if self.nt & 1 else 0)
+            request(r, "eid", "W", st["nqw"], low.WN, [[0, low.WN, 0]], low.WN, st["XF"], 2 if self.nt & 1 else 0)
         s(f"yn = L2_in[(i64)__shfl(ahead.eid, at + r) * {low.L2} + (ul < {low.L2} ? ul : {low.L2 - 1})];")
         for r in range(R):
-            request(r, "sender", f"L1_in + {st['x0']}" if st["x0"] else "L1_in", st["nqx"], low.L1, st["xn"], 0, 0)
+            request(r, "sender", "L1_in", st["nqx"], low.L1, st["runs"], st["xn"], 0, 0)
         s(f"handed += {R};")
         s.close()
 
@@ -368,9 +385,9 @@ class UvuEmitter:
         s(f"T* const sy = &s_stage[wave][{self.R * st['row']}] + r * {st['y']};")
         s(f"if (ul < {low.L2}) sy[ul] = yn;")
         for b in self.used_in1:
-            (off, ls), cs = self._lane_ptr(low.in1[b])
+            (_, ls), cs = self._lane_ptr(low.in1[b])
             for i in range(low.in1[b].d):
-                s(f"{buf}.x.b{b}[{i}] = sr[{off - st['x0'] + i * cs} + ul * {ls}];")
+                s(f"{buf}.x.b{b}[{i}] = sr[{st['xl'][b] + i * cs} + ul * {ls}];")
         for p in low.paths:
             V = low.in2[p.i2].mul
             for v in range(V):

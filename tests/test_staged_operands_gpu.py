@@ -32,6 +32,8 @@ PROBLEMS = {
     "lips": None,
     "middle": ("32x0e+32x1o+32x2e", "1o", "0e"),          # paths read one block of X, not the first
     "ragged-middle": ("30x0e+20x1o+24x2e+2x3o", "1o", "0e+3o"),  # two of the four, the first one off a 16-byte boundary
+    "holes": ("32x0e+32x1o+32x2e+32x3o", "0e", "0e+2e"),  # the first and the third block, across an instruction boundary
+    "ragged-holes": ("18x0e+32x1o+6x2e+20x1e+32x0o", "0e", "0e+2e+0o"),  # three runs, off 16-byte boundaries
     "chunks": ("128x0e+128x1o", "0e+1o+2e", "0e+1o+2e"),  # two waves to a node: dY of eight edges at a time
     "ragged-chunks": ("200x0e+100x1o", "0e+1o", "0e+1o+2e"),
 }
@@ -74,11 +76,14 @@ def test_these_problems_stage_their_rows(name):
     assert UvuEmitter(lower(_problem(name, np.float32, "mul_ir"))).rows_stage is not None
 
 
-@pytest.mark.parametrize("name,dtype,first,count", [("middle", np.float32, 32, 96), ("middle", np.float64, 32, 96),
-                                                    ("ragged-middle", np.float32, 28, 184), ("ragged-middle", np.float64, 30, 180)])
-def test_rows_are_staged_as_far_as_paths_read_them(name, dtype, first, count):
-    stage = UvuEmitter(lower(_problem(name, dtype, "mul_ir"))).rows_stage
-    assert (stage["x0"], stage["xn"]) == (first, count)
+@pytest.mark.parametrize("name,dtype,runs", [
+    ("rest", np.float32, [[0, 288, 0]]), ("middle", np.float32, [[32, 128, 0]]), ("middle", np.float64, [[32, 128, 0]]),
+    ("ragged-middle", np.float32, [[28, 212, 0]]), ("ragged-middle", np.float64, [[30, 210, 0]]),
+    ("holes", np.float32, [[0, 32, 0], [128, 288, 32]]),
+    ("ragged-holes", np.float32, [[0, 20, 0], [112, 144, 20], [204, 236, 52]]),
+    ("ragged-holes", np.float64, [[0, 18, 0], [114, 144, 18], [204, 236, 48]])])
+def test_rows_are_staged_as_far_as_paths_read_them(name, dtype, runs):
+    assert UvuEmitter(lower(_problem(name, dtype, "mul_ir"))).rows_stage["runs"] == runs
 
 
 @pytest.mark.parametrize("problem", [("32x0e+32x1o+32x2e", "0e+1o+2e+3o", "0e+0o+1e+1o+2e+2o"),
