@@ -3106,7 +3106,13 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     walk = mode != rt.CONV_ATOMIC  # kernels walk per-node edge segments
     em = UvuEmitter(low, acc_budget_words=t["conv_acc"], kahan=kahan)
     # (conv_rows: rows of two edges staged in LDS, bit 1 forward, 2 sender walk)
-    if not t["conv_rows"] & 1:
+    # Where the caller's edges are sorted, loads by the lanes go to consecutive rows and need no edge numbers: in single precision
+    # rows are not staged for up to three values of X and weights a lane and edge (forward, us, 20 000 nodes x 20 edges, staged / not, edges in
+    # any order and sorted: two values, 32x0e, 43.9 / 45.7 and 42.4 / 37.3; three, 32x0e with l <= 1 harmonics, 48.7 / 51.7 and
+    # 48.0 / 42.8; four 55.3 / 62.6 and 54.0 / 52.8; eight, 32x0e+32x1o, 62.5 / 67.5 and 61.3 / 61.2; three in double precision
+    # 63.4 / 70.8 and 62.3 / 62.4).
+    few = low.elem_size == 4 and sum(low.in1[b].d for b in em.used_in1) + em.n_wslots <= 3
+    if not t["conv_rows"] & 1 or (mode == rt.CONV_SORTED and few):
         em.rows_stage = None
     # fp64 with rows that fill the wave: when everything a node needs (accumulators or gradient slice, one
     # operand set) fits the 512 registers a lane has at one wave per SIMD, that beats walking the edges once

@@ -96,6 +96,17 @@ def test_rows_are_staged_where_that_takes_little_scratch_memory(problem, monkeyp
     assert rt.kernel_resources(rt.compile_source(conv_module(lower(p), True)[0]))["forward"][1] <= 80
 
 
+@pytest.mark.parametrize("in2,dtype,det,staged", [("0e+1o", np.float32, True, False), ("0e+1o", np.float32, False, True),
+                                                  ("0e+1o", np.float64, True, True), ("0e+1o+2e", np.float32, True, True)])
+def test_short_rows_of_sorted_edges_are_not_staged(in2, dtype, det, staged, monkeypatch):
+    monkeypatch.delenv("OEQ_AMD_TUNE", raising=False)
+    p = P.ChannelwiseTPP("32x0e", in2, "0e+1o+2e")
+    p.irrep_dtype = p.weight_dtype = dtype
+    src = conv_module(lower(p), det)[0]
+    forward = src[src.index(" void forward(i64"):]
+    assert ("global_load_lds" in forward[:forward.index("__global__")]) == staged
+
+
 @pytest.mark.parametrize("mul", [32, 64, 128])
 def test_single_values_in_double_precision_are_not_staged(mul):
     for dtype, in2, staged in ((np.float64, "0e", False), (np.float64, "0e+1o", True), (np.float32, "0e", True)):
