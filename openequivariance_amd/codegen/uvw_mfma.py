@@ -1,5 +1,9 @@
 """MFMA kernels for shared-weight 'uvw' tensor products (fp32 and fp64).
 
+First-order passes in fp32 over blocks of at most 64 channels run on the bf16 matrix instructions instead, with operands
+split in three (``uvw_split.py``; ``uvw_split=0`` switches that off); the kernels here are for fp64, wider blocks, tiles
+that are mostly padding and the second-order pair.
+
 With one weight tensor for the whole batch the channel mix of a path,
 ``Z[b][w,k] += sum_u W[u,w] * T[b][u,k]`` with ``T[b][u,k] = sum_ij c_ijk X[b][u,i] Y[b][j]``,
 is a dense GEMM once rows are batched: ``[(b,k)] x [u] x [w]``. These kernels
@@ -259,7 +263,7 @@ class MfmaEmitter:
         wpe = 2 if self.words == 1 else 1
         self.tune = tuning(dict(uvw_wf=wpe, uvw_wx=wpe, uvw_ww=wpe, uvw_blocks=2, uvw_pipe=1, uvw_regs=220,
                                 uvw_merge=1, uvw_fregs=232, uvw_wregs=232, uvw_xregs=215, uvw_mfma_dd=1, uvw_gdma=1,
-                                uvw_bf3=0))
+                                uvw_bf3=0, uvw_split=1))
         # Forward kernels in the split-operand form (see BF3_TERMS). Off by default: correct to the fp32 bound, but
         # its weight slices take 24 registers per path where the fp32 form takes 16, so config 4's forward becomes
         # four kernels instead of two, and what those cost is their passes over X and Z, not their multiplies
@@ -1248,11 +1252,23 @@ def tp_module(low: Lowered, compute_units: int = 256, edge_lists: bool = False):
       "__builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true)); }")
     s(utility_kernels(edge_lists=edge_lists))
     em._emit_path_fns(s)
-    fwd_names = em.emit_forward(s)
-    bwd_names = em.emit_backward(s)
     max_blocks = compute_units * em.tune["uvw_blocks"]
-    descs = [(rt.ROLE_TP_FORWARD, n, 64 * WAVES, RT, max_blocks) for n in fwd_names]
-    descs += [(rt.ROLE_TP_BACKWARD, n, 64 * WAVES, RT, max_blocks) for n in bwd_names]
+    from .uvw_split import DEVICE, SplitEmitter
+    sp = SplitEmitter(low)
+    on = bool(em.tune["uvw_split"]) and not em.bf3
+    split_f, split_b = on and sp.supported("forward"), on and sp.supported("dx")
+    if split_f or split_b:
+        s(DEVICE)
+    if split_f:
+        descs = [(rt.ROLE_TP_FORWARD, n, 64 * WAVES, RT, compute_units * sp.waves("forward"))
+                 for n in sp.emit_pass(s, "forward", "forward", em.FWD_SIG)]
+    else:
+        descs = [(rt.ROLE_TP_FORWARD, n, 64 * WAVES, RT, max_blocks) for n in em.emit_forward(s)]
+    if split_b:
+        descs += [(rt.ROLE_TP_BACKWARD, n, 64 * WAVES, RT, compute_units * sp.waves("dx"))
+                  for n in sp.emit_pass(s, "dx", "backward", em.BWD_SIG) + sp.emit_dw(s, "backward_w", em.BWD_SIG)]
+    else:
+        descs += [(rt.ROLE_TP_BACKWARD, n, 64 * WAVES, RT, max_blocks) for n in em.emit_backward(s)]
     if em.tune["uvw_mfma_dd"]:
         names_a, names_b = em.second_order_kernels(s)
         descs += [(rt.ROLE_DOUBLE_BACKWARD_A, n, 64 * WAVES, RT, max_blocks) for n in names_a]

@@ -1,0 +1,903 @@
+"""Split-operand matrix kernels for shared-weight 'uvw' tensor products in fp32: forward, dX / dY and dW.
+
+The fp32 matrix instructions share the datapath of the vector unit and give 157 TFLOP/s; the bf16 ones are a pipe of their
+own with 16 times that. Here every fp32 operand is the sum of three bf16 numbers (8 mantissa bits each: together the 24 of
+fp32; a remainder is exact), and a product the six cross products of weight 2^-16 and above, accumulated in fp32 by
+``v_mfma_f32_16x16x32_bf16``: 6 x 16 cycles for what takes the fp32 instruction 8 x 32. What is dropped is 2^-26 of a
+product, and 32 products are summed before they are rounded, so the results are nearer to 64 bits than those of the
+fp32 instruction. 64x{0e,1o,2e} (x) {0e,1o,2e} -> the same, relative errors of Z, dX, dY, dW at 100 003 rows, before
+and now: 2.9e-7, 1.6e-7, 1.7e-7, 5.4e-7 and 0.75e-7, 0.8e-7, 1.0e-7, 2.3e-7. An infinity in an operand gives NaN.
+
+Where the fp32 kernels (``uvw_mfma.py``) contract with the coupling coefficients first and multiply the result, forward and dX
+multiply first: the matrix cores form W^T x (or W dZ) component by component, the lanes contract what comes out. The
+operand that is split, written to LDS and read by every wave is then a row as it lies in memory - 9 components per channel
+at l <= 2, where the contraction of 11 paths has 35 - so that a tile's operands are prepared once, and X and dZ are read
+once per kernel.
+
+* Forward, dX: a block of 4 waves owns 16 rows at a time; wave w result channels 16 w .. 16 w + 15, with the weights
+  of all sub-paths of the kernel in registers. The threads split the next tile's rows into LDS (two copies) while
+  this one's components are multiplied. dY falls out of dX's products: summed over the lanes of a row in registers, over
+  the waves through LDS in wave order. As few kernels as the registers allow (``SplitEmitter.plan``).
+* dW: wave w owns input channels 16 w .. 16 w + 15, contracts X and Y for them in registers, eight rows a lane, in the
+  layout of the A operand; the output gradient's operands are split once per block. Products of 32 rows are summed from zero
+  and then added to the running sums by fp32 matrix instructions with the identity. The bf16 instruction cuts off what it aligns,
+  always downwards, and running sums of 12 steps drift by that: every second block works on negated values,
+  which the identity (with the same sign) turns back (dW above: 1.5e-6 on the running sums directly, 5.4e-7 from zero, 2.3e-7
+  with the signs).
+
+What bounds them (MI355X, the problem above, 100 003 rows): the registers of a SIMD hold one wave of these kernels, and
+a wave issues one instruction in about 2.1 ns, a matrix instruction takes 8 (less, and at a higher clock, where the data are
+zeros: random operands cost 20 % of the clock): forward 420 matrix and 1 060 other instructions a tile, 165 us at 100 003 rows
+against 328 us for the fp32 kernels; dX 270 against 461, dW 330 against 367; a pass through forward and backward 1 061 -> 719 us.
+So the order of the instructions is written out
+(``interleave``): vector, LDS and memory instructions go between the matrix instructions that hide them; left to the compiler they
+clump, and registers spill.
+"""
+
+from __future__ import annotations
+
+from dataclasses import dataclass
+from typing import List
+
+from .common import Src
+from .lower import Lowered, Path, float_literal
+
+WAVES = 4
+# (part of A, part of B), smallest products first
+TERMS = ((2, 0), (0, 2), (1, 1), (1, 0), (0, 1), (0, 0))
+LDS_BUDGET = 160 * 1024 - 1024
+# Estimated registers up to which result blocks share a kernel: what compiles without scratch memory (512 registers
+# a lane; the estimates are up to 30 below what the compiler takes, and above it for dW).
+MAX_REGS, MAX_REGS_DW = 500, 430
+# Weight operands kept in accumulation registers: 256 less the results of four sub-paths, twice.
+PARKED = 216
+# Two waves per SIMD (256 registers): up to this estimate. 64x0e+16x1o (x) 0e+1o -> the same, 150 000 rows, one wave / two:
+# forward 52 / 40 us, dX 71 / 54, dW 69 / 61.
+TWO_WAVES = 300
+# Components of Y that dW reads from LDS ahead of their use.
+AHEAD = 4
+
+
+def c16(n: int) -> int:
+    return (n + 15) // 16
+
+
+def c32(n: int) -> int:
+    return (n + 31) // 32
+
+
+@dataclass
+class Sub:
+    """One channel v of a path's second operand: a mul1 x mul3 weight matrix."""
+    index: int
+    p: Path
+    v: int
+
+
+DEVICE = r"""
+typedef float oeq_f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float oeq_f2u __attribute__((ext_vector_type(2), aligned(4)));
+// a and b as sums of three bf16 numbers each (round to nearest; the remainders are exact in fp32); q<i> holds the i-th
+// parts, a's in the low half. A remainder is one dot product with (-1, 0) or (0, -1).
+OEQ_DEV void oeq_split3(float a, float b, unsigned& q0, unsigned& q1, unsigned& q2)
+{
+    unsigned l = 0x0000bf80u, h = 0xbf800000u;
+    asm("" : "+s"(l), "+s"(h));
+    const oeq_bf2 lo = __builtin_bit_cast(oeq_bf2, l), hi = __builtin_bit_cast(oeq_bf2, h);
+    const oeq_bf2 p0 = __builtin_convertvector((oeq_f2{a, b}), oeq_bf2);
+    a = __builtin_amdgcn_fdot2_f32_bf16(p0, lo, a, false);
+    b = __builtin_amdgcn_fdot2_f32_bf16(p0, hi, b, false);
+    const oeq_bf2 p1 = __builtin_convertvector((oeq_f2{a, b}), oeq_bf2);
+    a = __builtin_amdgcn_fdot2_f32_bf16(p1, lo, a, false);
+    b = __builtin_amdgcn_fdot2_f32_bf16(p1, hi, b, false);
+    const oeq_bf2 p2 = __builtin_convertvector((oeq_f2{a, b}), oeq_bf2);
+    q0 = __builtin_bit_cast(unsigned, p0), q1 = __builtin_bit_cast(unsigned, p1), q2 = __builtin_bit_cast(unsigned, p2);
+}
+// Component I of eight channels (or rows) as three bf16 operands: r[e * D + I], e = 0..7.
+template <int D, int I> OEQ_DEV void oeq_split8(const float (&r)[8 * D], oeq_bf8 (&f)[3])
+{
+    unsigned q[3][4];
+    #pragma unroll
+    for (int m = 0; m < 4; ++m) oeq_split3(r[2 * m * D + I], r[(2 * m + 1) * D + I], q[0][m], q[1][m], q[2][m]);
+    #pragma unroll
+    for (int c = 0; c < 3; ++c) f[c] = __builtin_bit_cast(oeq_bf8, oeq_u4{q[c][0], q[c][1], q[c][2], q[c][3]});
+}
+// The same four registers as accumulation registers.
+OEQ_DEV oeq_bf8 oeq_park(oeq_bf8 v)
+{
+    const oeq_u4 q = __builtin_bit_cast(oeq_u4, v);
+    oeq_u4 r;
+    #pragma unroll
+    for (int m = 0; m < 4; ++m) { unsigned t; asm("v_accvgpr_write_b32 %0, %1" : "=a"(t) : "v"(q[m])); r[m] = t; }
+    return __builtin_bit_cast(oeq_bf8, r);
+}
+OEQ_DEV void oeq_block_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+"""
+
+
+class SplitEmitter:
+    def __init__(self, low: Lowered):
+        self.low = low
+        self.subs: List[Sub] = []
+        for p in low.paths:
+            for v in range(low.in2[p.i2].mul):
+                self.subs.append(Sub(len(self.subs), p, v))
+
+    # ------------------------------------------------------------------ shared
+    def yat(self, sub: Sub, j: int) -> int:
+        b2 = self.low.in2[sub.p.i2]
+        return b2.off + sub.v * b2.d + j
+
+    def wpos(self, sub: Sub, u: str, w: str) -> str:
+        V, wtot = self.low.in2[sub.p.i2].mul, self.low.out[sub.p.io].mul
+        return f"{sub.p.woff + sub.v * wtot} + ({u}) * {V * wtot} + ({w})"
+
+    def lit(self, v):
+        return float_literal(v, "float")
+
+    def sides(self, kind: str):
+        """(blocks contracted over, blocks of the result tiles, their index in a sub-path)"""
+        low = self.low
+        if kind == "forward":
+            return low.in1, low.out, (lambda q: q.p.i1), (lambda q: q.p.io)
+        return low.out, low.in1, (lambda q: q.p.io), (lambda q: q.p.i1)
+
+    def cut(self, blocks, block_of, fits):
+        """Sub-paths by kernel: consecutive blocks that fit one together."""
+        kernels = []
+        for t in range(len(blocks)):
+            mine = [q for q in self.subs if block_of(q) == t]
+            if mine and kernels and fits(kernels[-1] + mine):
+                kernels[-1] += mine
+            elif mine:
+                kernels.append(mine)
+        return kernels
+
+    def plan(self, kind: str):
+        A, T, ia, it = self.sides(kind)
+        return self.cut(T, it, lambda subs: self.registers(kind, subs) <= MAX_REGS and self.lds(kind, subs) <= LDS_BUDGET)
+
+    def plan_dw(self):
+        return self.cut(self.low.out, lambda q: q.p.io,
+                        lambda subs: self.registers_dw(subs) <= MAX_REGS_DW and self.lds_dw(subs) <= LDS_BUDGET)
+
+    def registers(self, kind: str, subs) -> int:
+        """Estimate for a forward or dX kernel: weights, sums, Y, operands on their way from LDS, results, rows on
+        their way from memory; for dX also X (this tile's and the next one's) and dY."""
+        A, T, ia, it = self.sides(kind)
+        S = lambda q: c32(A[ia(q)].mul)
+        used_a, used_t = {ia(q) for q in subs}, {it(q) for q in subs}
+        tacc = 4 * sum(T[t].d for t in used_t)
+        most = max(sum(1 for q in subs if ia(q) == a) for a in used_a)
+        regs = 12 * sum(S(q) for q in subs) + tacc + 4 * self.low.L2 + 24 * max(S(q) for q in subs) + 8 * most + \
+            sum(2 * A[a].d * c32(A[a].mul) for a in used_a) + 32
+        if kind != "forward":
+            regs += 2 * tacc + 4 * self.low.L2
+        return regs
+
+    def lds(self, kind: str, subs) -> int:
+        A, T, ia, it = self.sides(kind)
+        frags = sum(A[a].d * c32(A[a].mul) for a in {ia(q) for q in subs})
+        return 2 * (3072 * frags + 64 * self.low.L2 * (1 if kind == "forward" else 5))
+
+    def share(self, kind: str) -> float:
+        """Of the multiplies of a pass, those with weights that are not padding (a wave's 16 result channels times four,
+        32 contracted channels at a time)."""
+        A, T, ia, it = self.sides(kind)
+        return sum(A[ia(q)].d * A[ia(q)].mul * T[it(q)].mul for q in self.subs) / \
+            sum(A[ia(q)].d * 32 * c32(A[ia(q)].mul) * 64 for q in self.subs)
+
+    def waves(self, kind: str) -> int:
+        """Waves per SIMD of the kernels of a role: two where the largest of them comes under 256 registers and half
+        the LDS."""
+        kinds = [kind] if kind == "forward" else ["dx", "dw"]
+        need = [(self.registers_dw(s), self.lds_dw(s)) if k == "dw" else (self.registers(k, s), self.lds(k, s))
+                for k in kinds for s in (self.plan_dw() if k == "dw" else self.plan(k))]
+        return 2 if all(r <= TWO_WAVES and 2 * m <= LDS_BUDGET for r, m in need) else 1
+
+    def supported(self, kind: str) -> bool:
+        """Whether these kernels are the ones to use for a role ('forward', or 'dx' for the whole backward pass).
+
+        Not for blocks of more than 64 channels, whose weights a wave's registers do not hold, nor where a tile would be mostly
+        padding. Two waves per SIMD: the share of real multiplies 0.28 (24 channels, l <= 1, 60 000 rows) forward 26 -> 15 us,
+        backward 67 -> 49; 0.1 (33 and 17 -> 15 and 7 channels) 23 -> 16 and 54 -> 46; 0.03 (8 channels) 15 -> 14 and
+        42 -> 44. One wave: 0.5 (32 channels, l <= 2) 95 -> 59 and 233 -> 161; 0.38 / 0.30 (40, 30 -> 50, 20, 10 channels) 43 ->
+        30 and 95 -> 99; 0.12 (16 channels, l <= 2) 57 -> 56 and 133 -> 158."""
+        low = self.low
+        if low.elem_size != 4 or any(low.in1[q.p.i1].mul > 64 or low.out[q.p.io].mul > 64 for q in self.subs):
+            return False
+        A, T, ia, it = self.sides(kind)
+        for subs in self.plan(kind):
+            # (two components at least: the pipeline over them has a step that writes LDS and one that reads it)
+            if self.registers(kind, subs) > MAX_REGS or self.lds(kind, subs) > LDS_BUDGET or \
+                    sum(A[a].d for a in {ia(q) for q in subs}) < 2:
+                return False
+        # (scalars alone: one component of dX for many of dZ, 64x0e -> 64x0e+32x1o+16x2e backward 78 -> 81 us)
+        if sum(low.in1[a].d for a in {q.p.i1 for q in self.subs}) < 2:
+            return False
+        if kind != "forward" and any(self.registers_dw(s) > MAX_REGS_DW or self.lds_dw(s) > LDS_BUDGET or
+                                     len(self.stages_dw(s)) < 2 for s in self.plan_dw()):
+            return False
+        least = 0.08 if self.waves(kind) == 2 else 0.35 if kind == "forward" else 0.45
+        return self.share(kind) >= least
+
+    def open_kernel(self, s: Src, name: str, sig: str, waves: int):
+        s.open(f'extern "C" __global__ __launch_bounds__({64 * WAVES}) '
+               f'__attribute__((amdgpu_waves_per_eu({waves}, {waves}))) void {name}{sig}')
+        s("const int lane = oeq_lane(), wave = oeq_wave(), l16 = lane & 15, lq = lane >> 4;")
+        s("(void)lane; (void)wave; (void)l16; (void)lq;")
+
+    # ------------------------------------------------------------- forward and dX
+    def weights(self, s: Src, kind: str, q: Sub, park: int = 0):
+        """B operands of a sub-path in registers: the lane's result channel 16 wave + lane % 16 and, of every 32
+        contracted channels, the eight from 8 (lane / 16) on; zeros past either block."""
+        A, T, ia, it = self.sides(kind)
+        a, t = A[ia(q)], T[it(q)]
+        ld = self.low.in2[q.p.i2].mul * self.low.out[q.p.io].mul
+        cu, ct = (ld, 1) if kind == "forward" else (1, ld)   # distance of two contracted / two result channels
+        base = q.p.woff + q.v * self.low.out[q.p.io].mul
+        S = c32(a.mul)
+        s(f"oeq_bf8 w{q.index}[{S}][3];")
+        s.open("")
+        s(f"const int t = min(16 * wave + l16, {t.mul - 1});")
+        for st in range(S):
+            s.open("")
+            s("float r[8];")
+            for e in range(8):
+                full = 32 * st + 32 <= a.mul
+                u = f"{32 * st + e} + 8 * lq"
+                val = f"W[{base} + ({u if full else f'min({u}, {a.mul - 1})'}) * {cu} + t * {ct}]"
+                conds = ([] if t.mul >= 64 else [f"16 * wave + l16 < {t.mul}"]) + ([] if full else [f"{u} < {a.mul}"])
+                s(f"r[{e}] = " + (f"oeq_sel({' && '.join(conds)}, {val});" if conds else f"{val};"))
+            s(f"oeq_split8<1, 0>(r, w{q.index}[{st}]);")
+            if park > 0:
+                s(f"for (int c = 0; c < 3; ++c) w{q.index}[{st}][c] = oeq_park(w{q.index}[{st}][c]);")
+            park -= 12
+            s("__builtin_amdgcn_sched_barrier(0);")
+            s.close()
+        s.close()
+
+    def rows_request(self, kind: str, a: int, st: int):
+        """ra<a>_<st>: two neighbouring channels of one of the tile's 16 rows, for the thread to split (in scope:
+        ``rows``, the tile's first row, and ``own``, the byte offset of the thread's row from there)."""
+        b = self.sides(kind)[0][a]
+        if b.mul % 2 == 0:
+            ch = f"2 * (tid & 15) * {b.d}"
+            if 32 * st + 32 > b.mul:
+                ch = f"min(2 * (tid & 15), {b.mul - 2 - 32 * st}) * {b.d}"
+            out = f"{{ const float* ap = oeq_at(rows + {b.off + 32 * st * b.d}, own + 4u * (unsigned)({ch})); "
+            for m in range(b.d):
+                out += f"{{ const oeq_f2u v = *(const oeq_f2u*)(ap + {2 * m}); ra{a}_{st}[{2 * m}] = v[0]; ra{a}_{st}[{2 * m + 1}] = v[1]; }} "
+            return [(3, out + "}")]
+        out = []
+        for e in range(2):
+            t = f"{{ const float* ap = oeq_at(rows + {b.off}, own + 4u * (unsigned)(min({32 * st + e} + 2 * (tid & 15), {b.mul - 1}) * {b.d})); "
+            out.append((3, t + " ".join(f"ra{a}_{st}[{e * b.d + i}] = ap[{i}];" for i in range(b.d)) + " }"))
+        return out
+
+    def rows_write(self, kind: str, a: int, st: int, at: int, buf: str):
+        """ra<a>_<st> as A operands: (part, lane, pair) at 16 bytes a lane. The lanes of a quarter are turned by four
+        times its number, so that a wave's stores fall into 64 banks."""
+        b = self.sides(kind)[0][a]
+        out = []
+        for i in range(b.d):
+            v = [f"ra{a}_{st}[{e * b.d + i}]" for e in range(2)]
+            if 32 * st + 32 > b.mul:
+                # channels past the block meet zero weights: zeros here too, not other channels' values
+                v = [f"oeq_sel({32 * st + e} + 2 * (tid & 15) < {b.mul}, {v[e]})" for e in range(2)]
+            out.append((10, f"{{ unsigned q0, q1, q2; oeq_split3({v[0]}, {v[1]}, q0, q1, q2); " +
+                        " ".join(f"{buf}[{at + 768 * i + 256 * c} + put] = q{c};" for c in range(3)) + " }"))
+        return out
+
+    @staticmethod
+    def put(s: Src, tasks):
+        for _, line in tasks:
+            s(line)
+
+    @staticmethod
+    def spread_reads(reads, tasks):
+        """``reads`` from LDS at equal distances among the first two thirds of ``tasks``: the four waves of a block come
+        to them together."""
+        out, total = [], sum(w for w, _ in tasks)
+        done, at = 0, 0
+        for t in tasks:
+            while at < len(reads) and done * len(reads) * 3 >= 2 * total * at:
+                out.append(reads[at])
+                at += 1
+            out.append(t)
+            done += t[0]
+        return out + reads[at:]
+
+    @staticmethod
+    def interleave(s: Src, lead, tasks):
+        """The matrix instructions ``lead`` with ``tasks`` (weight, line) shared out between them, in this order:
+        the wave issues in order, and what is issued while the matrix cores are at work costs nothing."""
+        total, done, at = sum(w for w, _ in tasks) or 1, 0, 0
+        for n, m in enumerate(lead):
+            s(m)
+            some = False
+            while at < len(tasks) and (done + tasks[at][0] / 2) * len(lead) <= total * (n + 1):
+                s(tasks[at][1])
+                done += tasks[at][0]
+                at += 1
+                some = True
+            if some:
+                s("__builtin_amdgcn_sched_barrier(0);")
+        for w, line in tasks[at:]:
+            s(line)
+        s("__builtin_amdgcn_sched_barrier(0);")
+
+    def emit_pass(self, s: Src, kind: str, name: str, sig: str):
+        names = []
+        for n, subs in enumerate(self.plan(kind)):
+            names.append(name if n == 0 else f"{name}_{n}")
+            self.emit_kernel(s, kind, names[-1], sig, subs, n)
+        return names
+
+    def emit_kernel(self, s: Src, kind: str, name: str, sig: str, subs, number: int):
+        low = self.low
+        A, T, ia, it = self.sides(kind)
+        L2, fwd = low.L2, kind == "forward"
+        dst, LT = ("L3_out", low.L3) if fwd else ("L1_grad", low.L1)
+        used_a, used_t = sorted({ia(q) for q in subs}), sorted({it(q) for q in subs})
+        at, total = {}, 0
+        for a in used_a:
+            for st in range(c32(A[a].mul)):
+                at[(a, st)] = total
+                total += 768 * A[a].d
+        self.open_kernel(s, name, sig, self.waves(kind))
+        s("const int tid = (int)threadIdx.x;")
+        s(f"__shared__ __attribute__((aligned(16))) unsigned s_a[2][{total}];")
+        s(f"__shared__ __attribute__((aligned(16))) float s_y[2][{L2}][16];")
+        if not fwd:
+            s(f"__shared__ float s_dy[2][{WAVES}][{16 * L2}];")
+        s("const i64 ntiles = (num_batch + 15) / 16;")
+        # where a thread's pair of channels goes within an operand, and where a lane's operand lies
+        s("const int put = 4 * (((tid & 15) >> 2) * 16 + (((tid >> 4) + 4 * ((tid & 15) >> 2)) & 15)) + (tid & 3);")
+        s("const int get = 4 * (lq * 16 + ((l16 + 4 * lq) & 15));")
+        park = PARKED if self.waves(kind) == 1 else 0
+        for q in subs:
+            self.weights(s, kind, q, park)
+            park -= 12 * c32(A[ia(q)].mul)
+        for a in used_a:
+            for st in range(c32(A[a].mul)):
+                s(f"float ra{a}_{st}[{2 * A[a].d}];")
+        ny = (16 * L2 + 255) // 256
+        s(f"float ry[{ny}];")
+
+        src, LA = ("L1_in", low.L1) if fwd else ("L3_grad", low.L3)
+
+        def where(tile, const="const "):
+            """Where the rows of ``tile`` lie; past the batch: its last row."""
+            s(f"{const}first = min(({tile}) * 16, num_batch - 1);")
+            s(f"{'const int ' if const else ''}end = (int)min((i64)15, num_batch - 1 - first);")
+
+        def request_y():
+            for n in range(ny):
+                v = f"min(tid + {256 * n}, {16 * L2 - 1})"
+                s(f"ry[{n}] = *oeq_at(L2_in + first * {L2}, 4u * (unsigned)(min({v} / {L2}, end) * {L2} + {v} % {L2}));")
+
+        # (threads past the tile repeat its last value: a store under a lane's condition makes the compiler wait for more
+        # than it has to afterwards)
+        def write_y(buf):
+            for n in range(ny):
+                v = f"min(tid + {256 * n}, {16 * L2 - 1})"
+                s(f"s_y[{buf}][{v} % {L2}][{v} / {L2}] = ry[{n}];")
+
+        def request_x(t):
+            b = T[t]
+            s("#pragma unroll")
+            s.open("for (int r = 0; r < 4; ++r)")
+            s(f"const float* xp = oeq_at(L1_in + first * {low.L1} + {b.off}, 4u * (unsigned)(min(4 * lq + r, end) * {low.L1} + ch{t} * {b.d}));")
+            for i in range(b.d):
+                s(f"xn{t}[{i}][r] = xp[{i}];")
+            s.close()
+
+        for t in used_t:
+            s(f"const int ch{t} = min(16 * wave + l16, {T[t].mul - 1});")
+            if not fwd:
+                s(f"v4t xn{t}[{T[t].d}];")
+        units = [(a, st) for a in used_a for st in range(c32(A[a].mul))]
+        s.open("")
+        where("(i64)blockIdx.x", "const i64 ")
+        s(f"const float* rows = {src} + first * {LA};")
+        s(f"const unsigned own = (unsigned)min(tid >> 4, end) * {4 * LA}u;")
+        for a, st in units:
+            self.put(s, self.rows_request(kind, a, st))
+        request_y()
+        if not fwd:
+            for t in used_t:
+                request_x(t)
+        for a, st in units:
+            self.put(s, self.rows_write(kind, a, st, at[(a, st)], "s_a[0]"))
+        write_y("0")
+        s.close()
+        s.open("")
+        where("((i64)blockIdx.x + gridDim.x)", "const i64 ")
+        s(f"const float* rows = {src} + first * {LA};")
+        s(f"const unsigned own = (unsigned)min(tid >> 4, end) * {4 * LA}u;")
+        for a, st in units:
+            self.put(s, self.rows_request(kind, a, st))
+        request_y()
+        s.close()
+        # Software pipeline over the components of the contracted rows, across tiles: while the matrix cores work on one,
+        # the lanes contract the results of the one before with the coupling coefficients, and its successor's operands
+        # are on their way from LDS. The last component of a tile is contracted, and its rows are stored, beside the first
+        # matrix instructions of the next.
+        steps = [(a, i) for a in sorted(used_a, key=lambda a: -A[a].d) for i in range(A[a].d)]
+        mine = {a: [q for q in subs if ia(q) == a] for a in used_a}
+        N = len(steps)
+
+        def fetch(n, buf="cur"):
+            a, i = steps[n]
+            return [(1, f"f{n}[{st}][{c}] = __builtin_bit_cast(oeq_bf8, *(const oeq_u4*)(s_a[{buf}] + "
+                        f"{at[(a, st)] + 768 * i + 256 * c} + get));") for st in range(c32(A[a].mul)) for c in range(3)]
+
+        def contract(n):
+            a, i = steps[n]
+            out = []
+            for q in mine[a]:
+                names = {}
+                for (i1, j, k, c) in q.p.nnz:
+                    if (i1 if fwd else k) != i:
+                        continue
+                    key = self.lit(abs(c))
+                    if key not in names:
+                        names[key] = f"m{n}_{q.index}_{len(names)}"
+                        out.append((4 if len(names) > 1 else 8, f"const v4t {names[key]} = {key} * P{n}_{q.index};"))
+                    op, yj = "-=" if c < 0 else "+=", self.yat(q, j)
+                    if fwd:
+                        out.append((4, f"acc{it(q)}[{k}] {op} y[{yj}] * {names[key]};"))
+                    else:
+                        out.append((4, f"acc{it(q)}[{i1}] {op} y[{yj}] * {names[key]};"))
+                        out.append((4, f"dy[{yj}] {op} x{it(q)}[{i1}] * {names[key]};"))
+            return out
+
+        def store(row0, end):
+            """Rows past the batch repeat its last one, in what was read and so in the results, and write it again: no
+            store hangs on a lane's row."""
+            out = []
+            for t in used_t:
+                for r in range(4):
+                    text = f"float* op = oeq_at({dst} + {row0} * {LT} + {T[t].off}, 4u * (unsigned)(min(4 * lq + {r}, {end}) * {LT} + ch{t} * {T[t].d})); " + \
+                        " ".join(f"__builtin_nontemporal_store((float)acc{t}[{k}][{r}], op + {k});" for k in range(T[t].d))
+                    out.append((6, (f"if (16 * wave + l16 < {T[t].mul}) " if T[t].mul < 64 else "") + "{ " + text + " }"))
+            return out
+
+        def lead(n):
+            a, i = steps[n]
+            out = []
+            for ca, cb in TERMS:
+                for st in range(c32(A[a].mul)):
+                    for q in mine[a]:
+                        out.append(f"P{n}_{q.index} = oeq_mfma_bf(f{n}[{st}][{ca}], w{q.index}[{st}][{cb}], P{n}_{q.index}, 0, 0, 0);")
+            return out
+
+        for n, (a, i) in enumerate(steps):
+            if n in (0, N - 1):
+                for q in mine[a]:
+                    s(f"v4t P{n}_{q.index} = v4t{{}};")
+        s(f"oeq_bf8 f0[{c32(A[steps[0][0]].mul)}][3];")
+        s(f"v4t y[{L2}];")
+        for j in range(L2):
+            s(f"y[{j}] = v4t{{}};")
+        for t in used_t:
+            s(f"v4t acc{t}[{T[t].d}];")
+            for k in range(T[t].d):
+                s(f"acc{t}[{k}] = v4t{{}};")
+            if not fwd:
+                s(f"v4t x{t}[{T[t].d}];")
+                for k in range(T[t].d):
+                    s(f"x{t}[{k}] = v4t{{}};")
+        if not fwd:
+            s(f"v4t dy[{L2}];")
+            for j in range(L2):
+                s(f"dy[{j}] = v4t{{}};")
+
+            # dY of a tile: the waves' shares, in wave order, on top of what an earlier kernel has left there. Read beside
+            # one step and added up beside a later one, each element by one thread: accesses of the threads past the
+            # tile are out of the buffer's range, and no branch cuts a step in two. Without a tile to finish, as at first,
+            # the block's own first tile is written as it is, or with what its sums replace when they are there.
+            def finish(buf):
+                s("const int fend = (int)min((i64)15, num_batch - 1 - frow0);")
+                s(f"const __amdgpu_buffer_rsrc_t dyr = __builtin_amdgcn_make_buffer_rsrc(L2_grad + frow0 * {L2}, 0, (fend + 1) * {4 * L2}, 0x00027000);")
+                s(f"float sdy[{ny}][4], ody[{ny}];")
+                take, give = [], []
+                for n in range(ny):
+                    v = f"(tid + {256 * n})"
+                    take.append((8, " ".join(f"sdy[{n}][{q}] = s_dy[{buf}][{q}][min({v}, {16 * L2 - 1})];" for q in range(4))
+                                 + (f" ody[{n}] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(dyr, 4 * {v}, 0, 0));" if number else "")))
+                    tot = f"((sdy[{n}][0] + sdy[{n}][1]) + sdy[{n}][2]) + sdy[{n}][3]"
+                    if number:
+                        tot = f"ody[{n}] + (ready ? {tot} : 0.0f)"
+                    give.append((8, f"__builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, {tot}), dyr, 4 * {v}, 0, 0);"))
+                return take, give
+        s("int cur = 0;")
+        s("i64 prow0 = (i64)blockIdx.x * 16;  // first row of the tile whose results are still to be stored")
+        s("oeq_block_sync();")
+        self.put(s, fetch(0))
+        s.open("for (i64 tile = blockIdx.x; tile < ntiles; tile += gridDim.x, cur ^= 1)")
+        s("const i64 row0 = tile * 16;")
+        # the tile whose rows are requested during this one
+        where("(tile + 2 * (i64)gridDim.x)", "const i64 ")
+        s(f"const float* rows = {src} + first * {LA};")
+        s(f"const unsigned own = (unsigned)min(tid >> 4, end) * {4 * LA}u;")
+        s("const int pend = (int)min((i64)15, num_batch - 1 - prow0);")
+        take = give = []
+        if not fwd:
+            # (two tiles back: its shares were written beside the first component of the tile before)
+            s("const bool ready = tile >= (i64)blockIdx.x + 2 * (i64)gridDim.x;")
+            s("const i64 frow0 = (ready ? tile - 2 * (i64)gridDim.x : (i64)blockIdx.x) * 16;")
+            take, give = finish("cur")
+        # the step that writes an operand of the next tile: not the first, which has the rows of the tile before to store,
+        # nor the last, which reads them
+        writer = lambda m: min(1 + m * max(1, N - 4) // len(units), N - 2) if N > 2 else 0
+        for n, (a, i) in enumerate(steps):
+            tasks, reads = [], []
+            if n + 1 < N:
+                s(f"oeq_bf8 f{n + 1}[{c32(A[steps[n + 1][0]].mul)}][3];")
+                reads = fetch(n + 1)
+            # a share of the next tile's operands, and of the requests for the one after
+            for ua, ust in (units[m] for m in range(len(units)) if writer(m) == n):
+                tasks += self.rows_write(kind, ua, ust, at[(ua, ust)], "s_a[cur ^ 1]")
+                tasks += self.rows_request(kind, ua, ust)
+            tasks += contract((n or N) - 1)
+            if n == min(1, N - 1):
+                tasks += take
+            if n == N - 1:
+                tasks += give
+            if n == N - 1:
+                s("oeq_block_sync();  // the next tile's operands are written, this tile's are read")
+                reads = fetch(0, "cur ^ 1")
+            tasks = self.spread_reads(reads, tasks)
+            if n not in (0, N - 1):
+                for q in mine[a]:
+                    s(f"v4t P{n}_{q.index};")
+            pre = [f"P{n}_{q.index} = v4t{{}};" for q in mine[a]]
+            for line in pre:
+                s(line)
+            s("__builtin_amdgcn_sched_barrier(0);")
+            if n == 0:
+                half = lead(0)
+                cut = len(half) // 2
+                self.interleave(s, half[:cut], tasks)
+                tasks = store("prow0", "pend")
+                tasks += [(1, f"y[{j}] = *(const v4t*)&s_y[cur][{j}][4 * lq];") for j in range(L2)]
+                self.interleave(s, half[cut:], tasks)
+                if not fwd:
+                    self.reduce_dy(s, "s_dy[cur ^ 1]")
+                    for j in range(L2):
+                        s(f"dy[{j}] = v4t{{}};")
+                for t in used_t:
+                    for k in range(T[t].d):
+                        s(f"acc{t}[{k}] = v4t{{}};")
+                        if not fwd:
+                            s(f"x{t}[{k}] = xn{t}[{k}];")
+                if not fwd:
+                    s.open("")
+                    where("(tile + gridDim.x)", "const i64 ")
+                    for t in used_t:
+                        request_x(t)
+                    s.close()
+                write_y("cur ^ 1")
+                request_y()
+            else:
+                self.interleave(s, lead(n), tasks)
+        s("prow0 = row0;")
+        if number == 0:
+            for t in range(len(T)):
+                if not any(it(q) == t for q in self.subs):
+                    s.open(f"for (int z = tid; z < {16 * T[t].mul * T[t].d}; z += 256)")
+                    s(f"const i64 row = row0 + z / {T[t].mul * T[t].d};")
+                    s(f"if (row < num_batch) {dst}[row * {LT} + {T[t].off} + z % {T[t].mul * T[t].d}] = 0.0f;")
+                    s.close()
+        s.close()
+        s("const int pend = (int)min((i64)15, num_batch - 1 - prow0);")
+        self.put(s, contract(N - 1))
+        self.put(s, store("prow0", "pend"))
+        if not fwd:
+            self.reduce_dy(s, "s_dy[cur ^ 1]")
+            s("const i64 tiles_here = (ntiles - 1 - blockIdx.x) / gridDim.x + 1;")
+            s("oeq_block_sync();")
+            s("const bool ready = true;")
+            for back, buf in ((2, "cur"), (1, "cur ^ 1")):
+                s.open(f"if (tiles_here >= {back})")
+                s(f"const i64 frow0 = ((i64)blockIdx.x + (tiles_here - {back}) * gridDim.x) * 16;")
+                for part in finish(buf):
+                    self.put(s, part)
+                s.close()
+        s.close()
+
+    def reduce_dy(self, s: Src, into: str):
+        """Sum over the 16 lanes that hold a row's channels; a lane is left with n / 16 consecutive values of the
+        4 x L2 its group of lanes holds, which lie one after the other in memory, too."""
+        L2 = self.low.L2
+        n = 4 * L2
+        cur = (n + 15) // 16 * 16
+        s.open("")
+        s(f"float rv[{cur}];")
+        for o in range(cur):
+            s(f"rv[{o}] = {f'dy[{o % L2}][{o // L2}]' if o < n else '0.0f'};")
+        s("int at = 0;")
+        for ctrl, bit in (("0x140", 8), ("0x141", 4), ("0x1B", 2), ("0xB1", 1)):
+            half = cur // 2
+            s.open("")
+            s(f"const bool hi = (l16 & {bit}) != 0;")
+            for j in range(half):
+                s(f"{{ const float keep = hi ? rv[{j + half}] : rv[{j}]; const float send = hi ? rv[{j}] : rv[{j + half}]; "
+                  f"rv[{j}] = keep + oeq_dpp<{ctrl}>(send); }}")
+            s(f"at += hi ? {half} : 0;")
+            s.close()
+            cur = half
+        for t in range(cur):
+            s(f"if (at + {t} < {n}) {into}[wave][4 * lq * {L2} + at + {t}] = rv[{t}];")
+        s.close()
+
+    # ------------------------------------------------------------------------ dW
+    def split_dw(self, subs):
+        """(waves along the input channels, waves along the output channels, 16-channel tiles of a sub-path's outputs
+        that a wave sums)"""
+        most = max(c16(self.low.in1[q.p.i1].mul) for q in subs)
+        wu = 4 if most > 2 else most
+        return wu, 4 // wu, lambda q: (c16(self.low.out[q.p.io].mul) + 4 // wu - 1) // (4 // wu)
+
+    def registers_dw(self, subs) -> int:
+        low = self.low
+        _, _, per = self.split_dw(subs)
+        into = max(sum(4 * per(q) for q in subs if q.p.io == o) for o in {q.p.io for q in subs})
+        x = 8 * sum(low.in1[a].d for a in {q.p.i1 for q in subs})
+        g = 8 * sum(low.out[o].d for o in {q.p.io for q in subs})
+        return 4 * sum(per(q) for q in subs) + into + x + 16 + max(x, g) + 18 * max(per(q) for q in subs) + 32 + 32
+
+    def lds_dw(self, subs) -> int:
+        low = self.low
+        return 2 * (3072 * sum(low.out[o].d * c16(low.out[o].mul) for o in {q.p.io for q in subs}) + 128 * low.L2)
+
+    def stages_dw(self, subs):
+        """(output block, component, sub-path), in the order in which they are multiplied."""
+        out = self.low.out
+        return [(o, k, q) for o in sorted({q.p.io for q in subs}, key=lambda o: -out[o].d) for k in range(out[o].d)
+                for q in subs if q.p.io == o and any(kk == k for _, _, kk, _ in q.p.nnz)]
+
+    def emit_dw(self, s: Src, name: str, sig: str):
+        names = []
+        for n, subs in enumerate(self.plan_dw()):
+            names.append(name if n == 0 else f"{name}_{n}")
+            self.emit_dw_kernel(s, names[-1], sig, subs)
+        return names
+
+    def emit_dw_kernel(self, s: Src, name: str, sig: str, subs):
+        low = self.low
+        L2 = low.L2
+        WU, WW, per = self.split_dw(subs)
+        used_a, used_o = sorted({q.p.i1 for q in subs}), sorted({q.p.io for q in subs}, key=lambda o: -low.out[o].d)
+        where, total = {}, 0
+        for o in used_o:
+            for k in range(low.out[o].d):
+                where[(o, k)] = total
+                total += 768 * c16(low.out[o].mul)
+        self.open_kernel(s, name, sig, self.waves("dw"))
+        s("const int tid = (int)threadIdx.x;")
+        s(f"__shared__ __attribute__((aligned(16))) unsigned s_g[2][{total}];")
+        s(f"__shared__ __attribute__((aligned(16))) float s_y[2][{L2}][32];")
+        s(f"const int wu = wave % {WU}, ww = wave / {WU};")
+        s("(void)ww;")
+        # rows of the identity: a product with them adds a tile of sums to another one, rounding to nearest
+        s("const float sign = (blockIdx.x & 1) ? -1.0f : 1.0f;")
+        s("float eye[4];")
+        s("for (int i = 0; i < 4; ++i) eye[i] = l16 == 4 * lq + i ? sign : 0.0f;")
+        for q in subs:
+            s(f"v4t dw{q.index}[{per(q)}];")
+            for j in range(per(q)):
+                s(f"dw{q.index}[{j}] = v4t{{}};")
+        for o in used_o:
+            s(f"float g{o}[{8 * low.out[o].d}];")
+            s(f"const int gc{o} = min(16 * wave + l16, {low.out[o].mul - 1});")
+        for a in used_a:
+            s(f"float x{a}[8][{low.in1[a].d}], xn{a}[8][{low.in1[a].d}];")
+            s(f"const int xc{a} = min(16 * wu + l16, {low.in1[a].mul - 1});")
+        s(f"v4t yv[{AHEAD + 1}][2];  // a component of Y for the lane's eight rows, and the next ones")
+        ny = (32 * L2 + 255) // 256
+        s(f"float ry[{ny}];")
+        s("const i64 nsteps = (num_batch + 31) / 32;")
+
+        def rows_of(step):
+            s(f"const i64 first = min((i64)({step}) * 32, num_batch - 1);")
+            s("const int end = (int)min((i64)31, num_batch - 1 - first);")
+
+        def request_g(o, e):
+            b = low.out[o]
+            return [(4, f"{{ const float* gp = oeq_at(L3_grad + first * {low.L3} + {b.off}, 4u * (unsigned)(min(8 * lq + {e}, end) * {low.L3} + gc{o} * {b.d})); "
+                     + " ".join(f"g{o}[{e * b.d + k}] = gp[{k}];" for k in range(b.d)) + " }")]
+
+        def request_x(a, e):
+            b = low.in1[a]
+            return [(4, f"{{ const float* xp = oeq_at(L1_in + first * {low.L1} + {b.off}, 4u * (unsigned)(min(8 * lq + {e}, end) * {low.L1} + xc{a} * {b.d})); "
+                     + " ".join(f"xn{a}[{e}][{i}] = xp[{i}];" for i in range(b.d)) + " }")]
+
+        def request_y():
+            return [(4, f"ry[{n}] = *oeq_at(L2_in + first * {L2}, 4u * (unsigned)min(min(tid + {256 * n}, {32 * L2 - 1}), end * {L2} + {L2 - 1}));")
+                    for n in range(ny)]
+
+        def write_y(buf):
+            v = [f"min(tid + {256 * n}, {32 * L2 - 1})" for n in range(ny)]
+            return [(5, f"s_y[{buf}][{v[n]} % {L2}][{v[n]} / {L2}] = sign * ry[{n}];") for n in range(ny)]
+
+        def write_g(o, buf, n):
+            """dZ of the wave's columns of a block, zero past the batch (``n``: rows there are), as operands."""
+            b = low.out[o]
+            out = []
+            for k in range(b.d):
+                text = f"{{ float v[8]; " + " ".join(f"v[{e}] = oeq_sel({e} + 8 * lq < {n}, g{o}[{e * b.d + k}]);" for e in range(8)) + \
+                    " oeq_bf8 f[3]; oeq_split8<1, 0>(v, f); " + \
+                    " ".join(f"*(oeq_u4*)({buf} + {where[(o, k)] + 256 * c} + 768 * wave + 4 * lane) = __builtin_bit_cast(oeq_u4, f[{c}]);"
+                             for c in range(3)) + " }"
+                out.append((44, (f"if (16 * wave < {16 * c16(b.mul)}) " if b.mul <= 48 else "") + text))
+            return out
+
+        stages = self.stages_dw(subs)
+        first_k = {q.index: min(k for _, _, k, _ in q.p.nnz) for q in subs}
+        last_k = {q.index: max(k for _, _, k, _ in q.p.nnz) for q in subs}
+        N = len(stages)
+
+        # (stage, component of Y) in the order in which stages 1 .. N - 1 are contracted, and the first one's
+        js_of = lambda n: sorted({j for (_, j, kk, _) in stages[n % N][2].p.nnz if kk == stages[n % N][1]})
+        later = [(n, j) for n in range(1, N) for j in js_of(n)]
+        
+        def read_y(units, u, buf):
+            if u >= len(units):
+                return []
+            n, j = units[u]
+            row = f"{buf}[{self.yat(stages[n % N][2], j)}]"
+            return [(2, f"yv[{u % (AHEAD + 1)}][0] = *(const v4t*)&{row}[8 * lq]; "
+                        f"yv[{u % (AHEAD + 1)}][1] = *(const v4t*)&{row}[8 * lq + 4];")]
+
+        def t_tasks(n):
+            """The contraction of X and Y for stage n, eight rows a lane, as operands. Y comes from LDS, component by
+            component, two ahead of the sums."""
+            o, k, q = stages[n % N]
+            buf = "s_y[cur]" if n < N else "s_y[cur ^ 1]"
+            units = later if n % N else [(0, j) for j in js_of(0)]
+            out, first = [], True
+            for u, (m, j) in enumerate(units):
+                if m != n % N:
+                    continue
+                if u == 0:
+                    for v in range(AHEAD):
+                        out += read_y(units, v, buf)
+                out += read_y(units, u + AHEAD, buf)
+                for i, jj, kk, c in q.p.nnz:
+                    if (jj, kk) != (j, k):
+                        continue
+                    for h in range(2):
+                        out.append((8, " ".join(f"t[{4 * h + r}] {'=' if first else '+='} ({self.lit(c)} * yv[{u % (AHEAD + 1)}][{h}][{r}]) * "
+                                                f"x{q.p.i1}[{4 * h + r}][{i}];" for r in range(4))))
+                    first = False
+            return out + [(28, f"oeq_split8<1, 0>(t, ta[{n % 2}]);")]
+
+        def read_bg(n, pair, buf):
+            o, k, q = stages[n % N]
+            out = []
+            for j in pair:
+                nt = f"{j}" if WW == 1 else f"min(ww + {j * WW}, {c16(low.out[o].mul) - 1})"
+                for c in range(3):
+                    out.append((1, f"bg[{j}][{c}] = __builtin_bit_cast(oeq_bf8, *(const oeq_u4*)({buf} + {where[(o, k)] + 256 * c} + 768 * ({nt}) + 4 * lane));"))
+            return out
+
+        most = max(per(q) for q in subs)
+        pairs = lambda q: [list(range(j, min(j + 2, per(q)))) for j in range(0, per(q), 2)]
+
+        def lead(n, pair):
+            o, k, q = stages[n]
+            return [f"tm{q.index}[{j}] = oeq_mfma_bf(ta[{n % 2}][{ca}], bg[{j}][{cb}], tm{q.index}[{j}], 0, 0, 0);"
+                    for ca, cb in TERMS for j in pair]
+
+        # ---- the first step's operands
+        s("float t[8];")
+        s("oeq_bf8 ta[2][3];")
+        s(f"oeq_bf8 bg[{most}][3];")
+        for q in subs:
+            s(f"v4t tm{q.index}[{per(q)}];")
+        s.open("")
+        rows_of("blockIdx.x")
+        for o in used_o:
+            for e in range(8):
+                self.put(s, request_g(o, e))
+        for a in used_a:
+            for e in range(8):
+                self.put(s, request_x(a, e))
+        self.put(s, request_y())
+        s("const int rows = (int)min((i64)32, num_batch - (i64)blockIdx.x * 32);")
+        for o in used_o:
+            self.put(s, write_g(o, "s_g[0]", "rows"))
+        self.put(s, write_y("0"))
+        s.close()
+        for a in used_a:
+            for e in range(8):
+                for i in range(low.in1[a].d):
+                    s(f"x{a}[{e}][{i}] = xn{a}[{e}][{i}];")
+        s("int cur = 0;")
+        s("oeq_block_sync();")
+        self.put(s, t_tasks(0))
+        self.put(s, read_bg(0, pairs(stages[0][2])[0], "s_g[0]"))
+        s.open("for (i64 step = blockIdx.x; step < nsteps; step += gridDim.x, cur ^= 1)")
+        # the step whose rows are requested, and written to LDS, during this one
+        rows_of("step + gridDim.x")
+        s("const int rows = (int)max((i64)0, min((i64)32, num_batch - (step + (i64)gridDim.x) * 32));")
+        pending = []   # sums to be flushed beside a later stage's products
+        g_req = [t for o in used_o for e in range(8) for t in request_g(o, e)] + request_y()
+        g_put = [t for o in used_o for t in write_g(o, "s_g[cur ^ 1]", "rows")] + write_y("cur ^ 1")
+        x_req = [t for a in used_a for e in range(8) for t in request_x(a, e)]
+        # (stages over which these are spread: X is requested when dZ has left the registers)
+        spread = lambda items, n, lo, hi: items[max(0, n - lo) * len(items) // (hi - lo):(n + 1 - lo) * len(items) // (hi - lo)] \
+            if lo <= n < hi else []
+        req_end = max(1, 3 * N // 20)
+        put_from = min(max(req_end, 3 * N // 5), N - 2)
+        put_end = min(max(put_from + 1, 9 * N // 10), N - 1)
+        for n, (o, k, q) in enumerate(stages):
+            tasks = []
+            tasks += spread(g_req, n, 0, req_end) + spread(g_put, n, put_from, put_end) + spread(x_req, n, put_from, put_end)
+            if k == first_k[q.index]:
+                for j in range(per(q)):
+                    s(f"tm{q.index}[{j}] = v4t{{}};")
+            new_group = n + 1 == N or stages[n + 1][:2] != stages[n][:2]
+            group_start = n == 0 or stages[n - 1][:2] != stages[n][:2]
+            ps = pairs(q)
+            buf, nbuf = "s_g[cur]", "s_g[cur]" if n + 1 < N else "s_g[cur ^ 1]"
+            if n + 1 == N:
+                if group_start:
+                    # (read before the barrier: past it, other waves write over this step's operands)
+                    for pair in ps[1:]:
+                        self.put(s, read_bg(n, pair, buf))
+                s("oeq_block_sync();  // the next step's operands are written, this one's are read")
+                tasks += [(1, " ".join(f"x{a}[{e}][{i}] = xn{a}[{e}][{i}];" for i in range(low.in1[a].d)))
+                          for a in used_a for e in range(8)]
+            tasks += t_tasks(n + 1)
+            flush = [f"dw{p.index}[{j}] = oeq_mfma(eye[{i}], tm{p.index}[{j}][{i}], dw{p.index}[{j}], 0, 0, 0);"
+                     for p in pending for i in range(4) for j in range(per(p))]
+            pending = [q] if k == last_k[q.index] else []
+            seq = [lead(n, pair) for pair in ps]
+            # operands of this group that are not there yet (its second half), and the next group's first half once
+            # this stage is done with its own
+            weight = sum(w for w, _ in tasks)
+            cut = [[] for _ in seq]
+            at = 0
+            for m in range(len(seq)):
+                acc = 0
+                while at < len(tasks) and (m + 1 == len(seq) or acc + tasks[at][0] / 2 < weight / len(seq)):
+                    cut[m].append(tasks[at])
+                    acc += tasks[at][0]
+                    at += 1
+            for m in range(len(seq)):
+                extra = []
+                if group_start and m + 1 < len(ps) and n + 1 < N:
+                    extra = read_bg(n, ps[m + 1], buf)
+                if new_group and m > 0 and m == len(ps) - 1:
+                    extra = extra + read_bg(n + 1, pairs(stages[(n + 1) % N][2])[0], nbuf)
+                self.interleave(s, seq[m] + (flush if m + 1 == len(seq) else []), extra + cut[m])
+            if new_group and len(ps) == 1:
+                self.put(s, read_bg(n + 1, pairs(stages[(n + 1) % N][2])[0], nbuf))
+            if n + 1 == N:
+                for p in pending:
+                    for i in range(4):
+                        for j in range(per(p)):
+                            s(f"dw{p.index}[{j}] = oeq_mfma(eye[{i}], tm{p.index}[{j}][{i}], dw{p.index}[{j}], 0, 0, 0);")
+                if N % 2:
+                    s("for (int c = 0; c < 3; ++c) ta[0][c] = ta[1][c];")
+        s.close()
+        s(f"float* prow = wpartial + (i64)blockIdx.x * {low.WN};")
+        for q in subs:
+            U, Wn = low.in1[q.p.i1].mul, low.out[q.p.io].mul
+            for j in range(per(q)):
+                s("#pragma unroll")
+                s.open("for (int i = 0; i < 4; ++i)")
+                nt = f"{j}" if WW == 1 else f"(ww + {j * WW})"
+                s(f"const int u = 16 * wu + 4 * lq + i, w = 16 * {nt} + l16;")
+                s(f"if (u < {U} && w < {Wn}) prow[{self.wpos(q, 'u', 'w')}] = dw{q.index}[{j}][i];")
+                s.close()
+        s.close()

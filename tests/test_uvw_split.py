@@ -1,0 +1,106 @@
+"""Split-operand matrix kernels of shared-weight 'uvw' products (codegen/uvw_split.py): which problems they take, that their
+kernels cover every sub-path once, and their results at tile, step and grid boundaries against the float64 oracle."""
+
+import numpy as np
+import pytest
+import torch
+
+import openequivariance_amd as oeq
+from openequivariance_amd._torch.tensor_product import build_tp_module
+from openequivariance_amd.codegen.lower import lower
+from openequivariance_amd.codegen.uvw_split import SplitEmitter
+from openequivariance_amd.core import problems as P
+from oracle import e3nn_ref as R
+
+
+def _shared(in1, in2, out, dtype=np.float32):
+    return P.FullyConnectedTPProblem(in1, in2, out, shared_weights=True, internal_weights=False, label="split",
+                                     irrep_dtype=dtype, weight_dtype=dtype)
+
+
+def _gaps():  # an input irrep that no path reads, an output irrep that no path writes
+    return oeq.TPProblem("32x0e+48x1o+20x2e", "1x0e+1x1o", "32x0e+16x1e+64x1o",
+                         [(0, 0, 0, "uvw", True), (0, 1, 2, "uvw", True), (1, 0, 2, "uvw", True, 0.6),
+                          (1, 1, 0, "uvw", True)], shared_weights=True, internal_weights=False, label="split-gaps")
+
+
+# (name, problem, waves per SIMD of forward and backward)
+CASES = [
+    ("l2-64", P.config4_uvw_shared, 1, 1),
+    ("l2-32", lambda: _shared("32x0e+32x1o+32x2e", "1x0e+1x1o+1x2e", "32x0e+32x1o+32x2e"), 1, 1),
+    ("l1-64-16", lambda: _shared("64x0e+16x1o", "1x0e+1x1o", "64x0e+16x1o"), 2, 2),
+    ("odd-channels", lambda: _shared("33x0e+17x1o", "1x0e+1x1o", "15x0e+7x1o"), 2, 2),
+    ("two-channel-second-operand", lambda: _shared("64x0e+32x1o", "3x0e+2x1o", "64x0e+32x1o"), 1, 1),
+    ("gaps", _gaps, 2, 1),
+]
+
+
+@pytest.mark.parametrize("name,make,wf,wb", CASES, ids=[c[0] for c in CASES])
+def test_plan_covers_every_sub_path_once(name, make, wf, wb):
+    low = lower(make())
+    em = SplitEmitter(low)
+    assert em.supported("forward") and em.supported("dx")
+    assert (em.waves("forward"), em.waves("dx")) == (wf, wb)
+    for plan in (em.plan("forward"), em.plan("dx"), em.plan_dw()):
+        assert sorted(q.index for subs in plan for q in subs) == list(range(len(em.subs)))
+    for subs in em.plan_dw():
+        stages = em.stages_dw(subs)
+        assert {q.index for _, _, q in stages} == {q.index for q in subs}
+        assert all(any(k == kk for _, _, kk, _ in q.p.nnz) for _, k, q in stages)
+    src, _, descs = build_tp_module(make())
+    assert "oeq_split3(" in src and any(d[1] == "backward_w" for d in descs)
+
+
+def test_takes_only_what_it_is_made_for():
+    for problem in (_shared("64x0e+64x1o", "1x0e+1x1o", "64x0e+64x1o", np.float64),   # fp64
+                    _shared("128x0e+128x1o", "1x0e+1x1o", "64x0e+64x1o"),             # blocks of more than 64 channels
+                    _shared("8x0e+8x1o", "1x0e+1x1o", "8x0e+8x1o"),                   # tiles that are mostly padding
+                    _shared("64x0e", "1x0e", "64x0e")):                               # a single component
+        em = SplitEmitter(lower(problem))
+        assert not em.supported("forward") and not em.supported("dx")
+        assert "oeq_split3(" not in build_tp_module(problem)[0]
+
+
+# A result is a sum of at most some thirty roundings of 2^-24 of its size, or a sum over rows that are as near: 2-norm.
+TOL = 16 * 2.0 ** -24
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,make,wf,wb", CASES, ids=[c[0] for c in CASES])
+def test_boundaries_match_oracle(name, make, wf, wb):
+    """1 to 33 rows: below, at and past a tile of 16 and a step of 32. Then three tiles for some blocks and two for the
+    others, and a last tile of five rows; there the output gradient is zero but at rows where mistakes would hide, so that
+    the oracle's weight gradient needs these rows only."""
+    from openequivariance_amd._torch import ops
+    problem = make()
+    ref = R.Problem.from_spec(problem)
+    tp = oeq.TensorProduct(problem)
+    for B in (1, 15, 16, 17, 31, 32, 33, 16 * 256 * max(wf, wb) * 2 + 21):
+        gen = torch.Generator(device="cuda").manual_seed(B)
+        x, y, g = (torch.randn(B, d, device="cuda", generator=gen)
+                   for d in (problem.irreps_in1.dim, problem.irreps_in2.dim, problem.irreps_out.dim))
+        w = torch.randn(problem.weight_numel, device="cuda", generator=gen)
+        at = sorted({r for r in (0, 15, 16, 31, 32, 4095, 4096, 4111, 8191, 8192, B // 2, B - 21, B - 6, B - 5, B - 1)
+                     if 0 <= r < B}) if B > 33 else list(range(B))
+        if B > 33:
+            keep = torch.zeros(B, 1, device="cuda")
+            keep[at] = 1.0
+            g *= keep
+        z = ops.tp_forward(x, y, w, tp.kid)
+        dx, dy, dw = ops.tp_backward(x, y, w, g, tp.kid)
+        xs, ys, gs = (t[at].cpu().numpy() for t in (x, y, g))
+        want = (R.tp_forward(ref, xs, ys, w.cpu().numpy()), *R.tp_backward(ref, xs, ys, w.cpu().numpy(), gs))
+        for got, exact in zip((z[at], dx[at], dy[at], dw), want):
+            off = np.linalg.norm(got.cpu().numpy().astype(np.float64) - exact) / np.linalg.norm(exact)
+            assert off <= TOL, (name, B, off)
+        if B > 33:
+            assert not (dx * (1 - keep)).any() and not (dy * (1 - keep)).any()
+        again = ops.tp_backward(x, y, w, g, tp.kid)
+        assert all(torch.equal(a, b) for a, b in zip((dx, dy, dw), again))
+    # an infinity and a NaN stay in their rows
+    x[3, 0], x[20, 1] = float("inf"), float("nan")
+    z2 = ops.tp_forward(x, y, w, tp.kid)
+    rows = torch.arange(len(z2), device="cuda")
+    assert not torch.isfinite(z2[3]).all() and not torch.isfinite(z2[20]).all()
+    clean = (rows != 3) & (rows != 20)
+    assert torch.equal(z2[clean], z[clean])
