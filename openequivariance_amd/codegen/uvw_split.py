@@ -6,13 +6,16 @@ fp32; a remainder is exact), and a product the six cross products of weight 2^-1
 ``v_mfma_f32_16x16x32_bf16``: 6 x 16 cycles for what takes the fp32 instruction 8 x 32. What is dropped is 2^-26 of a
 product, and 32 products are summed before they are rounded, so the results are nearer to 64 bits than those of the
 fp32 instruction. 64x{0e,1o,2e} (x) {0e,1o,2e} -> the same, relative errors of Z, dX, dY, dW at 100 003 rows, before
-and now: 2.9e-7, 1.6e-7, 1.7e-7, 5.4e-7 and 0.75e-7, 0.8e-7, 1.0e-7, 2.3e-7. An infinity in an operand gives NaN.
+and now: 2.9e-7, 1.6e-7, 1.7e-7, 5.4e-7 and 0.75e-7, 0.8e-7, 1.0e-7, 1.7e-7. An infinity in an operand gives NaN.
 
 Where the fp32 kernels (``uvw_mfma.py``) contract with the coupling coefficients first and multiply the result, forward and dX
 multiply first: the matrix cores form W^T x (or W dZ) component by component, the lanes contract what comes out. The
 operand that is split, written to LDS and read by every wave is then a row as it lies in memory - 9 components per channel
 at l <= 2, where the contraction of 11 paths has 35 - so that a tile's operands are prepared once, and X and dZ are read
-once per kernel.
+once per kernel. The exception are paths whose other side has a single component, l x l -> 0 in the forward and 0 x l -> l in
+dW (there the output gradient's side): contracted on the way to LDS they are one product, not 2 l + 1 (``folds``; 35 -> 29
+products each; forward 182 -> 175 us, dW 332 -> 318). dX has no such path, since dY needs every component of W dZ. The most
+frequent coefficient of a path is a factor of its weights (``Sub.unit``).
 
 * Forward, dX: a block of 4 waves owns 16 rows at a time; wave w result channels 16 w .. 16 w + 15, with the weights
   of all sub-paths of the kernel in registers. The threads split the next tile's rows into LDS (two copies) while
@@ -23,20 +26,23 @@ once per kernel.
   and then added to the running sums by fp32 matrix instructions with the identity. The bf16 instruction cuts off what it aligns,
   always downwards, and running sums of 12 steps drift by that: every second block works on negated values,
   which the identity (with the same sign) turns back (dW above: 1.5e-6 on the running sums directly, 5.4e-7 from zero, 2.3e-7
-  with the signs).
+  with the signs, 1.7e-7 with the folds). Y lies in LDS times the coefficients it is met with, as zeros past the batch.
 
 What bounds them (MI355X, the problem above, 100 003 rows): the registers of a SIMD hold one wave of these kernels, and
-a wave issues one instruction in about 2.1 ns, a matrix instruction takes 8 (less, and at a higher clock, where the data are
-zeros: random operands cost 20 % of the clock): forward 420 matrix and 1 060 other instructions a tile, 165 us at 100 003 rows
-against 328 us for the fp32 kernels; dX 270 against 461, dW 330 against 367; a pass through forward and backward 1 061 -> 719 us.
-So the order of the instructions is written out
-(``interleave``): vector, LDS and memory instructions go between the matrix instructions that hide them; left to the compiler they
-clump, and registers spill.
+a wave issues an instruction in 2.1 ns, one that needs the result before it in 3.6, a matrix instruction takes 8. Counters of
+the forward: of 100 wave cycles 48 issue, 33 wait to issue, 19 wait for memory or LDS; matrix cores busy 54. Run back to back the
+kernels are also bound by power: random operands lower the clock (2.1 GHz, 2.4 on zeros), fewer matrix instructions raise it.
+So the order of the instructions is written out (``interleave``): vector, LDS and memory instructions go between the matrix
+instructions that hide them, and what takes several is cut in steps (a split of eight values as one piece: 714 us for a pass through
+forward and backward, in steps 695); left to the compiler they clump, and registers spill. The pass: fp32 kernels
+1 066 us, these 719 with 35 products each and without the steps, 683 now.
 """
 
 from __future__ import annotations
 
+from collections import Counter
 from dataclasses import dataclass
+from functools import cached_property
 from typing import List
 
 from .common import Src
@@ -73,6 +79,21 @@ class Sub:
     p: Path
     v: int
 
+    @property
+    def key(self):
+        return ("fold", self.index)
+
+    @cached_property
+    def unit(self) -> float:
+        """The magnitude that most coefficients of the path have (one coefficient in seven of the eleven paths up to
+        l = 2): a factor of the weights, before they are split, or of their gradient, after the sums."""
+        sizes = Counter(f"{abs(c):.12g}" for *_, c in self.p.nnz)
+        most = max(sizes.values())
+        return next(abs(c) for *_, c in self.p.nnz if sizes[f"{abs(c):.12g}"] == most)
+
+    def ratio(self, c: float) -> float:
+        return float(f"{abs(c) / self.unit:.12g}")
+
 
 DEVICE = r"""
 typedef float oeq_f4u __attribute__((ext_vector_type(4), aligned(4)));
@@ -93,6 +114,21 @@ OEQ_DEV void oeq_split3(float a, float b, unsigned& q0, unsigned& q1, unsigned& 
     const oeq_bf2 p2 = __builtin_convertvector((oeq_f2{a, b}), oeq_bf2);
     q0 = __builtin_bit_cast(unsigned, p0), q1 = __builtin_bit_cast(unsigned, p1), q2 = __builtin_bit_cast(unsigned, p2);
 }
+// The same in steps, for a caller that puts other instructions between them: q = the next parts of a and b, which keep the
+// remainders (a dependent instruction is issued after 3.6 ns, one that is not after 2.1).
+OEQ_DEV void oeq_split_part(float& a, float& b, unsigned& q)
+{
+    unsigned l = 0x0000bf80u, h = 0xbf800000u;
+    asm("" : "+s"(l), "+s"(h));
+    const oeq_bf2 p = __builtin_convertvector((oeq_f2{a, b}), oeq_bf2);
+    a = __builtin_amdgcn_fdot2_f32_bf16(p, __builtin_bit_cast(oeq_bf2, l), a, false);
+    b = __builtin_amdgcn_fdot2_f32_bf16(p, __builtin_bit_cast(oeq_bf2, h), b, false);
+    q = __builtin_bit_cast(unsigned, p);
+}
+OEQ_DEV void oeq_split_last(float a, float b, unsigned& q)
+{
+    q = __builtin_bit_cast(unsigned, __builtin_convertvector((oeq_f2{a, b}), oeq_bf2));
+}
 // Component I of eight channels (or rows) as three bf16 operands: r[e * D + I], e = 0..7.
 template <int D, int I> OEQ_DEV void oeq_split8(const float (&r)[8 * D], oeq_bf8 (&f)[3])
 {
@@ -111,6 +147,21 @@ OEQ_DEV oeq_bf8 oeq_park(oeq_bf8 v)
     for (int m = 0; m < 4; ++m) { unsigned t; asm("v_accvgpr_write_b32 %0, %1" : "=a"(t) : "v"(q[m])); r[m] = t; }
     return __builtin_bit_cast(oeq_bf8, r);
 }
+// r[n] = lo[n] + (lo[n] of the mirrored lane) in the lanes of the lower half, hi[n] + (hi[n] of it) in the others; r may be lo.
+// (Two wait states between the instruction that writes an operand and the one that reads it from other lanes, which the
+// compiler does not see.)
+#define OEQ_FOLD_LANES(r0, r1, r2, lo0, lo1, lo2, hi0, hi1, hi2, MIRROR, UPPER) \
+    { \
+        float f0 = lo0, f1 = lo1, f2 = lo2; \
+        asm("s_nop 1\n\tv_add_f32_dpp %0, %0, %0 " MIRROR " row_mask:0xf bank_mask:0xf\n\t" \
+            "v_add_f32_dpp %1, %1, %1 " MIRROR " row_mask:0xf bank_mask:0xf\n\t" \
+            "v_add_f32_dpp %2, %2, %2 " MIRROR " row_mask:0xf bank_mask:0xf\n\t" \
+            "v_add_f32_dpp %0, %3, %3 " MIRROR " row_mask:0xf bank_mask:" UPPER "\n\t" \
+            "v_add_f32_dpp %1, %4, %4 " MIRROR " row_mask:0xf bank_mask:" UPPER "\n\t" \
+            "v_add_f32_dpp %2, %5, %5 " MIRROR " row_mask:0xf bank_mask:" UPPER \
+            : "+v"(f0), "+v"(f1), "+v"(f2) : "v"(hi0), "v"(hi1), "v"(hi2)); \
+        r0 = f0, r1 = f1, r2 = f2; \
+    }
 OEQ_DEV void oeq_block_sync()
 {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -185,6 +236,20 @@ class SplitEmitter:
         frags = sum(A[a].d * c32(A[a].mul) for a in {ia(q) for q in subs})
         return 2 * (3072 * frags + 64 * self.low.L2 * (1 if kind == "forward" else 5))
 
+    def folds(self, kind: str, subs):
+        """Sub-paths of a forward kernel whose result has one component and whose operand has more (l x l -> 0): X and Y
+        are contracted by the threads that split the rows, and one component is multiplied, not 2 l + 1. As many as the LDS
+        has room for, and two more steps remain."""
+        A, T, ia, it = self.sides(kind)
+        out, room = [], LDS_BUDGET // self.waves(kind) - self.lds(kind, subs)
+        for q in sorted(subs, key=lambda q: -A[ia(q)].d):
+            if kind == "forward" and T[it(q)].d == 1 and A[ia(q)].d > 1:
+                room -= 2 * 3072 * c32(A[ia(q)].mul)
+                raw = {ia(p) for p in subs if p not in out and p is not q}
+                if room >= 0 and sum(A[a].d for a in raw) >= 2:
+                    out.append(q)
+        return out
+
     def share(self, kind: str) -> float:
         """Of the multiplies of a pass, those with weights that are not padding (a wave's 16 result channels times four,
         32 contracted channels at a time)."""
@@ -251,7 +316,7 @@ class SplitEmitter:
             for e in range(8):
                 full = 32 * st + 32 <= a.mul
                 u = f"{32 * st + e} + 8 * lq"
-                val = f"W[{base} + ({u if full else f'min({u}, {a.mul - 1})'}) * {cu} + t * {ct}]"
+                val = f"{self.lit(q.unit)} * W[{base} + ({u if full else f'min({u}, {a.mul - 1})'}) * {cu} + t * {ct}]"
                 conds = ([] if t.mul >= 64 else [f"16 * wave + l16 < {t.mul}"]) + ([] if full else [f"{u} < {a.mul}"])
                 s(f"r[{e}] = " + (f"oeq_sel({' && '.join(conds)}, {val});" if conds else f"{val};"))
             s(f"oeq_split8<1, 0>(r, w{q.index}[{st}]);")
@@ -290,9 +355,37 @@ class SplitEmitter:
             if 32 * st + 32 > b.mul:
                 # channels past the block meet zero weights: zeros here too, not other channels' values
                 v = [f"oeq_sel({32 * st + e} + 2 * (tid & 15) < {b.mul}, {v[e]})" for e in range(2)]
-            out.append((10, f"{{ unsigned q0, q1, q2; oeq_split3({v[0]}, {v[1]}, q0, q1, q2); " +
-                        " ".join(f"{buf}[{at + 768 * i + 256 * c} + put] = q{c};" for c in range(3)) + " }"))
+            out += self.split_pair(f"{a}_{st}_{i}", v, [f"{buf}[{at + 768 * i + 256 * c} + put]" for c in range(3)])
         return out
+
+    def fold_write(self, q: Sub, st: int, at: int, buf: str):
+        """The one component of a folded sub-path from ra<a>_<st> and yt<q>, as ``rows_write`` has it."""
+        b, n = self.low.in1[q.p.i1], q.index
+        out = []
+        for e in range(2):
+            for m, (i, j, _, c) in enumerate(q.p.nnz):
+                r = q.ratio(c)
+                y = f"yt{n}[{j}]" if r == 1.0 else f"({self.lit(r)} * yt{n}[{j}])"
+                op = ("= -" if c < 0 else "= ") if m == 0 else "-= " if c < 0 else "+= "
+                out.append((1, f"{'float ' if m == 0 else ''}tf{n}_{st}_{e} {op}{y} * ra{q.p.i1}_{st}[{e * b.d + i}];"))
+        v = [f"tf{n}_{st}_{e}" for e in range(2)]
+        if 32 * st + 32 > b.mul:
+            v = [f"oeq_sel({32 * st + e} + 2 * (tid & 15) < {b.mul}, {v[e]})" for e in range(2)]
+        return out + self.split_pair(f"f{n}_{st}", v, [f"{buf}[{at + 256 * c} + put]" for c in range(3)])
+
+    @staticmethod
+    def split_pair(name: str, v, to):
+        """Two values to three places, in steps."""
+        q = [f"q{name}_{c}" for c in range(3)]
+        return [(0, f"float s{name}_0 = {v[0]}, s{name}_1 = {v[1]}; unsigned {', '.join(q)};")] + \
+            [(3, f"oeq_split_part(s{name}_0, s{name}_1, {q[c]});") for c in range(2)] + \
+            [(1, f"oeq_split_last(s{name}_0, s{name}_1, {q[2]});")] + [(1, f"{to[c]} = {q[c]};") for c in range(3)]
+
+    @staticmethod
+    def split_tasks(v: str, q: str):
+        """Eight values as the parts ``q[part][pair]``, pair by pair and part by part; the values are used up."""
+        out = [(3, f"oeq_split_part({v}[{2 * m}], {v}[{2 * m + 1}], {q}[{c}][{m}]);") for c in range(2) for m in range(4)]
+        return out + [(1, f"oeq_split_last({v}[{2 * m}], {v}[{2 * m + 1}], {q}[2][{m}]);") for m in range(4)]
 
     @staticmethod
     def put(s: Src, tasks):
@@ -345,11 +438,17 @@ class SplitEmitter:
         L2, fwd = low.L2, kind == "forward"
         dst, LT = ("L3_out", low.L3) if fwd else ("L1_grad", low.L1)
         used_a, used_t = sorted({ia(q) for q in subs}), sorted({it(q) for q in subs})
+        folds = self.folds(kind, subs)
+        raw_a = sorted({ia(q) for q in subs if q not in folds})   # blocks whose components are multiplied
         at, total = {}, 0
-        for a in used_a:
+        for a in raw_a:
             for st in range(c32(A[a].mul)):
                 at[(a, st)] = total
                 total += 768 * A[a].d
+        for q in folds:
+            for st in range(c32(A[ia(q)].mul)):
+                at[(q.key, st)] = total
+                total += 768
         self.open_kernel(s, name, sig, self.waves(kind))
         s("const int tid = (int)threadIdx.x;")
         s(f"__shared__ __attribute__((aligned(16))) unsigned s_a[2][{total}];")
@@ -370,6 +469,16 @@ class SplitEmitter:
         ny = (16 * L2 + 255) // 256
         s(f"float ry[{ny}];")
 
+        # coefficients beside a path's most frequent one, in scalar registers: a constant in the instruction makes it
+        # twice as long, and the wave issues it in 3.4 ns, not 2.1
+        ratios = {}
+        for q in subs:
+            for *_, c in q.p.nnz:
+                key = self.lit(q.ratio(c))
+                if q.ratio(c) != 1.0 and key not in ratios:
+                    ratios[key] = f"c{len(ratios)}"
+                    s(f'float {ratios[key]} = {key}; asm("" : "+s"({ratios[key]}));')
+
         src, LA = ("L1_in", low.L1) if fwd else ("L3_grad", low.L3)
 
         def where(tile, const="const "):
@@ -380,7 +489,7 @@ class SplitEmitter:
         def request_y():
             for n in range(ny):
                 v = f"min(tid + {256 * n}, {16 * L2 - 1})"
-                s(f"ry[{n}] = *oeq_at(L2_in + first * {L2}, 4u * (unsigned)(min({v} / {L2}, end) * {L2} + {v} % {L2}));")
+                s(f"ry[{n}] = *oeq_at(L2_in + first * {L2}, 4u * (unsigned)min({v}, end * {L2} + {v} % {L2}));")
 
         # (threads past the tile repeat its last value: a store under a lane's condition makes the compiler wait for more
         # than it has to afterwards)
@@ -389,32 +498,58 @@ class SplitEmitter:
                 v = f"min(tid + {256 * n}, {16 * L2 - 1})"
                 s(f"s_y[{buf}][{v} % {L2}][{v} / {L2}] = ry[{n}];")
 
+        # byte offsets of the lane's four rows in a tile of X or the results; past the batch: its last row
+        s(f"unsigned lr[4];")
+        s(f"for (int r = 0; r < 4; ++r) lr[r] = {4 * LT}u * (4 * lq + r);")
+        row_at = lambda r, end: f"min(lr[{r}], {4 * LT}u * (unsigned){end})"
+
         def request_x(t):
             b = T[t]
-            s("#pragma unroll")
-            s.open("for (int r = 0; r < 4; ++r)")
-            s(f"const float* xp = oeq_at(L1_in + first * {low.L1} + {b.off}, 4u * (unsigned)(min(4 * lq + r, end) * {low.L1} + ch{t} * {b.d}));")
-            for i in range(b.d):
-                s(f"xn{t}[{i}][r] = xp[{i}];")
-            s.close()
+            return [(4, f"{{ const float* xp = oeq_at(L1_in + xfirst * {low.L1} + {b.off}, {row_at(r, 'xend')} + ch{t}); "
+                        + " ".join(f"xn{t}[{i}][{r}] = xp[{i}];" for i in range(b.d)) + " }") for r in range(4)]
 
         for t in used_t:
-            s(f"const int ch{t} = min(16 * wave + l16, {T[t].mul - 1});")
+            s(f"const unsigned ch{t} = {4 * T[t].d}u * min(16 * wave + l16, {T[t].mul - 1});")
             if not fwd:
                 s(f"v4t xn{t}[{T[t].d}];")
+        for q in folds:
+            s(f"float yt{q.index}[{low.in2[q.p.i2].d}];  // Y of the thread's row")
+
+        def y_request(q):
+            b2 = low.in2[q.p.i2]
+            return [(3, f"{{ const float* yp = oeq_at(L2_in + first * {L2} + {self.yat(q, 0)}, 4u * (unsigned)(min(tid >> 4, end) * {L2})); "
+                     + " ".join(f"yt{q.index}[{j}] = yp[{j}];" for j in range(b2.d)) + " }")]
+
+        def request(a, st):
+            """The rows of a unit, and the Y that its folds will meet once the last of them is written."""
+            out = self.rows_request(kind, a, st)
+            if st == c32(A[a].mul) - 1:
+                for q in folds:
+                    out += y_request(q) if ia(q) == a else []
+            return out
+
+        def write(a, st, buf):
+            out = self.rows_write(kind, a, st, at[(a, st)], buf) if a in raw_a else []
+            for q in folds:
+                if ia(q) == a:
+                    out += self.fold_write(q, st, at[(q.key, st)], buf)
+            return out
+
         units = [(a, st) for a in used_a for st in range(c32(A[a].mul))]
         s.open("")
         where("(i64)blockIdx.x", "const i64 ")
         s(f"const float* rows = {src} + first * {LA};")
         s(f"const unsigned own = (unsigned)min(tid >> 4, end) * {4 * LA}u;")
         for a, st in units:
-            self.put(s, self.rows_request(kind, a, st))
+            self.put(s, request(a, st))
         request_y()
         if not fwd:
+            s("const i64 xfirst = first;")
+            s("const int xend = end;")
             for t in used_t:
-                request_x(t)
+                self.put(s, request_x(t))
         for a, st in units:
-            self.put(s, self.rows_write(kind, a, st, at[(a, st)], "s_a[0]"))
+            self.put(s, write(a, st, "s_a[0]"))
         write_y("0")
         s.close()
         s.open("")
@@ -422,41 +557,53 @@ class SplitEmitter:
         s(f"const float* rows = {src} + first * {LA};")
         s(f"const unsigned own = (unsigned)min(tid >> 4, end) * {4 * LA}u;")
         for a, st in units:
-            self.put(s, self.rows_request(kind, a, st))
+            self.put(s, request(a, st))
         request_y()
         s.close()
         # Software pipeline over the components of the contracted rows, across tiles: while the matrix cores work on one,
         # the lanes contract the results of the one before with the coupling coefficients, and its successor's operands
         # are on their way from LDS. The last component of a tile is contracted, and its rows are stored, beside the first
         # matrix instructions of the next.
-        steps = [(a, i) for a in sorted(used_a, key=lambda a: -A[a].d) for i in range(A[a].d)]
-        mine = {a: [q for q in subs if ia(q) == a] for a in used_a}
+        steps = [(a, i) for a in sorted(raw_a, key=lambda a: -A[a].d) for i in range(A[a].d)] + [(q.key, 0) for q in folds]
+        mine = {a: [q for q in subs if ia(q) == a and q not in folds] for a in raw_a} | {q.key: [q] for q in folds}
+        slots = {a: c32(A[a].mul) for a in raw_a} | {q.key: c32(A[ia(q)].mul) for q in folds}
         N = len(steps)
 
         def fetch(n, buf="cur"):
             a, i = steps[n]
             return [(1, f"f{n}[{st}][{c}] = __builtin_bit_cast(oeq_bf8, *(const oeq_u4*)(s_a[{buf}] + "
-                        f"{at[(a, st)] + 768 * i + 256 * c} + get));") for st in range(c32(A[a].mul)) for c in range(3)]
+                        f"{at[(a, st)] + 768 * i + 256 * c} + get));") for st in range(slots[a]) for c in range(3)]
+
+        begun = {}  # sum -> the term that starts it, in the order of the steps
+
+        def add(sum_, term, c=1.0):
+            if begun.setdefault(sum_, term) == term:
+                return (4, f"{sum_} = {'-' if c < 0 else ''}{term};")
+            return (4, f"{sum_} {'-=' if c < 0 else '+='} {term};")
 
         def contract(n):
             a, i = steps[n]
             out = []
             for q in mine[a]:
-                names = {}
+                if q in folds:
+                    out.append(add(f"acc{it(q)}[0]", f"P{n}_{q.index}"))
+                    continue
+                names = {self.lit(1.0): f"P{n}_{q.index}"}
                 for (i1, j, k, c) in q.p.nnz:
                     if (i1 if fwd else k) != i:
                         continue
-                    key = self.lit(abs(c))
+                    key = self.lit(q.ratio(c))
                     if key not in names:
                         names[key] = f"m{n}_{q.index}_{len(names)}"
-                        out.append((4 if len(names) > 1 else 8, f"const v4t {names[key]} = {key} * P{n}_{q.index};"))
-                    op, yj = "-=" if c < 0 else "+=", self.yat(q, j)
-                    if fwd:
-                        out.append((4, f"acc{it(q)}[{k}] {op} y[{yj}] * {names[key]};"))
-                    else:
-                        out.append((4, f"acc{it(q)}[{i1}] {op} y[{yj}] * {names[key]};"))
-                        out.append((4, f"dy[{yj}] {op} x{it(q)}[{i1}] * {names[key]};"))
+                        out.append((4, f"const v4t {names[key]} = {ratios[key]} * P{n}_{q.index};"))
+                    yj = self.yat(q, j)
+                    out.append(add(f"acc{it(q)}[{k if fwd else i1}]", f"y[{yj}] * {names[key]}", c))
+                    if not fwd:
+                        out.append(add(f"dy[{yj}]", f"x{it(q)}[{i1}] * {names[key]}", c))
             return out
+
+        for n in range(N):
+            contract(n)
 
         def store(row0, end):
             """Rows past the batch repeat its last one, in what was read and so in the results, and write it again: no
@@ -464,7 +611,7 @@ class SplitEmitter:
             out = []
             for t in used_t:
                 for r in range(4):
-                    text = f"float* op = oeq_at({dst} + {row0} * {LT} + {T[t].off}, 4u * (unsigned)(min(4 * lq + {r}, {end}) * {LT} + ch{t} * {T[t].d})); " + \
+                    text = f"float* op = oeq_at({dst} + {row0} * {LT} + {T[t].off}, {row_at(r, end)} + ch{t}); " + \
                         " ".join(f"__builtin_nontemporal_store((float)acc{t}[{k}][{r}], op + {k});" for k in range(T[t].d))
                     out.append((6, (f"if (16 * wave + l16 < {T[t].mul}) " if T[t].mul < 64 else "") + "{ " + text + " }"))
             return out
@@ -473,7 +620,7 @@ class SplitEmitter:
             a, i = steps[n]
             out = []
             for ca, cb in TERMS:
-                for st in range(c32(A[a].mul)):
+                for st in range(slots[a]):
                     for q in mine[a]:
                         out.append(f"P{n}_{q.index} = oeq_mfma_bf(f{n}[{st}][{ca}], w{q.index}[{st}][{cb}], P{n}_{q.index}, 0, 0, 0);")
             return out
@@ -482,7 +629,7 @@ class SplitEmitter:
             if n in (0, N - 1):
                 for q in mine[a]:
                     s(f"v4t P{n}_{q.index} = v4t{{}};")
-        s(f"oeq_bf8 f0[{c32(A[steps[0][0]].mul)}][3];")
+        s(f"oeq_bf8 f0[{slots[steps[0][0]]}][3];")
         s(f"v4t y[{L2}];")
         for j in range(L2):
             s(f"y[{j}] = v4t{{}};")
@@ -540,15 +687,20 @@ class SplitEmitter:
         for n, (a, i) in enumerate(steps):
             tasks, reads = [], []
             if n + 1 < N:
-                s(f"oeq_bf8 f{n + 1}[{c32(A[steps[n + 1][0]].mul)}][3];")
+                s(f"oeq_bf8 f{n + 1}[{slots[steps[n + 1][0]]}][3];")
                 reads = fetch(n + 1)
             # a share of the next tile's operands, and of the requests for the one after
             for ua, ust in (units[m] for m in range(len(units)) if writer(m) == n):
-                tasks += self.rows_write(kind, ua, ust, at[(ua, ust)], "s_a[cur ^ 1]")
-                tasks += self.rows_request(kind, ua, ust)
+                tasks += write(ua, ust, "s_a[cur ^ 1]")
+                tasks += request(ua, ust)
             tasks += contract((n or N) - 1)
             if n == min(1, N - 1):
                 tasks += take
+                if not fwd:
+                    # X of the next tile, whose registers this tile's has left beside the step before
+                    s("const i64 xfirst = min((tile + gridDim.x) * 16, num_batch - 1);")
+                    s("const int xend = (int)min((i64)15, num_batch - 1 - xfirst);")
+                    tasks += [v for t in used_t for v in request_x(t)]
             if n == N - 1:
                 tasks += give
             if n == N - 1:
@@ -568,22 +720,13 @@ class SplitEmitter:
                 self.interleave(s, half[:cut], tasks)
                 tasks = store("prow0", "pend")
                 tasks += [(1, f"y[{j}] = *(const v4t*)&s_y[cur][{j}][4 * lq];") for j in range(L2)]
+                if not fwd:
+                    tasks += self.reduce_dy("s_dy[cur ^ 1]")
                 self.interleave(s, half[cut:], tasks)
                 if not fwd:
-                    self.reduce_dy(s, "s_dy[cur ^ 1]")
-                    for j in range(L2):
-                        s(f"dy[{j}] = v4t{{}};")
-                for t in used_t:
-                    for k in range(T[t].d):
-                        s(f"acc{t}[{k}] = v4t{{}};")
-                        if not fwd:
-                            s(f"x{t}[{k}] = xn{t}[{k}];")
-                if not fwd:
-                    s.open("")
-                    where("(tile + gridDim.x)", "const i64 ")
                     for t in used_t:
-                        request_x(t)
-                    s.close()
+                        for k in range(T[t].d):
+                            s(f"x{t}[{k}] = xn{t}[{k}];")
                 write_y("cur ^ 1")
                 request_y()
             else:
@@ -601,7 +744,7 @@ class SplitEmitter:
         self.put(s, contract(N - 1))
         self.put(s, store("prow0", "pend"))
         if not fwd:
-            self.reduce_dy(s, "s_dy[cur ^ 1]")
+            self.put(s, self.reduce_dy("s_dy[cur ^ 1]"))
             s("const i64 tiles_here = (ntiles - 1 - blockIdx.x) / gridDim.x + 1;")
             s("oeq_block_sync();")
             s("const bool ready = true;")
@@ -613,30 +756,29 @@ class SplitEmitter:
                 s.close()
         s.close()
 
-    def reduce_dy(self, s: Src, into: str):
-        """Sum over the 16 lanes that hold a row's channels; a lane is left with n / 16 consecutive values of the
-        4 x L2 its group of lanes holds, which lie one after the other in memory, too."""
+    def reduce_dy(self, into: str):
+        """Sum over the 16 lanes that hold a row's channels. A step adds the lanes of a mirrored half to the ones of the other
+        and leaves half as many values: a lane keeps those of the half it lies in. n / 16 consecutive ones of the 4 x L2
+        values of its group of lanes, which lie one after the other in memory, too, are a lane's in the end."""
         L2 = self.low.L2
         n = 4 * L2
         cur = (n + 15) // 16 * 16
-        s.open("")
-        s(f"float rv[{cur}];")
-        for o in range(cur):
-            s(f"rv[{o}] = {f'dy[{o % L2}][{o // L2}]' if o < n else '0.0f'};")
-        s("int at = 0;")
-        for ctrl, bit in (("0x140", 8), ("0x141", 4), ("0x1B", 2), ("0xB1", 1)):
+        val = [f"dy[{o % L2}][{o // L2}]" if o < n else "0.0f" for o in range(cur)]
+        out = [(0, f"float rv[{cur // 2 + 2}]; int at = 0;")]
+        for ctrl, bit, upper in (("row_mirror", 8, "0xc"), ("row_half_mirror", 4, "0xa"), ("0x1B", 2, None), ("0xB1", 1, None)):
             half = cur // 2
-            s.open("")
-            s(f"const bool hi = (l16 & {bit}) != 0;")
-            for j in range(half):
-                s(f"{{ const float keep = hi ? rv[{j + half}] : rv[{j}]; const float send = hi ? rv[{j}] : rv[{j + half}]; "
-                  f"rv[{j}] = keep + oeq_dpp<{ctrl}>(send); }}")
-            s(f"at += hi ? {half} : 0;")
-            s.close()
-            cur = half
-        for t in range(cur):
-            s(f"if (at + {t} < {n}) {into}[wave][4 * lq * {L2} + at + {t}] = rv[{t}];")
-        s.close()
+            for j in range(0, half, 1 if upper is None else 3):
+                if upper is None:
+                    out.append((3, f"{{ const bool hi = (l16 & {bit}) != 0; const float keep = hi ? {val[j + half]} : {val[j]}, send = hi ? {val[j]} : {val[j + half]}; "
+                                   f"rv[{j}] = keep + oeq_dpp<{ctrl}>(send); }}"))
+                    continue
+                # (three at a time; past the last pair: it once more)
+                at = [min(j + m, half - 1) for m in range(3)]
+                into_ = [f"rv[{j + m}]" if j + m < half else f"rv[{cur // 2}]" for m in range(3)]
+                out.append((7, f"OEQ_FOLD_LANES({', '.join(into_ + [val[m] for m in at] + [val[m + half] for m in at])}, \"{ctrl}\", \"{upper}\")"))
+            out.append((1, f"at += (l16 & {bit}) ? {half} : 0;"))
+            val, cur = [f"rv[{j}]" for j in range(half)], half
+        return out + [(1, f"if (at + {t} < {n}) {into}[wave][4 * lq * {L2} + at + {t}] = rv[{t}];") for t in range(cur)]
 
     # ------------------------------------------------------------------------ dW
     def split_dw(self, subs):
@@ -654,15 +796,32 @@ class SplitEmitter:
         g = 8 * sum(low.out[o].d for o in {q.p.io for q in subs})
         return 4 * sum(per(q) for q in subs) + into + x + 16 + max(x, g) + 18 * max(per(q) for q in subs) + 32 + 32
 
+    def table_dw(self, subs):
+        """(component of Y, ratio of a coefficient to its path's unit), each once."""
+        return sorted({(self.yat(q, j), q.ratio(c)) for q in subs for _, j, _, c in q.p.nnz})
+
     def lds_dw(self, subs) -> int:
         low = self.low
-        return 2 * (3072 * sum(low.out[o].d * c16(low.out[o].mul) for o in {q.p.io for q in subs}) + 128 * low.L2)
+        return 2 * (3072 * sum(low.out[o].d * c16(low.out[o].mul) for o in {q.p.io for q in subs}) + 192 * len(self.table_dw(subs)))
 
-    def stages_dw(self, subs):
-        """(output block, component, sub-path), in the order in which they are multiplied."""
+    def folds_dw(self, subs):
+        """Sub-paths whose input has one component and whose output has more (0 x l -> l): Y and dZ are contracted by the
+        threads that split dZ, and one component is multiplied, not 2 l + 1. As many as the LDS has room for, and three more
+        products remain."""
+        low, out, room = self.low, [], LDS_BUDGET // self.waves("dw") - self.lds_dw(subs)
+        for q in sorted(subs, key=lambda q: -low.out[q.p.io].d):
+            if low.in1[q.p.i1].d == 1 and low.out[q.p.io].d > 1:
+                room -= 2 * 3072 * c16(low.out[q.p.io].mul)
+                if room >= 0 and len(self.stages_dw([p for p in subs if p not in out and p is not q])) >= 3:
+                    out.append(q)
+        return out
+
+    def stages_dw(self, subs, folds=()):
+        """(output block, component, sub-path), in the order in which they are multiplied; first those that are folded."""
         out = self.low.out
-        return [(o, k, q) for o in sorted({q.p.io for q in subs}, key=lambda o: -out[o].d) for k in range(out[o].d)
-                for q in subs if q.p.io == o and any(kk == k for _, _, kk, _ in q.p.nnz)]
+        return [(q.p.io, q.key, q) for q in folds] + \
+            [(o, k, q) for o in sorted({q.p.io for q in subs}, key=lambda o: -out[o].d) for k in range(out[o].d)
+             for q in subs if q.p.io == o and q not in folds and any(kk == k for _, _, kk, _ in q.p.nnz)]
 
     def emit_dw(self, s: Src, name: str, sig: str):
         names = []
@@ -676,15 +835,20 @@ class SplitEmitter:
         L2 = low.L2
         WU, WW, per = self.split_dw(subs)
         used_a, used_o = sorted({q.p.i1 for q in subs}), sorted({q.p.io for q in subs}, key=lambda o: -low.out[o].d)
+        folds = self.folds_dw(subs)
+        stages = self.stages_dw(subs, folds)
         where, total = {}, 0
-        for o in used_o:
-            for k in range(low.out[o].d):
-                where[(o, k)] = total
-                total += 768 * c16(low.out[o].mul)
+        for o, k in dict.fromkeys((o, k) for o, k, _ in stages):
+            where[(o, k)] = total
+            total += 768 * c16(low.out[o].mul)
+        # components of Y times the coefficients they are met with: the rows of the tile's Y in LDS
+        table = self.table_dw(subs)
+        s(f"static __constant__ const float {name}_c[{len(table)}] = {{{', '.join(self.lit(r) for _, r in table)}}};")
+        s(f"static __constant__ const int {name}_j[{len(table)}] = {{{', '.join(str(j) for j, _ in table)}}};")
         self.open_kernel(s, name, sig, self.waves("dw"))
         s("const int tid = (int)threadIdx.x;")
         s(f"__shared__ __attribute__((aligned(16))) unsigned s_g[2][{total}];")
-        s(f"__shared__ __attribute__((aligned(16))) float s_y[2][{L2}][32];")
+        s(f"__shared__ __attribute__((aligned(16))) float s_y[3][{len(table)}][32];")
         s(f"const int wu = wave % {WU}, ww = wave / {WU};")
         s("(void)ww;")
         # rows of the identity: a product with them adds a tile of sums to another one, rounding to nearest
@@ -702,8 +866,15 @@ class SplitEmitter:
             s(f"float x{a}[8][{low.in1[a].d}], xn{a}[8][{low.in1[a].d}];")
             s(f"const int xc{a} = min(16 * wu + l16, {low.in1[a].mul - 1});")
         s(f"v4t yv[{AHEAD + 1}][2];  // a component of Y for the lane's eight rows, and the next ones")
-        ny = (32 * L2 + 255) // 256
-        s(f"float ry[{ny}];")
+        # (a thread's elements: row tid / 32 + 8 n of the table, row tid % 32 of the tile; past the table its last row again)
+        ny = (len(table) + 7) // 8
+        s(f"float ry[{ny}], yc[{ny}];")
+        s(f"int yj[{ny}];")
+        s("#pragma unroll")
+        s.open(f"for (int n = 0; n < {ny}; ++n)")
+        s(f"const int at = min((tid >> 5) + 8 * n, {len(table) - 1});")
+        s(f"yc[n] = sign * {name}_c[at], yj[n] = {name}_j[at];")
+        s.close()
         s("const i64 nsteps = (num_batch + 31) / 32;")
 
         def rows_of(step):
@@ -720,40 +891,61 @@ class SplitEmitter:
             return [(4, f"{{ const float* xp = oeq_at(L1_in + first * {low.L1} + {b.off}, 4u * (unsigned)(min(8 * lq + {e}, end) * {low.L1} + xc{a} * {b.d})); "
                      + " ".join(f"xn{a}[{e}][{i}] = xp[{i}];" for i in range(b.d)) + " }")]
 
-        def request_y():
-            return [(4, f"ry[{n}] = *oeq_at(L2_in + first * {L2}, 4u * (unsigned)min(min(tid + {256 * n}, {32 * L2 - 1}), end * {L2} + {L2 - 1}));")
+        # (Y is a step ahead of dZ, with which it is contracted on the way to LDS, and so has three copies)
+        def request_y(step):
+            s(f"const i64 yfirst = min((i64)({step}) * 32, num_batch - 1);")
+            s("const int yend = (int)min((i64)31, num_batch - 1 - yfirst);")
+            s(f"const int yrows = (int)max((i64)0, min((i64)32, num_batch - (i64)({step}) * 32));")
+            return [(4, f"ry[{n}] = *oeq_at(L2_in + yfirst * {L2}, 4u * (unsigned)(min(tid & 31, yend) * {L2} + yj[{n}]));")
                     for n in range(ny)]
 
         def write_y(buf):
-            v = [f"min(tid + {256 * n}, {32 * L2 - 1})" for n in range(ny)]
-            return [(5, f"s_y[{buf}][{v[n]} % {L2}][{v[n]} / {L2}] = sign * ry[{n}];") for n in range(ny)]
+            """Zeros for the rows past the batch, which repeat its last one otherwise."""
+            return [(5, f"s_y[{buf}][min((tid >> 5) + {8 * n}, {len(table) - 1})][tid & 31] = oeq_sel((tid & 31) < yrows, yc[{n}] * ry[{n}]);")
+                    for n in range(ny)]
 
-        def write_g(o, buf, n):
-            """dZ of the wave's columns of a block, zero past the batch (``n``: rows there are), as operands."""
-            b = low.out[o]
-            out = []
-            for k in range(b.d):
-                text = f"{{ float v[8]; " + " ".join(f"v[{e}] = oeq_sel({e} + 8 * lq < {n}, g{o}[{e * b.d + k}]);" for e in range(8)) + \
-                    " oeq_bf8 f[3]; oeq_split8<1, 0>(v, f); " + \
-                    " ".join(f"*(oeq_u4*)({buf} + {where[(o, k)] + 256 * c} + 768 * wave + 4 * lane) = __builtin_bit_cast(oeq_u4, f[{c}]);"
-                             for c in range(3)) + " }"
-                out.append((44, (f"if (16 * wave < {16 * c16(b.mul)}) " if b.mul <= 48 else "") + text))
+        def fold(q, v, buf):
+            """dZ and Y of a folded sub-path, for the lane's column and eight rows."""
+            o, terms, y = q.p.io, q.p.nnz, f"yf{q.index}"
+            get = lambda m: [(2, f"{y}[{m & 1}][{h}] = *(const v4t*)&{buf}[{at_of(q, terms[m][1], terms[m][3])}][8 * lq + {4 * h}];") for h in (0, 1)]
+            out = [(0, f"float {v}[8]; v4t {y}[2][2];")] + get(0)
+            for m, (_, j, k, c) in enumerate(terms):
+                out += get(m + 1) if m + 1 < len(terms) else []
+                op = ("= -" if c < 0 else "= ") if m == 0 else "-= " if c < 0 else "+= "
+                out += [(4, " ".join(f"{v}[{4 * h + r}] {op}{y}[{m & 1}][{h}][{r}] * g{o}[{(4 * h + r) * low.out[o].d + k}];" for r in range(4)))
+                        for h in (0, 1)]
             return out
 
-        stages = self.stages_dw(subs)
-        first_k = {q.index: min(k for _, _, k, _ in q.p.nnz) for q in subs}
-        last_k = {q.index: max(k for _, _, k, _ in q.p.nnz) for q in subs}
-        N = len(stages)
+        def write_g(o, buf, ynext):
+            """dZ of the wave's columns of a block as operands."""
+            b = low.out[o]
+            out = []
+            for k in [k for oo, k in where if oo == o]:
+                only = f"if (16 * wave < {16 * c16(b.mul)}) " if b.mul <= 48 else ""
+                q = next((q for q in folds if q.key == k), None)
+                v = f"v{o}_{k}" if q is None else f"vf{q.index}"
+                if q is None:
+                    out.append((0, f"float {v}[8]; " + " ".join(f"{v}[{e}] = g{o}[{e * b.d + k}];" for e in range(8))))
+                else:
+                    out += fold(q, v, ynext)
+                out += self.split_tasks(v, "tg")
+                out += [(1, only + f"*(oeq_u4*)({buf} + {where[(o, k)] + 256 * c} + 768 * wave + 4 * lane) = oeq_u4{{tg[{c}][0], tg[{c}][1], tg[{c}][2], tg[{c}][3]}};")
+                        for c in range(3)]
+            return out
 
-        # (stage, component of Y) in the order in which stages 1 .. N - 1 are contracted, and the first one's
-        js_of = lambda n: sorted({j for (_, j, kk, _) in stages[n % N][2].p.nnz if kk == stages[n % N][1]})
+        places = {q.index: [n for n, (_, _, p) in enumerate(stages) if p is q] for q in subs}
+        N = len(stages)
+        at_of = lambda q, j, c: table.index((self.yat(q, j), q.ratio(c)))
+
+        # (stage, row of the table) in the order in which stages 1 .. N - 1 are contracted, and the first one's
+        js_of = lambda n: sorted({at_of(stages[n % N][2], j, c) for (_, j, kk, c) in stages[n % N][2].p.nnz if kk == stages[n % N][1]})
         later = [(n, j) for n in range(1, N) for j in js_of(n)]
-        
+
         def read_y(units, u, buf):
             if u >= len(units):
                 return []
             n, j = units[u]
-            row = f"{buf}[{self.yat(stages[n % N][2], j)}]"
+            row = f"{buf}[{j}]"
             return [(2, f"yv[{u % (AHEAD + 1)}][0] = *(const v4t*)&{row}[8 * lq]; "
                         f"yv[{u % (AHEAD + 1)}][1] = *(const v4t*)&{row}[8 * lq + 4];")]
 
@@ -761,7 +953,10 @@ class SplitEmitter:
             """The contraction of X and Y for stage n, eight rows a lane, as operands. Y comes from LDS, component by
             component, two ahead of the sums."""
             o, k, q = stages[n % N]
-            buf = "s_y[cur]" if n < N else "s_y[cur ^ 1]"
+            if q in folds:
+                return [(4, " ".join(f"t[{4 * h + r}] = x{q.p.i1}[{4 * h + r}][0];" for r in range(4))) for h in (0, 1)] + \
+                    self.split_tasks("t", f"ta[{n % 2}]")
+            buf = "s_y[ycur]" if n < N else "s_y[ynext]"
             units = later if n % N else [(0, j) for j in js_of(0)]
             out, first = [], True
             for u, (m, j) in enumerate(units):
@@ -772,13 +967,16 @@ class SplitEmitter:
                         out += read_y(units, v, buf)
                 out += read_y(units, u + AHEAD, buf)
                 for i, jj, kk, c in q.p.nnz:
-                    if (jj, kk) != (j, k):
+                    if kk != k or at_of(q, jj, c) != j:
                         continue
+                    op = ("= -" if c < 0 else "= ") if first else "-= " if c < 0 else "+= "
                     for h in range(2):
-                        out.append((8, " ".join(f"t[{4 * h + r}] {'=' if first else '+='} ({self.lit(c)} * yv[{u % (AHEAD + 1)}][{h}][{r}]) * "
-                                                f"x{q.p.i1}[{4 * h + r}][{i}];" for r in range(4))))
+                        out.append((4, " ".join(f"t[{4 * h + r}] {op}yv[{u % (AHEAD + 1)}][{h}][{r}] * x{q.p.i1}[{4 * h + r}][{i}];"
+                                                for r in range(4))))
                     first = False
-            return out + [(28, f"oeq_split8<1, 0>(t, ta[{n % 2}]);")]
+            return out + self.split_tasks("t", f"ta[{n % 2}]")
+
+        operand = lambda q: f"__builtin_bit_cast(oeq_bf8, oeq_u4{{{', '.join(f'{q}[{m}]' for m in range(4))}}})"
 
         def read_bg(n, pair, buf):
             o, k, q = stages[n % N]
@@ -794,12 +992,12 @@ class SplitEmitter:
 
         def lead(n, pair):
             o, k, q = stages[n]
-            return [f"tm{q.index}[{j}] = oeq_mfma_bf(ta[{n % 2}][{ca}], bg[{j}][{cb}], tm{q.index}[{j}], 0, 0, 0);"
+            return [f"tm{q.index}[{j}] = oeq_mfma_bf({operand(f'ta[{n % 2}][{ca}]')}, bg[{j}][{cb}], tm{q.index}[{j}], 0, 0, 0);"
                     for ca, cb in TERMS for j in pair]
 
         # ---- the first step's operands
         s("float t[8];")
-        s("oeq_bf8 ta[2][3];")
+        s("unsigned ta[2][3][4], tg[3][4];")
         s(f"oeq_bf8 bg[{most}][3];")
         for q in subs:
             s(f"v4t tm{q.index}[{per(q)}];")
@@ -811,27 +1009,30 @@ class SplitEmitter:
         for a in used_a:
             for e in range(8):
                 self.put(s, request_x(a, e))
-        self.put(s, request_y())
-        s("const int rows = (int)min((i64)32, num_batch - (i64)blockIdx.x * 32);")
+        for n, step in enumerate(("blockIdx.x", "(i64)blockIdx.x + gridDim.x")):
+            s.open("")
+            self.put(s, request_y(step))
+            self.put(s, write_y(n))
+            s.close()
+        s("oeq_block_sync();")
         for o in used_o:
-            self.put(s, write_g(o, "s_g[0]", "rows"))
-        self.put(s, write_y("0"))
+            self.put(s, write_g(o, "s_g[0]", "s_y[0]"))
         s.close()
         for a in used_a:
             for e in range(8):
                 for i in range(low.in1[a].d):
                     s(f"x{a}[{e}][{i}] = xn{a}[{e}][{i}];")
-        s("int cur = 0;")
+        s("int cur = 0, ycur = 0;")
         s("oeq_block_sync();")
         self.put(s, t_tasks(0))
         self.put(s, read_bg(0, pairs(stages[0][2])[0], "s_g[0]"))
         s.open("for (i64 step = blockIdx.x; step < nsteps; step += gridDim.x, cur ^= 1)")
         # the step whose rows are requested, and written to LDS, during this one
         rows_of("step + gridDim.x")
-        s("const int rows = (int)max((i64)0, min((i64)32, num_batch - (step + (i64)gridDim.x) * 32));")
+        s("const int ynext = ycur == 2 ? 0 : ycur + 1, yput = ynext == 2 ? 0 : ynext + 1;")
         pending = []   # sums to be flushed beside a later stage's products
-        g_req = [t for o in used_o for e in range(8) for t in request_g(o, e)] + request_y()
-        g_put = [t for o in used_o for t in write_g(o, "s_g[cur ^ 1]", "rows")] + write_y("cur ^ 1")
+        g_req = [t for o in used_o for e in range(8) for t in request_g(o, e)] + request_y("step + 2 * (i64)gridDim.x")
+        g_put = [t for o in used_o for t in write_g(o, "s_g[cur ^ 1]", "s_y[ynext]")] + write_y("yput")
         x_req = [t for a in used_a for e in range(8) for t in request_x(a, e)]
         # (stages over which these are spread: X is requested when dZ has left the registers)
         spread = lambda items, n, lo, hi: items[max(0, n - lo) * len(items) // (hi - lo):(n + 1 - lo) * len(items) // (hi - lo)] \
@@ -842,7 +1043,7 @@ class SplitEmitter:
         for n, (o, k, q) in enumerate(stages):
             tasks = []
             tasks += spread(g_req, n, 0, req_end) + spread(g_put, n, put_from, put_end) + spread(x_req, n, put_from, put_end)
-            if k == first_k[q.index]:
+            if n == places[q.index][0]:
                 for j in range(per(q)):
                     s(f"tm{q.index}[{j}] = v4t{{}};")
             new_group = n + 1 == N or stages[n + 1][:2] != stages[n][:2]
@@ -860,7 +1061,7 @@ class SplitEmitter:
             tasks += t_tasks(n + 1)
             flush = [f"dw{p.index}[{j}] = oeq_mfma(eye[{i}], tm{p.index}[{j}][{i}], dw{p.index}[{j}], 0, 0, 0);"
                      for p in pending for i in range(4) for j in range(per(p))]
-            pending = [q] if k == last_k[q.index] else []
+            pending = [q] if n == places[q.index][-1] else []
             seq = [lead(n, pair) for pair in ps]
             # operands of this group that are not there yet (its second half), and the next group's first half once
             # this stage is done with its own
@@ -887,8 +1088,9 @@ class SplitEmitter:
                     for i in range(4):
                         for j in range(per(p)):
                             s(f"dw{p.index}[{j}] = oeq_mfma(eye[{i}], tm{p.index}[{j}][{i}], dw{p.index}[{j}], 0, 0, 0);")
+                s("ycur = ynext;")
                 if N % 2:
-                    s("for (int c = 0; c < 3; ++c) ta[0][c] = ta[1][c];")
+                    s("for (int c = 0; c < 3; ++c) for (int m = 0; m < 4; ++m) ta[0][c][m] = ta[1][c][m];")
         s.close()
         s(f"float* prow = wpartial + (i64)blockIdx.x * {low.WN};")
         for q in subs:
@@ -898,6 +1100,6 @@ class SplitEmitter:
                 s.open("for (int i = 0; i < 4; ++i)")
                 nt = f"{j}" if WW == 1 else f"(ww + {j * WW})"
                 s(f"const int u = 16 * wu + 4 * lq + i, w = 16 * {nt} + l16;")
-                s(f"if (u < {U} && w < {Wn}) prow[{self.wpos(q, 'u', 'w')}] = dw{q.index}[{j}][i];")
+                s(f"if (u < {U} && w < {Wn}) prow[{self.wpos(q, 'u', 'w')}] = {self.lit(q.unit)} * dw{q.index}[{j}][i];")
                 s.close()
         s.close()

@@ -51,6 +51,27 @@ def test_plan_covers_every_sub_path_once(name, make, wf, wb):
     assert "oeq_split3(" in src and any(d[1] == "backward_w" for d in descs)
 
 
+# (problem, sub-paths contracted before the product in the forward, and in each kernel of dW)
+FOLDS = [("l2-64", 2, [0, 1, 1]), ("l2-32", 2, [2]), ("l1-64-16", 1, [1]), ("odd-channels", 1, [1]),
+         ("two-channel-second-operand", 2, [2]), ("gaps", 1, [1])]
+
+
+@pytest.mark.parametrize("name,forward,dw", FOLDS, ids=[f[0] for f in FOLDS])
+def test_contracted_first_are_paths_with_one_component_on_the_other_side(name, forward, dw):
+    low = lower(next(c[1] for c in CASES if c[0] == name)())
+    em = SplitEmitter(low)
+    found = [q for subs in em.plan("forward") for q in em.folds("forward", subs)]
+    assert len(found) == forward and all(low.out[q.p.io].d == 1 < low.in1[q.p.i1].d for q in found)
+    assert not any(em.folds("dx", subs) for subs in em.plan("dx"))
+    assert [len(em.folds_dw(subs)) for subs in em.plan_dw()] == dw
+    for subs in em.plan_dw():
+        folds = em.folds_dw(subs)
+        assert all(low.in1[q.p.i1].d == 1 < low.out[q.p.io].d for q in folds)
+        stages = em.stages_dw(subs, folds)
+        assert {q.index for _, _, q in stages} == {q.index for q in subs} and len(stages) >= 3
+        assert [sum(q is f for _, _, q in stages) for f in folds] == [1] * len(folds)
+
+
 def test_takes_only_what_it_is_made_for():
     for problem in (_shared("64x0e+64x1o", "1x0e+1x1o", "64x0e+64x1o", np.float64),   # fp64
                     _shared("128x0e+128x1o", "1x0e+1x1o", "64x0e+64x1o"),             # blocks of more than 64 channels
