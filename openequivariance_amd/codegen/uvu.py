@@ -3335,7 +3335,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         (rt.ROLE_SEGMENT_PTR, "oeq_segment_ptr", 256, 256, compute_units * 16),
     ]
     if walk:
-        s(fixup_backward_kernel(low.L1, kahan, bool(em.nt & 4)))
+        s(fixup_backward_kernel(low.L1, kahan, bool(em.nt & 4), low.elem_size))
         descs += [
             (rt.ROLE_CONV_FORWARD, "forward", blk_f, G_f, 0, xcd),
             (rt.ROLE_CONV_BACKWARD, "backward", blk_b, G_b, compute_units * 8 if low.shared_weights else 0, xcd_b),

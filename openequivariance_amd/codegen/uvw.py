@@ -1247,7 +1247,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
         s(f"typedef oeq_wvec{n} oeq_wvec{n}_any __attribute__((aligned(sizeof(T))));")
     blk_f, G_f = em.emit_conv_forward(s, kahan)
     blk_b = em.emit_backward(s, conv=True)
-    s(fixup_backward_kernel(low.L1, kahan, True))
+    s(fixup_backward_kernel(low.L1, kahan, True, low.elem_size))
     cu = compute_units
     # shared weights: every wave of the backward grid writes one partial weight-gradient row (summed in order
     # by oeq_wreduce), so that grid is bounded
