@@ -35,7 +35,7 @@ kernels are also bound by power: random operands lower the clock (2.1 GHz, 2.4 o
 So the order of the instructions is written out (``interleave``): vector, LDS and memory instructions go between the matrix
 instructions that hide them, and what takes several is cut in steps (a split of eight values as one piece: 714 us for a pass through
 forward and backward, in steps 695); left to the compiler they clump, and registers spill. The pass: fp32 kernels
-1 066 us, these 719 with 35 products each and without the steps, 683 now.
+1 061 us, these 719 with 35 products each and without the steps, 661 now.
 """
 
 from __future__ import annotations
@@ -469,16 +469,6 @@ class SplitEmitter:
         ny = (16 * L2 + 255) // 256
         s(f"float ry[{ny}];")
 
-        # coefficients beside a path's most frequent one, in scalar registers: a constant in the instruction makes it
-        # twice as long, and the wave issues it in 3.4 ns, not 2.1
-        ratios = {}
-        for q in subs:
-            for *_, c in q.p.nnz:
-                key = self.lit(q.ratio(c))
-                if q.ratio(c) != 1.0 and key not in ratios:
-                    ratios[key] = f"c{len(ratios)}"
-                    s(f'float {ratios[key]} = {key}; asm("" : "+s"({ratios[key]}));')
-
         src, LA = ("L1_in", low.L1) if fwd else ("L3_grad", low.L3)
 
         def where(tile, const="const "):
@@ -595,7 +585,7 @@ class SplitEmitter:
                     key = self.lit(q.ratio(c))
                     if key not in names:
                         names[key] = f"m{n}_{q.index}_{len(names)}"
-                        out.append((4, f"const v4t {names[key]} = {ratios[key]} * P{n}_{q.index};"))
+                        out.append((4, f"const v4t {names[key]} = {key} * P{n}_{q.index};"))
                     yj = self.yat(q, j)
                     out.append(add(f"acc{it(q)}[{k if fwd else i1}]", f"y[{yj}] * {names[key]}", c))
                     if not fwd:
@@ -824,13 +814,37 @@ class SplitEmitter:
              for q in subs if q.p.io == o and q not in folds and any(kk == k for _, _, kk, _ in q.p.nnz)]
 
     def emit_dw(self, s: Src, name: str, sig: str):
-        names = []
-        for n, subs in enumerate(self.plan_dw()):
-            names.append(name if n == 0 else f"{name}_{n}")
-            self.emit_dw_kernel(s, names[-1], sig, subs)
-        return names
+        """One kernel, in which a block goes through the parts of ``plan_dw`` one after the other: the steps of 32 rows seldom
+        divide evenly among the blocks, and those that have one more of a part have one fewer of the next. Small batches have blocks to
+        spare, and their parts run side by side. 64x{0e,1o,2e}, forward and backward, a launch per part / one: 2 000 rows 85 /
+        72 - 81 us, 4 500 99 / 90, 20 000 187 / 171, 60 000 408 / 391, 100 003 and 131 072 the same."""
+        parts = self.plan_dw()
+        tables = [self.table_dw(subs) for subs in parts]
+        words = []
+        for n, (subs, table) in enumerate(zip(parts, tables)):
+            s(f"static __constant__ const float {name}_c{n}[{len(table)}] = {{{', '.join(self.lit(r) for _, r in table)}}};")
+            s(f"static __constant__ const int {name}_j{n}[{len(table)}] = {{{', '.join(str(j) for j, _ in table)}}};")
+            words.append(2 * sum(768 * c16(self.low.out[o].mul) for o, _ in self.operands_dw(subs)) + 96 * len(table))
+        self.open_kernel(s, name, sig, self.waves("dw"))
+        s("const int tid = (int)threadIdx.x;")
+        s(f"__shared__ __attribute__((aligned(16))) unsigned s_lds[{max(words)}];")
+        s("const i64 nsteps = (num_batch + 31) / 32;")
+        s("const int more = (int)(nsteps % gridDim.x);  // blocks with one step more")
+        for n, subs in enumerate(parts):
+            s.open("")
+            s(f"const i64 begin = (blockIdx.x + {n} * (gridDim.x - more)) % gridDim.x;  // the block's first step")
+            if n:
+                s("oeq_block_sync();")
+            self.emit_dw_part(s, f"{name}_c{n}", f"{name}_j{n}", subs, tables[n])
+            s.close()
+        s.close()
+        return [name]
 
-    def emit_dw_kernel(self, s: Src, name: str, sig: str, subs):
+    def operands_dw(self, subs):
+        """(output block, component or folded sub-path) whose operands are in LDS."""
+        return list(dict.fromkeys((o, k) for o, k, _ in self.stages_dw(subs, self.folds_dw(subs))))
+
+    def emit_dw_part(self, s: Src, coefficients: str, components: str, subs, table):
         low = self.low
         L2 = low.L2
         WU, WW, per = self.split_dw(subs)
@@ -838,17 +852,12 @@ class SplitEmitter:
         folds = self.folds_dw(subs)
         stages = self.stages_dw(subs, folds)
         where, total = {}, 0
-        for o, k in dict.fromkeys((o, k) for o, k, _ in stages):
+        for o, k in self.operands_dw(subs):
             where[(o, k)] = total
             total += 768 * c16(low.out[o].mul)
-        # components of Y times the coefficients they are met with: the rows of the tile's Y in LDS
-        table = self.table_dw(subs)
-        s(f"static __constant__ const float {name}_c[{len(table)}] = {{{', '.join(self.lit(r) for _, r in table)}}};")
-        s(f"static __constant__ const int {name}_j[{len(table)}] = {{{', '.join(str(j) for j, _ in table)}}};")
-        self.open_kernel(s, name, sig, self.waves("dw"))
-        s("const int tid = (int)threadIdx.x;")
-        s(f"__shared__ __attribute__((aligned(16))) unsigned s_g[2][{total}];")
-        s(f"__shared__ __attribute__((aligned(16))) float s_y[3][{len(table)}][32];")
+        # dZ's operands, and components of Y times the coefficients they are met with
+        s(f"unsigned (* const s_g)[{total}] = (unsigned (*)[{total}])s_lds;")
+        s(f"float (* const s_y)[{len(table)}][32] = (float (*)[{len(table)}][32])(s_lds + {2 * total});")
         s(f"const int wu = wave % {WU}, ww = wave / {WU};")
         s("(void)ww;")
         # rows of the identity: a product with them adds a tile of sums to another one, rounding to nearest
@@ -873,9 +882,8 @@ class SplitEmitter:
         s("#pragma unroll")
         s.open(f"for (int n = 0; n < {ny}; ++n)")
         s(f"const int at = min((tid >> 5) + 8 * n, {len(table) - 1});")
-        s(f"yc[n] = sign * {name}_c[at], yj[n] = {name}_j[at];")
+        s(f"yc[n] = sign * {coefficients}[at], yj[n] = {components}[at];")
         s.close()
-        s("const i64 nsteps = (num_batch + 31) / 32;")
 
         def rows_of(step):
             s(f"const i64 first = min((i64)({step}) * 32, num_batch - 1);")
@@ -996,20 +1004,21 @@ class SplitEmitter:
                     for ca, cb in TERMS for j in pair]
 
         # ---- the first step's operands
+        s.open("if (begin < nsteps)")
         s("float t[8];")
         s("unsigned ta[2][3][4], tg[3][4];")
         s(f"oeq_bf8 bg[{most}][3];")
         for q in subs:
             s(f"v4t tm{q.index}[{per(q)}];")
         s.open("")
-        rows_of("blockIdx.x")
+        rows_of("begin")
         for o in used_o:
             for e in range(8):
                 self.put(s, request_g(o, e))
         for a in used_a:
             for e in range(8):
                 self.put(s, request_x(a, e))
-        for n, step in enumerate(("blockIdx.x", "(i64)blockIdx.x + gridDim.x")):
+        for n, step in enumerate(("begin", "begin + gridDim.x")):
             s.open("")
             self.put(s, request_y(step))
             self.put(s, write_y(n))
@@ -1026,7 +1035,7 @@ class SplitEmitter:
         s("oeq_block_sync();")
         self.put(s, t_tasks(0))
         self.put(s, read_bg(0, pairs(stages[0][2])[0], "s_g[0]"))
-        s.open("for (i64 step = blockIdx.x; step < nsteps; step += gridDim.x, cur ^= 1)")
+        s.open("for (i64 step = begin; step < nsteps; step += gridDim.x, cur ^= 1)")
         # the step whose rows are requested, and written to LDS, during this one
         rows_of("step + gridDim.x")
         s("const int ynext = ycur == 2 ? 0 : ycur + 1, yput = ynext == 2 ? 0 : ynext + 1;")
@@ -1092,6 +1101,7 @@ class SplitEmitter:
                 if N % 2:
                     s("for (int c = 0; c < 3; ++c) for (int m = 0; m < 4; ++m) ta[0][c][m] = ta[1][c][m];")
         s.close()
+        s.close()
         s(f"float* prow = wpartial + (i64)blockIdx.x * {low.WN};")
         for q in subs:
             U, Wn = low.in1[q.p.i1].mul, low.out[q.p.io].mul
@@ -1102,4 +1112,3 @@ class SplitEmitter:
                 s(f"const int u = 16 * wu + 4 * lq + i, w = 16 * {nt} + l16;")
                 s(f"if (u < {U} && w < {Wn}) prow[{self.wpos(q, 'u', 'w')}] = {self.lit(q.unit)} * dw{q.index}[{j}][i];")
                 s.close()
-        s.close()
