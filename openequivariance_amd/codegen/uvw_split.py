@@ -35,7 +35,7 @@ kernels are also bound by power: random operands lower the clock (2.1 GHz, 2.4 o
 So the order of the instructions is written out (``interleave``): vector, LDS and memory instructions go between the matrix
 instructions that hide them, and what takes several is cut in steps (a split of eight values as one piece: 714 us for a pass through
 forward and backward, in steps 695); left to the compiler they clump, and registers spill. The pass: fp32 kernels
-1 061 us, these 719 with 35 products each and without the steps, 661 now.
+1 062 us, these 719 with 35 products each and without the steps, 647 now.
 """
 
 from __future__ import annotations
@@ -60,6 +60,9 @@ PARKED = 216
 # Two waves per SIMD (256 registers): up to this estimate. 64x0e+16x1o (x) 0e+1o -> the same, 150 000 rows, one wave / two:
 # forward 52 / 40 us, dX 71 / 54, dW 69 / 61.
 TWO_WAVES = 300
+# Operands of weights on their way from memory while one is split (64x{0e,1o,2e}, forward and backward, one after the other /
+# with these and the first tile's rows ahead: 4 500 rows 91 / 86 us, 20 000 173 / 167, 131 072 853 / 845).
+WEIGHTS_AHEAD = 6
 # Components of Y that dW reads from LDS ahead of their use.
 AHEAD = 4
 
@@ -298,34 +301,39 @@ class SplitEmitter:
         s("(void)lane; (void)wave; (void)l16; (void)lq;")
 
     # ------------------------------------------------------------- forward and dX
-    def weights(self, s: Src, kind: str, q: Sub, park: int = 0):
-        """B operands of a sub-path in registers: the lane's result channel 16 wave + lane % 16 and, of every 32
-        contracted channels, the eight from 8 (lane / 16) on; zeros past either block."""
+    def weights(self, s: Src, kind: str, subs, park: int = 0):
+        """B operands of the sub-paths in registers: the lane's result channel 16 wave + lane % 16 and, of every 32
+        contracted channels, the eight from 8 (lane / 16) on; zeros past either block. The first ``park`` registers of them go
+        to accumulation registers. Memory is WEIGHTS_AHEAD operands ahead of the splits."""
         A, T, ia, it = self.sides(kind)
-        a, t = A[ia(q)], T[it(q)]
-        ld = self.low.in2[q.p.i2].mul * self.low.out[q.p.io].mul
-        cu, ct = (ld, 1) if kind == "forward" else (1, ld)   # distance of two contracted / two result channels
-        base = q.p.woff + q.v * self.low.out[q.p.io].mul
-        S = c32(a.mul)
-        s(f"oeq_bf8 w{q.index}[{S}][3];")
-        s.open("")
-        s(f"const int t = min(16 * wave + l16, {t.mul - 1});")
-        for st in range(S):
-            s.open("")
-            s("float r[8];")
-            for e in range(8):
-                full = 32 * st + 32 <= a.mul
-                u = f"{32 * st + e} + 8 * lq"
-                val = f"{self.lit(q.unit)} * W[{base} + ({u if full else f'min({u}, {a.mul - 1})'}) * {cu} + t * {ct}]"
-                conds = ([] if t.mul >= 64 else [f"16 * wave + l16 < {t.mul}"]) + ([] if full else [f"{u} < {a.mul}"])
-                s(f"r[{e}] = " + (f"oeq_sel({' && '.join(conds)}, {val});" if conds else f"{val};"))
-            s(f"oeq_split8<1, 0>(r, w{q.index}[{st}]);")
-            if park > 0:
-                s(f"for (int c = 0; c < 3; ++c) w{q.index}[{st}][c] = oeq_park(w{q.index}[{st}][c]);")
-            park -= 12
-            s("__builtin_amdgcn_sched_barrier(0);")
-            s.close()
-        s.close()
+        loads, splits = [], []
+        for q in subs:
+            a, t, S = A[ia(q)], T[it(q)], c32(A[ia(q)].mul)
+            ld = self.low.in2[q.p.i2].mul * self.low.out[q.p.io].mul
+            cu, ct = (ld, 1) if kind == "forward" else (1, ld)   # distance of two contracted / two result channels
+            base = q.p.woff + q.v * self.low.out[q.p.io].mul
+            s(f"oeq_bf8 w{q.index}[{S}][3];")
+            for st in range(S):
+                r = f"r{q.index}_{st}"
+                get, use = [f"float {r}[8];"], []
+                for e in range(8):
+                    full = 32 * st + 32 <= a.mul
+                    u = f"{32 * st + e} + 8 * lq"
+                    get.append(f"{r}[{e}] = W[{base} + ({u if full else f'min({u}, {a.mul - 1})'}) * {cu} + min(16 * wave + l16, {t.mul - 1}) * {ct}];")
+                    conds = ([] if t.mul >= 64 else [f"16 * wave + l16 < {t.mul}"]) + ([] if full else [f"{u} < {a.mul}"])
+                    val = f"{self.lit(q.unit)} * {r}[{e}]"
+                    use.append(f"{r}[{e}] = " + (f"oeq_sel({' && '.join(conds)}, {val});" if conds else f"{val};"))
+                use.append(f"oeq_split8<1, 0>({r}, w{q.index}[{st}]);")
+                if park > 0:
+                    use.append(f"for (int c = 0; c < 3; ++c) w{q.index}[{st}][c] = oeq_park(w{q.index}[{st}][c]);")
+                park -= 12
+                loads.append(get)
+                splits.append(use)
+        for n in range(-WEIGHTS_AHEAD, len(loads)):
+            for line in (loads[n + WEIGHTS_AHEAD] if n + WEIGHTS_AHEAD < len(loads) else []) + (splits[n] if n >= 0 else []):
+                s(line)
+            if n >= 0:
+                s("__builtin_amdgcn_sched_barrier(0);")
 
     def rows_request(self, kind: str, a: int, st: int):
         """ra<a>_<st>: two neighbouring channels of one of the tile's 16 rows, for the thread to split (in scope:
@@ -460,9 +468,6 @@ class SplitEmitter:
         s("const int put = 4 * (((tid & 15) >> 2) * 16 + (((tid >> 4) + 4 * ((tid & 15) >> 2)) & 15)) + (tid & 3);")
         s("const int get = 4 * (lq * 16 + ((l16 + 4 * lq) & 15));")
         park = PARKED if self.waves(kind) == 1 else 0
-        for q in subs:
-            self.weights(s, kind, q, park)
-            park -= 12 * c32(A[ia(q)].mul)
         for a in used_a:
             for st in range(c32(A[a].mul)):
                 s(f"float ra{a}_{st}[{2 * A[a].d}];")
@@ -526,7 +531,6 @@ class SplitEmitter:
             return out
 
         units = [(a, st) for a in used_a for st in range(c32(A[a].mul))]
-        s.open("")
         where("(i64)blockIdx.x", "const i64 ")
         s(f"const float* rows = {src} + first * {LA};")
         s(f"const unsigned own = (unsigned)min(tid >> 4, end) * {4 * LA}u;")
@@ -538,10 +542,10 @@ class SplitEmitter:
             s("const int xend = end;")
             for t in used_t:
                 self.put(s, request_x(t))
+        self.weights(s, kind, subs, park)   # (the first tile's rows are on their way meanwhile)
         for a, st in units:
             self.put(s, write(a, st, "s_a[0]"))
         write_y("0")
-        s.close()
         s.open("")
         where("((i64)blockIdx.x + gridDim.x)", "const i64 ")
         s(f"const float* rows = {src} + first * {LA};")
