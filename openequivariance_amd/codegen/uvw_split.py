@@ -23,9 +23,9 @@ frequent coefficient of a path is a factor of its weights (``Sub.unit``).
   the waves through LDS in wave order. As few kernels as the registers allow (``SplitEmitter.plan``).
 * dW: wave w owns input channels 16 w .. 16 w + 15, contracts X and Y for them in registers, eight rows a lane, in the
   layout of the A operand; the output gradient's operands are split once per block. Products of 32 rows are summed from zero
-  and then added to the running sums by fp32 matrix instructions with the identity. The bf16 instruction cuts off what it aligns,
+  and then added to the running sums. The bf16 instruction cuts off what it aligns,
   always downwards, and running sums of 12 steps drift by that: every second block works on negated values,
-  which the identity (with the same sign) turns back (dW above: 1.5e-6 on the running sums directly, 5.4e-7 from zero, 2.3e-7
+  which the addition turns back (dW above: 1.5e-6 on the running sums directly, 5.4e-7 from zero, 2.3e-7
   with the signs, 1.7e-7 with the folds). Y lies in LDS times the coefficients it is met with, as zeros past the batch.
 
 What bounds them (MI355X, the problem above, 100 003 rows): the registers of a SIMD hold one wave of these kernels, and
@@ -35,7 +35,7 @@ kernels are also bound by power: random operands lower the clock (2.1 GHz, 2.4 o
 So the order of the instructions is written out (``interleave``): vector, LDS and memory instructions go between the matrix
 instructions that hide them, and what takes several is cut in steps (a split of eight values as one piece: 714 us for a pass through
 forward and backward, in steps 695); left to the compiler they clump, and registers spill. The pass: fp32 kernels
-1 062 us, these 719 with 35 products each and without the steps, 647 now.
+1 062 us, these 719 with 35 products each and without the steps, 630 now.
 """
 
 from __future__ import annotations
@@ -864,10 +864,7 @@ class SplitEmitter:
         s(f"float (* const s_y)[{len(table)}][32] = (float (*)[{len(table)}][32])(s_lds + {2 * total});")
         s(f"const int wu = wave % {WU}, ww = wave / {WU};")
         s("(void)ww;")
-        # rows of the identity: a product with them adds a tile of sums to another one, rounding to nearest
         s("const float sign = (blockIdx.x & 1) ? -1.0f : 1.0f;")
-        s("float eye[4];")
-        s("for (int i = 0; i < 4; ++i) eye[i] = l16 == 4 * lq + i ? sign : 0.0f;")
         for q in subs:
             s(f"v4t dw{q.index}[{per(q)}];")
             for j in range(per(q)):
@@ -1002,6 +999,11 @@ class SplitEmitter:
         most = max(per(q) for q in subs)
         pairs = lambda q: [list(range(j, min(j + 2, per(q)))) for j in range(0, per(q), 2)]
 
+        # A step's products into the running sums. By fp32 matrix instructions with the identity, which spare the moves out of the
+        # accumulation registers but keep the vector unit for 32 cycles a value where an addition and its moves take 14: dW
+        # 298 us, 281 by additions (64x{0e,1o,2e}, 100 003 rows; the pass 642 -> 630, 20 000 rows 165 -> 159).
+        flush = lambda p, j: " ".join(f"dw{p.index}[{j}][{i}] += sign * tm{p.index}[{j}][{i}];" for i in range(4))
+
         def lead(n, pair):
             o, k, q = stages[n]
             return [f"tm{q.index}[{j}] = oeq_mfma_bf({operand(f'ta[{n % 2}][{ca}]')}, bg[{j}][{cb}], tm{q.index}[{j}], 0, 0, 0);"
@@ -1072,8 +1074,7 @@ class SplitEmitter:
                 tasks += [(1, " ".join(f"x{a}[{e}][{i}] = xn{a}[{e}][{i}];" for i in range(low.in1[a].d)))
                           for a in used_a for e in range(8)]
             tasks += t_tasks(n + 1)
-            flush = [f"dw{p.index}[{j}] = oeq_mfma(eye[{i}], tm{p.index}[{j}][{i}], dw{p.index}[{j}], 0, 0, 0);"
-                     for p in pending for i in range(4) for j in range(per(p))]
+            tasks = [(4, flush(p, j)) for p in pending for j in range(per(p))] + tasks
             pending = [q] if n == places[q.index][-1] else []
             seq = [lead(n, pair) for pair in ps]
             # operands of this group that are not there yet (its second half), and the next group's first half once
@@ -1093,14 +1094,13 @@ class SplitEmitter:
                     extra = read_bg(n, ps[m + 1], buf)
                 if new_group and m > 0 and m == len(ps) - 1:
                     extra = extra + read_bg(n + 1, pairs(stages[(n + 1) % N][2])[0], nbuf)
-                self.interleave(s, seq[m] + (flush if m + 1 == len(seq) else []), extra + cut[m])
+                self.interleave(s, seq[m], extra + cut[m])
             if new_group and len(ps) == 1:
                 self.put(s, read_bg(n + 1, pairs(stages[(n + 1) % N][2])[0], nbuf))
             if n + 1 == N:
                 for p in pending:
-                    for i in range(4):
-                        for j in range(per(p)):
-                            s(f"dw{p.index}[{j}] = oeq_mfma(eye[{i}], tm{p.index}[{j}][{i}], dw{p.index}[{j}], 0, 0, 0);")
+                    for j in range(per(p)):
+                        s(flush(p, j))
                 s("ycur = ynext;")
                 if N % 2:
                     s("for (int c = 0; c < 3; ++c) for (int m = 0; m < 4; ++m) ta[0][c][m] = ta[1][c][m];")
