@@ -38,3 +38,48 @@ def test_double_precision_rows(channels):
     assert not got[-1].any()
     # a sum of some twenty terms: as many roundings of 2^-53
     assert float((got - want).abs().max()) <= 64 * 2.0 ** -53 * float(want.abs().max())
+
+
+def _wide(dtype, channels=64):
+    out = [(0, 0, 0), (1, 1, 0), (0, 1, 1), (1, 0, 1), (1, 2, 1), (0, 2, 2), (1, 1, 2), (1, 2, 2)]  # l of the three irreps
+    return oeq.TPProblem(f"{channels}x0e+{channels}x1o", "1x0e+1x1o+1x2e",
+                         "+".join(f"{channels}x{l}{'oe'[(a + b) % 2 == 0]}" for a, b, l in out),
+                         [(a, b, n, "uvu", True) for n, (a, b, _) in enumerate(out)],
+                         shared_weights=False, internal_weights=False, label="default-mode-terms",
+                         irrep_dtype=dtype, weight_dtype=dtype)
+
+
+@pytest.mark.parametrize("channels", [32, 64, 128])
+def test_floats_are_added_by_atomics_and_doubles_in_order(channels):
+    """Edges in any order. Rows that a wave's atomics cover without holes; others are summed in order in both precisions."""
+    from openequivariance_amd import runtime as rt
+    from openequivariance_amd._torch.tensor_product_conv import build_conv_module
+    modes = [build_conv_module(_wide(dtype, channels), False)[1]["dx_mode"] for dtype in (np.float32, np.float64)]
+    assert modes == [rt.DX_ATOMIC, rt.DX_TERMS]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("channels,nodes,edges", [(32, 40, 700), (64, 37, 900), (64, 9000, 20000), (128, 40, 700)])
+def test_double_precision_default_mode(channels, nodes, edges):
+    """Unsorted edges, the first half of them from one sender (more than a chunk of its sum holds), none from the last node; the
+    index in one launch, and in slices. Two passes agree in every bit."""
+    problem = _wide(np.float64, channels)
+    rng = np.random.default_rng(channels + nodes)
+    rows, cols = rng.integers(0, nodes, edges), rng.integers(0, nodes - 1, edges)
+    cols[:edges // 2] = 3
+    shuffle = rng.permutation(edges)
+    rows, cols = (torch.from_numpy(v[shuffle]).cuda() for v in (rows, cols))
+    gen = torch.Generator(device="cuda").manual_seed(channels)
+    x, y, w, g = (torch.randn(*s, generator=gen, device="cuda", dtype=torch.float64) for s in
+                  ((nodes, problem.irreps_in1.dim), (edges, 9), (edges, problem.weight_numel), (nodes, problem.irreps_out.dim)))
+    leaves = tuple(t.requires_grad_(True) for t in (x, y, w))
+    conv = oeq.TensorProductConv(problem)
+    got = torch.autograd.grad(conv(x, y, w, rows, cols), leaves, g)
+    again = torch.autograd.grad(conv(x, y, w, rows.clone(), cols.clone()), leaves, g)
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
+    want = torch.autograd.grad(oeq.TensorProduct(problem)(x[cols], y, w), leaves, g[rows])
+    assert not got[0][-1].any()
+    # sums of up to n terms, in another order: their roundings add up to n 2^-53 of the terms' sizes at most
+    n = int(torch.bincount(cols).max()) + 16
+    for a, b in zip(got, want):
+        assert float((a - b).abs().max()) <= n * 2.0 ** -53 * float(b.abs().max())
