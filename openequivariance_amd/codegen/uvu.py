@@ -3232,7 +3232,9 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     xcd = max(1, t["conv_xcd"])
     xcd_b = 1 if (walk and low.shared_weights) else xcd  # bounded grid: one partial dW row per wave group
     gres = None if t["conv_gres"] < 0 else bool(t["conv_gres"])
-    sender_walk = (9 * low.L1 >= 2 * (low.WN + low.L2 + low.L3) and not low.shared_weights and t["conv_dxm"] < 0
+    # (the ratio up to which it pays: see where dx_mode is chosen)
+    sender_ratio = (9 if low.elem_size == 4 else 7) / 2
+    sender_walk = (sender_ratio * low.L1 >= low.WN + low.L2 + low.L3 and not low.shared_weights and t["conv_dxm"] < 0
                    and t["conv_dxs"] < 0) or t["conv_dxs"] > 0
     forward_groups = width_groups = None
     # A wave per width pays where the row of all widths is much for one wave. Backward: two widths, whose waves wait for each
@@ -3303,7 +3305,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
             # (only where a row fills the wave and the atomics go through the LDS transpose, 64 consecutive
             # floats per instruction: per-lane atomics of packed or ragged rows are several times slower than
             # the ordered reduction)
-            # Single precision only: atomics on doubles run at 1.1 TB/s of the terms (mace-large 1 500 nodes x 32 edges, a step
+            # Single precision only: atomics on doubles take longer than the terms written and read again (mace-large 1 500 nodes x 32 edges, a step
             # 1 411 us by atomics, 837 by terms; 100 x 20 121 / 106, 3 000 x 40 3 481 / 2 031, 12 000 x 32 10 660 / 6 464;
             # mace-medium 300 x 30 147 / 107, 12 000 x 16 1 810 / 1 445; NequIP lips 1 000 x 24 475 / 338; SevenNet's first
             # layer 2 000 x 24 213 / 194). Floats: mace-large 300 x 40 125 / 159, 6 001 x 32 1 281 / 1 525, lips 1 000 x 24
@@ -3323,8 +3325,12 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
             # kernel of the adjoint problem (lower.adjoint). Measured over 128 problems on the config-5 graph,
             # backward op: ratio (WN + L2 + L3) / L1 of 1.1 .. 3.5: -16 % .. -57 %; 4.0 (NequIP aspirin, water):
             # -5 %; 4.6: -2 % .. -6 %; 5.1: +-3 %; 5.3 and more: slower, +27 % at config 5 (7.6).
-            auto = 9 * low.L1 >= 2 * (low.WN + low.L2 + low.L3) and not low.shared_weights and t["conv_dxm"] < 0
-            if (t["conv_dxs"] > 0) or (t["conv_dxs"] < 0 and auto):
+            # Double precision, where the terms are streamed at the rate of single precision but the second walk's
+            # forward kernel is slower: step, us, walk / terms, ratio 1 12 000 nodes x 20 edges 318 / 440; 2 (64x{0e,1o,2e})
+            # 1 500 x 30 164 / 196, 12 000 x 20 883 / 978; 3 (64x{0e,1o}) 109 / 112 and 574 / 559, (128x{0e,1o}) 199 / 208 and
+            # 1 124 / 1 079; 4 136 / 124 and 697 / 627, (128x{0e,1o}) 246 / 235 and 1 372 / 1 214, NequIP aspirin 1 000 x 24
+            # 169 / 162, 4 000 x 24 564 / 517, water 1 500 x 35 164 / 166, 20 000 x 20 1 167 / 1 043.
+            if sender_walk:
                 dx_mode = em.DX_SENDER_WALK
         if dx_mode == em.DX_ATOMIC and walk and low.elem_size == 4 and t["conv_wb"] == 2 and "conv_wb" not in user_tune:
             # With the dX terms leaving as atomics a third wave per SIMD pays where the compiler finds the registers

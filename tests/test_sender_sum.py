@@ -83,3 +83,16 @@ def test_double_precision_default_mode(channels, nodes, edges):
     n = int(torch.bincount(cols).max()) + 16
     for a, b in zip(got, want):
         assert float((a - b).abs().max()) <= n * 2.0 ** -53 * float(b.abs().max())
+
+
+@pytest.mark.parametrize("dtype,paths,walk", [(np.float32, 5, True), (np.float64, 4, True), (np.float64, 5, False)])
+def test_up_to_which_ratio_the_senders_are_walked(dtype, paths, walk):
+    """Words of an edge's weights and an output row against those of an X row: 3 with four paths, 4 with five."""
+    from openequivariance_amd import runtime as rt
+    from openequivariance_amd._torch.tensor_product_conv import build_conv_module
+    ins = [(0, 0, 0, "uvu", True), (0, 1, 1, "uvu", True), (1, 0, 2, "uvu", True), (1, 1, 3, "uvu", True), (1, 1, 4, "uvu", True)]
+    out = ["64x0e", "64x1o", "64x1o", "64x0e", "64x1e"]
+    problem = oeq.TPProblem("64x0e+64x1o", "1x0e+1x1o", "+".join(out[:paths]), ins[:paths], shared_weights=False,
+                            internal_weights=False, label="sender-ratio", irrep_dtype=dtype, weight_dtype=dtype)
+    for deterministic in (False, True):
+        assert (build_conv_module(problem, deterministic)[1]["dx_mode"] == rt.DX_SENDER_WALK) == walk
