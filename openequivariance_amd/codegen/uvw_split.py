@@ -688,8 +688,10 @@ class SplitEmitter:
                 tasks += write(ua, ust, "s_a[cur ^ 1]")
                 tasks += request(ua, ust)
             tasks += contract((n or N) - 1)
-            if n == min(1, N - 1):
+            if n == min(1, N - 2):
+                # (before the tile's barrier: the next tile's first step writes these shares over)
                 tasks += take
+            if n == min(1, N - 1):
                 if not fwd:
                     # X of the next tile, whose registers this tile's has left beside the step before
                     s("const i64 xfirst = min((tile + gridDim.x) * 16, num_batch - 1);")

@@ -32,6 +32,8 @@ CASES = [
     ("odd-channels", lambda: _shared("33x0e+17x1o", "1x0e+1x1o", "15x0e+7x1o"), 2, 2),
     ("two-channel-second-operand", lambda: _shared("64x0e+32x1o", "3x0e+2x1o", "64x0e+32x1o"), 1, 1),
     ("gaps", _gaps, 2, 1),
+    # two components of the output: two steps of dX's pipeline
+    ("two-scalars", lambda: _shared("64x0e+64x1o", "1x0e+1x1o", "64x0e+32x0e"), 2, 2),
 ]
 
 
@@ -51,9 +53,22 @@ def test_plan_covers_every_sub_path_once(name, make, wf, wb):
     assert "oeq_split3(" in src and any(d[1] == "backward_w" for d in descs)
 
 
+@pytest.mark.parametrize("name,make,wf,wb", CASES, ids=[c[0] for c in CASES])
+def test_shares_of_dy_are_read_before_the_barrier(name, make, wf, wb):
+    """A tile's step 0 writes the shares that the tile before reads: not one read of them past that tile's barrier."""
+    loops = build_tp_module(make())[0].split("tile += gridDim.x, cur ^= 1)")[1:]
+    found = 0
+    for loop in loops:
+        loop = loop[:loop.index("prow0 = row0;")]
+        reads = [at for at in range(len(loop)) if loop.startswith("s_dy[cur][", at)]
+        found += len(reads)
+        assert loop.count("oeq_block_sync();") == 1 and all(at < loop.index("oeq_block_sync();") for at in reads)
+    assert found
+
+
 # (problem, sub-paths contracted before the product in the forward, and in each kernel of dW)
 FOLDS = [("l2-64", 2, [0, 1, 1]), ("l2-32", 2, [2]), ("l1-64-16", 1, [1]), ("odd-channels", 1, [1]),
-         ("two-channel-second-operand", 2, [2]), ("gaps", 1, [1])]
+         ("two-channel-second-operand", 2, [2]), ("gaps", 1, [1]), ("two-scalars", 1, [0])]
 
 
 @pytest.mark.parametrize("name,forward,dw", FOLDS, ids=[f[0] for f in FOLDS])
