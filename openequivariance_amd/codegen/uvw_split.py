@@ -92,7 +92,8 @@ class Sub:
         l = 2): a factor of the weights, before they are split, or of their gradient, after the sums."""
         sizes = Counter(f"{abs(c):.12g}" for *_, c in self.p.nnz)
         most = max(sizes.values())
-        return next(abs(c) for *_, c in self.p.nnz if sizes[f"{abs(c):.12g}"] == most)
+        # (a path of weight zero keeps its coefficients, all of them zero)
+        return next(abs(c) for *_, c in self.p.nnz if sizes[f"{abs(c):.12g}"] == most) or 1.0
 
     def ratio(self, c: float) -> float:
         return float(f"{abs(c) / self.unit:.12g}")

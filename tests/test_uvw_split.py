@@ -24,6 +24,12 @@ def _gaps():  # an input irrep that no path reads, an output irrep that no path 
                           (1, 1, 0, "uvw", True)], shared_weights=True, internal_weights=False, label="split-gaps")
 
 
+def _zero_weight():  # a path that contributes nothing, and whose weights get no gradient
+    return oeq.TPProblem("64x0e+64x1o", "1x0e+1x1o", "64x0e+64x1o",
+                         [(0, 0, 0, "uvw", True), (0, 1, 1, "uvw", True, 0.0), (1, 0, 1, "uvw", True)],
+                         shared_weights=True, internal_weights=False, label="split-zero-weight")
+
+
 # (name, problem, waves per SIMD of forward and backward)
 CASES = [
     ("l2-64", P.config4_uvw_shared, 1, 1),
@@ -32,6 +38,7 @@ CASES = [
     ("odd-channels", lambda: _shared("33x0e+17x1o", "1x0e+1x1o", "15x0e+7x1o"), 2, 2),
     ("two-channel-second-operand", lambda: _shared("64x0e+32x1o", "3x0e+2x1o", "64x0e+32x1o"), 1, 1),
     ("gaps", _gaps, 2, 1),
+    ("zero-path-weight", _zero_weight, 2, 1),
     # two components of the output: two steps of dX's pipeline
     ("two-scalars", lambda: _shared("64x0e+64x1o", "1x0e+1x1o", "64x0e+32x0e"), 2, 2),
 ]
@@ -68,7 +75,7 @@ def test_shares_of_dy_are_read_before_the_barrier(name, make, wf, wb):
 
 # (problem, sub-paths contracted before the product in the forward, and in each kernel of dW)
 FOLDS = [("l2-64", 2, [0, 1, 1]), ("l2-32", 2, [2]), ("l1-64-16", 1, [1]), ("odd-channels", 1, [1]),
-         ("two-channel-second-operand", 2, [2]), ("gaps", 1, [1]), ("two-scalars", 1, [0])]
+         ("two-channel-second-operand", 2, [2]), ("gaps", 1, [1]), ("two-scalars", 1, [0]), ("zero-path-weight", 0, [1])]
 
 
 @pytest.mark.parametrize("name,forward,dw", FOLDS, ids=[f[0] for f in FOLDS])
