@@ -96,3 +96,22 @@ def test_up_to_which_ratio_the_senders_are_walked(dtype, paths, walk):
                             internal_weights=False, label="sender-ratio", irrep_dtype=dtype, weight_dtype=dtype)
     for deterministic in (False, True):
         assert (build_conv_module(problem, deterministic)[1]["dx_mode"] == rt.DX_SENDER_WALK) == walk
+
+
+@pytest.mark.parametrize("dtype,instruction", [(np.float32, "global_atomic_add_f32"), (np.float64, "global_atomic_add_f64")])
+def test_atomics_are_one_instruction(dtype, instruction, tmp_path, monkeypatch):
+    """Not a loop of compare-and-swap, whichever compiler it is."""
+    import subprocess
+    from pathlib import Path
+    from openequivariance_amd import runtime as rt
+    from openequivariance_amd._torch.tensor_product_conv import build_conv_module
+    objdump = Path("/opt/rocm/llvm/bin/llvm-objdump")
+    if not objdump.exists():
+        pytest.skip("no disassembler")
+    monkeypatch.setenv("OEQ_AMD_TUNE", "conv_dxm=1")
+    code = rt.unpack_code(rt.compile_source(build_conv_module(_wide(dtype, 64), False)[0]))
+    text = ""
+    for n, blob in enumerate(code):
+        (tmp_path / f"{n}.co").write_bytes(blob)
+        text += subprocess.run([objdump, "-d", "--mcpu=gfx950", tmp_path / f"{n}.co"], capture_output=True, text=True, check=True).stdout
+    assert instruction in text and "cmpswap" not in text
