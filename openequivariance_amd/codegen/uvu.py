@@ -3305,14 +3305,18 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
             # (only where a row fills the wave and the atomics go through the LDS transpose, 64 consecutive
             # floats per instruction: per-lane atomics of packed or ragged rows are several times slower than
             # the ordered reduction)
-            # Single precision only: atomics on doubles take longer than the terms written and read again (mace-large 1 500 nodes x 32 edges, a step
-            # 1 411 us by atomics, 837 by terms; 100 x 20 121 / 106, 3 000 x 40 3 481 / 2 031, 12 000 x 32 10 660 / 6 464;
-            # mace-medium 300 x 30 147 / 107, 12 000 x 16 1 810 / 1 445; NequIP lips 1 000 x 24 475 / 338; SevenNet's first
-            # layer 2 000 x 24 213 / 194). Floats: mace-large 300 x 40 125 / 159, 6 001 x 32 1 281 / 1 525, lips 1 000 x 24
-            # 134 / 141, mace-uvu 8 000 x 32 2 596 / 3 007, SevenNet's first layer 8 000 x 32 393 / 440.
+            # Atomics / terms, a step, us: mace-large 300 nodes x 40 edges 125 / 159, 6 001 x 32 1 281 / 1 525, lips 1 000 x 24
+            # 134 / 141, mace-uvu 8 000 x 32 2 596 / 3 007, SevenNet's first layer 8 000 x 32 393 / 440; double precision
+            # mace-large 300 x 16 175 / 190, 1 500 x 32 760 / 837, 12 000 x 32 5 910 / 6 524, mace-medium 3 000 x 40 730 / 874,
+            # lips 1 000 x 24 323 / 340, 3 000 x 40 1 135 / 1 225, mace-uvu 50 000 x 32 36.2 / 40.7 ms, SevenNet's first
+            # layer 2 000 x 24 177 / 196.
             coalesced = bool(t["conv_tra"]) and em._atomics_coalesce() and not em.ir_mul
+            # (in order all the same up to the ratio that single precision walks the senders to, where torch's deterministic
+            # algorithms may be asked of this mode)
+            in_order = low.elem_size == 8 and not low.shared_weights and t["conv_dxs"] < 0 and \
+                9 * low.L1 >= 2 * (low.WN + low.L2 + low.L3)
             dx_mode = t["conv_dxm"] if t["conv_dxm"] >= 0 else (
-                em.DX_ATOMIC if (mode == rt.CONV_GROUPED and coalesced and low.elem_size == 4) else em.DX_TERMS)
+                em.DX_ATOMIC if (mode == rt.CONV_GROUPED and coalesced and not in_order) else em.DX_TERMS)
             # arrival counting keeps an edge's terms lane-major, 64 values per (block, component) and chunk: they
             # fit the edge's row of dx_tmp only when no used block has lanes without a channel
             if dx_mode == em.DX_ARRIVAL and (em.R != 1 or 64 * em.NCH * em._term_slots()[1] > low.L1):
