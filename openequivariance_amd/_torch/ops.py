@@ -252,6 +252,21 @@ def _resolve(kid: int, spec: Optional[torch.Tensor]):
         second_order_kid=e.second_order_kid or 0, owner=e))
 
 
+def _without_terms(kid: int) -> int:
+    """Called by the native ops where a convolution's backward pass has no room for its terms per edge: the kernel set
+    of the same problem that walks the senders instead, where that is what the terms are the faster form of
+    (codegen/uvu.py: terms_for_walk); else 0."""
+    from ..codegen.lower import lower
+    from ..codegen.uvu import terms_for_walk
+    from ..core.spec import problem_from_dict
+    desc = json.loads(bytes(get_entry(kid).spec.tolist()).decode())
+    if desc["kind"] != "conv" or any(k in desc["tune"] for k in ("conv_dxs", "conv_dxm")) or \
+            not terms_for_walk(lower(problem_from_dict(desc["problem"]))):
+        return 0
+    walk = dict(desc, tune=(desc["tune"] + "," if desc["tune"] else "") + "conv_dxs=1")
+    return register_spec(json.dumps(walk, sort_keys=True, separators=(",", ":")).encode())
+
+
 # ---------------------------------------------------------------------------
 # batch tensor product
 # ---------------------------------------------------------------------------
@@ -597,7 +612,7 @@ def _conv_second_order(operands, cotangents, kid, spec):
 
 if _native is not None:
     _native.set_callbacks(dict(
-        resolve=_resolve, check_edges=_check_edges, build_index=_build_index, conv_forward=_composed_forward,
+        resolve=_resolve, without_terms=_without_terms, check_edges=_check_edges, build_index=_build_index, conv_forward=_composed_forward,
         conv_backward=_composed_backward, conv_double_backward=_composed_double_backward,
         tp_second_order=_tp_second_order, conv_second_order=_conv_second_order, error_type=rt.OeqError))
 

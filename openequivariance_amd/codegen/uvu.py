@@ -3233,9 +3233,8 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
     xcd_b = 1 if (walk and low.shared_weights) else xcd  # bounded grid: one partial dW row per wave group
     gres = None if t["conv_gres"] < 0 else bool(t["conv_gres"])
     # (the ratio up to which it pays: see where dx_mode is chosen)
-    sender_ratio = (9 if low.elem_size == 4 else 7) / 2
-    sender_walk = (sender_ratio * low.L1 >= low.WN + low.L2 + low.L3 and not low.shared_weights and t["conv_dxm"] < 0
-                   and t["conv_dxs"] < 0) or t["conv_dxs"] > 0
+    sender_walk = (9 * low.L1 >= 2 * (low.WN + low.L2 + low.L3) and not terms_for_walk(low) and not low.shared_weights
+                   and t["conv_dxm"] < 0 and t["conv_dxs"] < 0) or t["conv_dxs"] > 0
     forward_groups = width_groups = None
     # A wave per width pays where the row of all widths is much for one wave. Backward: two widths, whose waves wait for each
     # other least, and more than the smallest rows (step, us, one wave / a wave per width, by the estimate of that one
@@ -3313,8 +3312,7 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
             coalesced = bool(t["conv_tra"]) and em._atomics_coalesce() and not em.ir_mul
             # (in order all the same up to the ratio that single precision walks the senders to, where torch's deterministic
             # algorithms may be asked of this mode)
-            in_order = low.elem_size == 8 and not low.shared_weights and t["conv_dxs"] < 0 and \
-                9 * low.L1 >= 2 * (low.WN + low.L2 + low.L3)
+            in_order = terms_for_walk(low) and t["conv_dxs"] < 0
             dx_mode = t["conv_dxm"] if t["conv_dxm"] >= 0 else (
                 em.DX_ATOMIC if (mode == rt.CONV_GROUPED and coalesced and not in_order) else em.DX_TERMS)
             # arrival counting keeps an edge's terms lane-major, 64 values per (block, component) and chunk: they
@@ -3500,6 +3498,14 @@ def conv_module(low: Lowered, deterministic: bool, compute_units: int = 256, kah
                 return half
         descs = _small_graph_rules(src, descs, splits, compute_units, t, low.shared_weights, em.R, bool(forward_groups))
     return src, dims, descs
+
+
+def terms_for_walk(low: Lowered) -> bool:
+    """Whether sender gradients go through terms per edge where single precision walks the senders (the figures are
+    where conv_module chooses dx_mode). The walk needs no scratch memory: a call without room for the terms, L1 words an
+    edge, falls back on it."""
+    words = low.WN + low.L2 + low.L3
+    return low.mode == "uvu" and low.elem_size == 8 and not low.shared_weights and 7 * low.L1 < 2 * words <= 9 * low.L1
 
 
 class Split(NamedTuple):

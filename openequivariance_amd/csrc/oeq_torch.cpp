@@ -66,7 +66,7 @@ std::shared_mutex g_entries_mu;
 
 // Python functions of _torch/ops.py; held until the process ends (no destructor runs after the interpreter's).
 struct Callbacks {
-    py::object resolve, check_edges, build_index, conv_forward, conv_backward, conv_double_backward, tp_second_order,
+    py::object resolve, without_terms, check_edges, build_index, conv_forward, conv_backward, conv_double_backward, tp_second_order,
         conv_second_order, error_type;
 };
 Callbacks* g_py = nullptr;
@@ -82,6 +82,13 @@ EntryRef entry_of(int64_t kid, const OptTensor& spec) {
         g_py->resolve(kid, spec.has_value() ? py::cast(*spec) : py::object(py::none()));
     }
     TORCH_CHECK(false, "kernel id ", kid, " could not be registered");
+}
+
+// The kernel set of the same problem whose backward pass keeps no terms per edge in scratch memory, for a call that has
+// no room for them; 0: none.
+int64_t without_terms(int64_t kid) {
+    py::gil_scoped_acquire gil;
+    return g_py->without_terms(kid).cast<int64_t>();
 }
 
 void check(int rc, const char* what) {
@@ -426,7 +433,14 @@ Tensor3 conv_backward_gpu(const Tensor& L1_in, const Tensor& L2_in, const Tensor
     const Index ix = conv_index(e, kid, n, r, c, p, e.dx_mode != OEQ_DX_ATOMIC);
     const size_t nb = oeq_conv_backward_scratch_bytes(e.k, n.nodes, n.edges);
     Tensor ws;
-    if (nb) ws = scratch(x, nb);
+    try {
+        if (nb) ws = scratch(x, nb);
+    } catch (const c10::OutOfMemoryError&) {
+        const int64_t other = e.dx_mode == OEQ_DX_TERMS ? without_terms(kid) : 0;
+        if (!other) throw;
+        dx = dy = dw = Tensor();
+        return conv_backward_gpu(L1_in, L2_in, W, L3_grad, rows, cols, transpose_perm, other, std::nullopt);
+    }
     check(oeq_conv_backward_indexed(e.k, n.nodes, n.edges, x.data_ptr(), dx.data_ptr(), y.data_ptr(), dy.data_ptr(),
                                     w.data_ptr(), dw.data_ptr(), g.data_ptr(), r.data_ptr<int64_t>(),
                                     c.data_ptr<int64_t>(), pp, ix.data.data_ptr(), ix.data.numel(), ix.sender_side,
@@ -740,6 +754,7 @@ PYBIND11_MODULE(_oeq_torch, m) {
     m.def("set_callbacks", [](py::dict fns) {
         auto* c = new Callbacks();
         c->resolve = fns["resolve"];
+        c->without_terms = fns["without_terms"];
         c->check_edges = fns["check_edges"];
         c->build_index = fns["build_index"];
         c->conv_forward = fns["conv_forward"];

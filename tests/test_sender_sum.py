@@ -115,3 +115,39 @@ def test_atomics_are_one_instruction(dtype, instruction, tmp_path, monkeypatch):
         (tmp_path / f"{n}.co").write_bytes(blob)
         text += subprocess.run([objdump, "-d", "--mcpu=gfx950", tmp_path / f"{n}.co"], capture_output=True, text=True, check=True).stdout
     assert instruction in text and "cmpswap" not in text
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("deterministic", [False, True])
+def test_no_room_for_the_terms(deterministic):
+    """Double precision at a ratio of 4, where the terms are the faster form: without room for them the senders are walked."""
+    channels, edges, nodes = 64, 60000, 2000
+    ins = [(0, 0, 0, "uvu", True), (0, 1, 1, "uvu", True), (1, 0, 2, "uvu", True), (1, 1, 3, "uvu", True), (1, 1, 4, "uvu", True)]
+    problem = oeq.TPProblem(f"{channels}x0e+{channels}x1o", "1x0e+1x1o", "+".join(f"{channels}x{r}" for r in ("0e", "1o", "1o", "0e", "1e")),
+                            ins, shared_weights=False, internal_weights=False, label="no-room", irrep_dtype=np.float64,
+                            weight_dtype=np.float64)
+    rng = np.random.default_rng(5)
+    rows, cols = np.sort(rng.integers(0, nodes, edges)), rng.integers(0, nodes, edges)
+    order = np.lexsort((cols, rows))
+    rows, cols = rows[order], cols[order]
+    where = [torch.from_numpy(v).cuda() for v in (rows, cols, np.argsort(cols, kind="stable"))][:3 if deterministic else 2]
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    x, y, w, g = (torch.randn(*s, generator=gen, device="cuda", dtype=torch.float64) for s in
+                  ((nodes, problem.irreps_in1.dim), (edges, 4), (edges, problem.weight_numel), (nodes, problem.irreps_out.dim)))
+    leaves = tuple(t.requires_grad_(True) for t in (x, y, w))
+    conv = oeq.TensorProductConv(problem, deterministic=deterministic)
+    backward = lambda: torch.autograd.grad(conv(*leaves, *where), leaves, g)
+    want = backward()
+    terms = edges * problem.irreps_in1.dim * 8  # bytes; the results take nearly as many again
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + sum(t.nbytes for t in want) + terms * 0.6) / total)
+        got = backward()
+        assert torch.cuda.memory_reserved() < torch.cuda.memory_allocated() + terms
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    n = int(torch.bincount(where[1]).max()) + 16
+    for a, b in zip(got, want):
+        assert float((a - b).abs().max()) <= n * 2.0 ** -53 * float(b.abs().max())
