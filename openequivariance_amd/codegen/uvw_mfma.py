@@ -64,7 +64,7 @@ kernels once per weight tensor (W, then the cotangent of dW, adding to the first
 from __future__ import annotations
 
 from dataclasses import dataclass
-from typing import List
+from typing import Dict, List, Optional
 
 from .common import Src, prelude, utility_kernels
 from .lower import Lowered, Path, float_literal
@@ -1215,7 +1215,17 @@ class MfmaEmitter:
         return names_a, names_b
 
 
-def tp_module(low: Lowered, compute_units: int = 256, edge_lists: bool = False):
+# Scratch memory (bytes a lane) up to which a split-operand kernel is the faster one, by its waves per SIMD. At two waves past
+# it: one wave where the tiles are full enough for that (SplitEmitter.supported), and the fp32 instructions else. 60 000 rows,
+# us, two waves / one / fp32: forward 12 B 68 / - / 73, 28 B 49 / - / 62, 32 B 72 / 66 / 87, 100 B 73 / 68 / 87, 120 B 68 / - / 70
+# (2 000 rows 10.1 / - / 9.1), 124 B 53 / - / 39, 164 B 85 / - / 88 (12.3 / - / 9.5), 312 B 139 / - / 90, 360 B 134 / 62 / 78;
+# backward 16 B 66 / - / 81, 76 B 104 / - / 97 and 109 / - / 100, 116 B 116 / 77 / 94. One wave / fp32: backward 80 B 176 / 264,
+# 256 B 154 / 156 (2 000 rows 32 / 34); forward 664 B 324 / 203.
+SPLIT_SCRATCH = {2: 28, 1: 256}
+
+
+def tp_module(low: Lowered, compute_units: int = 256, edge_lists: bool = False, split_waves: Optional[Dict[str, int]] = None):
+    """``split_waves``: waves per SIMD of a role's split-operand kernels, 0 for none; others by rule."""
     from .. import runtime as rt
 
     em = MfmaEmitter(low)
@@ -1254,9 +1264,10 @@ def tp_module(low: Lowered, compute_units: int = 256, edge_lists: bool = False):
     em._emit_path_fns(s)
     max_blocks = compute_units * em.tune["uvw_blocks"]
     from .uvw_split import DEVICE, SplitEmitter
-    sp = SplitEmitter(low)
+    split_waves = split_waves or {}
+    sp = SplitEmitter(low, split_waves)
     on = bool(em.tune["uvw_split"]) and not em.bf3
-    split_f, split_b = on and sp.supported("forward"), on and sp.supported("dx")
+    split_f, split_b = (on and split_waves.get(kind) != 0 and sp.supported(kind) for kind in ("forward", "dx"))
     if split_f or split_b:
         s(DEVICE)
     if split_f:
@@ -1269,6 +1280,8 @@ def tp_module(low: Lowered, compute_units: int = 256, edge_lists: bool = False):
                   for n in sp.emit_pass(s, "dx", "backward", em.BWD_SIG) + sp.emit_dw(s, "backward_w", em.BWD_SIG)]
     else:
         descs += [(rt.ROLE_TP_BACKWARD, n, 64 * WAVES, RT, max_blocks) for n in em.emit_backward(s)]
+    own = {kind: [d[1] for d in descs if d[0] == role] for kind, role, on in
+           (("forward", rt.ROLE_TP_FORWARD, split_f), ("dx", rt.ROLE_TP_BACKWARD, split_b)) if on}
     if em.tune["uvw_mfma_dd"]:
         names_a, names_b = em.second_order_kernels(s)
         descs += [(rt.ROLE_DOUBLE_BACKWARD_A, n, 64 * WAVES, RT, max_blocks) for n in names_a]
@@ -1279,4 +1292,13 @@ def tp_module(low: Lowered, compute_units: int = 256, edge_lists: bool = False):
     ]
     dims = dict(L1_dim=low.L1, L2_dim=low.L2, L3_dim=low.L3, weight_numel=low.WN, elem_size=low.elem_size,
                 shared_weights=1, deterministic=0, wpartial_per_block=1)
-    return s.text(), dims, descs
+    src = s.text()
+    if own:
+        # The estimates of registers that admit a plan are off by some: the code object says what it took (compiled here,
+        # cached like any other).
+        res = rt.kernel_resources(rt.compile_source(src))
+        fewer = {kind: sp.waves(kind) - 1 for kind, names in own.items()
+                 if max(res[n][1] for n in names) > SPLIT_SCRATCH[sp.waves(kind)]}
+        if fewer:
+            return tp_module(low, compute_units, edge_lists, dict(split_waves, **fewer))
+    return src, dims, descs

@@ -43,7 +43,7 @@ from __future__ import annotations
 from collections import Counter
 from dataclasses import dataclass
 from functools import cached_property
-from typing import List
+from typing import Dict, List, Optional
 
 from .common import Src
 from .lower import Lowered, Path, float_literal
@@ -52,8 +52,9 @@ WAVES = 4
 # (part of A, part of B), smallest products first
 TERMS = ((2, 0), (0, 2), (1, 1), (1, 0), (0, 1), (0, 0))
 LDS_BUDGET = 160 * 1024 - 1024
-# Estimated registers up to which result blocks share a kernel: what compiles without scratch memory (512 registers
-# a lane; the estimates are up to 30 below what the compiler takes, and above it for dW).
+# Estimated registers up to which result blocks share a kernel: what mostly compiles without scratch memory (512 registers
+# a lane; the estimates are seldom more than 30 below what the compiler takes, and above it for dW). Where one does not,
+# uvw_mfma.tp_module finds out.
 MAX_REGS, MAX_REGS_DW = 500, 430
 # Weight operands kept in accumulation registers: 256 less the results of four sub-paths, twice.
 PARKED = 216
@@ -176,8 +177,10 @@ OEQ_DEV void oeq_block_sync()
 
 
 class SplitEmitter:
-    def __init__(self, low: Lowered):
+    def __init__(self, low: Lowered, waves: Optional[Dict[str, int]] = None):
+        """``waves``: waves per SIMD of a role ('forward', or 'dx' for the backward pass) where that is not left to the rule."""
         self.low = low
+        self.given = {kind: n for kind, n in (waves or {}).items() if n}
         self.subs: List[Sub] = []
         for p in low.paths:
             for v in range(low.in2[p.i2].mul):
@@ -265,6 +268,8 @@ class SplitEmitter:
         """Waves per SIMD of the kernels of a role: two where the largest of them comes under 256 registers and half
         the LDS."""
         kinds = [kind] if kind == "forward" else ["dx", "dw"]
+        if kinds[0] in self.given:
+            return self.given[kinds[0]]
         need = [(self.registers_dw(s), self.lds_dw(s)) if k == "dw" else (self.registers(k, s), self.lds(k, s))
                 for k in kinds for s in (self.plan_dw() if k == "dw" else self.plan(k))]
         return 2 if all(r <= TWO_WAVES and 2 * m <= LDS_BUDGET for r, m in need) else 1

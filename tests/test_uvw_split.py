@@ -147,3 +147,29 @@ def test_boundaries_match_oracle(name, make, wf, wb):
     assert not torch.isfinite(z2[3]).all() and not torch.isfinite(z2[20]).all()
     clean = (rows != 3) & (rows != 20)
     assert torch.equal(z2[clean], z[clean])
+
+
+# (problem, kernels on split operands of the forward and the backward pass, waves per SIMD of each)
+SPILLS = [
+    # as estimated, forward 664 bytes a lane at one wave per SIMD; 124 at two, a tile that is mostly padding
+    (("8x0e+20x1o+48x2e", "1x0e+1x1o+1x2e+2x3o", "64x0o+40x0o+64x2o+32x3o"), 0, 1),
+    (("40x0o+16x2o", "1x0e+1x1o+1x2e+1x3o", "64x0e+40x1o+8x1e"), 0, 0),
+    # at two waves forward 360 and backward 116 bytes, none at one
+    (("40x0e+40x2o", "1x0e+2x1o", "64x0o+48x1o+64x2e"), 1, 1),
+    (("48x0e+48x1o", "1x0e+1x1o", "48x0e+48x1o"), 2, 1),
+]
+
+
+@pytest.mark.parametrize("irreps,wf,wb", SPILLS)
+def test_kernels_that_spill_are_not_used(irreps, wf, wb):
+    from openequivariance_amd import runtime as rt
+    from openequivariance_amd.codegen.uvw_mfma import SPLIT_SCRATCH
+    src, _, descs = build_tp_module(_shared(*irreps))
+    scratch = rt.kernel_resources(rt.compile_source(src))
+    for role, name, waves in ((rt.ROLE_TP_FORWARD, "forward", wf), (rt.ROLE_TP_BACKWARD, "backward", wb)):
+        kernels = [d for d in descs if d[0] == role]
+        body = src.split(f"void {name}(")[1].split('extern "C"')[0]
+        assert ("oeq_split8" in body or "oeq_split_part" in body) == bool(waves)
+        if waves:
+            assert f"amdgpu_waves_per_eu({waves}, {waves})" in src.split(f"void {name}(")[0].split('extern "C"')[-1]
+            assert all(d[4] == 256 * waves and scratch[d[1]][1] <= SPLIT_SCRATCH[waves] for d in kernels)
