@@ -6,7 +6,13 @@ fp32; a remainder is exact), and a product the six cross products of weight 2^-1
 ``v_mfma_f32_16x16x32_bf16``: 6 x 16 cycles for what takes the fp32 instruction 8 x 32. What is dropped is 2^-26 of a
 product, and 32 products are summed before they are rounded, so the results are nearer to 64 bits than those of the
 fp32 instruction. 64x{0e,1o,2e} (x) {0e,1o,2e} -> the same, relative errors of Z, dX, dY, dW at 100 003 rows, before
-and now: 2.9e-7, 1.6e-7, 1.7e-7, 5.4e-7 and 0.75e-7, 0.8e-7, 1.0e-7, 1.7e-7. An infinity in an operand gives NaN.
+and now: 2.9e-7, 1.6e-7, 1.7e-7, 5.4e-7 and 0.75e-7, 0.8e-7, 1.0e-7, 1.7e-7.
+
+Three parts hold an operand of magnitude 2^-110 (7.7e-34) to 3.39e38, and zero. Forward and dX look at what is left of every
+operand after its third part: rows with one outside that range, an infinity or NaN among them, are formed once more by fp32
+instructions (``emit_redo``). The look costs the forward 2 to 5 % (100 003 rows of the problem above 147 / 149 us, 4 500
+19.6 / 20.2) and the backward 1 % (470 / 474, 65 / 68); at two waves per SIMD up to 12 % where it fills the registers
+(64x{0e,1o} (x) l <= 2 52 / 59).
 
 Where the fp32 kernels (``uvw_mfma.py``) contract with the coupling coefficients first and multiply the result, forward and dX
 multiply first: the matrix cores form W^T x (or W dZ) component by component, the lanes contract what comes out. The
@@ -56,8 +62,9 @@ LDS_BUDGET = 160 * 1024 - 1024
 # a lane; the estimates are seldom more than 30 below what the compiler takes, and above it for dW). Where one does not,
 # uvw_mfma.tp_module finds out.
 MAX_REGS, MAX_REGS_DW = 500, 430
-# Weight operands kept in accumulation registers: 256 less the results of four sub-paths, twice.
-PARKED = 216
+# Registers of weight operands kept as accumulation registers, of 256; the others hold results (64x{0e,1o,2e}, forward, 100 003 rows:
+# 144 149 us, 192 and 204, with 8 bytes of scratch memory a lane, 152).
+PARKED = 144
 # Two waves per SIMD (256 registers): up to this estimate. 64x0e+16x1o (x) 0e+1o -> the same, 150 000 rows, one wave / two:
 # forward 52 / 40 us, dX 71 / 54, dW 69 / 61.
 TWO_WAVES = 300
@@ -105,7 +112,10 @@ typedef float oeq_f4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float oeq_f2u __attribute__((ext_vector_type(2), aligned(4)));
 // a and b as sums of three bf16 numbers each (round to nearest; the remainders are exact in fp32); q<i> holds the i-th
 // parts, a's in the low half. A remainder is one dot product with (-1, 0) or (0, -1).
-OEQ_DEV void oeq_split3(float a, float b, unsigned& q0, unsigned& q1, unsigned& q2)
+// What remains of a and b after the last part is zero, unless three parts do not hold them: below 2^-110 (7.7e-34), where bf16
+// has no bits for the last one, above 3.39e38, where the first is an infinity, an infinity itself, NaN. lost gathers its
+// bits; its sign says nothing.
+OEQ_DEV void oeq_split3(float a, float b, unsigned& q0, unsigned& q1, unsigned& q2, unsigned& lost)
 {
     unsigned l = 0x0000bf80u, h = 0xbf800000u;
     asm("" : "+s"(l), "+s"(h));
@@ -117,6 +127,9 @@ OEQ_DEV void oeq_split3(float a, float b, unsigned& q0, unsigned& q1, unsigned& 
     a = __builtin_amdgcn_fdot2_f32_bf16(p1, lo, a, false);
     b = __builtin_amdgcn_fdot2_f32_bf16(p1, hi, b, false);
     const oeq_bf2 p2 = __builtin_convertvector((oeq_f2{a, b}), oeq_bf2);
+    a = __builtin_amdgcn_fdot2_f32_bf16(p2, lo, a, false);
+    b = __builtin_amdgcn_fdot2_f32_bf16(p2, hi, b, false);
+    lost |= __builtin_bit_cast(unsigned, a) | __builtin_bit_cast(unsigned, b);
     q0 = __builtin_bit_cast(unsigned, p0), q1 = __builtin_bit_cast(unsigned, p1), q2 = __builtin_bit_cast(unsigned, p2);
 }
 // The same in steps, for a caller that puts other instructions between them: q = the next parts of a and b, which keep the
@@ -134,12 +147,19 @@ OEQ_DEV void oeq_split_last(float a, float b, unsigned& q)
 {
     q = __builtin_bit_cast(unsigned, __builtin_convertvector((oeq_f2{a, b}), oeq_bf2));
 }
+OEQ_DEV void oeq_split_last(float a, float b, unsigned& q, unsigned& lost)
+{
+    oeq_split_part(a, b, q);
+    lost |= __builtin_bit_cast(unsigned, a) | __builtin_bit_cast(unsigned, b);
+}
+// Whether any lane of the wave has lost something.
+OEQ_DEV bool oeq_any_lost(unsigned lost) { return __builtin_amdgcn_ballot_w64((lost << 1) != 0) != 0; }
 // Component I of eight channels (or rows) as three bf16 operands: r[e * D + I], e = 0..7.
-template <int D, int I> OEQ_DEV void oeq_split8(const float (&r)[8 * D], oeq_bf8 (&f)[3])
+template <int D, int I> OEQ_DEV void oeq_split8(const float (&r)[8 * D], oeq_bf8 (&f)[3], unsigned& lost)
 {
     unsigned q[3][4];
     #pragma unroll
-    for (int m = 0; m < 4; ++m) oeq_split3(r[2 * m * D + I], r[(2 * m + 1) * D + I], q[0][m], q[1][m], q[2][m]);
+    for (int m = 0; m < 4; ++m) oeq_split3(r[2 * m * D + I], r[(2 * m + 1) * D + I], q[0][m], q[1][m], q[2][m], lost);
     #pragma unroll
     for (int c = 0; c < 3; ++c) f[c] = __builtin_bit_cast(oeq_bf8, oeq_u4{q[c][0], q[c][1], q[c][2], q[c][3]});
 }
@@ -172,6 +192,15 @@ OEQ_DEV void oeq_block_sync()
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+// One value of four rows, at these byte offsets.
+OEQ_DEV v4t oeq_rows4(const float* p, const unsigned (&at)[4]) { return v4t{*oeq_at(p, at[0]), *oeq_at(p, at[1]), *oeq_at(p, at[2]), *oeq_at(p, at[3])}; }
+// oeq_block_sync with the block's accesses to memory as well.
+OEQ_DEV void oeq_block_sync_all()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 """
 
@@ -329,7 +358,7 @@ class SplitEmitter:
                     conds = ([] if t.mul >= 64 else [f"16 * wave + l16 < {t.mul}"]) + ([] if full else [f"{u} < {a.mul}"])
                     val = f"{self.lit(q.unit)} * {r}[{e}]"
                     use.append(f"{r}[{e}] = " + (f"oeq_sel({' && '.join(conds)}, {val});" if conds else f"{val};"))
-                use.append(f"oeq_split8<1, 0>({r}, w{q.index}[{st}]);")
+                use.append(f"oeq_split8<1, 0>({r}, w{q.index}[{st}], wlost);")
                 if park > 0:
                     use.append(f"for (int c = 0; c < 3; ++c) w{q.index}[{st}][c] = oeq_park(w{q.index}[{st}][c]);")
                 park -= 12
@@ -377,15 +406,21 @@ class SplitEmitter:
         b, n = self.low.in1[q.p.i1], q.index
         out = []
         for e in range(2):
-            for m, (i, j, _, c) in enumerate(q.p.nnz):
-                r = q.ratio(c)
-                y = f"yt{n}[{j}]" if r == 1.0 else f"({self.lit(r)} * yt{n}[{j}])"
-                op = ("= -" if c < 0 else "= ") if m == 0 else "-= " if c < 0 else "+= "
-                out.append((1, f"{'float ' if m == 0 else ''}tf{n}_{st}_{e} {op}{y} * ra{q.p.i1}_{st}[{e * b.d + i}];"))
+            out += [(1, line) for line in self.fold_terms(q, f"tf{n}_{st}_{e}", lambda i: f"ra{q.p.i1}_{st}[{e * b.d + i}]")]
         v = [f"tf{n}_{st}_{e}" for e in range(2)]
         if 32 * st + 32 > b.mul:
             v = [f"oeq_sel({32 * st + e} + 2 * (tid & 15) < {b.mul}, {v[e]})" for e in range(2)]
         return out + self.split_pair(f"f{n}_{st}", v, [f"{buf}[{at + 256 * c} + put]" for c in range(3)])
+
+    def fold_terms(self, q: Sub, name: str, x):
+        """The sum of a folded sub-path's terms; ``x(i)``: component i of the channel, yt<q>: Y of its row."""
+        out = []
+        for m, (i, j, _, c) in enumerate(q.p.nnz):
+            r = q.ratio(c)
+            y = f"yt{q.index}[{j}]" if r == 1.0 else f"({self.lit(r)} * yt{q.index}[{j}])"
+            op = ("= -" if c < 0 else "= ") if m == 0 else "-= " if c < 0 else "+= "
+            out.append(f"{'float ' if m == 0 else ''}{name} {op}{y} * {x(i)};")
+        return out
 
     @staticmethod
     def split_pair(name: str, v, to):
@@ -393,7 +428,7 @@ class SplitEmitter:
         q = [f"q{name}_{c}" for c in range(3)]
         return [(0, f"float s{name}_0 = {v[0]}, s{name}_1 = {v[1]}; unsigned {', '.join(q)};")] + \
             [(3, f"oeq_split_part(s{name}_0, s{name}_1, {q[c]});") for c in range(2)] + \
-            [(1, f"oeq_split_last(s{name}_0, s{name}_1, {q[2]});")] + [(1, f"{to[c]} = {q[c]};") for c in range(3)]
+            [(4, f"oeq_split_last(s{name}_0, s{name}_1, {q[2]}, lost);")] + [(1, f"{to[c]} = {q[c]};") for c in range(3)]
 
     @staticmethod
     def split_tasks(v: str, q: str):
@@ -536,6 +571,9 @@ class SplitEmitter:
                     out += self.fold_write(q, st, at[(q.key, st)], buf)
             return out
 
+        # Tiles with operands that three parts do not hold: a bit each, by the tile's number among the block's modulo 32.
+        # lost: what the thread's splits of the next tile left over; next: that tile's bit.
+        s("unsigned lost = 0, wlost = 0, redo = 0, next = 2;")
         units = [(a, st) for a in used_a for st in range(c32(A[a].mul))]
         where("(i64)blockIdx.x", "const i64 ")
         s(f"const float* rows = {src} + first * {LA};")
@@ -552,6 +590,9 @@ class SplitEmitter:
         for a, st in units:
             self.put(s, write(a, st, "s_a[0]"))
         write_y("0")
+        s("const unsigned wrows = oeq_any_lost(wlost) ? 0xffffu : 0u;")
+        s("redo = wrows ? ~0u : oeq_any_lost(lost) ? 1u : 0u;")
+        s("lost = 0;")
         s.open("")
         where("((i64)blockIdx.x + gridDim.x)", "const i64 ")
         s(f"const float* rows = {src} + first * {LA};")
@@ -692,6 +733,7 @@ class SplitEmitter:
             # a share of the next tile's operands, and of the requests for the one after
             for ua, ust in (units[m] for m in range(len(units)) if writer(m) == n):
                 tasks += write(ua, ust, "s_a[cur ^ 1]")
+                tasks.append((1, "redo |= oeq_any_lost(lost) ? next : 0u; lost = 0;"))
                 tasks += request(ua, ust)
             tasks += contract((n or N) - 1)
             if n == min(1, N - 2):
@@ -733,6 +775,7 @@ class SplitEmitter:
                 request_y()
             else:
                 self.interleave(s, lead(n), tasks)
+        s("next = (next << 1) | (next >> 31);")
         s("prow0 = row0;")
         if number == 0:
             for t in range(len(T)):
@@ -756,6 +799,157 @@ class SplitEmitter:
                 for part in finish(buf):
                     self.put(s, part)
                 s.close()
+        self.emit_redo(s, kind, subs, number, folds, where)
+        s.close()
+
+    def emit_redo(self, s: Src, kind: str, subs, number: int, folds, where):
+        """Rows with an operand that three bf16 parts do not hold, all rows of the block if a weight is one: once more with fp32
+        matrix instructions, after the last tile, on operands straight from memory. It costs nothing where there are none: beside
+        the splits' remainders the loop has one ballot a tile. dY of such a row is formed anew from the sub-paths of the
+        kernels before this one too, whose sums the first pass has written over."""
+        low = self.low
+        A, T, ia, it = self.sides(kind)
+        L2, fwd = low.L2, kind == "forward"
+        src, LA = ("L1_in", low.L1) if fwd else ("L3_grad", low.L3)
+        dst, LT = ("L3_out", low.L3) if fwd else ("L1_grad", low.L1)
+        used_a = sorted({ia(q) for q in subs})
+        mine = sorted(subs, key=it)
+        every = mine if fwd else [q for k in self.plan(kind)[:number] for q in sorted(k, key=it)] + mine
+        s("__shared__ unsigned s_redo[8];")
+        s("s_redo[wave] = redo, s_redo[4 + wave] = wrows;")
+        s("oeq_block_sync();")
+        s("redo = __builtin_amdgcn_readfirstlane(s_redo[0] | s_redo[1] | s_redo[2] | s_redo[3]);")
+        s("const unsigned whole = __builtin_amdgcn_readfirstlane(s_redo[4] | s_redo[5] | s_redo[6] | s_redo[7]);")
+        s("if (!redo) return;")
+        s("oeq_block_sync_all();  // (behind the stores of the rows that are written once more)")
+        # (lane numbers anew: kept, they would take registers in the loop above)
+        s.open("")
+        s("const int id = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));")
+        s("const int tid = 64 * wave + id, l16 = id & 15, lq = id >> 4;")
+        s("unsigned turn = 0;")
+        s.open("for (i64 tile = blockIdx.x; tile < ntiles; tile += gridDim.x, ++turn)")
+        s("if (!(redo >> (turn & 31) & 1)) continue;")
+        where("tile", "const i64 ")
+        s(f"const float* rows = {src} + first * {LA};")
+        # which rows: the splits again (tiles 32 turns apart share a bit)
+        s("unsigned gone = 0;")
+        s.open("")
+        s(f"const float* ap = rows + min(tid >> 4, end) * {LA};")
+        s("unsigned q;")
+        for a in used_a:
+            s(f"for (int z = tid & 15; z < {A[a].mul * A[a].d}; z += 16) oeq_split3(ap[{A[a].off} + z], 0.0f, q, q, q, gone);")
+        for q in folds:
+            b, b2 = A[ia(q)], low.in2[q.p.i2]
+            s(f"const float* yp{q.index} = L2_in + (first + min(tid >> 4, end)) * {L2} + {self.yat(q, 0)};")
+            s(f"const float yt{q.index}[{b2.d}] = {{{', '.join(f'yp{q.index}[{j}]' for j in range(b2.d))}}};")
+            s.open(f"for (int z = tid & 15; z < {b.mul}; z += 16)")
+            for line in self.fold_terms(q, "v", lambda i: f"ap[{b.off} + {b.d} * z + {i}]"):
+                s(line)
+            s("oeq_split3(v, 0.0f, q, q, q, gone);")
+            s.close()
+        s.close()
+        s("const unsigned long long rows_gone = __builtin_amdgcn_ballot_w64((gone << 1) != 0);")
+        s("unsigned four = 0;")
+        s("for (int r = 0; r < 4; ++r) four |= (rows_gone >> (16 * r) & 0xffff) ? 1u << r : 0u;")
+        s("oeq_block_sync();  // (the words of the tile before are read)")
+        s("s_redo[wave] = four << (4 * wave);")
+        s("oeq_block_sync();")
+        s("const unsigned bad = whole | __builtin_amdgcn_readfirstlane(s_redo[0] | s_redo[1] | s_redo[2] | s_redo[3]);")
+        s("if (!bad) continue;")
+        s("int col = 16 * wave + l16;")
+        s(f"const float* ap = rows + min(l16, end) * {LA};")
+        opaque = "asm volatile(\"\" : \"+v\"(col));  // (no address is worked out ahead: registers)"
+        if not fwd:
+            # (Y as it is met: its components together with those of dY would be too many registers)
+            s("unsigned yr[4];")
+            s(f"for (int r = 0; r < 4; ++r) yr[r] = {4 * L2}u * min(4 * lq + r, end);")
+            s(f"const float* yp = L2_in + first * {L2};")
+            s(f"v4t dy[{L2}];")
+            s(" ".join(f"dy[{j}] = v4t{{}};" for j in range(L2)))
+        at = 0
+        while at < len(every):
+            t, own = it(every[at]), any(every[at] is q for q in mine)
+            group = []
+            while at < len(every) and it(every[at]) == t:
+                group.append(every[at])
+                at += 1
+            b = T[t]
+            s.open("")
+            if own:
+                s(f"v4t acc[{b.d}];")
+                s(" ".join(f"acc[{k}] = v4t{{}};" for k in range(b.d)))
+            if not fwd:
+                s(f"v4t x[{b.d}];")
+                for i in range(b.d):
+                    s(f"for (int r = 0; r < 4; ++r) x[{i}][r] = oeq_sel(col < {b.mul}, "
+                      f"L1_in[(first + min(4 * lq + r, end)) * {low.L1} + {b.off + i} + min(col, {b.mul - 1}) * {b.d}]);")
+                s("__builtin_amdgcn_sched_barrier(0);")
+            for q in group:
+                a = A[ia(q)]
+                ld = low.in2[q.p.i2].mul * low.out[q.p.io].mul
+                cu, ct = (ld, 1) if fwd else (1, ld)
+                base = q.p.woff + q.v * low.out[q.p.io].mul
+                if fwd:
+                    # contracted first, as the fp32 kernels do: what a small Y brings back into range stays in it
+                    b2 = low.in2[q.p.i2]
+                    s.open("")
+                    s(f"const float* yp = L2_in + (first + min(l16, end)) * {L2} + {self.yat(q, 0)};")
+                    s(f"const float y[{b2.d}] = {{{', '.join(f'yp[{j}]' for j in range(b2.d))}}};")
+                    for kk in sorted({k for _, _, k, _ in q.p.nnz}):
+                        s(opaque)
+                        s("#pragma unroll 4")
+                        s.open(f"for (int u0 = 0; u0 < {a.mul}; u0 += 4)")
+                        s(f"const int u = min(u0 + lq, {a.mul - 1});")
+                        s(f"const float* xp = ap + {a.off} + {a.d} * u;")
+                        terms = " + ".join(f"{self.lit(c)} * y[{j}] * xp[{i}]" for i, j, k, c in q.p.nnz if k == kk)
+                        s(f"const float av = oeq_sel(u0 + lq < {a.mul}, {terms});")
+                        s(f"const float bv = oeq_sel(u0 + lq < {a.mul} && col < {b.mul}, W[{base} + u * {cu} + min(col, {b.mul - 1}) * {ct}]);")
+                        s(f"acc[{kk}] = oeq_mfma(av, bv, acc[{kk}], 0, 0, 0);")
+                        s.close()
+                        s("__builtin_amdgcn_sched_barrier(0);")
+                    s.close()
+                    continue
+                for i in sorted({k for _, _, k, _ in q.p.nnz}):
+                    s.open("")
+                    s("v4t P = v4t{};")
+                    s(opaque)
+                    s("#pragma unroll 4")
+                    s.open(f"for (int u0 = 0; u0 < {a.mul}; u0 += 4)")
+                    s(f"const int u = min(u0 + lq, {a.mul - 1});")
+                    s(f"const float av = oeq_sel(u0 + lq < {a.mul}, ap[{a.off + i} + {a.d} * u]);")
+                    s(f"const float bv = oeq_sel(u0 + lq < {a.mul} && col < {b.mul}, W[{base} + u * {cu} + min(col, {b.mul - 1}) * {ct}]);")
+                    s("P = oeq_mfma(av, bv, P, 0, 0, 0);")
+                    s.close()
+                    for (i1, j, k, c) in q.p.nnz:
+                        if k != i:
+                            continue
+                        if own:
+                            s(f"acc[{i1}] += {self.lit(c)} * oeq_rows4(yp + {self.yat(q, j)}, yr) * P;")
+                        s(f"dy[{self.yat(q, j)}] += {self.lit(c)} * x[{i1}] * P;")
+                    s("__builtin_amdgcn_sched_barrier(0);")
+                    s.close()
+            if own:
+                s.open("for (int r = 0; r < 4; ++r)")
+                s(f"float* op = {dst} + (first + 4 * lq + r) * {LT} + {b.off} + {b.d} * col;")
+                s(f"if (4 * lq + r <= end && (bad >> (4 * lq + r) & 1) && col < {b.mul}) {{ "
+                  + " ".join(f"op[{k}] = acc[{k}][r];" for k in range(b.d)) + " }")
+                s.close()
+            s.close()
+        if not fwd:
+            for j in range(L2):
+                s.open("for (int r = 0; r < 4; ++r)")
+                s(f"float v = dy[{j}][r];")
+                for ctrl in ("0x140", "0x141", "0x1B", "0xB1"):
+                    s(f"v += oeq_dpp<{ctrl}>(v);")
+                s(f"if (l16 == 0) s_dy[0][wave][(4 * lq + r) * {L2} + {j}] = v;")
+                s.close()
+            s("oeq_block_sync();")
+            s.open(f"for (int z = tid; z < {16 * L2}; z += 256)")
+            s(f"const float v = ((s_dy[0][0][z] + s_dy[0][1][z]) + s_dy[0][2][z]) + s_dy[0][3][z];")
+            s(f"if (z / {L2} <= end && (bad >> (z / {L2}) & 1)) L2_grad[first * {L2} + z] = v;")
+            s.close()
+            s("oeq_block_sync();")
+        s.close()
         s.close()
 
     def reduce_dy(self, into: str):

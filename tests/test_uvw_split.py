@@ -173,3 +173,66 @@ def test_kernels_that_spill_are_not_used(irreps, wf, wb):
         if waves:
             assert f"amdgpu_waves_per_eu({waves}, {waves})" in src.split(f"void {name}(")[0].split('extern "C"')[-1]
             assert all(d[4] == 256 * waves and scratch[d[1]][1] <= SPLIT_SCRATCH[waves] for d in kernels)
+
+
+def _fp32(problem):
+    """The kernel set of the problem on fp32 matrix instructions."""
+    from openequivariance_amd._torch import ops
+    with ops._tune_env("uvw_split=0"):
+        return ops.register_spec(ops.make_spec("tp", problem))
+
+
+def _off(got, want):
+    """The 2-norm of the difference. Infinities in the same places, NaN nowhere else (the fp32 kernels have some more: zeros
+    that pad a tile meet infinities)."""
+    known = ~torch.isnan(want)
+    got, want = got[known], want[known]
+    assert not torch.isnan(got).any() and torch.equal(torch.isinf(got), torch.isinf(want))
+    assert torch.equal(got[torch.isinf(got)], want[torch.isinf(want)])
+    a, b = got[torch.isfinite(got)].double(), want[torch.isfinite(got)].double()
+    return float((a - b).norm() / b.norm()) if bool(b.any()) else float(a.norm())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,make,wf,wb", CASES, ids=[c[0] for c in CASES])
+def test_operands_that_three_parts_do_not_hold(name, make, wf, wb):
+    """Infinities, the largest numbers, numbers near the smallest: rows that have one are what the fp32 instructions make of
+    them, rows beside them keep their bits."""
+    from openequivariance_amd._torch import ops
+    problem = make()
+    tp, plain = oeq.TensorProduct(problem), _fp32(problem)
+    for B in (40, 16 * 256 * max(wf, wb) * 2 + 21) + ((16 * 512 * 33 + 5,) if name == "two-scalars" else ()):
+        gen = torch.Generator(device="cuda").manual_seed(B)
+        x, y, g = (torch.randn(B, d, device="cuda", generator=gen)
+                   for d in (problem.irreps_in1.dim, problem.irreps_in2.dim, problem.irreps_out.dim))
+        w = torch.randn(problem.weight_numel, device="cuda", generator=gen)
+        z, (dx, dy, _) = ops.tp_forward(x, y, w, tp.kid), ops.tp_backward(x, y, w, g, tp.kid)
+        rows = dict(zip(("inf", "-inf", "large x", "large dZ", "small", "smallest", "nan"), (3, 17, B // 2, B // 2 + 1, B - 9, B - 2, B - 1)))
+        clean = torch.ones(B, dtype=torch.bool, device="cuda")
+        clean[list(rows.values())] = False
+        xs, gs, ys = x.clone(), g.clone(), y.clone()
+        for t in (xs, gs):
+            t[rows["inf"], 0], t[rows["-inf"], -1], t[rows["nan"], 1] = float("inf"), float("-inf"), float("nan")
+            t[rows["small"]] *= 2.0 ** -112
+            t[rows["smallest"]] *= 2.0 ** -124
+        xs[rows["large x"], 0] = gs[rows["large dZ"], 0] = 3.4e38
+        # (the other operands small, so that no result is near the end of the range)
+        ys[rows["large x"]] *= 2.0 ** -40
+        gs[rows["large x"]] *= 2.0 ** -40
+        ys[rows["large dZ"]] *= 2.0 ** -40
+        xs[rows["large dZ"]] *= 2.0 ** -40
+        got = (ops.tp_forward(xs, ys, w, tp.kid), *ops.tp_backward(xs, ys, w, gs, tp.kid)[:2])
+        want = (ops.tp_forward(xs, ys, w, plain), *ops.tp_backward(xs, ys, w, gs, plain)[:2])
+        for n, (a, b, before) in enumerate(zip(got, want, (z, dx, dy))):
+            assert torch.equal(a[clean], before[clean]), (B, n)
+            for kind, r in rows.items():
+                # (results near 2^-124 are sums of some hundred terms, each of which is rounded to multiples of 2^-149)
+                assert _off(a[r], b[r]) <= (TOL if kind != "smallest" else 100 * 2.0 ** -25), (B, n, kind)
+        # a weight that three parts do not hold: every row
+        for value in (2.0 ** -120 * 1.37, float("inf")):
+            wt = w.clone()
+            wt[5] = value
+            got = (ops.tp_forward(x, y, wt, tp.kid), *ops.tp_backward(x, y, wt, g, tp.kid)[:2])
+            want = (ops.tp_forward(x, y, wt, plain), *ops.tp_backward(x, y, wt, g, plain)[:2])
+            for a, b in zip(got, want):
+                assert _off(a, b) <= TOL
