@@ -12,7 +12,8 @@ Three parts hold an operand of magnitude 2^-110 (7.7e-34) to 3.39e38, and zero. 
 operand after its third part: rows with one outside that range, an infinity or NaN among them, are formed once more by fp32
 instructions (``emit_redo``). The look costs the forward 2 to 5 % (100 003 rows of the problem above 147 / 149 us, 4 500
 19.6 / 20.2) and the backward 1 % (470 / 474, 65 / 68); at two waves per SIMD up to 12 % where it fills the registers
-(64x{0e,1o} (x) l <= 2 52 / 59).
+(64x{0e,1o} (x) l <= 2 52 / 59). dW scales its operands by 2^20, which brings the smallest numbers into the range; where its sums
+are not finite, a wave forms them once more by fp32 instructions (``emit_redo_dw``).
 
 Where the fp32 kernels (``uvw_mfma.py``) contract with the coupling coefficients first and multiply the result, forward and dX
 multiply first: the matrix cores form W^T x (or W dZ) component by component, the lanes contract what comes out. The
@@ -73,6 +74,9 @@ TWO_WAVES = 300
 WEIGHTS_AHEAD = 6
 # Components of Y that dW reads from LDS ahead of their use.
 AHEAD = 4
+# dW's operands are multiplied by this before they are split, so that three parts hold every normal number: with Y's coefficients, in
+# place of a copy of X in folded sub-paths, and for dZ (100 003 rows of 64x{0e,1o,2e}: 72 multiplications in a step of 32 rows).
+SCALE = 2.0 ** 20
 
 
 def c16(n: int) -> int:
@@ -1085,7 +1089,7 @@ class SplitEmitter:
         s("#pragma unroll")
         s.open(f"for (int n = 0; n < {ny}; ++n)")
         s(f"const int at = min((tid >> 5) + 8 * n, {len(table) - 1});")
-        s(f"yc[n] = sign * {coefficients}[at], yj[n] = {components}[at];")
+        s(f"yc[n] = {self.lit(SCALE)} * sign * {coefficients}[at], yj[n] = {components}[at];")
         s.close()
 
         def rows_of(step):
@@ -1136,7 +1140,8 @@ class SplitEmitter:
                 q = next((q for q in folds if q.key == k), None)
                 v = f"v{o}_{k}" if q is None else f"vf{q.index}"
                 if q is None:
-                    out.append((0, f"float {v}[8]; " + " ".join(f"{v}[{e}] = g{o}[{e * b.d + k}];" for e in range(8))))
+                    out.append((0, f"float {v}[8];"))
+                    out += [(4, " ".join(f"{v}[{e}] = {self.lit(SCALE)} * g{o}[{e * b.d + k}];" for e in range(h, h + 4))) for h in (0, 4)]
                 else:
                     out += fold(q, v, ynext)
                 out += self.split_tasks(v, "tg")
@@ -1165,7 +1170,7 @@ class SplitEmitter:
             component, two ahead of the sums."""
             o, k, q = stages[n % N]
             if q in folds:
-                return [(4, " ".join(f"t[{4 * h + r}] = x{q.p.i1}[{4 * h + r}][0];" for r in range(4))) for h in (0, 1)] + \
+                return [(4, " ".join(f"t[{4 * h + r}] = {self.lit(SCALE)} * x{q.p.i1}[{4 * h + r}][0];" for r in range(4))) for h in (0, 1)] + \
                     self.split_tasks("t", f"ta[{n % 2}]")
             buf = "s_y[ycur]" if n < N else "s_y[ynext]"
             units = later if n % N else [(0, j) for j in js_of(0)]
@@ -1308,6 +1313,15 @@ class SplitEmitter:
                     s("for (int c = 0; c < 3; ++c) for (int m = 0; m < 4; ++m) ta[0][c][m] = ta[1][c][m];")
         s.close()
         s.close()
+        # Operands above the range that three parts hold, and infinities, have made NaN of the sums they met.
+        s("float off = 0.0f;")
+        for q in subs:
+            s("#pragma unroll")
+            s(f"for (int j = 0; j < {per(q)}; ++j) for (int i = 0; i < 4; ++i) off += 0.0f * dw{q.index}[j][i];")
+        s("const bool again = __builtin_amdgcn_ballot_w64(off != off) != 0;")
+        s.open("if (again)")
+        self.emit_redo_dw(s, subs)
+        s.close()
         s(f"float* prow = wpartial + (i64)blockIdx.x * {low.WN};")
         for q in subs:
             U, Wn = low.in1[q.p.i1].mul, low.out[q.p.io].mul
@@ -1316,5 +1330,32 @@ class SplitEmitter:
                 s.open("for (int i = 0; i < 4; ++i)")
                 nt = f"{j}" if WW == 1 else f"(ww + {j * WW})"
                 s(f"const int u = 16 * wu + 4 * lq + i, w = 16 * {nt} + l16;")
-                s(f"if (u < {U} && w < {Wn}) prow[{self.wpos(q, 'u', 'w')}] = {self.lit(q.unit)} * dw{q.index}[{j}][i];")
+                s(f"if (u < {U} && w < {Wn}) prow[{self.wpos(q, 'u', 'w')}] = (again ? 1.0f : {self.lit(q.unit / SCALE ** 2)}) * dw{q.index}[{j}][i];")
                 s.close()
+
+    def emit_redo_dw(self, s: Src, subs):
+        """The wave's sums once more with fp32 matrix instructions, on operands straight from memory; no other wave is waited
+        for."""
+        low = self.low
+        _, WW, per = self.split_dw(subs)
+        for q in subs:
+            a, b2, o = low.in1[q.p.i1], low.in2[q.p.i2], low.out[q.p.io]
+            s(" ".join(f"dw{q.index}[{j}] = v4t{{}};" for j in range(per(q))))
+            s.open("for (i64 step = begin; step < nsteps; step += gridDim.x)")
+            s("#pragma unroll 1")
+            s.open("for (int r0 = 0; r0 < 32; r0 += 4)")
+            s("const i64 row = min(step * 32 + r0 + lq, num_batch - 1);")
+            s(f"const bool there = step * 32 + r0 + lq < num_batch, in = there && 16 * wu + l16 < {a.mul};")
+            s(f"const float* xp = L1_in + row * {low.L1} + {a.off} + {a.d} * min(16 * wu + l16, {a.mul - 1});")
+            s(f"const float* yp = L2_in + row * {low.L2} + {self.yat(q, 0)};")
+            s(f"const float* gp = L3_grad + row * {low.L3} + {o.off};")
+            for kk in sorted({k for _, _, k, _ in q.p.nnz}):
+                s.open("")
+                terms = " + ".join(f"{self.lit(c)} * yp[{j}] * xp[{i}]" for i, j, k, c in q.p.nnz if k == kk)
+                s(f"const float av = oeq_sel(in, {terms});")
+                for j in range(per(q)):
+                    w = f"16 * (ww + {j * WW}) + l16"
+                    s(f"dw{q.index}[{j}] = oeq_mfma(av, oeq_sel(there && {w} < {o.mul}, gp[{o.d} * min({w}, {o.mul - 1}) + {kk}]), dw{q.index}[{j}], 0, 0, 0);")
+                s.close()
+            s.close()
+            s.close()

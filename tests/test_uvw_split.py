@@ -236,3 +236,30 @@ def test_operands_that_three_parts_do_not_hold(name, make, wf, wb):
             want = (ops.tp_forward(x, y, wt, plain), *ops.tp_backward(x, y, wt, g, plain)[:2])
             for a, b in zip(got, want):
                 assert _off(a, b) <= TOL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,make,wf,wb", CASES, ids=[c[0] for c in CASES])
+def test_weight_gradients_of_operands_that_three_parts_do_not_hold(name, make, wf, wb):
+    from openequivariance_amd._torch import ops
+    problem = make()
+    tp, plain = oeq.TensorProduct(problem), _fp32(problem)
+    for B in (40, 16 * 256 * max(wf, wb) * 2 + 21):
+        gen = torch.Generator(device="cuda").manual_seed(B)
+        x, y, g = (torch.randn(B, d, device="cuda", generator=gen)
+                   for d in (problem.irreps_in1.dim, problem.irreps_in2.dim, problem.irreps_out.dim))
+        w = torch.randn(problem.weight_numel, device="cuda", generator=gen)
+        gradient = lambda x, y, g, kid=tp.kid: ops.tp_backward(x, y, w, g, kid)[2]
+        dw = gradient(x, y, g)
+        # powers of two change no bit: numbers near the smallest, and large ones
+        for sx, sg in ((2.0 ** -100, 1.0), (1.0, 2.0 ** -100), (2.0 ** 40, 2.0 ** 20)):
+            assert torch.equal(gradient(x * sx, y, g * sg) * (1 / sx) * (1 / sg), dw), (B, sx, sg)
+        # sums that leave the range on the way, and come back; x near the smallest; the largest numbers, infinities, NaN
+        for sx, sg in ((2.0 ** 60, 2.0 ** 40), (2.0 ** -124, 2.0 ** 30)):
+            assert _off(gradient(x * sx, y, g * sg), gradient(x * sx, y, g * sg, plain)) <= 2 * TOL, (B, sx, sg)
+        for where, value in ((x, 3.4e38), (g, -3.4e38), (x, float("inf")), (g, float("-inf")), (y, float("inf")), (x, float("nan"))):
+            small = [t * 2.0 ** -40 if abs(value) < 1e39 else t for t in (x, y, g)]
+            at = [t is where for t in (x, y, g)].index(True)
+            small[at] = where.clone()
+            small[at][B - 3, 0] = value
+            assert _off(gradient(*small), gradient(*small, plain)) <= 2 * TOL, (B, at, value)
