@@ -263,3 +263,25 @@ def test_weight_gradients_of_operands_that_three_parts_do_not_hold(name, make, w
             small[at] = where.clone()
             small[at][B - 3, 0] = value
             assert _off(gradient(*small), gradient(*small, plain)) <= 2 * TOL, (B, at, value)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("irreps", [("64x0e+64x1o+64x2e", "1x0e+1x1o+1x2e"), ("64x0e+16x1o", "1x0e+1x1o")])
+def test_errors_have_no_mean(irreps):
+    """Y of l = 0 is one, as spherical harmonics are: nothing else gives an error either sign. Against the kernels in double
+    precision, on an even number of blocks of as many tiles each."""
+    from openequivariance_amd._torch import ops
+    kids = [oeq.TensorProduct(_shared(*irreps, irreps[0], dtype)).kid for dtype in (np.float32, np.float64)]
+    problem = _shared(*irreps, irreps[0])
+    B = 16 * 512 * 4
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    x, y, g = (torch.randn(B, d, device="cuda", generator=gen)
+               for d in (problem.irreps_in1.dim, problem.irreps_in2.dim, problem.irreps_out.dim))
+    y[:, 0] = 1.0
+    w = torch.randn(problem.weight_numel, device="cuda", generator=gen)
+    both = [(ops.tp_forward(*[t.to(d) for t in (x, y, w)], kid), ops.tp_backward(*[t.to(d) for t in (x, y, w, g)], kid)[0])
+            for kid, d in zip(kids, (torch.float32, torch.float64))]
+    for got, exact in zip(*both):
+        off = got.double() - exact
+        # (six standard deviations; columns of a row share the errors of its operands: a few times more)
+        assert abs(float(off.mean())) <= 12 * float(off.std()) / off.numel() ** 0.5
