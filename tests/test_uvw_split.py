@@ -39,6 +39,8 @@ CASES = [
     ("two-channel-second-operand", lambda: _shared("64x0e+32x1o", "3x0e+2x1o", "64x0e+32x1o"), 1, 1),
     ("gaps", _gaps, 2, 1),
     ("zero-path-weight", _zero_weight, 2, 1),
+    # sixteen input channels: the waves of dW side by side along the output channels
+    ("narrow-input", lambda: _shared("16x0e+16x1o", "1x0e+1x1o", "64x0e+32x1o"), 2, 2),
     # two components of the output: two steps of dX's pipeline
     ("two-scalars", lambda: _shared("64x0e+64x1o", "1x0e+1x1o", "64x0e+32x0e"), 2, 2),
 ]
@@ -75,7 +77,7 @@ def test_shares_of_dy_are_read_before_the_barrier(name, make, wf, wb):
 
 # (problem, sub-paths contracted before the product in the forward, and in each kernel of dW)
 FOLDS = [("l2-64", 2, [0, 1, 1]), ("l2-32", 2, [2]), ("l1-64-16", 1, [1]), ("odd-channels", 1, [1]),
-         ("two-channel-second-operand", 2, [2]), ("gaps", 1, [1]), ("two-scalars", 1, [0]), ("zero-path-weight", 0, [1])]
+         ("two-channel-second-operand", 2, [2]), ("gaps", 1, [1]), ("two-scalars", 1, [0]), ("zero-path-weight", 0, [1]), ("narrow-input", 1, [1])]
 
 
 @pytest.mark.parametrize("name,forward,dw", FOLDS, ids=[f[0] for f in FOLDS])
@@ -173,6 +175,38 @@ def test_kernels_that_spill_are_not_used(irreps, wf, wb):
         if waves:
             assert f"amdgpu_waves_per_eu({waves}, {waves})" in src.split(f"void {name}(")[0].split('extern "C"')[-1]
             assert all(d[4] == 256 * waves and scratch[d[1]][1] <= SPLIT_SCRATCH[waves] for d in kernels)
+
+
+def test_cases_cover_the_forms_of_dw():
+    """Waves along input and output channels, and numbers of stages, whose parity decides which operands a step begins with."""
+    forms, stages = set(), set()
+    for _, make, _, _ in CASES:
+        em = SplitEmitter(lower(make()))
+        for subs in em.plan_dw():
+            forms.add(em.split_dw(subs)[:2])
+            stages.add(len(em.stages_dw(subs, em.folds_dw(subs))) % 2)
+    assert forms == {(4, 1), (2, 2), (1, 4)} and stages == {0, 1}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,make,wf,wb", CASES, ids=[c[0] for c in CASES])
+def test_many_steps_a_block(name, make, wf, wb):
+    """Four or five steps of dW for every block and nine or ten tiles: buffers in turn and the third copy of Y come around again.
+    Against the kernels in double precision, all of the results."""
+    from openequivariance_amd import runtime as rt
+    from openequivariance_amd._torch import ops
+    problem, double = make(), make()
+    double.irrep_dtype = double.weight_dtype = np.float64
+    kid, exact_kid = oeq.TensorProduct(problem).kid, oeq.TensorProduct(double).kid
+    blocks = max(d[4] for d in build_tp_module(problem)[2] if d[0] in (rt.ROLE_TP_FORWARD, rt.ROLE_TP_BACKWARD))
+    B = 32 * (4 * blocks + 21) + 5
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    x, y, g = (torch.randn(B, d, device="cuda", generator=gen)
+               for d in (problem.irreps_in1.dim, problem.irreps_in2.dim, problem.irreps_out.dim))
+    w = torch.randn(problem.weight_numel, device="cuda", generator=gen)
+    run = lambda kid, x, y, w, g: (ops.tp_forward(x, y, w, kid), *ops.tp_backward(x, y, w, g, kid))
+    for got, exact in zip(run(kid, x, y, w, g), run(exact_kid, *(t.double() for t in (x, y, w, g)))):
+        assert float((got.double() - exact).norm() / exact.norm()) <= TOL
 
 
 def _fp32(problem):
