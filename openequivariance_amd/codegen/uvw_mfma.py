@@ -1217,11 +1217,11 @@ class MfmaEmitter:
 
 # Scratch memory (bytes a lane) up to which a split-operand kernel is the faster one, by its waves per SIMD. At two waves past
 # it: one wave where the tiles are full enough for that (SplitEmitter.supported), and the fp32 instructions else. 60 000 rows,
-# us, two waves / one / fp32: forward 12 B 68 / - / 73, 28 B 49 / - / 62, 32 B 72 / 66 / 87, 100 B 73 / 68 / 87, 120 B 68 / - / 70
-# (2 000 rows 10.1 / - / 9.1), 124 B 53 / - / 39, 164 B 85 / - / 88 (12.3 / - / 9.5), 312 B 139 / - / 90, 360 B 134 / 62 / 78;
-# backward 16 B 66 / - / 81, 76 B 104 / - / 97 and 109 / - / 100, 116 B 116 / 77 / 94. One wave / fp32: backward 80 B 176 / 264,
-# 256 B 154 / 156 (2 000 rows 32 / 34); forward 664 B 324 / 203.
-SPLIT_SCRATCH = {2: 28, 1: 256}
+# us, two waves / one / fp32: forward 12 B 68 / - / 73, 28 B 49 / - / 62, 40 B 52 / - / 63, 48 B 72 / 66 / 87, 100 B 73 / 68 / 87, 120 B
+# 68 / - / 70 (2 000 rows 10.1 / - / 9.1), 124 B 53 / - / 39, 164 B 85 / - / 88 (12.3 / - / 9.5), 312 B 139 / - / 90, 360 B
+# 134 / 62 / 78; backward 16 B 66 / - / 81, 40 B 78 / - / 83, 76 B 104 / - / 97 and 109 / - / 100, 100 B 126 / 80 / 94. One wave
+# / fp32: backward 80 B 176 / 264, 256 B 154 / 156 (2 000 rows 32 / 34); forward 664 B 324 / 203.
+SPLIT_SCRATCH = {2: 40, 1: 256}
 
 
 def tp_module(low: Lowered, compute_units: int = 256, edge_lists: bool = False, split_waves: Optional[Dict[str, int]] = None):

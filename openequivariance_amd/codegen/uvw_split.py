@@ -3,17 +3,17 @@
 The fp32 matrix instructions share the datapath of the vector unit and give 157 TFLOP/s; the bf16 ones are a pipe of their
 own with 16 times that. Here every fp32 operand is the sum of three bf16 numbers (8 mantissa bits each: together the 24 of
 fp32; a remainder is exact), and a product the six cross products of weight 2^-16 and above, accumulated in fp32 by
-``v_mfma_f32_16x16x32_bf16``: 6 x 16 cycles for what takes the fp32 instruction 8 x 32. What is dropped is 2^-26 of a
-product, and 32 products are summed before they are rounded, so the results are nearer to 64 bits than those of the
+``v_mfma_f32_16x16x32_bf16``: 6 x 16 cycles for what takes the fp32 instruction 8 x 32. What is dropped is 2^-24.3 of a
+product at most and 2^-27.4 root mean square, and 32 products are summed before they are rounded, so the results are nearer to 64 bits than those of the
 fp32 instruction. 64x{0e,1o,2e} (x) {0e,1o,2e} -> the same, relative errors of Z, dX, dY, dW at 100 003 rows, before
 and now: 2.9e-7, 1.6e-7, 1.7e-7, 5.4e-7 and 0.75e-7, 0.8e-7, 1.0e-7, 1.7e-7.
 
-Three parts hold an operand of magnitude 2^-110 (7.7e-34) to 3.39e38, and zero. Forward and dX look at what is left of every
-operand after its third part: rows with one outside that range, an infinity or NaN among them, are formed once more by fp32
-instructions (``emit_redo``). The look costs the forward 2 to 5 % (100 003 rows of the problem above 147 / 149 us, 4 500
-19.6 / 20.2) and the backward 1 % (470 / 474, 65 / 68); at two waves per SIMD up to 12 % where it fills the registers
-(64x{0e,1o} (x) l <= 2 52 / 59). dW scales its operands by 2^20, which brings the smallest numbers into the range; where its sums
-are not finite, a wave forms them once more by fp32 instructions (``emit_redo_dw``).
+Three parts hold a magnitude of 2^-110 (7.7e-34) to 3.39e38, and zero. Rows are multiplied by 2^20 on the way and weights divided by it
+(``SCALE``): all normal numbers below 1.6e32 = 2^107 are held, and weights from 8.1e-28 on. Forward and dX watch
+the largest operand; rows with a larger one or an infinity, and all rows where a weight is not held, are formed once more by fp32
+instructions (``emit_redo``). Where dW's sums are not finite, a wave forms them once more (``emit_redo_dw``). That costs, on the
+problem above, forward / backward, without / with, us: 500 rows 12.6 / 13.7 and 45.6 / 49.1, 4 500 19.7 / 21.1 and 64 / 70, 100 003
+155 / 159 and 505 / 502; such rows in every tile take 8 times as long as with the fp32 kernels (2 364 / 311, 6 454 / 772).
 
 Where the fp32 kernels (``uvw_mfma.py``) contract with the coupling coefficients first and multiply the result, forward and dX
 multiply first: the matrix cores form W^T x (or W dZ) component by component, the lanes contract what comes out. The
@@ -52,6 +52,8 @@ from dataclasses import dataclass
 from functools import cached_property
 from typing import Dict, List, Optional
 
+import numpy as np
+
 from .common import Src
 from .lower import Lowered, Path, float_literal
 
@@ -63,9 +65,9 @@ LDS_BUDGET = 160 * 1024 - 1024
 # a lane; the estimates are seldom more than 30 below what the compiler takes, and above it for dW). Where one does not,
 # uvw_mfma.tp_module finds out.
 MAX_REGS, MAX_REGS_DW = 500, 430
-# Registers of weight operands kept as accumulation registers, of 256; the others hold results (64x{0e,1o,2e}, forward, 100 003 rows:
-# 144 149 us, 192 and 204, with 8 bytes of scratch memory a lane, 152).
-PARKED = 144
+# Registers of weight operands kept as accumulation registers, of 256; the others hold results (64x{0e,1o,2e}, forward: with 168 to
+# 204 no scratch memory, 8 to 24 bytes a lane below and 72 above).
+PARKED = 180
 # Two waves per SIMD (256 registers): up to this estimate. 64x0e+16x1o (x) 0e+1o -> the same, 150 000 rows, one wave / two:
 # forward 52 / 40 us, dX 71 / 54, dW 69 / 61.
 TWO_WAVES = 300
@@ -74,8 +76,9 @@ TWO_WAVES = 300
 WEIGHTS_AHEAD = 6
 # Components of Y that dW reads from LDS ahead of their use.
 AHEAD = 4
-# dW's operands are multiplied by this before they are split, so that three parts hold every normal number: with Y's coefficients, in
-# place of a copy of X in folded sub-paths, and for dZ (100 003 rows of 64x{0e,1o,2e}: 72 multiplications in a step of 32 rows).
+# Operands are multiplied by this before they are split, so that three parts hold every normal number; in forward and dX the
+# weights are divided by it, in dW the sums by its square. (dW: with Y's coefficients, in place of a copy of X in folded
+# sub-paths, and dZ.)
 SCALE = 2.0 ** 20
 
 
@@ -116,10 +119,7 @@ typedef float oeq_f4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float oeq_f2u __attribute__((ext_vector_type(2), aligned(4)));
 // a and b as sums of three bf16 numbers each (round to nearest; the remainders are exact in fp32); q<i> holds the i-th
 // parts, a's in the low half. A remainder is one dot product with (-1, 0) or (0, -1).
-// What remains of a and b after the last part is zero, unless three parts do not hold them: below 2^-110 (7.7e-34), where bf16
-// has no bits for the last one, above 3.39e38, where the first is an infinity, an infinity itself, NaN. lost gathers its
-// bits; its sign says nothing.
-OEQ_DEV void oeq_split3(float a, float b, unsigned& q0, unsigned& q1, unsigned& q2, unsigned& lost)
+OEQ_DEV void oeq_split3(float a, float b, unsigned& q0, unsigned& q1, unsigned& q2)
 {
     unsigned l = 0x0000bf80u, h = 0xbf800000u;
     asm("" : "+s"(l), "+s"(h));
@@ -131,9 +131,6 @@ OEQ_DEV void oeq_split3(float a, float b, unsigned& q0, unsigned& q1, unsigned& 
     a = __builtin_amdgcn_fdot2_f32_bf16(p1, lo, a, false);
     b = __builtin_amdgcn_fdot2_f32_bf16(p1, hi, b, false);
     const oeq_bf2 p2 = __builtin_convertvector((oeq_f2{a, b}), oeq_bf2);
-    a = __builtin_amdgcn_fdot2_f32_bf16(p2, lo, a, false);
-    b = __builtin_amdgcn_fdot2_f32_bf16(p2, hi, b, false);
-    lost |= __builtin_bit_cast(unsigned, a) | __builtin_bit_cast(unsigned, b);
     q0 = __builtin_bit_cast(unsigned, p0), q1 = __builtin_bit_cast(unsigned, p1), q2 = __builtin_bit_cast(unsigned, p2);
 }
 // The same in steps, for a caller that puts other instructions between them: q = the next parts of a and b, which keep the
@@ -151,19 +148,31 @@ OEQ_DEV void oeq_split_last(float a, float b, unsigned& q)
 {
     q = __builtin_bit_cast(unsigned, __builtin_convertvector((oeq_f2{a, b}), oeq_bf2));
 }
-OEQ_DEV void oeq_split_last(float a, float b, unsigned& q, unsigned& lost)
+// The largest magnitude of those seen (NaN does not count; from the compiler, with an instruction to quiet each operand), and whether
+// any lane of the wave has met one that three parts do not hold.
+OEQ_DEV float oeq_top(float top, float a, float b)
 {
-    oeq_split_part(a, b, q);
-    lost |= __builtin_bit_cast(unsigned, a) | __builtin_bit_cast(unsigned, b);
+    float r;
+    asm("v_max3_f32 %0, %1, abs(%2), abs(%3)" : "=v"(r) : "v"(top), "v"(a), "v"(b));
+    return r;
 }
-// Whether any lane of the wave has lost something.
-OEQ_DEV bool oeq_any_lost(unsigned lost) { return __builtin_amdgcn_ballot_w64((lost << 1) != 0) != 0; }
+OEQ_DEV bool oeq_too_large(float top) { return __builtin_amdgcn_ballot_w64(top >= 3.39e38f) != 0; }
+// Of eight values: the largest magnitude, and twice the bits of the smallest, zeros aside, less one.
+OEQ_DEV void oeq_extent(const float (&r)[8], float& top, unsigned& least)
+{
+    unsigned v[8];
+    #pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = (__builtin_bit_cast(unsigned, r[e]) << 1) - 1u;
+    const unsigned a = min(min(v[0], v[1]), v[2]), b = min(min(v[3], v[4]), v[5]);
+    least = min(min(min(v[6], v[7]), a), b);
+    top = oeq_top(top, oeq_top(0.0f, r[0], r[1]), oeq_top(oeq_top(oeq_top(0.0f, r[2], r[3]), r[4], r[5]), r[6], r[7]));
+}
 // Component I of eight channels (or rows) as three bf16 operands: r[e * D + I], e = 0..7.
-template <int D, int I> OEQ_DEV void oeq_split8(const float (&r)[8 * D], oeq_bf8 (&f)[3], unsigned& lost)
+template <int D, int I> OEQ_DEV void oeq_split8(const float (&r)[8 * D], oeq_bf8 (&f)[3])
 {
     unsigned q[3][4];
     #pragma unroll
-    for (int m = 0; m < 4; ++m) oeq_split3(r[2 * m * D + I], r[(2 * m + 1) * D + I], q[0][m], q[1][m], q[2][m], lost);
+    for (int m = 0; m < 4; ++m) oeq_split3(r[2 * m * D + I], r[(2 * m + 1) * D + I], q[0][m], q[1][m], q[2][m]);
     #pragma unroll
     for (int c = 0; c < 3; ++c) f[c] = __builtin_bit_cast(oeq_bf8, oeq_u4{q[c][0], q[c][1], q[c][2], q[c][3]});
 }
@@ -354,15 +363,18 @@ class SplitEmitter:
             s(f"oeq_bf8 w{q.index}[{S}][3];")
             for st in range(S):
                 r = f"r{q.index}_{st}"
-                get, use = [f"float {r}[8];"], []
+                get, use = [f"float {r}[8];"], [f"oeq_extent({r}, top, least);"]
                 for e in range(8):
                     full = 32 * st + 32 <= a.mul
                     u = f"{32 * st + e} + 8 * lq"
                     get.append(f"{r}[{e}] = W[{base} + ({u if full else f'min({u}, {a.mul - 1})'}) * {cu} + min(16 * wave + l16, {t.mul - 1}) * {ct}];")
                     conds = ([] if t.mul >= 64 else [f"16 * wave + l16 < {t.mul}"]) + ([] if full else [f"{u} < {a.mul}"])
-                    val = f"({self.lit(q.unit)} * sign) * {r}[{e}]"
+                    val = f"({self.lit(q.unit / SCALE)} * sign) * {r}[{e}]"
                     use.append(f"{r}[{e}] = " + (f"oeq_sel({' && '.join(conds)}, {val});" if conds else f"{val};"))
-                use.append(f"oeq_split8<1, 0>({r}, w{q.index}[{st}], wlost);")
+                use.append(f"oeq_split8<1, 0>({r}, w{q.index}[{st}]);")
+                # (a weight that is 2^-110 or more when it is split is held by three parts)
+                small = 2 * int(np.float32(2.0 ** -110 * SCALE / q.unit).view(np.uint32))
+                use.insert(1, f"wout |= __builtin_amdgcn_ballot_w64(least < {small}u) != 0;")
                 if park > 0:
                     use.append(f"for (int c = 0; c < 3; ++c) w{q.index}[{st}][c] = oeq_park(w{q.index}[{st}][c]);")
                 park -= 12
@@ -428,11 +440,12 @@ class SplitEmitter:
 
     @staticmethod
     def split_pair(name: str, v, to):
-        """Two values to three places, in steps."""
-        q = [f"q{name}_{c}" for c in range(3)]
-        return [(0, f"float s{name}_0 = {v[0]}, s{name}_1 = {v[1]}; unsigned {', '.join(q)};")] + \
+        """Two values, times SCALE, to three places, in steps."""
+        q, large = [f"q{name}_{c}" for c in range(3)], float_literal(SCALE, "float")
+        return [(2, f"float s{name}_0 = {large} * {v[0]}, s{name}_1 = {large} * {v[1]}; unsigned {', '.join(q)};"),
+                (1, f"top = oeq_top(top, s{name}_0, s{name}_1);")] + \
             [(3, f"oeq_split_part(s{name}_0, s{name}_1, {q[c]});") for c in range(2)] + \
-            [(4, f"oeq_split_last(s{name}_0, s{name}_1, {q[2]}, lost);")] + [(1, f"{to[c]} = {q[c]};") for c in range(3)]
+            [(1, f"oeq_split_last(s{name}_0, s{name}_1, {q[2]});")] + [(1, f"{to[c]} = {q[c]};") for c in range(3)]
 
     @staticmethod
     def split_tasks(v: str, q: str):
@@ -580,8 +593,10 @@ class SplitEmitter:
         # the results' size, without / with: Z -5.7e-9 / 0.04e-9, dX -3.8e-9 / -0.02e-9 (errors of elements 6e-8).
         s("const float sign = (blockIdx.x & 1) ? -1.0f : 1.0f;")
         # Tiles with operands that three parts do not hold: a bit each, by the tile's number among the block's modulo 32.
-        # lost: what the thread's splits of the next tile left over; next: that tile's bit.
-        s("unsigned lost = 0, wlost = 0, redo = 0, next = 2;")
+        # top: the largest operand of the next tile that the thread has split; next: that tile's bit.
+        s("unsigned redo = 0, next = 2, least;")
+        s("float top = 0.0f;")
+        s("bool wout = false;  // a weight is not held")
         units = [(a, st) for a in used_a for st in range(c32(A[a].mul))]
         where("(i64)blockIdx.x", "const i64 ")
         s(f"const float* rows = {src} + first * {LA};")
@@ -595,12 +610,13 @@ class SplitEmitter:
             for t in used_t:
                 self.put(s, request_x(t))
         self.weights(s, kind, subs, park)   # (the first tile's rows are on their way meanwhile)
+        s("const unsigned wrows = wout || oeq_too_large(top) ? 0xffffu : 0u;")
+        s("top = 0.0f;")
         for a, st in units:
             self.put(s, write(a, st, "s_a[0]"))
         write_y("0")
-        s("const unsigned wrows = oeq_any_lost(wlost) ? 0xffffu : 0u;")
-        s("redo = wrows ? ~0u : oeq_any_lost(lost) ? 1u : 0u;")
-        s("lost = 0;")
+        s("redo = wrows ? ~0u : oeq_too_large(top) ? 1u : 0u;")
+        s("top = 0.0f;")
         s.open("")
         where("((i64)blockIdx.x + gridDim.x)", "const i64 ")
         s(f"const float* rows = {src} + first * {LA};")
@@ -741,7 +757,7 @@ class SplitEmitter:
             # a share of the next tile's operands, and of the requests for the one after
             for ua, ust in (units[m] for m in range(len(units)) if writer(m) == n):
                 tasks += write(ua, ust, "s_a[cur ^ 1]")
-                tasks.append((1, "redo |= oeq_any_lost(lost) ? next : 0u; lost = 0;"))
+                tasks.append((1, "redo |= oeq_too_large(top) ? next : 0u; top = 0.0f;"))
                 tasks += request(ua, ust)
             tasks += contract((n or N) - 1)
             if n == min(1, N - 2):
@@ -812,9 +828,8 @@ class SplitEmitter:
 
     def emit_redo(self, s: Src, kind: str, subs, number: int, folds, where):
         """Rows with an operand that three bf16 parts do not hold, all rows of the block if a weight is one: once more with fp32
-        matrix instructions, after the last tile, on operands straight from memory. It costs nothing where there are none: beside
-        the splits' remainders the loop has one ballot a tile. dY of such a row is formed anew from the sub-paths of the
-        kernels before this one too, whose sums the first pass has written over."""
+        matrix instructions, after the last tile, on operands straight from memory. dY of such a row is formed anew from the
+        sub-paths of the kernels before this one too, whose sums the first pass has written over."""
         low = self.low
         A, T, ia, it = self.sides(kind)
         L2, fwd = low.L2, kind == "forward"
@@ -840,12 +855,11 @@ class SplitEmitter:
         where("tile", "const i64 ")
         s(f"const float* rows = {src} + first * {LA};")
         # which rows: the splits again (tiles 32 turns apart share a bit)
-        s("unsigned gone = 0;")
+        s("float gone = 0.0f;")
         s.open("")
         s(f"const float* ap = rows + min(tid >> 4, end) * {LA};")
-        s("unsigned q;")
         for a in used_a:
-            s(f"for (int z = tid & 15; z < {A[a].mul * A[a].d}; z += 16) oeq_split3(ap[{A[a].off} + z], 0.0f, q, q, q, gone);")
+            s(f"for (int z = tid & 15; z < {A[a].mul * A[a].d}; z += 16) gone = oeq_top(gone, {self.lit(SCALE)} * ap[{A[a].off} + z], 0.0f);")
         for q in folds:
             b, b2 = A[ia(q)], low.in2[q.p.i2]
             s(f"const float* yp{q.index} = L2_in + (first + min(tid >> 4, end)) * {L2} + {self.yat(q, 0)};")
@@ -853,10 +867,10 @@ class SplitEmitter:
             s.open(f"for (int z = tid & 15; z < {b.mul}; z += 16)")
             for line in self.fold_terms(q, "v", lambda i: f"ap[{b.off} + {b.d} * z + {i}]"):
                 s(line)
-            s("oeq_split3(v, 0.0f, q, q, q, gone);")
+            s(f"gone = oeq_top(gone, {self.lit(SCALE)} * v, 0.0f);")
             s.close()
         s.close()
-        s("const unsigned long long rows_gone = __builtin_amdgcn_ballot_w64((gone << 1) != 0);")
+        s("const unsigned long long rows_gone = __builtin_amdgcn_ballot_w64(gone >= 3.39e38f);")
         s("unsigned four = 0;")
         s("for (int r = 0; r < 4; ++r) four |= (rows_gone >> (16 * r) & 0xffff) ? 1u << r : 0u;")
         s("oeq_block_sync();  // (the words of the tile before are read)")

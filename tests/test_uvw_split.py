@@ -153,10 +153,10 @@ def test_boundaries_match_oracle(name, make, wf, wb):
 
 # (problem, kernels on split operands of the forward and the backward pass, waves per SIMD of each)
 SPILLS = [
-    # as estimated, forward 664 bytes a lane at one wave per SIMD; 124 at two, a tile that is mostly padding
+    # as estimated, forward 712 bytes a lane at one wave per SIMD; 120 at two, a tile that is mostly padding
     (("8x0e+20x1o+48x2e", "1x0e+1x1o+1x2e+2x3o", "64x0o+40x0o+64x2o+32x3o"), 0, 1),
     (("40x0o+16x2o", "1x0e+1x1o+1x2e+1x3o", "64x0e+40x1o+8x1e"), 0, 0),
-    # at two waves forward 360 and backward 116 bytes, none at one
+    # at two waves forward 472 and backward 100 bytes, none at one
     (("40x0e+40x2o", "1x0e+2x1o", "64x0o+48x1o+64x2e"), 1, 1),
     (("48x0e+48x1o", "1x0e+1x1o", "48x0e+48x1o"), 2, 1),
 ]
