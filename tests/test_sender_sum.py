@@ -142,7 +142,13 @@ def test_no_room_for_the_terms(deterministic, monkeypatch):
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
     total = torch.cuda.get_device_properties(0).total_memory
+    fill = []
     try:
+        # (room in what torch holds already is filled first)
+        torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() / total)
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            while True:
+                fill.append(torch.empty(terms // 8, dtype=torch.uint8, device="cuda"))
         torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + sum(t.nbytes for t in want) + terms * 0.6) / total)
         got = backward()
     finally:
