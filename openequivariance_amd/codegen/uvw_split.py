@@ -38,12 +38,12 @@ frequent coefficient of a path is a factor of its weights (``Sub.unit``).
 
 What bounds them (MI355X, the problem above, 100 003 rows): the registers of a SIMD hold one wave of these kernels, and
 a wave issues an instruction in 2.1 ns, one that needs the result before it in 3.6, a matrix instruction takes 8. Counters of
-the forward: of 100 wave cycles 48 issue, 33 wait to issue, 19 wait for memory or LDS; matrix cores busy 54. Run back to back the
+the forward: of 100 wave cycles 54 issue, 31 wait to issue, 15 wait for memory or LDS; matrix cores busy 42. Run back to back the
 kernels are also bound by power: random operands lower the clock (2.1 GHz, 2.4 on zeros), fewer matrix instructions raise it.
 So the order of the instructions is written out (``interleave``): vector, LDS and memory instructions go between the matrix
 instructions that hide them, and what takes several is cut in steps (a split of eight values as one piece: 714 us for a pass through
 forward and backward, in steps 695); left to the compiler they clump, and registers spill. The pass: fp32 kernels
-1 062 us, these 719 with 35 products each and without the steps, 630 now.
+1 062 us, these 719 with 35 products each and without the steps, 633 with both, 647 with what keeps operands in range.
 """
 
 from __future__ import annotations
@@ -1186,7 +1186,7 @@ class SplitEmitter:
 
         def t_tasks(n):
             """The contraction of X and Y for stage n, eight rows a lane, as operands. Y comes from LDS, component by
-            component, two ahead of the sums."""
+            component, AHEAD of the sums."""
             o, k, q = stages[n % N]
             if q in folds:
                 return [(4, " ".join(f"t[{4 * h + r}] = {self.lit(SCALE)} * x{q.p.i1}[{4 * h + r}][0];" for r in range(4))) for h in (0, 1)] + \
